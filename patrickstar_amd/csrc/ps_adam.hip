@@ -208,6 +208,8 @@ int for_each_batch(const ChunkList& a, F launch)
     return 0;
 }
 
+constexpr FirstCall kNoFirstCall{-1, 0, 0, 0, 0, 0, 0};
+
 // Validated copy of a ps_call_pattern: how many operator calls the reference makes in the step and
 // which elements its first call covers, as a chunk index over the call's whole list.
 struct Calls {
@@ -218,11 +220,15 @@ struct Calls {
     // The span as the launch of chunks [batch_first, batch_first + n) sees it.
     FirstCall in_batch(int64_t batch_first, int n) const
     {
-        FirstCall fc{-1, 0, 0};
+        FirstCall fc = kNoFirstCall;
         if (first_chunk >= batch_first && first_chunk < batch_first + n) {
             fc.chunk = (int)(first_chunk - batch_first);
             fc.lo = lo;
             fc.hi = hi;
+            fc.lo_tile = (uint32_t)(lo / kTile);
+            fc.hi_tile = (uint32_t)((hi + kTile - 1) / kTile);
+            fc.in_lo = (uint32_t)((lo + kTile - 1) / kTile);
+            fc.in_hi = (uint32_t)(hi / kTile);
         }
         return fc;
     }
@@ -276,7 +282,7 @@ void launch_adam_batch(int arith, const ChunkBatch& b, dim3 grid, const StepCons
                        hipStream_t s)
 {
     if (arith == PS_ARITH_TORCH)
-        launch_adam_batch_arith<PS_ARITH_TORCH>(b, grid, c, FirstCall{-1, 0, 0}, s);
+        launch_adam_batch_arith<PS_ARITH_TORCH>(b, grid, c, kNoFirstCall, s);
     else
         launch_adam_batch_arith<PS_ARITH_OPERATOR>(b, grid, c, fc, s);
 }
@@ -302,7 +308,7 @@ void launch_gated_batch(int arith, const ChunkBatch& b, dim3 grid, size_t chunk_
                         hipStream_t s)
 {
     if (arith == PS_ARITH_TORCH)
-        launch_gated_batch_arith<PS_ARITH_TORCH>(b, grid, chunk_numel, ga, FirstCall{-1, 0, 0}, d_state, s);
+        launch_gated_batch_arith<PS_ARITH_TORCH>(b, grid, chunk_numel, ga, kNoFirstCall, d_state, s);
     else
         launch_gated_batch_arith<PS_ARITH_OPERATOR>(b, grid, chunk_numel, ga, fc, d_state, s);
 }

@@ -217,9 +217,11 @@ __device__ __forceinline__ void element_any(const StepConsts& c, float step_size
 }
 
 // Which elements of a launch belong to the step's first operator call: elements [lo, hi) of chunk
-// `chunk` of the launch's batch (-1: none of them).
+// `chunk` of the launch's batch (-1: none of them).  In tiles: [in_lo, in_hi) lie wholly inside the span,
+// [lo_tile, hi_tile) are the ones it touches.
 struct FirstCall {
     int chunk;
+    uint32_t lo_tile, hi_tile, in_lo, in_hi;
     uint64_t lo, hi;
 };
 
