@@ -3,10 +3,10 @@
 The reference's hybrid Adam keeps some chunks' optimizer state in host memory and
 updates them with the CPU operator (``patrickstar/ops/fp16_cpu_adam.py:415-428``,
 ``patrickstar/ops/chunk_io_buff.py:214-255``).  On MI355X those chunks are instead
-copied into double-buffered HBM staging by ``hipMemcpyAsync`` on side streams,
-updated by the same fused kernel as resident chunks, and copied back, all ordered
-by events inside ``ps_adam_step_hybrid``; the Python side only owns the
-staging buffers.  A position's fp16 payload may stay in HBM (where forward and
+updated by the same fused kernel as resident chunks: up to 8 of them where they
+are, over the link, more of them copied into HBM staging by ``hipMemcpyAsync`` on
+side streams and copied back, all ordered by events inside
+``ps_adam_step_hybrid``; the Python side only owns the staging buffers.  A position's fp16 payload may stay in HBM (where forward and
 backward use it, as in the reference); it is then updated in place and only the
 optimizer state (12 B/element each way) crosses the link.
 """
