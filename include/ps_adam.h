@@ -455,6 +455,16 @@ int ps_overflow_scan_chunks_noalloc(const ps_chunk* chunks, int n_chunks, size_t
 int ps_grad_to_chunk(const void* d_grad, int grad_is_half, uint16_t* d_slot_fp16, size_t numel,
                      ps_step_state* d_state, ps_stream_t stream);
 
+/* The same for a list of gradients: one kernel launch for up to 64 of them.  `copies` is a host array, read before the
+ * call returns.  Slots must not overlap one another or any gradient of the list. */
+typedef struct ps_grad_copy {
+    const void* d_grad;    /* fp16 (grad_is_half != 0) or fp32, numel elements */
+    uint16_t* d_slot_fp16;
+    uint64_t numel;        /* 0: nothing is copied */
+    int64_t grad_is_half;
+} ps_grad_copy;
+int ps_grads_to_chunks(const ps_grad_copy* copies, int n_copies, ps_step_state* d_state, ps_stream_t stream);
+
 #define PS_FLAG_FALSE 0
 #define PS_FLAG_TRUE 1
 #define PS_FLAG_FROM_DEVICE 2

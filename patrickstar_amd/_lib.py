@@ -90,6 +90,15 @@ class ps_tensor_call(ctypes.Structure):
     ]
 
 
+class ps_grad_copy(ctypes.Structure):
+    _fields_ = [
+        ("d_grad", ctypes.c_void_p),
+        ("d_slot_fp16", ctypes.c_void_p),
+        ("numel", ctypes.c_uint64),
+        ("grad_is_half", ctypes.c_int64),
+    ]
+
+
 class ps_scale_record(ctypes.Structure):
     _fields_ = [
         ("scale_after", ctypes.c_double),
@@ -103,6 +112,7 @@ assert ctypes.sizeof(ps_step_state) == 256
 assert ctypes.sizeof(ps_call_pattern) == 32
 assert ctypes.sizeof(ps_scale_record) == 16
 assert ctypes.sizeof(ps_tensor_call) == 56
+assert ctypes.sizeof(ps_grad_copy) == 32
 
 _f, _d, _i, _i64, _sz, _vp = (
     ctypes.c_float,
@@ -138,6 +148,7 @@ SIGNATURES = {
     "ps_overflow_scan_f32": (_i, [_vp, _sz, _vp, _vp]),
     "ps_overflow_scan_chunks": (_i, [_vp, _i, _sz, _vp, _vp, _vp]),
     "ps_overflow_scan_chunks_noalloc": (_i, [_vp, _i, _sz, _vp, _vp]),
+    "ps_grads_to_chunks": (_i, [_vp, _i, _vp, _vp]),
     "ps_grad_to_chunk": (_i, [_vp, _i, _vp, _sz, _vp, _vp]),
     "ps_scaler_update": (_i, [_vp, _i, _vp, _i64, _i64, _vp]),
     "ps_state_read": (_i, [_vp, ctypes.POINTER(ps_step_state), _vp]),
@@ -184,6 +195,13 @@ def current_stream_handle():
     import torch
 
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def raw_stream(device):
+    """The current stream of a GPU as an integer handle, without the wrapper object."""
+    import torch
+
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def call_pattern(n_calls, first_chunk=0, first_offset=0, first_numel=0):

@@ -368,6 +368,14 @@ class PatrickStarClient:
             )
         return view
 
+    def data_address(self, param):
+        """``access_data(param).data_ptr()`` of a chunk tensor, without making the view."""
+        info = self.chunk_tensor_index.get_tensor_info(param.ps_attr.data_id())
+        payload = self.chunk_list[info.chunk_id].payload
+        if payload is None:
+            return self.access_data(param).data_ptr()
+        return payload.data_ptr() + info.start_offset * payload.element_size()
+
     def release_data(self, param, reset_state=None):
         return None
 

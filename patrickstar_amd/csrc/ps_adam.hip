@@ -144,6 +144,8 @@ std::shared_ptr<HostAdam> find_opt(int id)
 constexpr size_t kMaxGridX = 0xFFFFFFFFull / 64;
 static_assert(kBlock == 64 && kScanBlock == 64, "kMaxGridX is for 64-thread workgroups");
 
+constexpr size_t kMaxCopyBlocks = 0xFFFFFFFFull / kCopyBlock;  // of the gradient copy (2^24 - 1 spans of 2048 elements)
+
 unsigned grid_1d(size_t n_blocks, size_t block_threads)
 {
     const size_t most = 0xFFFFFFFFull / block_threads;
@@ -1657,56 +1659,54 @@ int ps_overflow_scan_chunks_noalloc(const ps_chunk* chunks, int n_chunks, size_t
     return 0;
 }
 
+int ps_grads_to_chunks(const ps_grad_copy* copies, int n_copies, ps_step_state* d_state, ps_stream_t stream)
+{
+    if (n_copies < 0) return fail(PS_ERR_BAD_ARG, "n_copies = %d is negative", n_copies);
+    if (n_copies > 0 && !copies) return fail(PS_ERR_BAD_ARG, "copies is NULL");
+    for (int i = 0; i < n_copies; ++i) {
+        if (copies[i].numel > 0 && (!copies[i].d_grad || !copies[i].d_slot_fp16))
+            return fail(PS_ERR_BAD_ARG, "copy %d has a NULL address", i);
+        if (copies[i].numel > (size_t)kCopySpan * kMaxCopyBlocks)
+            return fail(PS_ERR_BAD_ARG, "copy %d: numel = %zu is beyond the launch grid", i, (size_t)copies[i].numel);
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    int next = 0;
+    while (next < n_copies) {
+        GradBatch b;
+        memset(&b, 0, sizeof(b));
+        memset(b.first_block, 0xFF, sizeof(b.first_block));
+        size_t blocks = 0;
+        int in_batch = 0;
+        for (; next < n_copies && in_batch < kGradBatch; ++next) {
+            const ps_grad_copy& c = copies[next];
+            if (c.numel == 0) continue;
+            const size_t more = (c.numel + kCopySpan - 1) / kCopySpan;
+            if (blocks + more > kMaxCopyBlocks) break;  // the next launch starts with this gradient
+            b.src[in_batch] = c.d_grad;
+            b.dst[in_batch] = c.d_slot_fp16;
+            b.numel_half[in_batch] = 2 * (uint64_t)c.numel + (c.grad_is_half ? 1 : 0);
+            b.first_block[in_batch] = (uint32_t)blocks;
+            blocks += more;
+            in_batch += 1;
+        }
+        if (in_batch == 0) continue;
+        const dim3 grid((unsigned)blocks), block(kCopyBlock);
+        if (in_batch == 1)
+            hipLaunchKernelGGL(grads_to_chunks_kernel<true>, grid, block, 0, s, b, d_state);
+        else
+            hipLaunchKernelGGL(grads_to_chunks_kernel<false>, grid, block, 0, s, b, d_state);
+        PS_HIP(hipGetLastError());
+    }
+    return 0;
+}
+
 int ps_grad_to_chunk(const void* d_grad, int grad_is_half, uint16_t* d_slot_fp16, size_t numel,
                      ps_step_state* d_state, ps_stream_t stream)
 {
     if (numel == 0) return 0;
     if (!d_grad || !d_slot_fp16) return fail(PS_ERR_BAD_ARG, "ps_grad_to_chunk: NULL pointer");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t esz = grad_is_half ? 2 : 4;
-    const char* gbytes = static_cast<const char*>(d_grad);
-
-    auto scalar_span = [&](size_t lo, size_t hi) {
-        if (hi <= lo) return;
-        const size_t n = hi - lo;
-        size_t blocks = (n + (size_t)kAuxBlock * 4 - 1) / ((size_t)kAuxBlock * 4);
-        dim3 grid(grid_1d(blocks, kAuxBlock)), block(kAuxBlock);
-        const void* src = gbytes + lo * esz;
-        if (grad_is_half)
-            hipLaunchKernelGGL(grad_to_chunk_kernel<true>, grid, block, 0, s, src, d_slot_fp16 + lo, n, d_state);
-        else
-            hipLaunchKernelGGL(grad_to_chunk_kernel<false>, grid, block, 0, s, src, d_slot_fp16 + lo, n, d_state);
-    };
-
-    const uintptr_t dst = reinterpret_cast<uintptr_t>(d_slot_fp16);
-    const uintptr_t src = reinterpret_cast<uintptr_t>(d_grad);
-    const bool addressable = (dst % 2 == 0) && (src % esz == 0);
-    if (!addressable || numel < 4096) {
-        scalar_span(0, numel);
-    } else {
-        // elements before the slot's first 16-byte boundary, whole 8-element vectors, remainder: one launch, whose
-        // last workgroup does the at most 14 elements in front of and behind the vectors
-        const size_t head = (size_t)(((16 - dst % 16) % 16) / 2);
-        const size_t n_vec = (numel - head) / 8;
-        const size_t body_end = head + n_vec * 8;
-        const CopyEdges edges{d_grad, d_slot_fp16, head, body_end, numel};
-        size_t blocks = (n_vec + kCopyBlock - 1) / kCopyBlock;
-        unsigned body_blocks = grid_1d(blocks, kCopyBlock);
-        if (((size_t)body_blocks + 1) * kCopyBlock > 0xFFFFFFFFull) body_blocks -= 1;  // room for the edge workgroup
-        dim3 grid(body_blocks + 1), block(kCopyBlock);
-        uint16_t* dst_al = d_slot_fp16 + head;
-        if (grad_is_half) {
-            const uintptr_t first = src + head * 2;
-            const int shift = (int)((first % 16) / 2);
-            const uint16_t* src_al = reinterpret_cast<const uint16_t*>(first - (uintptr_t)shift * 2);
-            hipLaunchKernelGGL(grad_to_chunk_f16_vec_kernel, grid, block, kCopyLdsBytes, s, src_al, shift, dst_al, n_vec, edges, d_state);
-        } else {
-            hipLaunchKernelGGL(grad_to_chunk_f32_vec_kernel, grid, block, kCopyLdsBytes, s,
-                               static_cast<const float*>(d_grad) + head, dst_al, n_vec, edges, d_state);
-        }
-    }
-    PS_HIP(hipGetLastError());
-    return 0;
+    const ps_grad_copy c{d_grad, d_slot_fp16, numel, grad_is_half != 0};
+    return ps_grads_to_chunks(&c, 1, d_state, stream);
 }
 
 int ps_scaler_update(ps_step_state* d_state, int flag_mode, ps_scale_record* d_log,

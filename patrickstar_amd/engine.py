@@ -5,9 +5,9 @@ Only the configuration surface and the optimizer / loss-scaler wiring of
 are kept; the reference's hook-driven chunk movement, memory tracer and
 collectives are not part of this path.  With 288 GB of HBM every chunk stays
 resident: module parameters are fp16 views into the fp16 chunk payloads, so
-forward and backward are ordinary PyTorch; during ``backward`` each gradient is
-written over its parameter's chunk slot as soon as it is complete, probed for
-inf/nan in the same pass (one fused kernel per parameter, no host sync), which
+forward and backward are ordinary PyTorch; during ``backward`` the gradients are
+written over their parameters' chunk slots as they are completed, a few at a time,
+and probed for inf/nan in the same pass (one fused kernel, no host sync), which
 is the state ``optimizer.step()`` expects.
 """
 import torch
@@ -93,7 +93,11 @@ class PatrickStarEngine(torch.nn.Module):
         )
         self.client.init(self.module, self.optimizer)
         self.iteration_cnt_ = 0
-        self._copied = set()  # parameters whose gradient already sits in its chunk slot (this backward)
+        self._copied = set()  # parameters whose gradient sits in its chunk slot already, or waits to be copied there (this backward)
+        self._pending = {}  # parameter -> gradient that waits to be copied (see _gradient_to_chunk)
+        self._pending_elements = 0
+        self._pending_stream = None
+        self._pending_task = None  # the backward pass at whose end _end_of_backward will run
         for p in self.client.chunk_based_param_fp16:
             if p.requires_grad:
                 p.register_post_accumulate_grad_hook(self._on_gradient_ready)
@@ -102,29 +106,69 @@ class PatrickStarEngine(torch.nn.Module):
         return self.module(*inputs, **kwargs)
 
     # -- backward-side producer ---------------------------------------------------------
+    # Gradients that wait for one copy kernel: at most this many (what one launch takes), and at most this many elements
+    # besides the last one's.  With a launch of its own every gradient cost 7 us more of host time, and every bias 2.5 us
+    # on the device: BERT-base dimensions, 1024 tokens, 199 gradients: 11.3 - 12.3 ms an iteration, 10.2 - 10.4 now.
+    PENDING_GRADIENTS = 64
+    PENDING_ELEMENTS = 16 * 1024 * 1024
+
     def _gradient_to_chunk(self, p):
-        """Write ``p.grad`` over ``p``'s fp16 chunk slot, probing it for inf/nan in the same pass, and drop it."""
+        """Take ``p.grad`` off ``p`` and put it down to be written over ``p``'s fp16 chunk slot and probed for inf/nan in
+        the same pass, by a kernel it shares with its neighbours.  The list holds on to the gradients until that kernel is queued, on
+        the stream they were put down on, so their memory is not handed out before it has run."""
         g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
         if g.dtype not in (torch.half, torch.float):
             raise TypeError(f"gradient dtype {g.dtype} is not supported")
+        stream = _lib.raw_stream(self.client.device)
+        if self._pending and (p in self._pending or stream != self._pending_stream.cuda_stream):
+            self._flush_gradients()
+        if not self._pending:
+            self._pending_stream = torch.cuda.current_stream(self.client.device)
+            self._pending_elements = 0
+        self._pending[p] = g
+        self._pending_elements += g.numel()
+        p.grad = None
+        if len(self._pending) >= self.PENDING_GRADIENTS or self._pending_elements >= self.PENDING_ELEMENTS:
+            self._flush_gradients()
+
+    def _flush_gradients(self):
+        """Queue the copy of every gradient that waits, on the stream they belong to."""
+        if not self._pending:
+            return
+        pending, self._pending = self._pending, {}
         scaler = self.loss_scaler
         state_ptr = scaler.state_ptr if isinstance(scaler, DynamicLossScaler) else None
-        slot = self.client.access_data(p)
+        rows = [(g.data_ptr(), self.client.data_address(p), g.numel(), g.dtype == torch.half) for p, g in pending.items()]
         with torch.cuda.device(self.client.device):
             _lib.check(
-                _lib.load().ps_grad_to_chunk(
-                    g.data_ptr(), int(g.dtype == torch.half), slot.data_ptr(), g.numel(), state_ptr,
-                    _lib.current_stream_handle(),
+                _lib.load().ps_grads_to_chunks(
+                    (_lib.ps_grad_copy * len(rows))(*rows), len(rows), state_ptr, self._pending_stream.cuda_stream
                 ),
-                "ps_grad_to_chunk",
+                "ps_grads_to_chunks",
             )
-        p.grad = None
+
+    def _end_of_backward(self):
+        """Runs once when the backward pass that put the pending gradients down ends, whoever started it: the caller's
+        stream has been put behind the streams of backward by then, so a copy queued only now needs the same."""
+        stream, waiting = self._pending_stream, bool(self._pending)
+        self._flush_gradients()
+        if waiting:
+            current = torch.cuda.current_stream(self.client.device)
+            if current.cuda_stream != stream.cuda_stream:
+                current.wait_stream(stream)
 
     def _on_gradient_ready(self, p):
         """Post-accumulate-grad hook: runs during backward, as soon as ``p``'s gradient is complete (every use of the
         parameter has been differentiated, so nothing in the rest of backward reads its value any more).  The
         reference does the same copy in its post-backward module hook (``patrickstar/core/hook.py:200-230``); the
         copies overlap the rest of backward and no second full set of gradients stays alive."""
+        task = torch._C._current_graph_task_id()
+        if task != self._pending_task:
+            # another backward pass than the one whose end the list waits for (a nested one, or the next one after a
+            # pass that failed)
+            self._flush_gradients()
+            self._pending_task = task
+            torch.autograd.Variable._execution_engine.queue_callback(self._end_of_backward)
         self._gradient_to_chunk(p)
         self._copied.add(p)
 
@@ -142,11 +186,13 @@ class PatrickStarEngine(torch.nn.Module):
             else:
                 # the slot still holds the fp16 parameter, which step() would read as a gradient
                 self.client.access_data(p).zero_()
+        self._end_of_backward()
         self._copied.clear()
 
     def backward(self, loss):
         self.optimizer.zero_grad()
         self._copied.clear()
+        self._pending.clear()  # left by a pass that failed
         if self.loss_scaler:
             self.loss_scaler.backward(loss)
         else:
