@@ -858,7 +858,8 @@ struct TensorItem {
     size_t body, tiles;
     int cls;  // the class of calls it belongs to (steps whose tensors carry their own numbers; 0 otherwise)
 };
-static_assert(kTile <= 256, "TensorBatch::numel_head keeps the head length (up to kTile - 1 elements) in 8 bits");
+static_assert(kTile <= 256, "TensorBatch::lengths keeps the head length (up to kTile - 1 elements) in 8 bits");
+static_assert(kMaxGridX * kTile <= kNumelMask, "TensorBatch::lengths keeps a length in 40 bits");
 
 int check_tensor_list(const ps_chunk* tensors, const size_t* numels, int n_tensors)
 {
@@ -868,7 +869,7 @@ int check_tensor_list(const ps_chunk* tensors, const size_t* numels, int n_tenso
         const ps_chunk& t = tensors[i];
         if (numels[i] > 0 && (!t.param_fp32 || !t.exp_avg || !t.exp_avg_sq || !t.param_fp16))
             return fail(PS_ERR_BAD_ARG, "tensor %d has a NULL address", i);
-        if ((numels[i] + kTile - 1) / kTile >= kMaxGridX || numels[i] > kNumelMask)
+        if (numels[i] > kNumelMask || (numels[i] + kTile - 1) / kTile >= kMaxGridX)
             return fail(PS_ERR_BAD_ARG, "tensor %d: numel = %zu is beyond the launch grid", i, numels[i]);
     }
     return 0;
@@ -889,10 +890,9 @@ TensorItem tensor_item(const ps_chunk* tensors, const size_t* numels, int i, boo
 // list) of the tensor that is the step's first operator call, marked in its batch; -1: none.
 //
 // `classes`: which class each tensor of the batch belongs to.  max_classes == 0: the items' own class numbers.
-// max_classes > 0: a launch takes at most that many distinct classes; classes.k[] then numbers them 0, 1, ... in the
+// max_classes > 0: a launch takes at most that many distinct classes; its tensors' numbers are then 0, 1, ... in the
 // order of their first tensor in the batch and classes.of[] says which of the items' classes each one is.
 struct BatchClasses {
-    ClassIndex k;
     int of[kTensorBatch];
     int n;
 };
@@ -915,6 +915,7 @@ int for_each_tensor_batch(std::vector<TensorItem>& items, const ps_chunk* tensor
         while (next < items.size() && in_batch < kTensorBatch &&
                (items[next].tiles * 10 >= widest * 9 || widest <= kShortTensorTiles)) {
             const TensorItem& it = items[next];
+            int cls = it.cls;
             if (max_classes > 0) {
                 int j = 0;
                 while (j < bc.n && bc.of[j] != it.cls) ++j;
@@ -922,9 +923,7 @@ int for_each_tensor_batch(std::vector<TensorItem>& items, const ps_chunk* tensor
                     if (bc.n == max_classes) break;  // the next launch starts with this tensor
                     bc.of[bc.n++] = it.cls;
                 }
-                bc.k.k[in_batch] = (uint16_t)j;
-            } else {
-                bc.k.k[in_batch] = (uint16_t)it.cls;
+                cls = j;
             }
             ps_chunk t = tensors[it.index];
             t.param_fp32 += it.head;
@@ -932,7 +931,7 @@ int for_each_tensor_batch(std::vector<TensorItem>& items, const ps_chunk* tensor
             t.exp_avg_sq += it.head;
             t.param_fp16 += it.head;
             b.t[in_batch] = t;
-            b.numel_head[in_batch] = (uint64_t)it.body | ((uint64_t)it.head << 56);
+            b.lengths[in_batch] = (uint64_t)it.body | ((uint64_t)cls << 40) | ((uint64_t)it.head << 56);
             if (it.index == first_tensor) b.first_call = in_batch;
             in_batch += 1;
             next += 1;
@@ -952,26 +951,26 @@ int wd_mode_of(int arith, double wd, bool adamw)
 }
 
 template <int ARITH, int WD>
-void launch_tensors_planned_wd(const TensorBatch& b, dim3 grid, const ClassIndex& ci, bool grad_f32,
+void launch_tensors_planned_wd(const TensorBatch& b, dim3 grid, bool grad_f32,
                                const PlannedConsts* d_consts, const ps_step_state* d_state, hipStream_t s)
 {
     dim3 block(kBlock);
     if (grad_f32)
-        hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, ci, d_consts, d_state);
+        hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
     else
-        hipLaunchKernelGGL((adam_tensors_planned_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, ci, d_consts, d_state);
+        hipLaunchKernelGGL((adam_tensors_planned_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
 }
 
 template <int ARITH>
-void launch_tensors_planned_arith(const TensorBatch& b, dim3 grid, const ClassIndex& ci, int wd_mode, bool grad_f32,
+void launch_tensors_planned_arith(const TensorBatch& b, dim3 grid, int wd_mode, bool grad_f32,
                                   const PlannedConsts* d_consts, const ps_step_state* d_state, hipStream_t s)
 {
     if (wd_mode == WD_DECOUPLED)
-        launch_tensors_planned_wd<ARITH, WD_DECOUPLED>(b, grid, ci, grad_f32, d_consts, d_state, s);
+        launch_tensors_planned_wd<ARITH, WD_DECOUPLED>(b, grid, grad_f32, d_consts, d_state, s);
     else if (wd_mode == WD_L2)
-        launch_tensors_planned_wd<ARITH, WD_L2>(b, grid, ci, grad_f32, d_consts, d_state, s);
+        launch_tensors_planned_wd<ARITH, WD_L2>(b, grid, grad_f32, d_consts, d_state, s);
     else
-        launch_tensors_planned_wd<ARITH, WD_NONE>(b, grid, ci, grad_f32, d_consts, d_state, s);
+        launch_tensors_planned_wd<ARITH, WD_NONE>(b, grid, grad_f32, d_consts, d_state, s);
 }
 
 // Numbers the distinct records (classes of calls) of a step by their bytes; records are zero-filled before they are
@@ -1016,38 +1015,38 @@ bool key_grad_f32(int key) { return (key & 2) != 0; }
 static_assert(PS_ARITH_OPERATOR == 0 && PS_ARITH_TORCH == 1, "class_key keeps the arithmetic in one bit");
 
 template <int ARITH, int WD, int UNS>
-void launch_tensors_each_uns(const TensorBatch& b, dim3 grid, const ClassIndex& ci, const ConstsBatch& cb, bool grad_f32,
+void launch_tensors_each_uns(const TensorBatch& b, dim3 grid, const ConstsBatch& cb, bool grad_f32,
                              hipStream_t s)
 {
     dim3 block(kBlock);
     if (grad_f32)
-        hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, ci, cb);
+        hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
     else
-        hipLaunchKernelGGL((adam_tensors_each_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, ci, cb);
+        hipLaunchKernelGGL((adam_tensors_each_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
 }
 
 template <int ARITH, int WD>
-void launch_tensors_each_wd(const TensorBatch& b, dim3 grid, const ClassIndex& ci, const ConstsBatch& cb,
+void launch_tensors_each_wd(const TensorBatch& b, dim3 grid, const ConstsBatch& cb,
                             const Flavour& f, hipStream_t s)
 {
     if (f.unscale == UNSCALE_MUL)
-        launch_tensors_each_uns<ARITH, WD, UNSCALE_MUL>(b, grid, ci, cb, f.grad_f32, s);
+        launch_tensors_each_uns<ARITH, WD, UNSCALE_MUL>(b, grid, cb, f.grad_f32, s);
     else if (ARITH == PS_ARITH_OPERATOR && f.unscale == UNSCALE_DIV)  // the torch formula never divides
-        launch_tensors_each_uns<ARITH, WD, UNSCALE_DIV>(b, grid, ci, cb, f.grad_f32, s);
+        launch_tensors_each_uns<ARITH, WD, UNSCALE_DIV>(b, grid, cb, f.grad_f32, s);
     else
-        launch_tensors_each_uns<ARITH, WD, UNSCALE_NONE>(b, grid, ci, cb, f.grad_f32, s);
+        launch_tensors_each_uns<ARITH, WD, UNSCALE_NONE>(b, grid, cb, f.grad_f32, s);
 }
 
 template <int ARITH>
-void launch_tensors_each_arith(const TensorBatch& b, dim3 grid, const ClassIndex& ci, const ConstsBatch& cb,
+void launch_tensors_each_arith(const TensorBatch& b, dim3 grid, const ConstsBatch& cb,
                                const Flavour& f, hipStream_t s)
 {
     if (f.wd_mode == WD_DECOUPLED)
-        launch_tensors_each_wd<ARITH, WD_DECOUPLED>(b, grid, ci, cb, f, s);
+        launch_tensors_each_wd<ARITH, WD_DECOUPLED>(b, grid, cb, f, s);
     else if (f.wd_mode == WD_L2)
-        launch_tensors_each_wd<ARITH, WD_L2>(b, grid, ci, cb, f, s);
+        launch_tensors_each_wd<ARITH, WD_L2>(b, grid, cb, f, s);
     else
-        launch_tensors_each_wd<ARITH, WD_NONE>(b, grid, ci, cb, f, s);
+        launch_tensors_each_wd<ARITH, WD_NONE>(b, grid, cb, f, s);
 }
 
 }  // namespace
@@ -1192,9 +1191,9 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     memset(&cb, 0, sizeof(cb));
                     for (int q = 0; q < bc.n; ++q) cb.c[q] = consts[bc.of[q]];
                     if (f.arith == PS_ARITH_TORCH)
-                        launch_tensors_each_arith<PS_ARITH_TORCH>(b, grid, bc.k, cb, f, s);
+                        launch_tensors_each_arith<PS_ARITH_TORCH>(b, grid, cb, f, s);
                     else
-                        launch_tensors_each_arith<PS_ARITH_OPERATOR>(b, grid, bc.k, cb, f, s);
+                        launch_tensors_each_arith<PS_ARITH_OPERATOR>(b, grid, cb, f, s);
                 });
                 if (rc) return rc;
             }
@@ -1282,11 +1281,11 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     }
                     if (items.empty()) continue;
                     int rc = for_each_tensor_batch(items, tensors, -1, 0,
-                                                   [&](const TensorBatch& b, dim3 grid, const BatchClasses& bc) {
+                                                   [&](const TensorBatch& b, dim3 grid, const BatchClasses&) {
                         if (key_arith(key) == PS_ARITH_TORCH)
-                            launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, bc.k, wd_mode, grad_f32, table + window, d_state, s);
+                            launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, wd_mode, grad_f32, table + window, d_state, s);
                         else
-                            launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, bc.k, wd_mode, grad_f32, table + window, d_state, s);
+                            launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, wd_mode, grad_f32, table + window, d_state, s);
                     });
                     if (rc) return rc;
                 }
