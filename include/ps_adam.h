@@ -482,6 +482,15 @@ int ps_grads_to_chunks(const ps_grad_copy* copies, int n_copies, ps_step_state* 
 int ps_scaler_update(ps_step_state* d_state, int flag_mode, ps_scale_record* d_log,
                      int64_t log_capacity, int64_t operator_calls, ps_stream_t stream);
 
+/* A whole device-decided step over HBM-resident chunks in one call: ps_overflow_scan_chunks (if probe
+ * != 0), ps_adam_step_chunks_gated, ps_scaler_update(..., PS_FLAG_FROM_DEVICE, ...), with the same
+ * results.  A list of at most 80 tiles of 256 elements (every chunk counted as long as the
+ * longest) is one kernel launch instead of three.  All arguments are checked before anything is queued. */
+int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
+                                const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
+                                const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
+                                int64_t log_capacity, int64_t operator_calls, ps_stream_t stream);
+
 /* Copy *d_state to host memory and wait for it: the only synchronising call. */
 int ps_state_read(const ps_step_state* d_state, ps_step_state* host_out, ps_stream_t stream);
 

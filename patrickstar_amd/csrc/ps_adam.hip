@@ -315,6 +315,29 @@ void launch_gated_batch(int arith, const ChunkBatch& b, dim3 grid, size_t chunk_
         launch_gated_batch_arith<PS_ARITH_OPERATOR>(b, grid, chunk_numel, ga, fc, d_state, s);
 }
 
+template <int ARITH>
+void launch_small_step_arith(const ChunkBatch& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
+                             ps_step_state* d_state, hipStream_t s)
+{
+    dim3 grid(1), block(kBlock, kSmallWaves);
+    const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
+    if (decay && ga.adamw)
+        hipLaunchKernelGGL((adam_small_step_kernel<ARITH, WD_DECOUPLED>), grid, block, 0, s, b, a, ga, fc, d_state);
+    else if (decay)
+        hipLaunchKernelGGL((adam_small_step_kernel<ARITH, WD_L2>), grid, block, 0, s, b, a, ga, fc, d_state);
+    else
+        hipLaunchKernelGGL((adam_small_step_kernel<ARITH, WD_NONE>), grid, block, 0, s, b, a, ga, fc, d_state);
+}
+
+void launch_small_step(int arith, const ChunkBatch& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
+                       ps_step_state* d_state, hipStream_t s)
+{
+    if (arith == PS_ARITH_TORCH)
+        launch_small_step_arith<PS_ARITH_TORCH>(b, a, ga, kNoFirstCall, d_state, s);
+    else
+        launch_small_step_arith<PS_ARITH_OPERATOR>(b, a, ga, fc, d_state, s);
+}
+
 template <int ARITH, int WD>
 void launch_tensors_wd(const TensorBatch& b, dim3 grid, const StepConsts& c, hipStream_t s)
 {
@@ -1721,6 +1744,39 @@ int ps_scaler_update(ps_step_state* d_state, int flag_mode, ps_scale_record* d_l
                        operator_calls);
     PS_HIP(hipGetLastError());
     return 0;
+}
+
+int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
+                                const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
+                                const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
+                                int64_t log_capacity, int64_t operator_calls, ps_stream_t stream)
+{
+    auto o = find_opt(optimizer_id);
+    if (!o) return fail(PS_ERR_UNKNOWN_ID, "optimizer id %d was never created", optimizer_id);
+    if (!d_state) return fail(PS_ERR_BAD_ARG, "d_state is NULL");
+    if (d_log != nullptr && log_capacity <= 0)
+        return fail(PS_ERR_BAD_ARG, "log_capacity must be positive when d_log is given");
+    if (operator_calls < 0) return fail(PS_ERR_BAD_ARG, "operator_calls = %lld is negative", (long long)operator_calls);
+    ChunkList a;
+    if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kTile)) return rc;
+    Calls k;
+    if (int rc = make_calls(k, calls, n_chunks, chunk_numel)) return rc;
+    size_t tiles = 0;
+    for (int i = 0; i < n_chunks; ++i) tiles = std::max(tiles, (a.numel_of(i) + kTile - 1) / kTile);
+    if (n_chunks <= kBatch && tiles > 0 && tiles <= kSmallTiles / n_chunks) {
+        const GatedArgs ga = gated_args(*o, lr, epsilon, weight_decay, bias_correction, k.n_calls);
+        const SmallStep step{(uint32_t)tiles, (uint32_t)(tiles * n_chunks), (uint32_t)((((uint64_t)1 << 32) + tiles - 1) / tiles), chunk_numel, probe != 0, d_log, log_capacity, operator_calls};
+        const int arith = o->arith;
+        return for_each_batch(a, [&](const ChunkBatch& b, dim3, int) {
+            launch_small_step(arith, b, step, ga, k.in_batch(0, n_chunks), d_state, static_cast<hipStream_t>(stream));
+        });
+    }
+    if (probe)
+        if (int rc = ps_overflow_scan_chunks(chunks, n_chunks, chunk_numel, used_numel, d_state, stream)) return rc;
+    if (int rc = ps_adam_step_chunks_gated(optimizer_id, lr, epsilon, weight_decay, bias_correction, chunks, n_chunks,
+                                           chunk_numel, used_numel, calls, d_state, stream))
+        return rc;
+    return ps_scaler_update(d_state, PS_FLAG_FROM_DEVICE, d_log, log_capacity, operator_calls, stream);
 }
 
 int ps_state_read(const ps_step_state* d_state, ps_step_state* host_out, ps_stream_t stream)

@@ -35,6 +35,9 @@
 #ifndef PS_COPY_BLOCK
 #define PS_COPY_BLOCK 256  // threads per workgroup of the backward-side gradient copy (64: 43 us instead of 40 for 64 Mi fp16 elements off the slot's phase)
 #endif
+#ifndef PS_SMALL_TILES
+#define PS_SMALL_TILES 80  // longest list (256-element tiles) that one workgroup probes, steps and rescales in one launch
+#endif
 #if PS_MAX_WAVES_PER_EU > 0
 #define PS_OCCUPANCY __attribute__((amdgpu_waves_per_eu(1, PS_MAX_WAVES_PER_EU)))
 #else

@@ -930,16 +930,12 @@ __global__ void state_set_scaler_kernel(ps_step_state* st, double cur_scale, int
     }
 }
 
-// DynamicLossScaler.update_scale (loss_scaler.py:158-182), one lane.  `operator_calls`: how many times the
-// step that was just queued called the native operator in the reference's terms (its tensors; 0 when every
-// chunk took the torch formula): a clean step moves the operator's own step / beta^t state accordingly
-// (Adam_Optimizer::IncrementStep, cpu_adam.h:143-162), a skipped step never reaches the operator.
-__global__ void scaler_update_kernel(ps_step_state* st, int flag_mode, ps_scale_record* log,
-                                     int64_t log_capacity, int64_t operator_calls)
+// What DynamicLossScaler.update_scale (loss_scaler.py:158-182) makes of the state, formed by one whole wave (every lane
+// the same, except that lanes 0 to 3 raise one beta each).  `operator_calls`: how many times the step that was just queued called the native operator in the
+// reference's terms (its tensors; 0 when every chunk took the torch formula): a clean step moves the operator's own step /
+// beta^t state accordingly (Adam_Optimizer::IncrementStep, cpu_adam.h:143-162), a skipped step never reaches the operator.
+__device__ __forceinline__ ps_step_state scaler_updated(ps_step_state s, bool overflow, int64_t operator_calls)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    ps_step_state s = *st;
-    const bool overflow = flag_mode == PS_FLAG_FROM_DEVICE ? (s.overflow != 0) : (flag_mode != 0);
     if (overflow) {
         if (s.delayed_shift == 1 || s.cur_hysteresis == 1) {
             // Python: max(cur_scale / scale_factor, min_scale) -- true division gives a
@@ -984,28 +980,140 @@ __global__ void scaler_update_kernel(ps_step_state* st, int flag_mode, ps_scale_
             s.operator_beta2 = s.beta2;
         }
         // step t + 1: every call after the first evaluates (float)pow((double)beta, t + 1); the first call
-        // multiplies the held value by beta if the object's step is t, else it evaluates pow as well
-        s.beta1_t_rest = (float)pow_int((double)s.beta1, t + 1);
-        s.beta2_t_rest = (float)pow_int((double)s.beta2, t + 1);
+        // multiplies the held value by beta if the object's step is t, else it evaluates pow as well.  And
+        // fp16_cpu_adam.py:412-413 for that step: the powers of the betas that are no floats
+        const int j = threadIdx.x & 3;
+        const double power = pow_int(j == 0 ? (double)s.beta1 : j == 1 ? (double)s.beta2 : j == 2 ? s.beta1_f64 : s.beta2_f64, t + 1);
+        s.beta1_t_rest = (float)__shfl(power, 0, 64);
+        s.beta2_t_rest = (float)__shfl(power, 1, 64);
         const bool follows = s.operator_step == t && s.operator_beta1 == s.beta1 && s.operator_beta2 == s.beta2;
         s.beta1_t_next = follows ? s.beta1_t_cur * s.beta1 : s.beta1_t_rest;
         s.beta2_t_next = follows ? s.beta2_t_cur * s.beta2 : s.beta2_t_rest;
-        // fp16_cpu_adam.py:412-413 for the next step
-        s.bias_correction1_next = 1.0 - pow_int(s.beta1_f64, s.adam_step + 1);
-        s.bias_correction2_next = 1.0 - pow_int(s.beta2_f64, s.adam_step + 1);
-    }
-    if (log != nullptr && log_capacity > 0) {
-        ps_scale_record r;
-        r.scale_after = s.cur_scale;
-        r.overflow = overflow ? 1u : 0u;
-        r.scale_is_int = (uint32_t)s.scale_is_int;
-        log[s.cur_iter % log_capacity] = r;
+        s.bias_correction1_next = 1.0 - __shfl(power, 2, 64);
+        s.bias_correction2_next = 1.0 - __shfl(power, 3, 64);
     }
     s.cur_iter += 1;
     s.last_skipped = overflow ? 1u : 0u;
     s.overflow = 0;
     s.pending_operator_step = 0;
+    return s;
+}
+
+// One lane's work: the state as it now is, and the log's record of the iteration.
+__device__ __forceinline__ void scaler_store(ps_step_state* st, const ps_step_state& s, ps_scale_record* log, int64_t log_capacity)
+{
+    if (log != nullptr && log_capacity > 0) {
+        ps_scale_record r;
+        r.scale_after = s.cur_scale;
+        r.overflow = s.last_skipped;
+        r.scale_is_int = (uint32_t)s.scale_is_int;
+        log[(s.cur_iter - 1) % log_capacity] = r;
+    }
     *st = s;
+}
+
+__global__ void __launch_bounds__(64)
+    scaler_update_kernel(ps_step_state* st, int flag_mode, ps_scale_record* log, int64_t log_capacity, int64_t operator_calls)
+{
+    const ps_step_state before = *st;
+    const bool overflow = flag_mode == PS_FLAG_FROM_DEVICE ? (before.overflow != 0) : (flag_mode != 0);
+    const ps_step_state after = scaler_updated(before, overflow, operator_calls);
+    if (threadIdx.x == 0) scaler_store(st, after, log, log_capacity);
+}
+
+// ------------------------------------------- a whole device-decided step over a short chunk list
+//
+// Probe, update (or restore) and scale update of a list of at most kSmallTiles tiles by ONE workgroup of 16 waves.  As
+// three kernels they take three launches whatever the list's length, and the GPU waits for each.  The probe's flag crosses
+// the waves through LDS; waves 0 to 14 then go over the tiles, the last one meanwhile forms the next state, which
+// replaces the old one when nobody reads that any more.
+// Bound by launching: the host needs 17 us for a step in one launch, 21 us for one in three.  On the device one CU's
+// arithmetic takes 4 us + 0.12 us a tile (12.9 us for 75 tiles), the three kernels 10.6 us and the gaps between them: a
+// step waited for takes 27 / 31 / 33 / 36 us at 30 / 60 / 75 / 90 tiles, in three launches 32 us; among others 17.2 us at
+// all of them against 21.5.  The line lies where both together are about even.
+constexpr int kSmallWaves = 16;
+constexpr unsigned kSmallTiles = PS_SMALL_TILES;
+struct SmallStep {
+    uint32_t tiles, n_tiles;  // of one chunk (as wide as the widest, like the grid of the chunk-list kernels), of the list
+    uint32_t per_tile;        // 2^32 / tiles, rounded up: t * per_tile / 2^32 is t / tiles for every t of so short a list; 0: one tile each
+    size_t chunk_numel;
+    int probe;
+    ps_scale_record* log;
+    int64_t log_capacity, operator_calls;
+};
+
+struct SmallTile {
+    ps_chunk c;
+    size_t base, numel;  // the tile's first element in its chunk; the chunk's elements
+    uint32_t k;
+};
+__device__ __forceinline__ SmallTile small_tile(const ChunkBatch& b, const SmallStep& a, uint32_t t)
+{
+    SmallTile w;
+    w.k = a.per_tile ? __umulhi(t, a.per_tile) : t;  // t / tiles
+    w.c = b.c[w.k];
+    w.base = (size_t)(t - w.k * a.tiles) * kTile;
+    w.numel = b.n[w.k];
+    return w;
+}
+
+template <int ARITH, int WD>
+__global__ void __launch_bounds__(64 * kSmallWaves)
+    adam_small_step_kernel(ChunkBatch b, SmallStep a, GatedArgs ga, FirstCall fc, ps_step_state* st)
+{
+    static_assert(kBlock == 64 && kLaneElems == 4 && kUnroll == 1, "tiles of one wave, four elements per lane");
+    __shared__ uint32_t wave_hit[kSmallWaves];
+    __shared__ ps_step_state next;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.y), lane = threadIdx.x;
+    const StateView sv = view_state(st);
+    uint32_t hit = 0;
+    if (a.probe) {
+        for (uint32_t t = wave; t < a.n_tiles; t += kSmallWaves) {
+            const SmallTile w = small_tile(b, a, t);
+            if (w.base >= w.numel) continue;
+            const PS_GLOBAL uint16_t* h = (const PS_GLOBAL uint16_t*)w.c.param_fp16 + w.base;
+            if (w.base + kTile <= w.numel && ((uintptr_t)w.c.param_fp16 & 7u) == 0) {
+                const uint2v x = ((const guint2v*)h)[lane];
+                hit |= nonfinite_halves(x[0]) | nonfinite_halves(x[1]);
+                continue;
+            }
+            const uint32_t n = w.numel - w.base < kTile ? (uint32_t)(w.numel - w.base) : kTile;
+#pragma unroll
+            for (int e = 0; e < kTile / kBlock; ++e) hit |= nonfinite_halves(h[lane + e * kBlock < n ? lane + e * kBlock : n - 1]);
+        }
+    }
+    // the constants do not wait for the flag; the first call's pair is formed if the list holds any of that call
+    const StepConsts c_rest = gated_consts<ARITH>(ga, sv, false);
+    const StepConsts c = fc.chunk >= 0 ? gated_consts<ARITH>(ga, sv, true) : c_rest;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) hit |= (uint32_t)__shfl_xor((int)hit, off, 64);
+    if (lane == 0) wave_hit[wave] = hit;
+    __syncthreads();
+    uint32_t any = sv.overflow;
+#pragma unroll
+    for (int w = 0; w < kSmallWaves; ++w) any |= wave_hit[w];
+    const bool overflow = __builtin_amdgcn_readfirstlane(any) != 0;
+    if (wave == kSmallWaves - 1) {
+        const ps_step_state after = scaler_updated(*st, overflow, a.operator_calls);
+        if (lane == 0) next = after;
+    } else {
+        for (uint32_t t = wave; t < a.n_tiles; t += kSmallWaves - 1) {
+            const SmallTile w = small_tile(b, a, t);
+            if (overflow) {
+                restore_tile(w.c.param_fp32, w.c.param_fp16, w.base, w.numel);
+                continue;
+            }
+            const bool here = fc.chunk == (int)w.k;
+            size_t numel = w.numel;
+            if (w.base + kTile > numel && numel < a.chunk_numel) {  // as in adam_chunks_gated_kernel
+                if (!zeros_are_a_fixed_point(here ? c : c_rest)) numel = a.chunk_numel;
+                if (w.base >= numel) continue;
+            }
+            adam_tile<ARITH, WD, UNSCALE_RUNTIME>(c, w.c, w.base, numel, here ? (size_t)fc.lo : 0, here ? (size_t)fc.hi : 0);
+        }
+    }
+    __syncthreads();
+    if (wave == kSmallWaves - 1 && lane == 0) scaler_store(st, next, a.log, a.log_capacity);
 }
 
 }  // namespace

@@ -703,6 +703,17 @@ class FP16Adam(torch.optim.Optimizer):
             chunk_numel = self.client.default_chunk_size
             if self._dynamic:
                 scaler = self.loss_scaler
+                if n_dev and not host_positions and self._stages is None and self._tensor_table is None:
+                    # HBM-resident chunks, all of them whole: probe, step and scale update in one call
+                    _lib.check(
+                        self._lib.ps_adam_step_chunks_dynamic(
+                            self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls,
+                            int(self.scan_in_step), scaler.state_ptr, *scaler.log_arguments(), self._operator_calls, stream,
+                        ),
+                        "ps_adam_step_chunks_dynamic",
+                    )
+                    self._steps_dirty = True
+                    return loss
                 if self.scan_in_step:
                     self.check_overflow_chunks()
                 if self._stages is not None:
@@ -719,14 +730,6 @@ class FP16Adam(torch.optim.Optimizer):
                 elif host_positions:
                     self._streamer.step(self.opt_id, 0, lr, beta1, beta2, eps, weight_decay, -1.0, table, n_dev,
                                         self._calls, scaler, self._used_all)
-                elif n_dev:
-                    _lib.check(
-                        self._lib.ps_adam_step_chunks_gated(
-                            self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls,
-                            scaler.state_ptr, stream,
-                        ),
-                        "ps_adam_step_chunks_gated",
-                    )
                 # consume the device flag; a clean step advances state["step"] and takes the operator object
                 # through this step's calls
                 scaler.update_scale(None, operator_calls=self._operator_calls)

@@ -295,18 +295,20 @@ class DynamicLossScaler:
         return probe.overflow_flag
 
     # -- state machine ----------------------------------------------------------------
+    def log_arguments(self):
+        """Address (None: no log) and capacity of the device log, as the entry points take them."""
+        return (self._log.data_ptr() if self._log is not None else None), self._log_capacity
+
     def update_scale(self, overflow, operator_calls=1):
         """``overflow`` is a bool, or None to consume the sticky device flag; asynchronous.
         ``operator_calls``: how many tensors the optimizer step behind this call handed to the native operator in the
         reference's terms; a clean step takes the operator's step / beta^t state through that many calls."""
         self.materialize()
         mode = _lib.PS_FLAG_FROM_DEVICE if overflow is None else (_lib.PS_FLAG_TRUE if overflow else _lib.PS_FLAG_FALSE)
-        log_ptr = self._log.data_ptr() if self._log is not None else None
         with torch.cuda.device(self._state.device):
             _lib.check(
                 _lib.load().ps_scaler_update(
-                    self._state.data_ptr(), mode, log_ptr, self._log_capacity, int(operator_calls),
-                    _lib.current_stream_handle()
+                    self._state.data_ptr(), mode, *self.log_arguments(), int(operator_calls), _lib.current_stream_handle()
                 ),
                 "ps_scaler_update",
             )
