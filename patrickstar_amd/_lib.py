@@ -2,6 +2,7 @@
 
 There is no CPU fallback: if the library has not been built, loading raises.
 """
+import contextlib
 import ctypes
 import os
 
@@ -192,17 +193,29 @@ def check(rc, what):
         raise RuntimeError(f"{what} failed (code {rc}): {msg.decode() if msg else ''}")
 
 
-def current_stream_handle():
-    import torch
-
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
 def raw_stream(device):
     """The current stream of a GPU as an integer handle, without the wrapper object."""
     import torch
 
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
+
+
+def current_stream_handle():
+    import torch
+
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+
+
+_NO_GUARD = contextlib.nullcontext()
+
+
+def on_device(device):
+    """``torch.cuda.device(device)`` where the current device is another one; nothing to enter or leave where it is not."""
+    import torch
+
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _NO_GUARD
+    return torch.cuda.device(device)
 
 
 def call_pattern(n_calls, first_chunk=0, first_offset=0, first_numel=0):

@@ -11,6 +11,8 @@ import torch
 
 from . import _lib
 
+_FLOAT, _HALF = torch.float, torch.half
+
 
 def create_adam(optimizer_id, alpha=1e-3, betta1=0.9, betta2=0.999, eps=1e-8, weight_decay=0.0, adamw_mode=True,
                 should_log=False):
@@ -35,6 +37,29 @@ def adam_update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bia
     CPU tensors here, ``fp16_cpu_adam.py:222-225``); ``grads``: float32 or float16, never written;
     ``loss_scale <= 0``: no unscale.
     """
+    n = params.numel()
+    if not (
+        params.is_cuda and grads.is_cuda and exp_avg.is_cuda and exp_avg_sq.is_cuda
+        and params.dim() == 1 and grads.dim() == 1 and exp_avg.dim() == 1 and exp_avg_sq.dim() == 1
+        and params.is_contiguous() and grads.is_contiguous() and exp_avg.is_contiguous() and exp_avg_sq.is_contiguous()
+        and params.dtype is _FLOAT and exp_avg.dtype is _FLOAT and exp_avg_sq.dtype is _FLOAT
+        and (grads.dtype is _FLOAT or grads.dtype is _HALF)
+        and grads.numel() == n and exp_avg.numel() == n and exp_avg_sq.numel() == n
+    ):
+        _refuse(params, grads, exp_avg, exp_avg_sq)
+    with _lib.on_device(params.device):
+        rc = _lib.load().ps_adam_update(
+            optimizer_id, int(step), lr, beta1, beta2, epsilon, weight_decay, 1 if bias_correction else 0,
+            params.data_ptr(), grads.data_ptr(), 1 if grads.dtype is _HALF else 0, exp_avg.data_ptr(),
+            exp_avg_sq.data_ptr(), n, float(loss_scale), None, _lib.raw_stream(params.device),
+        )
+    if rc:
+        _lib.check(rc, "adam_update")
+    return 0
+
+
+def _refuse(params, grads, exp_avg, exp_avg_sq):
+    """Say which of adam_update's demands its tensors do not meet."""
     for name, t in (("params", params), ("grads", grads), ("exp_avg", exp_avg), ("exp_avg_sq", exp_avg_sq)):
         if not t.is_cuda:
             raise RuntimeError(f"adam_update: {name} must be a GPU tensor (got {t.device})")
@@ -44,16 +69,4 @@ def adam_update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bia
         raise TypeError("adam_update: params, exp_avg and exp_avg_sq must be float32")
     if grads.dtype not in (torch.float, torch.half):
         raise TypeError(f"adam_update: grads must be float32 or float16, got {grads.dtype}")
-    n = params.size(0)
-    if not (grads.size(0) == exp_avg.size(0) == exp_avg_sq.size(0) == n):
-        raise RuntimeError("adam_update: tensors differ in length")
-    with torch.cuda.device(params.device):
-        _lib.check(
-            _lib.load().ps_adam_update(
-                optimizer_id, int(step), lr, beta1, beta2, epsilon, weight_decay, int(bool(bias_correction)),
-                params.data_ptr(), grads.data_ptr(), int(grads.dtype == torch.half), exp_avg.data_ptr(),
-                exp_avg_sq.data_ptr(), n, float(loss_scale), None, _lib.current_stream_handle(),
-            ),
-            "adam_update",
-        )
-    return 0
+    raise RuntimeError("adam_update: tensors differ in length")

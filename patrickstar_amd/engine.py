@@ -139,7 +139,7 @@ class PatrickStarEngine(torch.nn.Module):
         scaler = self.loss_scaler
         state_ptr = scaler.state_ptr if isinstance(scaler, DynamicLossScaler) else None
         rows = [(g.data_ptr(), self.client.data_address(p), g.numel(), g.dtype == torch.half) for p, g in pending.items()]
-        with torch.cuda.device(self.client.device):
+        with _lib.on_device(self.client.device):
             _lib.check(
                 _lib.load().ps_grads_to_chunks(
                     (_lib.ps_grad_copy * len(rows))(*rows), len(rows), state_ptr, self._pending_stream.cuda_stream

@@ -479,7 +479,7 @@ class FP16Adam(torch.optim.Optimizer):
             if pos.fp32 is not None and cl[pos.fp32].payload is not None
         ]
         if rows:
-            with torch.cuda.device(self.client.device):
+            with _lib.on_device(self.client.device):
                 # pinned host payloads of host-resident positions are device-accessible: the kernel reads / writes them in place
                 _lib.check(
                     self._lib.ps_restore_fp16_chunks(
@@ -689,7 +689,7 @@ class FP16Adam(torch.optim.Optimizer):
             if self._dynamic:
                 self.loss_scaler.update_scale(None, operator_calls=0)
             return loss
-        with torch.cuda.device(self.client.device):
+        with _lib.on_device(self.client.device):
             stream = _lib.current_stream_handle()
             if plan["kind"] == "each":
                 if self._dynamic and self.scan_in_step:

@@ -145,7 +145,7 @@ class DynamicLossScaler:
         at ``adam_step`` with the same betas (``cpu_adam.h:143-162``)."""
         if betas is not None:
             self._betas = (float(betas[0]), float(betas[1]))
-        with torch.cuda.device(self._state.device):
+        with _lib.on_device(self._state.device):
             _lib.check(
                 _lib.load().ps_state_seed_step(
                     self._state.data_ptr(), int(adam_step), self._betas[0], self._betas[1], int(bool(fresh_operator)),
@@ -183,7 +183,7 @@ class DynamicLossScaler:
 
     def _read(self, notify=True):
         host = _lib.ps_step_state()
-        with torch.cuda.device(self._state.device):
+        with _lib.on_device(self._state.device):
             _lib.check(
                 _lib.load().ps_state_read(self._state.data_ptr(), ctypes.byref(host), _lib.current_stream_handle()),
                 "ps_state_read",
@@ -305,7 +305,7 @@ class DynamicLossScaler:
         reference's terms; a clean step takes the operator's step / beta^t state through that many calls."""
         self.materialize()
         mode = _lib.PS_FLAG_FROM_DEVICE if overflow is None else (_lib.PS_FLAG_TRUE if overflow else _lib.PS_FLAG_FALSE)
-        with torch.cuda.device(self._state.device):
+        with _lib.on_device(self._state.device):
             _lib.check(
                 _lib.load().ps_scaler_update(
                     self._state.data_ptr(), mode, *self.log_arguments(), int(operator_calls), _lib.current_stream_handle()
@@ -351,7 +351,7 @@ class DynamicLossScaler:
             self._read()  # outcomes recorded so far belong to the run that is being replaced: hand them on now
             self._log_start = self._log_seen = int(sd["cur_iter"])
             self._scale_seen = sd["cur_scale"]
-        with torch.cuda.device(self._state.device):
+        with _lib.on_device(self._state.device):
             _lib.check(
                 _lib.load().ps_state_set_scaler(
                     self._state.data_ptr(), float(sd["cur_scale"]), int(_is_int(sd["cur_scale"])), int(sd["cur_iter"]),
