@@ -23,8 +23,8 @@ static_assert(sizeof(ps_chunk) == 32 && sizeof(ps_step_state) == 256 && sizeof(p
 // What a workgroup needs before its first data load, fetched from the kernel arguments in one go.  Left to itself the
 // compiler loads the length, tests it, loads the call span, tests it, and only then loads the addresses: three waits
 // for scalar memory in a row in front of every tile's data loads.  The empty asm asks for all of them at once: 7.19 ->
-// 7.15 ms for 24 x 64 Mi elements, 313 -> 310 us for one chunk.  (The device-decided kernel keeps the plain order: with
-// this one its clean step gained 0.4 % and its skipped step, a single load per tile, lost 1.8 %.)
+// 7.15 ms for 24 x 64 Mi elements, 313 -> 310 us for one chunk.  The device-decided kernel had five such rounds and has
+// three (arguments, step state, constants): 2603 -> 2593 us for a clean step over 8 x 64 Mi elements, probe included.
 struct TileSource {
     float *p32, *m32, *v32;
     uint16_t* h16;
@@ -154,23 +154,31 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_chunks_gated_kernel(ChunkBatch b, size_t chunk_numel, GatedArgs ga, FirstCall fc,
                              const ps_step_state* __restrict__ st)
 {
-    const ps_chunk& ch = b.c[blockIdx.y];
+    const TileSource t = tile_source(b.c[blockIdx.y], b.n[blockIdx.y]);
+    const CallSpan s = call_span(fc);
     const size_t base = (size_t)blockIdx.x * kTile;
-    size_t numel = b.n[blockIdx.y];  // what lies behind it is zeros in all four lists
-    const StateView sv = view_state(st);
-    if (sv.overflow) {
-        restore_tile(ch.param_fp32, ch.param_fp16, base, numel);  // RNE(0) = 0 is already there
+    StateView sv = view_state(st);  // asked for at once, as in tile_source
+    asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
+    if (__builtin_expect(sv.overflow, 0)) {
+        if (restore_leader()) restore_tiles(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
         return;
     }
-    const bool here = fc.chunk == (int)blockIdx.y;
-    const size_t lo = here ? (size_t)fc.lo : 0, hi = here ? (size_t)fc.hi : 0;
+    if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
+        LaneTile r;
+        tile_load(r, t.p32, t.m32, t.v32, t.h16, base);
+        const StepConsts c = gated_consts<ARITH>(ga, sv, s.here);
+        tile_finish<ARITH, WD, UNSCALE_RUNTIME>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r,
+                                                t.p32, t.m32, t.v32, t.h16, base);
+        return;
+    }
+    size_t numel = t.numel;  // what lies behind it is zeros in all four lists
     if (base + kTile > numel && numel < chunk_numel) {
         // a tile that reaches into the padding: leave the zeros alone only if they are a fixed point of this step
-        if (!zeros_are_a_fixed_point(gated_consts<ARITH>(ga, sv, here))) numel = chunk_numel;
-        if (base >= numel) return;
+        if (!zeros_are_a_fixed_point(gated_consts<ARITH>(ga, sv, s.here))) numel = chunk_numel;
     }
-    adam_tile_late_consts<ARITH, WD, UNSCALE_RUNTIME>([&]() { return gated_consts<ARITH>(ga, sv, here); }, ch, base,
-                                                      numel, lo, hi);
+    if (base >= numel) return;
+    adam_tile_late_consts<ARITH, WD, UNSCALE_RUNTIME>([&]() { return gated_consts<ARITH>(ga, sv, s.here); }, as_chunk(t), base,
+                                                      numel, s.here ? fc.lo : 0, s.here ? fc.hi : 0);
 }
 
 // ------------------------------------------------------- tensor-list kernels
@@ -243,15 +251,18 @@ __device__ __forceinline__ void adam_head(const StepConsts& c, const ps_chunk& t
     }
 }
 
-// fp16 <- RNE(fp32) of this workgroup's tile (a skipped step).
-__device__ __forceinline__ void restore_tensor_tile(const ps_chunk& t, const TensorView& w)
+// fp16 <- RNE(fp32) of this workgroup's tiles (a skipped step).
+__device__ __forceinline__ void restore_tensor_tiles(const ps_chunk& t, const TensorView& w)
 {
+    if (!restore_leader()) return;
     if (w.tile >= 0) {
-        restore_tile(t.param_fp32, t.param_fp16, (size_t)w.tile * kTile, w.numel);
+        restore_tiles(t.param_fp32, t.param_fp16, (size_t)w.tile * kTile, w.numel);
         return;
     }
-    for (int j = threadIdx.x; j < w.head; j += kBlock)
-        t.param_fp16[(ptrdiff_t)j - w.head] = (uint16_t)float_to_half_bits(t.param_fp32[(ptrdiff_t)j - w.head]);
+    // workgroup 0 of a tensor with elements in front of its tile grid: those, and the tiles it leads
+    restore_tile(t.param_fp32 - w.head, t.param_fp16 - w.head, 0, (size_t)w.head);
+#pragma unroll 1
+    for (unsigned u = 1; u < kRestoreTiles; ++u) restore_tile(t.param_fp32, t.param_fp16, (size_t)(u * kRestoreStride - 1) * kTile, w.numel);
 }
 
 template <int ARITH, int WD, int UNS>
@@ -279,8 +290,8 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     const size_t base = w.tile < 0 ? 0 : (size_t)w.tile * kTile;
     if (w.tile >= 0 && base >= w.numel) return;
     const StateView sv = view_state(st);
-    if (sv.overflow) {
-        restore_tensor_tile(t, w);
+    if (__builtin_expect(sv.overflow, 0)) {
+        restore_tensor_tiles(t, w);
         return;
     }
     if (w.tile < 0) {
@@ -350,8 +361,8 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     const ps_chunk t = as_chunk(w.t);
     const size_t base = w.tile < 0 ? 0 : (size_t)w.tile * kTile;
     if (w.tile >= 0 && base >= w.numel) return;
-    if (st->overflow) {
-        restore_tensor_tile(t, w);
+    if (__builtin_expect(st->overflow, 0)) {
+        restore_tensor_tiles(t, w);
         return;
     }
     if (w.tile < 0) {

@@ -406,6 +406,41 @@ __device__ __forceinline__ void restore_tile(const float* __restrict__ p32,
     }
 }
 
+// The restore of a skipped step, inside kernels whose grid has a workgroup for every tile and whose cap on resident
+// workgroups suits the update: one load per wave is then too few in flight (3.2 TB/s).  The first kRestoreStride of every
+// kRestoreTiles * kRestoreStride workgroups restore kRestoreTiles tiles each, kRestoreStride apart, all of them loaded
+// before the first is stored; the others leave.  Workgroups go round the 8 XCDs and, inside each, round the 4 shader
+// engines: leaders that recur with a shorter period all land on the same few of the 32 (one in 4: 1136 us, one in 8 of
+// consecutive ones: 1197).  8 x 64 Mi elements, 3.2 GB, under the cap of 9: 950 us with a tile each; 2 / 4 / 8 tiles 32
+// apart 579 / 499 / 513 us, 4 tiles 64 / 256 / 2048 apart 494 / 494 / 633.  (A launch of which every workgroup leaves at
+// once takes 441 us; the stand-alone write-back, uncapped, moves the same bytes in 495.)
+constexpr unsigned kRestoreTiles = 4, kRestoreStride = 32;
+__device__ __forceinline__ bool restore_leader() { return blockIdx.x % (kRestoreTiles * kRestoreStride) < kRestoreStride; }
+
+// base: the first of the workgroup's tiles
+__device__ __forceinline__ void restore_tiles(const float* __restrict__ p32, uint16_t* __restrict__ h16, size_t base, size_t numel)
+{
+    static_assert(kLaneElems == 4 && kUnroll == 1, "one 16-byte load per lane and tile");
+    constexpr size_t step = (size_t)kRestoreStride * kTile;
+    if (base + (kRestoreTiles - 1) * step + kTile <= numel && (((uintptr_t)p32 | (uintptr_t)h16) & 15u) == 0) {
+        const size_t i = base + (size_t)threadIdx.x * kLaneElems;
+        float4v a[kRestoreTiles];
+#pragma unroll
+        for (unsigned u = 0; u < kRestoreTiles; ++u) a[u] = ld_f4(p32 + i + u * step);
+        __builtin_amdgcn_sched_barrier(0);  // the compiler converts each tile before it asks for the next otherwise
+#pragma unroll
+        for (unsigned u = 0; u < kRestoreTiles; ++u) {
+            HalfWords out;
+            out.w[0] = float_to_half_bits(a[u][0]) | (float_to_half_bits(a[u][1]) << 16);
+            out.w[1] = float_to_half_bits(a[u][2]) | (float_to_half_bits(a[u][3]) << 16);
+            st_halves(h16 + i + u * step, out);
+        }
+        return;
+    }
+#pragma unroll 1
+    for (unsigned u = 0; u < kRestoreTiles; ++u) restore_tile(p32, h16, base + u * step, numel);
+}
+
 }  // namespace
 
 #endif  // PS_TILE_H
