@@ -10,6 +10,8 @@ written over their parameters' chunk slots as they are completed, a few at a tim
 and probed for inf/nan in the same pass (one fused kernel, no host sync), which
 is the state ``optimizer.step()`` expects.
 """
+import threading
+
 import torch
 
 from . import _lib
@@ -66,6 +68,34 @@ def parse_config(config):
     return optim_type, optim_params, loss_scaler, gradient_clipping
 
 
+class _Waiting:
+    """Gradients that wait to be copied into their chunk slots by one kernel."""
+
+    __slots__ = ("gradients", "elements", "stream", "handle")
+
+    def __init__(self):
+        self.gradients = {}  # parameter -> gradient
+        self.elements = 0
+        self.stream = self.handle = None  # the stream the gradients belong to
+
+
+class _EndOfPass:
+    """What autograd calls when a backward pass ends.  The pass holds the only reference to it, so it lives as long as the
+    pass: if that fails and never calls it, what still waits is dropped and copied nowhere.  (The caller restores the
+    parameters after a failed pass; a gradient written into a slot later would be read as a weight by the next pass.)"""
+
+    __slots__ = ("engine", "task")
+
+    def __init__(self, engine, task):
+        self.engine, self.task = engine, task
+
+    def __call__(self):
+        self.engine._end_of_backward(self.task)
+
+    def __del__(self):
+        self.engine._pending.pop(self.task, None)
+
+
 class PatrickStarEngine(torch.nn.Module):
     def __init__(self, model, client, config):
         super().__init__()
@@ -94,10 +124,8 @@ class PatrickStarEngine(torch.nn.Module):
         self.client.init(self.module, self.optimizer)
         self.iteration_cnt_ = 0
         self._copied = set()  # parameters whose gradient sits in its chunk slot already, or waits to be copied there (this backward)
-        self._pending = {}  # parameter -> gradient that waits to be copied (see _gradient_to_chunk)
-        self._pending_elements = 0
-        self._pending_stream = None
-        self._pending_task = None  # the backward pass at whose end _end_of_backward will run
+        self._pending = {}  # backward pass that is under way (autograd's number of it) -> the gradients of it that wait to be copied
+        self._pending_lock = threading.RLock()  # hooks run on autograd's threads, the callback at a pass's end on its caller's
         for p in self.client.chunk_based_param_fp16:
             if p.requires_grad:
                 p.register_post_accumulate_grad_hook(self._on_gradient_ready)
@@ -112,50 +140,53 @@ class PatrickStarEngine(torch.nn.Module):
     PENDING_GRADIENTS = 64
     PENDING_ELEMENTS = 16 * 1024 * 1024
 
-    def _gradient_to_chunk(self, p):
-        """Take ``p.grad`` off ``p`` and put it down to be written over ``p``'s fp16 chunk slot and probed for inf/nan in
-        the same pass, by a kernel it shares with its neighbours.  The list holds on to the gradients until that kernel is queued, on
-        the stream they were put down on, so their memory is not handed out before it has run."""
+    def _gradient_to_chunk(self, p, waiting):
+        """Take ``p.grad`` off ``p`` and put it down in ``waiting``, to be written over ``p``'s fp16 chunk slot and probed for
+        inf/nan in the same pass, by a kernel it shares with its neighbours.  The list holds on to the gradients until that kernel is
+        queued, on the stream they were put down on, so their memory is not handed out before it has run."""
         g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
         if g.dtype not in (torch.half, torch.float):
             raise TypeError(f"gradient dtype {g.dtype} is not supported")
-        stream = _lib.raw_stream(self.client.device)
-        if self._pending and (p in self._pending or stream != self._pending_stream.cuda_stream):
-            self._flush_gradients()
-        if not self._pending:
-            self._pending_stream = torch.cuda.current_stream(self.client.device)
-            self._pending_elements = 0
-        self._pending[p] = g
-        self._pending_elements += g.numel()
-        p.grad = None
-        if len(self._pending) >= self.PENDING_GRADIENTS or self._pending_elements >= self.PENDING_ELEMENTS:
-            self._flush_gradients()
+        handle = _lib.raw_stream(self.client.device)
+        with self._pending_lock:
+            for other in tuple(self._pending.values()):
+                if other is not waiting and p in other.gradients:
+                    self._flush_gradients(other)  # a parameter of two passes: the gradient that comes later stays
+            if waiting.gradients and (p in waiting.gradients or handle != waiting.handle):
+                self._flush_gradients(waiting)
+            if not waiting.gradients:
+                waiting.stream, waiting.handle = torch.cuda.current_stream(self.client.device), handle
+            waiting.gradients[p] = g
+            waiting.elements += g.numel()
+            p.grad = None
+            if len(waiting.gradients) >= self.PENDING_GRADIENTS or waiting.elements >= self.PENDING_ELEMENTS:
+                self._flush_gradients(waiting)
 
-    def _flush_gradients(self):
-        """Queue the copy of every gradient that waits, on the stream they belong to."""
-        if not self._pending:
+    def _flush_gradients(self, waiting):
+        """Queue the copy of every gradient of a list, on the stream they belong to."""
+        with self._pending_lock:
+            pending, waiting.gradients, waiting.elements = waiting.gradients, {}, 0
+            if not pending:
+                return
+            scaler = self.loss_scaler
+            state_ptr = scaler.state_ptr if isinstance(scaler, DynamicLossScaler) else None
+            rows = [(g.data_ptr(), self.client.data_address(p), g.numel(), g.dtype == torch.half) for p, g in pending.items()]
+            with _lib.on_device(self.client.device):
+                _lib.check(
+                    _lib.load().ps_grads_to_chunks((_lib.ps_grad_copy * len(rows))(*rows), len(rows), state_ptr, waiting.handle),
+                    "ps_grads_to_chunks",
+                )
+
+    def _end_of_backward(self, task):
+        """Runs once when a backward pass that put gradients down ends, whoever started it: the caller's stream has been put
+        behind the streams of backward by then, so a copy queued only now needs the same."""
+        waiting = self._pending.pop(task, None)
+        if waiting is None or not waiting.gradients:
             return
-        pending, self._pending = self._pending, {}
-        scaler = self.loss_scaler
-        state_ptr = scaler.state_ptr if isinstance(scaler, DynamicLossScaler) else None
-        rows = [(g.data_ptr(), self.client.data_address(p), g.numel(), g.dtype == torch.half) for p, g in pending.items()]
-        with _lib.on_device(self.client.device):
-            _lib.check(
-                _lib.load().ps_grads_to_chunks(
-                    (_lib.ps_grad_copy * len(rows))(*rows), len(rows), state_ptr, self._pending_stream.cuda_stream
-                ),
-                "ps_grads_to_chunks",
-            )
-
-    def _end_of_backward(self):
-        """Runs once when the backward pass that put the pending gradients down ends, whoever started it: the caller's
-        stream has been put behind the streams of backward by then, so a copy queued only now needs the same."""
-        stream, waiting = self._pending_stream, bool(self._pending)
-        self._flush_gradients()
-        if waiting:
-            current = torch.cuda.current_stream(self.client.device)
-            if current.cuda_stream != stream.cuda_stream:
-                current.wait_stream(stream)
+        self._flush_gradients(waiting)
+        current = torch.cuda.current_stream(self.client.device)
+        if current.cuda_stream != waiting.handle:
+            current.wait_stream(waiting.stream)
 
     def _on_gradient_ready(self, p):
         """Post-accumulate-grad hook: runs during backward, as soon as ``p``'s gradient is complete (every use of the
@@ -163,18 +194,18 @@ class PatrickStarEngine(torch.nn.Module):
         reference does the same copy in its post-backward module hook (``patrickstar/core/hook.py:200-230``); the
         copies overlap the rest of backward and no second full set of gradients stays alive."""
         task = torch._C._current_graph_task_id()
-        if task != self._pending_task:
-            # another backward pass than the one whose end the list waits for (a nested one, or the next one after a
-            # pass that failed)
-            self._flush_gradients()
-            self._pending_task = task
-            torch.autograd.Variable._execution_engine.queue_callback(self._end_of_backward)
-        self._gradient_to_chunk(p)
+        waiting = self._pending.get(task)
+        if waiting is None:
+            # every pass has a list of its own: passes nest (reentrant checkpoints), run beside one another (threads) and fail
+            waiting = self._pending[task] = _Waiting()
+            torch.autograd.Variable._execution_engine.queue_callback(_EndOfPass(self, task))
+        self._gradient_to_chunk(p, waiting)
         self._copied.add(p)
 
     def _finish_gradients(self):
         """After backward: parameters whose hook did not fire (no gradient this iteration, or a gradient that was
         assigned by hand)."""
+        waiting = _Waiting()
         for p in self.client.chunk_based_param_fp16:
             if p in self._copied:
                 continue
@@ -182,17 +213,16 @@ class PatrickStarEngine(torch.nn.Module):
                 # a frozen parameter: the optimizer skips it (fp16_cpu_adam.py:566-569), its slot keeps the parameter
                 continue
             if p.grad is not None:
-                self._gradient_to_chunk(p)
+                self._gradient_to_chunk(p, waiting)
             else:
                 # the slot still holds the fp16 parameter, which step() would read as a gradient
                 self.client.access_data(p).zero_()
-        self._end_of_backward()
+        self._flush_gradients(waiting)
         self._copied.clear()
 
     def backward(self, loss):
         self.optimizer.zero_grad()
         self._copied.clear()
-        self._pending.clear()  # left by a pass that failed
         if self.loss_scaler:
             self.loss_scaler.backward(loss)
         else:

@@ -1,0 +1,214 @@
+"""The engine's lists of waiting gradients, on the CPU: the engine's own hooks and bookkeeping, with a stand-in for the
+kernel that copies the gradients of a list into their chunk slots."""
+import copy
+import ctypes
+import threading
+import types
+
+import pytest
+import torch
+from torch.utils.checkpoint import checkpoint
+
+import patrickstar_amd as ps
+from patrickstar_amd import _lib, engine as engine_module
+
+
+class _Net(torch.nn.Module):
+    def __init__(self, n=5):
+        super().__init__()
+        self.layers = torch.nn.ModuleList([torch.nn.Linear(6, 6) for _ in range(n)])
+        self.nested = ()
+
+    def forward(self, x):
+        for i, layer in enumerate(self.layers):
+            f = lambda y, m=layer: torch.tanh(m(y)) + y
+            x = checkpoint(f, x, use_reentrant=True) if i in self.nested else f(x)
+        return x.float().pow(2).mean()
+
+
+def _tensor_at(address, numel, half):
+    """The elements at an address, as a tensor that shares them."""
+    raw = (ctypes.c_int16 * numel).from_address(address) if half else (ctypes.c_float * numel).from_address(address)
+    return torch.frombuffer(raw, dtype=torch.half if half else torch.float)
+
+
+class _Library:
+    """What the engine calls of the native library, on host memory."""
+
+    def __init__(self):
+        self.flag = False  # the sticky overflow flag
+        self.launches = []  # gradients in each
+
+    def ps_grads_to_chunks(self, copies, n, state, stream):
+        self.launches.append(n)
+        for c in copies[:n]:
+            if c.numel:
+                slot = _tensor_at(c.d_slot_fp16, c.numel, True)
+                slot.copy_(_tensor_at(c.d_grad, c.numel, c.grad_is_half != 0))
+                self.flag = self.flag or not bool(torch.isfinite(slot).all())
+        return 0
+
+
+@pytest.fixture
+def host(monkeypatch):
+    """(engine, params, slots, library): an engine over a net on the CPU."""
+    library = _Library()
+    native = _lib.load()
+    monkeypatch.setattr(engine_module, "_lib", types.SimpleNamespace(
+        load=lambda: library, check=_lib.check, ps_grad_copy=_lib.ps_grad_copy, raw_stream=lambda device: 0, on_device=lambda device: _lib._NO_GUARD,
+    ))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: types.SimpleNamespace(cuda_stream=0))
+    assert native is not library
+    torch.manual_seed(0)
+    config = {"optimizer": {"type": "Adam", "params": {"lr": 1e-3, "betas": (0.9, 0.999), "eps": 1e-8, "weight_decay": 0}},
+              "fp16": {"enabled": True, "loss_scale": 64}}
+    client = ps.PatrickStarClient(0, 512, device="cpu")
+    model = client.register_model(_Net())
+    engine = ps.PatrickStarEngine(model=model, client=client, config=config)
+    params = list(engine.module.parameters())
+    return engine, params, [client.access_data(p) for p in params], library
+
+
+def _expected(engine, x, params):
+    nested, engine.module.nested = engine.module.nested, ()
+    want = torch.autograd.grad(engine(x) * 64, params)  # no hooks fire for autograd.grad
+    engine.module.nested = nested
+    return want
+
+
+def _input(seed=1):
+    return torch.randn(3, 6, generator=torch.Generator().manual_seed(seed)).half().requires_grad_()
+
+
+def _same(slots, want):
+    return [bool(torch.equal(s.view(w.shape), w)) for s, w in zip(slots, want)]
+
+
+class _Refused(Exception):
+    pass
+
+
+def _failing_pass(engine, x, start, inf=False):
+    """A backward pass that raises after every parameter's hook has run (``start`` begins it)."""
+    y = x.detach().clone().requires_grad_()
+
+    def refuse(grad):
+        raise _Refused
+
+    y.register_hook(refuse)  # the last gradient of the pass
+    with pytest.raises(_Refused):
+        start(engine(y) * (float("inf") if inf else 64))
+
+
+# 1: a copy for every gradient; 3: some copied, some waiting; 64: all of them waiting when the pass fails
+@pytest.mark.parametrize("at_once", [1, 3, 64])
+@pytest.mark.parametrize("nested", [(), (1, 2), (0, 3)])
+@pytest.mark.parametrize("retry", ["plain backward", "engine"])
+def test_gradients_of_a_failed_pass_stay_out_of_the_next_one(host, monkeypatch, at_once, nested, retry):
+    engine, params, slots, library = host
+    monkeypatch.setattr(type(engine), "PENDING_GRADIENTS", at_once)
+    x = _input()
+    engine.module.nested = nested
+    kept = [s.clone() for s in slots]
+    want = _expected(engine, x, params)
+    _failing_pass(engine, _input(2), lambda loss: loss.backward(), inf=True)
+    assert not engine._pending
+    library.flag = False  # the caller clears the flag and restores the parameters
+    for s, k in zip(slots, kept):
+        s.copy_(k)
+    if retry == "engine":
+        engine.backward(engine(x))
+    else:
+        (engine(x) * 64).backward()
+    assert all(_same(slots, want))
+    assert not library.flag and not engine._pending and all(p.grad is None for p in params)
+
+
+@pytest.mark.parametrize("nested", [(1, 2), (0, 3), (4,), (0, 1, 2, 3, 4)])
+def test_a_nested_pass_leaves_the_outer_list_waiting(host, nested):
+    engine, params, slots, library = host
+    engine.module.nested = nested
+    x = _input()
+    want = _expected(engine, x, params)
+    engine.backward(engine(x))
+    assert all(_same(slots, want)) and not engine._pending
+    # one copy at the end of each nested pass, one at the end of the outer one if it had gradients of its own
+    assert len(library.launches) == len(nested) + (len(nested) < len(engine.module.layers))
+
+
+def test_two_failed_passes_and_a_failed_nested_one(host):
+    engine, params, slots, library = host
+    x = _input()
+    kept = [s.clone() for s in slots]
+    want = _expected(engine, x, params)
+    engine.module.nested = (0, 1)
+
+    def refuse(grad):
+        raise _Refused
+
+    for _ in range(2):
+        handle = engine.module.layers[0].weight.register_hook(refuse)  # raises inside the nested pass over layer 0
+        with pytest.raises(_Refused):
+            engine.backward(engine(x))
+        handle.remove()
+        assert not engine._pending
+        for s, k in zip(slots, kept):
+            s.copy_(k)
+        for p in params:
+            p.grad = None
+    (engine(x) * 64).backward()
+    assert all(_same(slots, want)) and not engine._pending
+
+
+@pytest.mark.parametrize("inf_in_first", [False, True])
+def test_a_parameter_of_two_passes_keeps_the_later_gradient(host, inf_in_first):
+    """A layer outside a nested pass (its gradient comes first, and waits) and inside it: two gradients for one slot."""
+    engine, params, slots, library = host
+    first = engine.module.layers[0]
+    twin = copy.deepcopy(first)
+
+    def forward(x, inner):
+        f = lambda y: torch.tanh(engine.module.layers[1](inner(y)))
+        x = checkpoint(f, x, use_reentrant=True) if inner is first else f(x)
+        x = torch.tanh(first(engine.module.layers[2](x)))
+        return x.float().pow(2).mean() * 64
+
+    x = _input()
+    want = torch.autograd.grad(forward(x, twin), list(twin.parameters()))
+    if inf_in_first:
+        first.weight.register_hook(lambda g: g * float("inf") if not library.launches and not seen.append(1) else g)
+    seen = []
+    forward(x, first).backward()
+    assert bool(seen) == inf_in_first == library.flag and not engine._pending
+    if not inf_in_first:
+        assert all(_same(slots[:2], want))
+
+
+def test_passes_of_two_threads_keep_their_gradients_apart(host):
+    engine, params, slots, library = host
+    x = _input()
+    halves = [engine.module.layers[:2], engine.module.layers[2:]]
+    want, losses = [], []
+    for layers in halves:
+        y = x
+        for layer in layers:
+            y = torch.tanh(layer(y))
+        losses.append(y.float().pow(2).mean() * 64)
+        want += torch.autograd.grad(losses[-1], [p for layer in layers for p in layer.parameters()], retain_graph=True)
+    both = threading.Barrier(2)
+    for i, layers in enumerate(halves):
+        layers[0].weight.register_hook(lambda g: (both.wait(30), None)[1])  # neither pass ends before the other's last gradient
+    errors = []
+
+    def run(loss):
+        try:
+            loss.backward()
+        except Exception as e:
+            errors.append(e)
+
+    workers = [threading.Thread(target=run, args=(loss,)) for loss in losses]
+    for w in workers:
+        w.start()
+    for w in workers:
+        w.join(60)
+    assert not errors and all(_same(slots, want)) and not engine._pending

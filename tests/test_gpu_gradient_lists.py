@@ -110,3 +110,36 @@ def test_every_gradient_is_in_its_slot_when_backward_returns(how, monkeypatch):
         assert torch.equal(a, b), k
     optimizer.step()
     assert torch.isfinite(engine(x))
+
+
+@pytest.mark.parametrize("nested", [False, True])
+def test_a_plain_backward_after_a_failed_pass(nested):
+    """The failed pass leaves gradients that were never copied (45 layers, 90 of them, 64 to a launch): they stay out of the
+    slots, which the next pass reads as weights, and out of the overflow flag."""
+    torch.manual_seed(0)
+    config = {
+        "optimizer": {"type": "Adam", "params": {"lr": 1e-3, "betas": (0.9, 0.999), "eps": 1e-8, "weight_decay": 0}},
+        "fp16": {"enabled": True, "loss_scale": 0, "initial_scale_power": 6},
+        "default_chunk_size": 4096,
+    }
+    engine, optimizer = ps.initialize_engine(model_func=lambda: _Net(False), local_rank=0, config=config)
+    params = list(engine.module.parameters())
+    slots = [engine.client.access_data(p) for p in params]
+    x = torch.randn(8, 24, device="cuda").half().requires_grad_()
+    expected = torch.autograd.grad(engine(x) * 64, params)
+    kept = [s.clone() for s in slots]
+    engine.module.reentrant = nested
+
+    def refuse(grad):
+        raise ValueError("refused")
+
+    y = x.detach().clone().requires_grad_()
+    y.register_hook(refuse)
+    with pytest.raises(ValueError):
+        (engine(y) * float("inf")).backward()
+    for s, k in zip(slots, kept):
+        s.copy_(k)
+    optimizer.has_overflow = False
+    (engine(x) * 64).backward()
+    assert all(torch.equal(a, b) for a, b in zip(slots, expected))
+    assert optimizer.has_overflow is False and not engine._pending
