@@ -87,6 +87,7 @@ class PatrickStarClient:
         self.margin_use_ratio = 0.8  # the reference's default share of the margin (memtracer.py:190-214)
         self.staging_slots = 3  # what the optimizer streams host-resident positions through (FP16Adam.staging_slots)
         self.placement = None  # what plan_placement decided, for inspection
+        self.gradient_writer = None  # the engine's: called by settle_gradients
         if config is not None:
             self.opt_config.update(config.get("opts", {}))
             if "host_chunk_policy" in config:
@@ -353,6 +354,7 @@ class PatrickStarClient:
         """The tensor of ``param`` inside its chunk payload (a view; nothing moves)."""
         if param.ps_attr.param_type == ParamType.TORCH_BASED:
             return param.data  # PyTorch's own tensor (patrickstar/core/client.py:552-553)
+        self.settle_gradients(param)
         info = self.chunk_tensor_index.get_tensor_info(param.ps_attr.data_id())
         payload = self.chunk_list[info.chunk_id].payload
         if payload is None:
@@ -367,6 +369,14 @@ class PatrickStarClient:
                 f"{param.ps_attr.name} lives on {view.device}; this client does not move chunks (asked for {device})"
             )
         return view
+
+    def settle_gradients(self, param=None):
+        """During backward: queue the copies of gradients that are complete and wait to be written into their chunk slots
+        (the one of ``param``, with what waits beside it; None: all of them).  Work queued on the current stream afterwards
+        finds them there.  ``access_data``, the optimizer's ``step`` and whatever reads the overflow flag do this by themselves;
+        code that looks at a payload, or at a view of it taken earlier, before backward has returned calls it first."""
+        if self.gradient_writer is not None:
+            self.gradient_writer(param)
 
     def data_address(self, param):
         """``access_data(param).data_ptr()`` of a chunk tensor, without making the view."""

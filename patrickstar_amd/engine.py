@@ -125,6 +125,9 @@ class PatrickStarEngine(torch.nn.Module):
         self.iteration_cnt_ = 0
         self._copied = set()  # parameters whose gradient sits in its chunk slot already, or waits to be copied there (this backward)
         self._pending = {}  # backward pass that is under way (autograd's number of it) -> the gradients of it that wait to be copied
+        self.client.gradient_writer = self._settle_gradients
+        if isinstance(self.loss_scaler, DynamicLossScaler):
+            self.loss_scaler.before_flag = self._settle_gradients
         self._pending_lock = threading.RLock()  # hooks run on autograd's threads, the callback at a pass's end on its caller's
         for p in self.client.chunk_based_param_fp16:
             if p.requires_grad:
@@ -183,10 +186,23 @@ class PatrickStarEngine(torch.nn.Module):
         waiting = self._pending.pop(task, None)
         if waiting is None or not waiting.gradients:
             return
+        self._flush_in_front(waiting)
+
+    def _flush_in_front(self, waiting):
+        """Queue the copies of a list in front of what the current stream gets next."""
         self._flush_gradients(waiting)
         current = torch.cuda.current_stream(self.client.device)
         if current.cuda_stream != waiting.handle:
             current.wait_stream(waiting.stream)
+
+    def _settle_gradients(self, param=None):
+        """``PatrickStarClient.settle_gradients``."""
+        if not self._pending:
+            return
+        with self._pending_lock:
+            for waiting in tuple(self._pending.values()):
+                if waiting.gradients and (param is None or param in waiting.gradients):
+                    self._flush_in_front(waiting)
 
     def _on_gradient_ready(self, p):
         """Post-accumulate-grad hook: runs during backward, as soon as ``p``'s gradient is complete (every use of the

@@ -446,12 +446,14 @@ class FP16Adam(torch.optim.Optimizer):
     # -- overflow flag ------------------------------------------------------------
     @property
     def has_overflow(self):
+        self.client.settle_gradients()
         if self._dynamic:
             return self.loss_scaler.overflow_flag
         return self._host_overflow
 
     @has_overflow.setter
     def has_overflow(self, value):
+        self.client.settle_gradients()
         if self._dynamic:
             self.loss_scaler.materialize(self.client.device)
             off = _lib.ps_step_state.overflow.offset
@@ -494,6 +496,7 @@ class FP16Adam(torch.optim.Optimizer):
         """Probe the fp16 gradient payload of every chunk (asynchronous)."""
         if not self._dynamic:
             return
+        self.client.settle_gradients()
         table, n_dev, host_positions = self._tables or self._build_tables()
         stream = _lib.current_stream_handle()
         if n_dev:
@@ -678,6 +681,7 @@ class FP16Adam(torch.optim.Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
+        self.client.settle_gradients()
         # which parameters are trainable is looked at every step, as the reference does (fp16_cpu_adam.py:569-571):
         # freezing or unfreezing a parameter between steps makes a new plan (descriptor tables, call pattern, and
         # whether every tensor can still share one step number)

@@ -98,6 +98,8 @@ class DynamicLossScaler:
         # completed since the last time: records = [(iteration, overflow, scale before, scale after)], lost = how
         # many iterations fell out of the ring unseen.  A callable, or a weak reference to one.  Needs enable_log.
         self.on_read = None
+        # Called before the sticky flag is read or consumed: the engine queues the copies of gradients that wait to be probed.
+        self.before_flag = None
         self._betas = (0.9, 0.999)
 
     # -- device state ---------------------------------------------------------
@@ -247,6 +249,8 @@ class DynamicLossScaler:
     @property
     def overflow_flag(self):
         """The sticky device flag of the step being assembled (synchronises)."""
+        if self.before_flag is not None:
+            self.before_flag()
         return False if self._state is None else bool(self._read().overflow)
 
     @property
@@ -303,6 +307,8 @@ class DynamicLossScaler:
         """``overflow`` is a bool, or None to consume the sticky device flag; asynchronous.
         ``operator_calls``: how many tensors the optimizer step behind this call handed to the native operator in the
         reference's terms; a clean step takes the operator's step / beta^t state through that many calls."""
+        if self.before_flag is not None:
+            self.before_flag()
         self.materialize()
         mode = _lib.PS_FLAG_FROM_DEVICE if overflow is None else (_lib.PS_FLAG_TRUE if overflow else _lib.PS_FLAG_FALSE)
         with _lib.on_device(self._state.device):

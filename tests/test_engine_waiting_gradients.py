@@ -212,3 +212,65 @@ def test_passes_of_two_threads_keep_their_gradients_apart(host):
     for w in workers:
         w.join(60)
     assert not errors and all(_same(slots, want)) and not engine._pending
+
+
+def _readers(engine, params):
+    """What a program may do in the middle of a backward pass to see the gradients that are complete."""
+    client, optimizer = engine.client, engine.optimizer
+    optimizer._plan, optimizer._trainable_seen = {"kind": "empty"}, tuple(p.requires_grad for p in optimizer.param_groups[0]["params"])
+    return {
+        "access_data": lambda p: client.access_data(p),
+        "settle all": lambda p: client.settle_gradients(),
+        "settle one": lambda p: client.settle_gradients(p),
+        "has_overflow": lambda p: optimizer.has_overflow,
+        "clear the flag": lambda p: setattr(optimizer, "has_overflow", False),
+        "reset": lambda p: optimizer.has_overflow_and_reset_param(),
+        "step": lambda p: optimizer.step(),
+    }
+
+
+@pytest.mark.parametrize("how", ["access_data", "settle all", "settle one", "has_overflow", "clear the flag", "reset", "step"])
+def test_a_complete_gradient_is_in_its_slot_for_whoever_looks_during_backward(host, how):
+    engine, params, slots, library = host
+    x = _input()
+    want = _expected(engine, x, params)
+    look, seen = _readers(engine, params)[how], []
+
+    def hook(p):
+        i = [q is p for q in params].index(True)
+        look(p)
+        seen.append((i, slots[i].clone()))
+
+    for p in params:
+        p.register_post_accumulate_grad_hook(hook)  # behind the engine's own
+    engine.backward(engine(x))
+    assert sorted(i for i, _ in seen) == list(range(len(params)))
+    assert all(torch.equal(s.view(want[i].shape), want[i]) for i, s in seen)
+
+
+@pytest.mark.parametrize("how", ["access_data", "step"])
+def test_gradients_are_in_their_slots_for_a_callback_that_runs_before_the_engines(host, how):
+    engine, params, slots, library = host
+    x = _input()
+    want = _expected(engine, x, params)
+    look, seen = _readers(engine, params)[how], []
+
+    def at_end():
+        for p in params:
+            look(p)
+        seen.extend(s.clone() for s in slots)
+
+    loss = engine(x) * 64
+    loss.register_hook(lambda g: torch.autograd.Variable._execution_engine.queue_callback(at_end))
+    loss.backward()
+    assert len(seen) == len(params) and all(_same(seen, want)) and not engine._pending
+
+
+def test_a_dynamic_scaler_asks_for_waiting_gradients_before_its_flag_is_read():
+    scaler, asked = ps.DynamicLossScaler(), []
+    scaler.before_flag = lambda: asked.append(1)
+    assert scaler.overflow_flag is False and asked == [1]
+    scaler.materialize = lambda: (_ for _ in ()).throw(_Refused())
+    with pytest.raises(_Refused):
+        scaler.update_scale(None)
+    assert asked == [1, 1]
