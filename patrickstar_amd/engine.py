@@ -10,6 +10,7 @@ written over their parameters' chunk slots as they are completed, a few at a tim
 and probed for inf/nan in the same pass (one fused kernel, no host sync), which
 is the state ``optimizer.step()`` expects.
 """
+import sys
 import threading
 
 import torch
@@ -146,7 +147,9 @@ class PatrickStarEngine(torch.nn.Module):
     def _gradient_to_chunk(self, p, waiting):
         """Take ``p.grad`` off ``p`` and put it down in ``waiting``, to be written over ``p``'s fp16 chunk slot and probed for
         inf/nan in the same pass, by a kernel it shares with its neighbours.  The list holds on to the gradients until that kernel is
-        queued, on the stream they were put down on, so their memory is not handed out before it has run."""
+        queued, on the stream they were put down on, so their memory is not handed out before it has run.  Memory that somebody else
+        holds too (a workspace that a backward function uses again, a piece of the caller's own tensor, a gradient that another hook
+        has kept) may be written before the pass ends: a gradient in it does not wait."""
         g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
         if g.dtype not in (torch.half, torch.float):
             raise TypeError(f"gradient dtype {g.dtype} is not supported")
@@ -162,7 +165,9 @@ class PatrickStarEngine(torch.nn.Module):
             waiting.gradients[p] = g
             waiting.elements += g.numel()
             p.grad = None
-            if len(waiting.gradients) >= self.PENDING_GRADIENTS or waiting.elements >= self.PENDING_ELEMENTS:
+            # (3: `g`, the list's reference and the argument; 2: the gradient's own use of its memory and the handle made here)
+            shared = sys.getrefcount(g) > 3 or torch._C._storage_Use_Count(g.untyped_storage()._cdata) > 2
+            if shared or len(waiting.gradients) >= self.PENDING_GRADIENTS or waiting.elements >= self.PENDING_ELEMENTS:
                 self._flush_gradients(waiting)
 
     def _flush_gradients(self, waiting):

@@ -274,3 +274,61 @@ def test_a_dynamic_scaler_asks_for_waiting_gradients_before_its_flag_is_read():
     with pytest.raises(_Refused):
         scaler.update_scale(None)
     assert asked == [1, 1]
+
+
+class _Product(torch.autograd.Function):
+    """x @ w.T whose weight gradient is formed in a workspace that every call uses again."""
+
+    @staticmethod
+    def forward(ctx, x, w, workspace):
+        ctx.save_for_backward(x, w)
+        ctx.workspace = workspace
+        return x @ w.t()
+
+    @staticmethod
+    def backward(ctx, g):
+        x, w = ctx.saved_tensors
+        torch.mm(g.t(), x, out=ctx.workspace.view(w.shape))
+        return g @ w, ctx.workspace.view(w.shape), None
+
+
+@pytest.mark.parametrize("how", ["workspace", "pieces of one tensor", "kept by a hook"])
+def test_a_gradient_in_memory_that_others_hold_is_copied_before_they_use_it_again(host, how):
+    engine, params, slots, library = host
+    weights = [layer.weight for layer in engine.module.layers]
+    workspace = torch.zeros(36, dtype=torch.half)
+    x = _input()
+
+    def forward(product):
+        y = x
+        for w in weights:
+            y = torch.tanh(product(y, w)) + y
+        return y.float().pow(2).mean() * 64
+
+    want = torch.autograd.grad(forward(lambda y, w: y @ w.t()), weights)
+    if how == "workspace":
+        forward(lambda y, w: _Product.apply(y, w, workspace)).backward()
+    elif how == "kept by a hook":
+        kept = []
+        for w in weights:
+            ready, w._post_accumulate_grad_hooks = w._post_accumulate_grad_hooks, None
+            w.register_post_accumulate_grad_hook(lambda p: kept.append(p.grad))  # in front of the engine's
+            for hook in ready.values():
+                w.register_post_accumulate_grad_hook(hook)
+        weights[0].register_post_accumulate_grad_hook(lambda p: ([g.zero_() for g in kept], None)[1])
+        forward(lambda y, w: y @ w.t()).backward()
+    else:
+        whole = torch.zeros(len(weights), 6, 6, dtype=torch.half)
+        for w, piece in zip(weights, whole):
+            w.grad = piece  # accumulated into, in place
+        # once the last gradient is complete, and before the pass ends, their owner clears the tensor for the next pass
+        weights[0].register_post_accumulate_grad_hook(lambda p: (whole.zero_(), None)[1])
+        forward(lambda y, w: y @ w.t()).backward()
+    got = [engine.client.access_data(w) for w in weights]
+    assert all(_same(got, want))
+
+
+def test_ordinary_gradients_share_a_launch(host):
+    engine, params, slots, library = host
+    engine.backward(engine(_input()))
+    assert library.launches == [len(params)]
