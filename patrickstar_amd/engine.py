@@ -216,6 +216,12 @@ class PatrickStarEngine(torch.nn.Module):
         copies overlap the rest of backward and no second full set of gradients stays alive."""
         task = torch._C._current_graph_task_id()
         waiting = self._pending.get(task)
+        if task < 0:  # the node that accumulates a gradient was called by itself: there is no pass whose end a list could wait for
+            waiting = _Waiting()
+            self._gradient_to_chunk(p, waiting)
+            self._flush_gradients(waiting)
+            self._copied.add(p)
+            return
         if waiting is None:
             # every pass has a list of its own: passes nest (reentrant checkpoints), run beside one another (threads) and fail
             waiting = self._pending[task] = _Waiting()

@@ -332,3 +332,13 @@ def test_ordinary_gradients_share_a_launch(host):
     engine, params, slots, library = host
     engine.backward(engine(_input()))
     assert library.launches == [len(params)]
+
+
+def test_a_gradient_accumulated_outside_any_backward_pass_is_copied_at_once(host):
+    engine, params, slots, library = host
+    for p, slot in zip(params, slots):
+        accumulate = p.view_as(p).grad_fn.next_functions[0][0]
+        g = torch.randn(p.shape).half()
+        accumulate(g.clone())
+        assert torch.equal(slot, g) and p.grad is None
+    assert not engine._pending
