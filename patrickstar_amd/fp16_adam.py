@@ -510,6 +510,13 @@ class FP16Adam(torch.optim.Optimizer):
             self._streamer.scan_gradients(self.loss_scaler)
 
     # -- the step -----------------------------------------------------------------
+    def _parts_are_our_own(self):
+        """Whether probe and scale update are this package's (nobody has put another method in their place), so that one
+        native call may stand for them and the step."""
+        return getattr(self.loss_scaler.update_scale, "__func__", None) is DynamicLossScaler.update_scale and (
+            not self.scan_in_step or getattr(self.check_overflow_chunks, "__func__", None) is FP16Adam.check_overflow_chunks
+        )
+
     def _entries(self, p):
         """(lr, betas, eps, weight_decay, step) of one parameter as its ``state[p]`` holds them."""
         g, st = dict.__getitem__, self.state[p]
@@ -707,8 +714,9 @@ class FP16Adam(torch.optim.Optimizer):
             chunk_numel = self.client.default_chunk_size
             if self._dynamic:
                 scaler = self.loss_scaler
-                if n_dev and not host_positions and self._stages is None and self._tensor_table is None:
-                    # HBM-resident chunks, all of them whole: probe, step and scale update in one call
+                whole_in_hbm = n_dev and not host_positions and self._stages is None and self._tensor_table is None
+                if whole_in_hbm and self._parts_are_our_own():
+                    # probe, step and scale update in one call
                     _lib.check(
                         self._lib.ps_adam_step_chunks_dynamic(
                             self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls,
@@ -734,6 +742,14 @@ class FP16Adam(torch.optim.Optimizer):
                 elif host_positions:
                     self._streamer.step(self.opt_id, 0, lr, beta1, beta2, eps, weight_decay, -1.0, table, n_dev,
                                         self._calls, scaler, self._used_all)
+                elif n_dev:
+                    _lib.check(
+                        self._lib.ps_adam_step_chunks_gated(
+                            self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls,
+                            scaler.state_ptr, stream,
+                        ),
+                        "ps_adam_step_chunks_gated",
+                    )
                 # consume the device flag; a clean step advances state["step"] and takes the operator object
                 # through this step's calls
                 scaler.update_scale(None, operator_calls=self._operator_calls)

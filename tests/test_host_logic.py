@@ -724,3 +724,72 @@ def test_per_parameter_step_counts_follow_the_reference_under_random_schedules()
                 trainable = [p for p in params if p.requires_grad]
                 assert len({want[p] for p in trainable}) <= 1 or tuple(p.requires_grad for p in params) != opt._trainable_seen
         assert [opt.state[p]["step"] for p in params] == [want[p] for p in params], case
+
+
+class _StepCalls:
+    """A stand-in for the native library: which of its step functions are called, and in what order."""
+
+    def __init__(self):
+        self.names = []
+
+    def __getattr__(self, name):
+        if not name.startswith("ps_"):
+            raise AttributeError(name)
+        return lambda *args: self.names.append(name) or 0
+
+
+def _device_decided_step_on_the_cpu(monkeypatch, scaler, optimizer_class=ps.FP16Adam):
+    """(optimizer, library stand-in): a device-decided step over two chunks whose native calls only leave their names."""
+    client = ps.PatrickStarClient(0, 1000, device="cpu")
+    optimizer = optimizer_class(client, client.append_flat_chunks(2), loss_scaler=scaler)
+    library = _StepCalls()
+    monkeypatch.setattr(_lib, "current_stream_handle", lambda: None)
+    monkeypatch.setattr(_lib, "load", lambda: library)
+    scaler._state = torch.zeros(256, dtype=torch.uint8)
+    optimizer._lib = library
+    monkeypatch.setattr(optimizer, "_make_plan", lambda: None)
+    optimizer._trainable_seen = tuple(p.requires_grad for p in optimizer.param_groups[0]["params"])
+    optimizer._plan = {"kind": "uniform", "hyper": (1e-3, (0.9, 0.999), 1e-8, 0.0)}
+    return optimizer, library
+
+
+def test_a_device_decided_step_over_whole_hbm_chunks_is_one_call(monkeypatch):
+    optimizer, library = _device_decided_step_on_the_cpu(monkeypatch, ps.DynamicLossScaler())
+    optimizer.step()
+    assert library.names == ["ps_adam_step_chunks_dynamic"]
+
+
+@pytest.mark.parametrize("how", ["subclass", "instance"])
+def test_a_step_goes_through_a_scalers_own_update_scale(monkeypatch, how):
+    seen = []
+
+    class Counting(ps.DynamicLossScaler):
+        def update_scale(self, overflow, operator_calls=1):
+            seen.append((overflow, operator_calls))
+            super().update_scale(overflow, operator_calls)
+
+    scaler = Counting() if how == "subclass" else ps.DynamicLossScaler()
+    if how == "instance":
+        own = scaler.update_scale
+        scaler.update_scale = lambda overflow, operator_calls=1: (seen.append((overflow, operator_calls)), own(overflow, operator_calls))[1]
+    optimizer, library = _device_decided_step_on_the_cpu(monkeypatch, scaler)
+    optimizer.step()
+    assert seen == [(None, 2)]
+    assert library.names == ["ps_overflow_scan_chunks", "ps_adam_step_chunks_gated", "ps_scaler_update"]
+
+
+def test_a_step_goes_through_an_optimizers_own_probe(monkeypatch):
+    seen = []
+
+    class Probing(ps.FP16Adam):
+        def check_overflow_chunks(self):
+            seen.append(1)
+            super().check_overflow_chunks()
+
+    optimizer, library = _device_decided_step_on_the_cpu(monkeypatch, ps.DynamicLossScaler(), Probing)
+    optimizer.step()
+    assert seen == [1]
+    assert library.names == ["ps_overflow_scan_chunks", "ps_adam_step_chunks_gated", "ps_scaler_update"]
+    optimizer.scan_in_step = False  # the caller feeds the flag: there is no probe to go through
+    optimizer.step()
+    assert seen == [1] and library.names[3:] == ["ps_adam_step_chunks_dynamic"]
