@@ -1688,28 +1688,31 @@ int ps_grads_to_chunks(const ps_grad_copy* copies, int n_copies, ps_step_state* 
     for (int i = 0; i < n_copies; ++i) {
         if (copies[i].numel > 0 && (!copies[i].d_grad || !copies[i].d_slot_fp16))
             return fail(PS_ERR_BAD_ARG, "copy %d has a NULL address", i);
-        if (copies[i].numel > (size_t)kCopySpan * kMaxCopyBlocks)
-            return fail(PS_ERR_BAD_ARG, "copy %d: numel = %zu is beyond the launch grid", i, (size_t)copies[i].numel);
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     int next = 0;
+    size_t done = 0;  // elements of copies[next] that earlier launches have taken
     while (next < n_copies) {
         GradBatch b;
         memset(&b, 0, sizeof(b));
         memset(b.first_block, 0xFF, sizeof(b.first_block));
         size_t blocks = 0;
         int in_batch = 0;
-        for (; next < n_copies && in_batch < kGradBatch; ++next) {
+        while (next < n_copies && in_batch < kGradBatch && blocks < kMaxCopyBlocks) {
             const ps_grad_copy& c = copies[next];
-            if (c.numel == 0) continue;
-            const size_t more = (c.numel + kCopySpan - 1) / kCopySpan;
-            if (blocks + more > kMaxCopyBlocks) break;  // the next launch starts with this gradient
-            b.src[in_batch] = c.d_grad;
-            b.dst[in_batch] = c.d_slot_fp16;
-            b.numel_half[in_batch] = 2 * (uint64_t)c.numel + (c.grad_is_half ? 1 : 0);
-            b.first_block[in_batch] = (uint32_t)blocks;
-            blocks += more;
-            in_batch += 1;
+            // what is left of a gradient if that fits into the launch grid, else whole spans, and the rest in the next launch
+            const size_t left = c.numel - done, room = (kMaxCopyBlocks - blocks) * kCopySpan;
+            const size_t numel = std::min(left, room);
+            if (numel > 0) {
+                b.src[in_batch] = static_cast<const char*>(c.d_grad) + done * (c.grad_is_half ? 2 : 4);
+                b.dst[in_batch] = c.d_slot_fp16 + done;
+                b.numel_half[in_batch] = 2 * (uint64_t)numel + (c.grad_is_half ? 1 : 0);
+                b.first_block[in_batch] = (uint32_t)blocks;
+                blocks += (numel + kCopySpan - 1) / kCopySpan;
+                in_batch += 1;
+            }
+            done += numel;
+            if (done == c.numel) next += 1, done = 0;
         }
         if (in_batch == 0) continue;
         const dim3 grid((unsigned)blocks), block(kCopyBlock);

@@ -51,6 +51,31 @@ def test_lists_of_gradients_land_in_adjacent_slots_and_nowhere_else(kind, count)
             grads[i][at] = keep
 
 
+def test_a_gradient_longer_than_one_launch_can_take():
+    """A launch's grid ends at 2^24 - 1 spans of 2048 elements: the rest of the gradient goes into the next one."""
+    n = (2**24 - 1) * 2048 + 4099
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 5 * n:
+        pytest.skip("two tensors of 64 GiB do not fit")
+    grad = torch.zeros(n, dtype=torch.half, device="cuda")
+    slot = torch.full((n + 3,), 7.0, dtype=torch.half, device="cuda")
+    marks = [0, 6, 7, 8, n - 4100, n - 4099, n - 4098, n - 2051, n - 1]
+    for i, at in enumerate(marks):
+        grad[at] = i + 1.0
+    scaler = ps.DynamicLossScaler(init_scale=2**4)
+    _copy([grad], [slot[1 : 1 + n]], scaler.state_ptr)
+    assert scaler.overflow_flag is False
+    assert [float(slot[1 + at]) for at in marks] == [i + 1.0 for i in range(len(marks))]
+    assert float(slot[0]) == 7.0 and slot[1 + n :].tolist() == [7.0, 7.0]
+    held = sum(int(torch.count_nonzero(slot[lo : lo + 2**30])) for lo in range(0, n + 3, 2**30))
+    assert held == len(marks) + 3  # every other element has been copied
+    grad[n - 1] = float("inf")
+    _copy([grad], [slot[1 : 1 + n]], scaler.state_ptr)
+    assert scaler.overflow_flag is True
+    del grad, slot
+    torch.cuda.empty_cache()
+
+
 class _Net(torch.nn.Module):
     def __init__(self, reentrant):
         super().__init__()
