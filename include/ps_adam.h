@@ -339,8 +339,9 @@ int ps_restore_fp16_chunks(const ps_chunk* chunks, int n_chunks, size_t chunk_nu
  * staging their fp16 gradients (chunk_io_buff.py:214-255) and casts the result
  * back through a GPU buffer (chunk_io_buff.py:85-151).  Here such chunks are
  * updated by the GPU.  Up to 8 of them in place, the kernel reading and writing the pinned
- * payloads over the link (if one of them is not mapped at its own address on the current
- * device: as if there were more).  More are streamed through HBM: for chunk k, slot k % n_slots
+ * payloads over the link, where that is no slower (not beside resident chunks that take longer
+ * than copies would leave the link idle) and every one of them is mapped at its own address on the
+ * current device.  Otherwise they are streamed through HBM: for chunk k, slot k % n_slots
  * of `staging` receives fp16 grad + fp32 param/m/v by hipMemcpyAsync on a side stream
  * (14 B/element), the fused kernel runs on it, and fp32 param/m/v + fp16 param
  * go back on another side stream (14 B/element); events order the three, so

@@ -569,10 +569,39 @@ int fp16_payloads_in_hbm(const ps_chunk* host_chunks, int n, bool* in_hbm, bool*
 // Few host chunks are updated where they are: the kernel reads and writes the pinned payloads over the link, both
 // directions busy from the first tile to the last, where the copies leave one of them idle while the first chunk
 // comes in and while the last one goes out.  In place moves 45.0 GB/s each way (whatever the launch shape: 1 to 4 tiles
-// per workgroup, 2 to 32 workgroups per CU: 42.9 to 45.0), copies 57.1 one way and 48.3 each way when both are busy.
-// For n chunks that take u to copy one way: in place 57.1 / 45.0 n u; copied 2 u + 57.1 / 48.3 (n - 1) u; the same at
-// n = 9.  Two chunks of 32 Mi elements, 12 B/element each way: 22.8 -> 17.9 ms.
+// per workgroup, 2 to 32 workgroups per CU: 42.9 to 45.0) if the payloads start on KiB boundaries (from 64 bytes on 39,
+// at any element 35), copies 57.1 one way and 48.3 each way when both are busy.  Chunks of 8 Mi elements, 12 B/element
+// each way, copied / in place: one 3.73 / 2.47 ms, two 5.82 / 4.67, four 9.88 / 9.07, eight 18.11 / 17.90, nine 20.17 /
+// 20.09, ten 22.21 / 22.28, twelve 26.34 / 26.69.
 constexpr int kMaxInPlaceChunks = 8;
+
+// Whether the update in place is no slower than the copies.  It shares the CUs with the resident chunks' kernels and is
+// dispatched behind them, so the two take about as long as one after the other; copies run beside those kernels.  Two
+// chunks of 8 Mi elements on the host, copied / in place: with 24 such chunks in HBM 5.81 / 5.22 ms, with 32 5.84 / 5.45,
+// with 120 5.85 / 8.69; eight with 24 18.1 / 18.3.  At one element from a KiB boundary four chunks of 4 Mi 5.06 / 5.19 ms
+// (at 4 elements), eight of 2 Mi 4.86 / 5.57.  Copies of small chunks are bound by their launches: 6267 elements 119 us
+// for one, 172 for two, 416 for eight.
+bool in_place_pays(const ChunkList& host, const bool* fp16_in_hbm, const ChunkList& resident)
+{
+    const double kUs = 1e-6, kGB = 1e9;
+    double bytes = 0, longest = 0, resident_bytes = 0;  // of the host chunks: each way
+    int n = 0;
+    uintptr_t phase = 0;
+    for (int i = 0; i < host.n_chunks; ++i) {
+        if (host.numel_of(i) == 0) continue;
+        const ps_chunk& c = host.chunks[i];
+        const double b = (fp16_in_hbm[i] ? 12.0 : 14.0) * (double)host.numel_of(i);
+        bytes += b;
+        longest = std::max(longest, b);
+        n += 1;
+        phase |= (uintptr_t)c.param_fp32 | (uintptr_t)c.exp_avg | (uintptr_t)c.exp_avg_sq;
+        if (!fp16_in_hbm[i]) phase |= (uintptr_t)c.param_fp16;
+    }
+    for (int i = 0; i < resident.n_chunks; ++i) resident_bytes += 28.0 * (double)resident.numel_of(i);
+    const double link = bytes / ((phase & 1023) == 0 ? 45.0 * kGB : 35.0 * kGB);
+    const double copies = std::max(60 * kUs + 40 * kUs * n, 2 * longest / (57.1 * kGB) + (bytes - longest) / (48.3 * kGB));
+    return link + resident_bytes / (6200 * kGB) <= copies;
+}
 
 // Whether every payload of the list can be used by a kernel on the current device under the address the caller gave:
 // pinned host memory of this device's making, mapped at its own address, or device memory.  (hipMemcpyAsync takes
@@ -1398,7 +1427,7 @@ int ps_adam_step_hybrid(int optimizer_id, size_t step, double lr, double beta1, 
     std::unique_lock<std::mutex> turn;
     bool in_place = false;
     if (stream_host) {
-        if (n_host_chunks <= kMaxInPlaceChunks)
+        if (n_host_chunks <= kMaxInPlaceChunks && in_place_pays(host, fp16_in_hbm.get(), resident))
             if (int rc = mapped_in_place(host_chunks, n_host_chunks, &in_place)) return rc;
         if (int rc = get_pipeline(&p)) return rc;
         turn = std::unique_lock<std::mutex>(p->in_use);

@@ -65,3 +65,52 @@ def test_in_place_and_copied_host_chunks_agree_bit_for_bit(n, offset, fp16_on_ho
         for name, x, y in zip(("fp32 param", "exp_avg", "exp_avg_sq", "fp16"), a, b):
             assert torch.equal(x.view(torch.int16 if x.dtype == torch.half else torch.int32),
                                y.view(torch.int16 if y.dtype == torch.half else torch.int32)), name
+
+
+MI = 1 << 20
+
+
+@pytest.mark.parametrize("n_host,offset,n_resident,in_place", [
+    (1, 0, 0, True), (2, 0, 0, True), (8, 0, 0, True), (9, 0, 0, False),
+    (2, 0, 8, True), (2, 0, 40, False),  # resident chunks that take as long as the copies would save: 31 of this size
+    (1, 1, 0, True), (8, 1, 0, False), (8, 16, 0, False),  # accesses that straddle the link's lines
+])
+def test_host_chunks_are_updated_in_place_where_that_is_no_slower(n_host, offset, n_resident, in_place):
+    """Which route a list takes, told by whether the staging slots have been written, and the same bits on both as for the
+    same chunks in HBM."""
+    gen = torch.Generator(device="cuda:0").manual_seed(n_host)
+    made = [[torch.randn(MI, generator=gen, device="cuda:0") * 0.02, torch.randn(MI, generator=gen, device="cuda:0") * 1e-4,
+             (torch.randn(MI, generator=gen, device="cuda:0") * 1e-4).square(), (torch.randn(MI, generator=gen, device="cuda:0") * 4).half()]
+            for _ in range(n_host)]
+    host = []
+    for c in made:
+        views = [torch.zeros(MI + 16, pin_memory=True)[offset : offset + MI] for _ in range(3)]
+        for v, x in zip(views, c):
+            v.copy_(x)
+        host.append(views + [c[3].clone()])
+    zeros = [torch.zeros(MI, device="cuda:0") for _ in range(3)] + [torch.zeros(MI, dtype=torch.half, device="cuda:0")]
+    kept = [[u.clone() for u in zeros] for _ in range(n_resident)]
+    resident = [[t.data_ptr() for t in c] for c in kept]
+    slots = [[torch.full((MI,), 7.0, device="cuda:0") for _ in range(3)] + [torch.empty(0, dtype=torch.half, device="cuda:0")] for _ in range(2)]
+    lib = _lib.load()
+    args = (1, 1e-3, 0.9, 0.999, 1e-8, 0.01, 1)
+    calls = _lib.call_pattern(n_resident + n_host)
+    for opt in (OPT, OPT + 1):
+        adam_op.create_adam(opt, 1e-3, 0.9, 0.999, 1e-8, 0.01, True, False)
+    rows = lambda chunks: _lib.chunk_array([[t.data_ptr() for t in c] for c in chunks])
+    rc = lib.ps_adam_step_hybrid(
+        OPT, *args, _lib.chunk_array(resident) if resident else None, n_resident, rows(host), n_host, MI, None,
+        _lib.chunk_array([[t.data_ptr() for t in s[:3]] + [None] for s in slots]), 2, calls, 1000.0, None, _lib.current_stream_handle(),
+    )
+    _lib.check(rc, "ps_adam_step_hybrid")
+    rc = lib.ps_adam_step_chunks(OPT + 1, *args, rows(made), n_host, MI, None, calls, 1000.0, _lib.current_stream_handle())
+    _lib.check(rc, "ps_adam_step_chunks")
+    torch.cuda.synchronize()
+    for opt in (OPT, OPT + 1):
+        adam_op.destroy_adam(opt)
+    untouched = all(bool((t == 7.0).all()) for s in slots for t in s[:3])
+    assert untouched == in_place
+    for got, want in zip(host, made):
+        for g, w in zip(got, want):
+            as_int = torch.int16 if w.dtype == torch.half else torch.int32
+            assert torch.equal(g.cuda().view(as_int), w.view(as_int))
