@@ -228,7 +228,8 @@ int main()
         uint16_t* h = nullptr;  // pinned host memory, or NULL when the fp16 payload stays in HBM
     };
     PinnedChunk pinned[C];
-    ps_chunk host_table[2], staging[2];
+    ps_chunk host_table[9], staging[2];
+    const size_t used[10] = {n, n, n, 0, 0, 0, 0, 0, 0, 0};
     for (int c = 1; c < C; ++c) {
         HIP_OK(hipHostMalloc((void**)&pinned[c].p, n * 4, hipHostMallocDefault));
         HIP_OK(hipHostMalloc((void**)&pinned[c].m, n * 4, hipHostMallocDefault));
@@ -239,6 +240,7 @@ int main()
         host_table[c - 1].exp_avg_sq = pinned[c].v;
         host_table[c - 1].param_fp16 = c == 2 ? pinned[c].h : dev[c].h;
     }
+    for (int c = 2; c < 9; ++c) host_table[c] = host_table[0];
     for (int s = 0; s < 2; ++s) {
         HIP_OK(hipMalloc((void**)&staging[s].param_fp32, n * 4));
         HIP_OK(hipMalloc((void**)&staging[s].exp_avg, n * 4));
@@ -262,8 +264,11 @@ int main()
                     HIP_OK(hipMemcpy(dev[c].h, host[c].h.data(), n * 2, hipMemcpyHostToDevice));
             }
         }
-        PS_OK(ps_adam_step_hybrid(33, step, lr, b1, b2, eps, wd, 1, table, 1, host_table, 2, n, nullptr, staging, 2, &calls, scale,
-                                  NULL, stream));
+        // (with seven more descriptors that hold nothing the list is long enough to be copied through the slots; without
+        // them it is updated in place)
+        const bool copied = step == 2;
+        PS_OK(ps_adam_step_hybrid(33, step, lr, b1, b2, eps, wd, 1, table, 1, host_table, copied ? 9 : 2, n, copied ? used : nullptr,
+                                  staging, 2, &calls, scale, NULL, stream));
         HIP_OK(hipStreamSynchronize(stream));
         for (int c = 0; c < C; ++c) {
             oracle_adam_advance(&native, step, b1, b2);

@@ -168,3 +168,22 @@ def test_a_plain_backward_after_a_failed_pass(nested):
     (engine(x) * 64).backward()
     assert all(torch.equal(a, b) for a, b in zip(slots, expected))
     assert optimizer.has_overflow is False and not engine._pending
+
+
+def test_gradients_of_ordinary_layers_wait_for_a_launch_they_share(monkeypatch):
+    """None of them is held by anybody else."""
+    def model():
+        return torch.nn.Sequential(torch.nn.Embedding(50, 32), torch.nn.TransformerEncoderLayer(32, 2, 64, dropout=0.0, batch_first=True),
+                                   torch.nn.LayerNorm(32), torch.nn.Linear(32, 32), torch.nn.Conv1d(7, 7, 3))
+
+    config = {
+        "optimizer": {"type": "Adam", "params": {"lr": 1e-3, "betas": (0.9, 0.999), "eps": 1e-8, "weight_decay": 0}},
+        "fp16": {"enabled": True, "loss_scale": 64},
+        "default_chunk_size": 8192,
+    }
+    engine, optimizer = ps.initialize_engine(model_func=model, local_rank=0, config=config)
+    flush, lists = engine._flush_gradients, []
+    monkeypatch.setattr(engine, "_flush_gradients", lambda waiting: (lists.append(len(waiting.gradients)), flush(waiting))[1])
+    engine.backward(engine(torch.randint(0, 50, (3, 7), device="cuda")).float().pow(2).mean())
+    n = sum(1 for _ in engine.module.parameters())
+    assert sorted(k for k in lists if k) == [n]

@@ -26,26 +26,28 @@ def _payloads(n, offset, fp16_on_host, seed):
     return out
 
 
-def _step(n, offset, fp16_on_host, used, empty_chunks, state):
-    """One step over two host chunks, with ``empty_chunks`` further ones that hold nothing."""
+def _step(n, offset, fp16_on_host, used, empty_chunks, state, n_slots):
+    """One step over two host chunks, with ``empty_chunks`` further ones that hold nothing: what they hold then, and whether
+    the staging slots have been written."""
     chunks = [_payloads(n, offset, fp16_on_host, seed) for seed in (1, 2)]
     chunks[1][0][1][used:] = chunks[1][1][1][used:] = chunks[1][2][1][used:] = chunks[1][3][1][used:] = 0.0
     rows = [[view.data_ptr() for _, view in c] for c in chunks]
     rows += [rows[0]] * empty_chunks
-    slots = [[torch.empty(n, device="cuda:0") for _ in range(3)] + [torch.empty(n, dtype=torch.half, device="cuda:0")] for _ in range(2)]
+    slots = [[torch.full((n,), 7.0, device="cuda:0") for _ in range(3)] + [torch.empty(n, dtype=torch.half, device="cuda:0")] for _ in range(n_slots)]
     used_numel = (ctypes.c_size_t * len(rows))(n, used, *[0] * empty_chunks)
     lib = _lib.load()
     adam_op.create_adam(OPT, 1e-3, 0.9, 0.999, 1e-8, 0.01, True, False)
     torch.cuda.synchronize()
     rc = lib.ps_adam_step_hybrid(
         OPT, 1, 1e-3, 0.9, 0.999, 1e-8, 0.01, 1, None, 0, _lib.chunk_array(rows), len(rows), n, used_numel,
-        _lib.chunk_array([[t.data_ptr() for t in s] for s in slots]), 2, _lib.call_pattern(3, 0, 1, max(1, n // 3)) if n > 1 else None,
+        _lib.chunk_array([[t.data_ptr() for t in s] for s in slots]), n_slots, _lib.call_pattern(3, 0, 1, max(1, n // 3)) if n > 1 else None,
         1000.0, state, _lib.current_stream_handle(),
     )
     _lib.check(rc, "ps_adam_step_hybrid")
     torch.cuda.synchronize()
     adam_op.destroy_adam(OPT)
-    return [[whole.cpu().clone() for whole, _ in c] for c in chunks]
+    copied = [any(bool((t != 7.0).any()) for t in s[:3]) for s in slots]
+    return [[whole.cpu().clone() for whole, _ in c] for c in chunks], copied
 
 
 @pytest.mark.parametrize("decided", ["host", "device", "skipped"])
@@ -53,18 +55,21 @@ def _step(n, offset, fp16_on_host, used, empty_chunks, state):
 @pytest.mark.parametrize("n,offset", [(1, 0), (255, 0), (256, 0), (257, 4), (6267, 0), (4096 + 77, 1), (70001, 2)])
 def test_in_place_and_copied_host_chunks_agree_bit_for_bit(n, offset, fp16_on_host, decided):
     got = []
-    for empty_chunks in (0, 7):  # two chunks: in place; nine: through the staging slots
+    for empty_chunks, n_slots in ((0, 2), (7, 2), (7, 1)):  # two chunks: in place; nine: through the staging slots, or through one, used again
         state = None
         if decided != "host":
             scaler = DynamicLossScaler(init_scale=1000.0).materialize("cuda:0", betas=(0.9, 0.999))
             if decided == "skipped":
                 scaler._state[_lib.ps_step_state.overflow.offset :][:4].view(torch.int32).fill_(1)
             state = scaler.state_ptr
-        got.append(_step(n, offset, fp16_on_host, n - n // 4, empty_chunks, state))
-    for a, b in zip(*got):
-        for name, x, y in zip(("fp32 param", "exp_avg", "exp_avg_sq", "fp16"), a, b):
-            assert torch.equal(x.view(torch.int16 if x.dtype == torch.half else torch.int32),
-                               y.view(torch.int16 if y.dtype == torch.half else torch.int32)), name
+        chunks, copied = _step(n, offset, fp16_on_host, n - n // 4, empty_chunks, state, n_slots)
+        assert copied == [empty_chunks > 0] * n_slots
+        got.append(chunks)
+    for a, *others in zip(*got):
+        for b in others:
+            for name, x, y in zip(("fp32 param", "exp_avg", "exp_avg_sq", "fp16"), a, b):
+                assert torch.equal(x.view(torch.int16 if x.dtype == torch.half else torch.int32),
+                                   y.view(torch.int16 if y.dtype == torch.half else torch.int32)), name
 
 
 MI = 1 << 20

@@ -38,11 +38,12 @@ def test_hybrid_static_bit_exact(host_positions, chunk_size, host_keeps_fp16):
         h.compare(oc, what=f"hybrid step {step}")
 
 
+@pytest.mark.parametrize("more", [0, 8])  # a few host positions are updated in place, more than eight copied through the slots
 @pytest.mark.parametrize("host_keeps_fp16", [True, False])
-def test_hybrid_dynamic_skips_and_restores_host_chunks_too(host_keeps_fp16):
+def test_hybrid_dynamic_skips_and_restores_host_chunks_too(host_keeps_fp16, more):
     kw = dict(init_scale=2**10, scale_factor=2, scale_window=3, min_scale=1)
     scaler = ps.DynamicLossScaler(**kw)
-    h = HybridHarness(4, 2048 * 2 + 9, [1, 2], scaler, seed=12, host_keeps_fp16=host_keeps_fp16, lr=1e-3, weight_decay=0.01)
+    h = HybridHarness(4 + more, 2048 * 2 + 9, [1, 2, *range(4, 4 + more)], scaler, seed=12, host_keeps_fp16=host_keeps_fp16, lr=1e-3, weight_decay=0.01)
     h.fill_state()
     oc = h.oracle_chunks()
     oscaler = oracle.ScalerOracle(**kw)
@@ -509,20 +510,23 @@ def test_engine_refuses_host_placement_without_hybrid_adam():
     assert not any(q.on_host for q in engine.client.positions())
 
 
-def test_two_host_threads_stream_host_chunks_on_one_gpu_at_the_same_time():
+@pytest.mark.parametrize("more", [0, 8])  # in place / copied, as above
+def test_two_host_threads_stream_host_chunks_on_one_gpu_at_the_same_time(more):
     """Two optimizers with host-resident positions, stepped by two host threads on two streams of the same GPU at the
     same moment (a barrier in front of every step; ctypes drops the GIL inside the call).  Both use the library's
     one set of side streams for that GPU: the calls take turns there, and both must match the oracle bit for bit."""
     import threading
 
-    n, steps = 256 * 1024 + 77, 4
+    n, steps, n_chunks = 256 * 1024 + 77, 4, 5 + more
     cases = [
         dict(host=[1, 2, 4], keeps=True, scaler=lambda: ps.LossScaler(2**10), oscaler=lambda: oracle.StaticScalerOracle(2**10),
              kw=dict(lr=1e-3, weight_decay=0.01, use_adamw=True)),
         dict(host=[0, 3], keeps=False, scaler=lambda: ps.DynamicLossScaler(init_scale=2**8, scale_factor=2, scale_window=2),
              oscaler=lambda: oracle.ScalerOracle(init_scale=2**8, scale_factor=2, scale_window=2), kw=dict(lr=1e-4, weight_decay=0.0)),
     ]
-    hs = [HybridHarness(5, n, c["host"], c["scaler"](), seed=31 + i, host_keeps_fp16=c["keeps"], **c["kw"]) for i, c in enumerate(cases)]
+    for c in cases:
+        c["host"] += range(5, n_chunks)
+    hs = [HybridHarness(n_chunks, n, c["host"], c["scaler"](), seed=31 + i, host_keeps_fp16=c["keeps"], **c["kw"]) for i, c in enumerate(cases)]
     for h in hs:
         h.opt.staging_slots = 2
         h.fill_state()
@@ -540,7 +544,7 @@ def test_two_host_threads_stream_host_chunks_on_one_gpu_at_the_same_time():
                     h.fill_grads(1e-3, scale)
                     if t == 1 and step == 1:
                         h.payloads(3)[3][n - 1] = float("inf")  # last element of a host position's fp16 payload
-                    grads[t].append([h.download(i)[3] for i in range(5)])
+                    grads[t].append([h.download(i)[3] for i in range(n_chunks)])
                     barrier.wait(timeout=60)
                     h.opt.step()
             stream.synchronize()
@@ -694,7 +698,8 @@ def test_freezing_and_unfreezing_parameters_between_steps():
     assert optimizer.state[module.fc2.bias]["step"] == 2
 
 
-def test_a_failed_launch_in_the_streamed_step_leaves_the_pipeline_usable():
+@pytest.mark.parametrize("more", [0, 8])  # in place / copied, as above
+def test_a_failed_launch_in_the_streamed_step_leaves_the_pipeline_usable(more):
     """ps_adam_step_hybrid makes its side streams wait for the caller's stream before it queues anything; if queuing then
     stops half way (here: the resident chunks' launch reports an error) the caller's stream must still be put behind
     the side streams before the call returns.  The failure is forced from outside, without any fault on the GPU: the
@@ -705,7 +710,7 @@ def test_a_failed_launch_in_the_streamed_step_leaves_the_pipeline_usable():
 
     hip = ctypes.CDLL("libamdhip64.so")
     akw = dict(lr=1e-3, weight_decay=0.01, use_adamw=True)
-    h = HybridHarness(4, 2048 * 2 + 9, [1, 3], ps.LossScaler(2**8), seed=31, **akw)
+    h = HybridHarness(4 + more, 2048 * 2 + 9, [1, 3, *range(4, 4 + more)], ps.LossScaler(2**8), seed=31, **akw)
     h.fill_state()
     h.fill_grads(1e-3, 2**8)
     h.opt.step()  # a good step first: the side streams exist and have been used
@@ -724,7 +729,7 @@ def test_a_failed_launch_in_the_streamed_step_leaves_the_pipeline_usable():
         pytest.skip("this HIP runtime forgets a refused call's error at the next successful call: a launch failure "
                     "cannot be forced from outside")
     # the pipeline of this process (one per device) goes on working
-    g = HybridHarness(4, 2048 * 2 + 9, [0, 2], ps.LossScaler(2**8), seed=32, **akw)
+    g = HybridHarness(4 + more, 2048 * 2 + 9, [0, 2, *range(4, 4 + more)], ps.LossScaler(2**8), seed=32, **akw)
     g.fill_state()
     oc = g.oracle_chunks()
     oopt = oracle.OptimizerStepOracle(oc, oracle.StaticScalerOracle(2**8), lr=1e-3, weight_decay=0.01, use_adamw=True)
