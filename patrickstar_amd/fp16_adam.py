@@ -511,10 +511,12 @@ class FP16Adam(torch.optim.Optimizer):
 
     # -- the step -----------------------------------------------------------------
     def _parts_are_our_own(self):
-        """Whether probe and scale update are this package's (nobody has put another method in their place), so that one
-        native call may stand for them and the step."""
-        return getattr(self.loss_scaler.update_scale, "__func__", None) is DynamicLossScaler.update_scale and (
-            not self.scan_in_step or getattr(self.check_overflow_chunks, "__func__", None) is FP16Adam.check_overflow_chunks
+        """Whether probe and scale update are this package's (nobody has put another method in their place, in a class or on
+        an object), so that one native call may stand for them and the step."""
+        scaler = self.loss_scaler
+        return (type(scaler).update_scale is _UPDATE_SCALE and "update_scale" not in scaler.__dict__) and (
+            not self.scan_in_step
+            or (type(self).check_overflow_chunks is _CHECK_OVERFLOW_CHUNKS and "check_overflow_chunks" not in self.__dict__)
         )
 
     def _entries(self, p):
@@ -688,7 +690,8 @@ class FP16Adam(torch.optim.Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        self.client.settle_gradients()
+        if self.client.gradient_writer is not None:
+            self.client.settle_gradients()
         # which parameters are trainable is looked at every step, as the reference does (fp16_cpu_adam.py:569-571):
         # freezing or unfreezing a parameter between steps makes a new plan (descriptor tables, call pattern, and
         # whether every tensor can still share one step number)
@@ -852,3 +855,6 @@ class FP16Adam(torch.optim.Optimizer):
             self.loss_scaler.materialize(self.client.device)
             if "loss_scaler" in state_dict:
                 self.loss_scaler.load_state_dict(state_dict["loss_scaler"])
+
+
+_UPDATE_SCALE, _CHECK_OVERFLOW_CHUNKS = DynamicLossScaler.update_scale, FP16Adam.check_overflow_chunks

@@ -759,7 +759,7 @@ def test_a_device_decided_step_over_whole_hbm_chunks_is_one_call(monkeypatch):
     assert library.names == ["ps_adam_step_chunks_dynamic"]
 
 
-@pytest.mark.parametrize("how", ["subclass", "instance"])
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
 def test_a_step_goes_through_a_scalers_own_update_scale(monkeypatch, how):
     seen = []
 
@@ -772,13 +772,18 @@ def test_a_step_goes_through_a_scalers_own_update_scale(monkeypatch, how):
     if how == "instance":
         own = scaler.update_scale
         scaler.update_scale = lambda overflow, operator_calls=1: (seen.append((overflow, operator_calls)), own(overflow, operator_calls))[1]
+    if how == "class":
+        replaced = ps.DynamicLossScaler.update_scale
+        monkeypatch.setattr(ps.DynamicLossScaler, "update_scale", lambda self, overflow, operator_calls=1: (
+            seen.append((overflow, operator_calls)), replaced(self, overflow, operator_calls))[1])
     optimizer, library = _device_decided_step_on_the_cpu(monkeypatch, scaler)
     optimizer.step()
     assert seen == [(None, 2)]
     assert library.names == ["ps_overflow_scan_chunks", "ps_adam_step_chunks_gated", "ps_scaler_update"]
 
 
-def test_a_step_goes_through_an_optimizers_own_probe(monkeypatch):
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_a_step_goes_through_an_optimizers_own_probe(monkeypatch, how):
     seen = []
 
     class Probing(ps.FP16Adam):
@@ -786,7 +791,13 @@ def test_a_step_goes_through_an_optimizers_own_probe(monkeypatch):
             seen.append(1)
             super().check_overflow_chunks()
 
-    optimizer, library = _device_decided_step_on_the_cpu(monkeypatch, ps.DynamicLossScaler(), Probing)
+    optimizer, library = _device_decided_step_on_the_cpu(monkeypatch, ps.DynamicLossScaler(), Probing if how == "subclass" else ps.FP16Adam)
+    if how == "instance":
+        own = optimizer.check_overflow_chunks
+        optimizer.check_overflow_chunks = lambda: (seen.append(1), own())[1]
+    if how == "class":
+        replaced = ps.FP16Adam.check_overflow_chunks
+        monkeypatch.setattr(ps.FP16Adam, "check_overflow_chunks", lambda self: (seen.append(1), replaced(self))[1])
     optimizer.step()
     assert seen == [1]
     assert library.names == ["ps_overflow_scan_chunks", "ps_adam_step_chunks_gated", "ps_scaler_update"]
