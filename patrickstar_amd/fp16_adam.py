@@ -510,15 +510,6 @@ class FP16Adam(torch.optim.Optimizer):
             self._streamer.scan_gradients(self.loss_scaler)
 
     # -- the step -----------------------------------------------------------------
-    def _parts_are_our_own(self):
-        """Whether probe and scale update are this package's (nobody has put another method in their place, in a class or on
-        an object), so that one native call may stand for them and the step."""
-        scaler = self.loss_scaler
-        return (type(scaler).update_scale is _UPDATE_SCALE and "update_scale" not in scaler.__dict__) and (
-            not self.scan_in_step
-            or (type(self).check_overflow_chunks is _CHECK_OVERFLOW_CHUNKS and "check_overflow_chunks" not in self.__dict__)
-        )
-
     def _entries(self, p):
         """(lr, betas, eps, weight_decay, step) of one parameter as its ``state[p]`` holds them."""
         g, st = dict.__getitem__, self.state[p]
@@ -717,19 +708,24 @@ class FP16Adam(torch.optim.Optimizer):
             chunk_numel = self.client.default_chunk_size
             if self._dynamic:
                 scaler = self.loss_scaler
-                whole_in_hbm = n_dev and not host_positions and self._stages is None and self._tensor_table is None
-                if whole_in_hbm and self._parts_are_our_own():
-                    # probe, step and scale update in one call
+                scan = self.scan_in_step
+                if (
+                    n_dev and not host_positions and self._stages is None and self._tensor_table is None
+                    # (nobody has put a method of their own in place of the scale update or the probe, in a class or on an object)
+                    and type(scaler).update_scale is _UPDATE_SCALE and "update_scale" not in scaler.__dict__
+                    and (not scan or (type(self).check_overflow_chunks is _CHECK_OVERFLOW_CHUNKS and "check_overflow_chunks" not in self.__dict__))
+                ):
+                    # HBM-resident chunks, all of them whole: probe, step and scale update in one call
                     _lib.check(
                         self._lib.ps_adam_step_chunks_dynamic(
                             self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls,
-                            int(self.scan_in_step), scaler.state_ptr, *scaler.log_arguments(), self._operator_calls, stream,
+                            int(scan), scaler.state_ptr, *scaler.log_arguments(), self._operator_calls, stream,
                         ),
                         "ps_adam_step_chunks_dynamic",
                     )
                     self._steps_dirty = True
                     return loss
-                if self.scan_in_step:
+                if scan:
                     self.check_overflow_chunks()
                 if self._stages is not None:
                     self._run_stages(0, hyper, -1.0, scaler, stream)
