@@ -355,7 +355,8 @@ int ps_restore_fp16_chunks(const ps_chunk* chunks, int n_chunks, size_t chunk_nu
  *                14 B/element cross the link each way); the library asks the HIP runtime which
  *   staging      host array of n_slots (1..8) descriptors of DEVICE buffers of
  *                chunk_numel elements each, owned by the caller; param_fp16 may be NULL when
- *                every host chunk keeps its fp16 payload in HBM
+ *                every host chunk keeps its fp16 payload in HBM.  Asked for whichever way the list
+ *                takes; not written where the chunks are updated in place
  *   used_numel   as for ps_adam_step_chunks, over chunks[] followed by host_chunks[] (NULL: all full);
  *                only the used part of a host chunk crosses the link
  *   calls        as for ps_adam_step_chunks, over chunks[] followed by host_chunks[]; with

@@ -22,9 +22,11 @@ static_assert(sizeof(ps_chunk) == 32 && sizeof(ps_step_state) == 256 && sizeof(p
 
 // What a workgroup needs before its first data load, fetched from the kernel arguments in one go.  Left to itself the
 // compiler loads the length, tests it, loads the call span, tests it, and only then loads the addresses: three waits
-// for scalar memory in a row in front of every tile's data loads.  The empty asm asks for all of them at once: 7.19 ->
-// 7.15 ms for 24 x 64 Mi elements, 313 -> 310 us for one chunk.  The device-decided kernel had five such rounds and has
-// three (arguments, step state, constants): 2603 -> 2593 us for a clean step over 8 x 64 Mi elements, probe included.
+// for scalar memory in a row in front of every tile's data loads.  The empty asm asks for all of them at once; the
+// device-decided kernel had five such rounds and has three (arguments, step state, constants).  What that is worth is about
+// what one run and the next differ by: both forms alternated on one box, 7207 and 7187 us for 24 x 64 Mi elements, 308 and
+// 305 us for one chunk, 2602 and 2595 us for a clean device-decided step over eight, probe included; the same step on other
+// boxes takes 7.10 to 7.35 ms.
 struct TileSource {
     float *p32, *m32, *v32;
     uint16_t* h16;
@@ -682,7 +684,7 @@ __global__ void __launch_bounds__(kReduceBlock)
 //
 // Bound by memory where it is long: one gradient of 64 Mi elements 38.0 us (fp16), 68.4 us (fp32), with the look-up
 // 38.7 and 69.1 us; with the look-up and 2, 4 and 8 vectors per lane 39.4 / 39.6 / 40.0 and 70.1 / 71.6 / 78.0 us.  The
-// 199 gradients of a BERT-base-sized module, a kernel for each: 613 us (2.5 us for every bias); in five launches: 78 us.
+// 199 gradients of a BERT-base-sized module, a kernel for each: 613 us (2.5 us for every bias); in five launches: 80 us.
 constexpr int kGradBatch = 64;
 constexpr int kCopyBlock = PS_COPY_BLOCK;
 constexpr unsigned kCopySpan = kCopyBlock * 8;  // elements per workgroup
@@ -942,9 +944,10 @@ __global__ void state_set_scaler_kernel(ps_step_state* st, double cur_scale, int
 }
 
 // What DynamicLossScaler.update_scale (loss_scaler.py:158-182) makes of the state, formed by one whole wave (every lane
-// the same, except that lanes 0 to 3 raise one beta each).  `operator_calls`: how many times the step that was just queued called the native operator in the
-// reference's terms (its tensors; 0 when every chunk took the torch formula): a clean step moves the operator's own step /
-// beta^t state accordingly (Adam_Optimizer::IncrementStep, cpu_adam.h:143-162), a skipped step never reaches the operator.
+// the same, except that lanes 0 to 3 raise one beta each; the shuffles that hand the powers round need all 64 of them).
+// `operator_calls`: how many times the step that was just queued called the native operator in the reference's terms (its
+// tensors; 0 when every chunk took the torch formula): a clean step moves the operator's own step / beta^t state accordingly
+// (Adam_Optimizer::IncrementStep, cpu_adam.h:143-162), a skipped step never reaches the operator.
 __device__ __forceinline__ ps_step_state scaler_updated(ps_step_state s, bool overflow, int64_t operator_calls)
 {
     if (overflow) {
@@ -1038,10 +1041,12 @@ __global__ void __launch_bounds__(64)
 // three kernels they take three launches whatever the list's length, and the GPU waits for each.  The probe's flag crosses
 // the waves through LDS; waves 0 to 14 then go over the tiles, the last one meanwhile forms the next state, which
 // replaces the old one when nobody reads that any more.
-// Bound by launching: the host needs 17 us for a step in one launch, 21 us for one in three.  On the device one CU's
-// arithmetic takes 4 us + 0.12 us a tile (12.9 us for 75 tiles), the three kernels 10.6 us and the gaps between them: a
-// step waited for takes 27 / 31 / 33 / 36 us at 30 / 60 / 75 / 90 tiles, in three launches 32 us; among others 17.2 us at
-// all of them against 21.5.  The line lies where both together are about even.
+// Bound by the host and one launch up to about 80 tiles, by one CU's arithmetic (4 us + 0.12 us a tile, 12.8 us for 75
+// tiles) from there on; the three kernels take 10.6 us and the gaps between them.  FP16Adam.step(), in one launch / in three:
+// waited for, at 1 / 30 / 60 / 75 / 81 / 90 / 120 tiles 25.4 / 25.4 / 28.7 / 30.5 / 30.8 / 33.9 / 36.2 us against 29.8 to
+// 30.7 at all of them; among other steps 14.5 / 13.9 / 13.7 / 13.8 / 13.8 / 16.7 / 19.0 against 18.5 to 20.7.  The line is
+// the last length at which a step that is waited for is no slower (by more than the 0.4 us that runs differ by) and the
+// kernel still hides behind the host's work for the next step.
 constexpr int kSmallWaves = 16;
 constexpr unsigned kSmallTiles = PS_SMALL_TILES;
 struct SmallStep {

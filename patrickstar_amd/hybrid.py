@@ -1,14 +1,17 @@
-"""Host-resident chunk positions: streamed through HBM staging slots by the C ABI.
+"""Host-resident chunk positions, handed to the C ABI together with HBM staging slots.
 
 The reference's hybrid Adam keeps some chunks' optimizer state in host memory and
 updates them with the CPU operator (``patrickstar/ops/fp16_cpu_adam.py:415-428``,
 ``patrickstar/ops/chunk_io_buff.py:214-255``).  On MI355X those chunks are instead
 updated by the same fused kernel as resident chunks: up to 8 of them where they
-are, over the link, more of them copied into HBM staging by ``hipMemcpyAsync`` on
-side streams and copied back, all ordered by events inside
-``ps_adam_step_hybrid``; the Python side only owns the staging buffers.  A position's fp16 payload may stay in HBM (where forward and
-backward use it, as in the reference); it is then updated in place and only the
-optimizer state (12 B/element each way) crosses the link.
+are, over the link, if that is no slower (the library decides it for every step
+from the two lists); otherwise they are copied into HBM staging by
+``hipMemcpyAsync`` on side streams and copied back, all ordered by events inside
+``ps_adam_step_hybrid``.  The Python side owns the staging buffers, and keeps them
+also where every step so far was made in place.  A position's fp16 payload may
+stay in HBM (where forward and backward use it, as in the reference); it is then
+updated in place and only the optimizer state (12 B/element each way) crosses the
+link.
 """
 import torch
 
@@ -17,7 +20,7 @@ from . import _lib
 
 class HostChunkStreamer:
     def __init__(self, client, host_positions, n_slots=3, step_indices=None, used=None):
-        """``step_indices``: which of ``host_positions`` ``step()`` streams (default: all of them); the gradient probe
+        """``step_indices``: which of ``host_positions`` ``step()`` updates (default: all of them); the gradient probe
         always covers every position.  ``used``: per position, the elements in front of its zero padding (only those
         cross the link); default: whole chunks."""
         self.client = client
@@ -69,7 +72,7 @@ class HostChunkStreamer:
 
     def step(self, opt_id, step_no, lr, beta1, beta2, eps, weight_decay, loss_scale, resident, n_resident, calls=None,
              scaler=None, used=None):
-        """One optimizer step over the resident chunk array AND the host-resident chunks.
+        """One optimizer step over the resident chunk array AND the host-resident chunks (in place or through the slots).
         ``calls``: the step's ps_call_pattern over both lists (resident positions counted first).
         ``scaler`` (a device-resident DynamicLossScaler) selects the device-gated form.
         ``used``: size_t array over the resident positions followed by the streamed ones (None: whole chunks)."""
