@@ -1746,9 +1746,9 @@ int ps_grads_to_chunks(const ps_grad_copy* copies, int n_copies, ps_step_state* 
         if (in_batch == 0) continue;
         const dim3 grid((unsigned)blocks), block(kCopyBlock);
         if (in_batch == 1)
-            hipLaunchKernelGGL(grads_to_chunks_kernel<true>, grid, block, 0, s, b, d_state);
+            hipLaunchKernelGGL(grad_to_chunk_kernel, grid, block, 0, s, b.src[0], b.dst[0], b.numel_half[0], d_state);
         else
-            hipLaunchKernelGGL(grads_to_chunks_kernel<false>, grid, block, 0, s, b, d_state);
+            hipLaunchKernelGGL(grads_to_chunks_kernel, grid, block, 0, s, b, d_state);
         PS_HIP(hipGetLastError());
     }
     return 0;

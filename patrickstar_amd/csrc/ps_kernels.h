@@ -748,20 +748,25 @@ __device__ __forceinline__ uint32_t copy_span(const void* src, uint16_t* dst, si
     return hit;
 }
 
-// ONE: the launch has one gradient, so there is nothing to look up.
-template <bool ONE>
+__device__ __forceinline__ void copy_and_probe(const void* src, uint16_t* dst, uint64_t numel_half, uint32_t block, ps_step_state* st)
+{
+    const uint32_t hit = (numel_half & 1u) ? copy_span<true>(src, dst, numel_half >> 1, block) : copy_span<false>(src, dst, numel_half >> 1, block);
+    if (st != nullptr) block_flag_commit<kCopyBlock>(hit, &st->overflow);
+}
+
 __global__ void __launch_bounds__(kCopyBlock) grads_to_chunks_kernel(GradBatch b, ps_step_state* st)
 {
-    int k = 0;
-    uint32_t block = blockIdx.x;
-    if (!ONE) {
-        const uint64_t begun = __ballot(b.first_block[threadIdx.x & 63] <= blockIdx.x);
-        k = __builtin_amdgcn_readfirstlane(__popcll(begun) - 1);  // gradient 0 begins at workgroup 0: never -1
-        block -= b.first_block[k];
-    }
-    const uint64_t nh = b.numel_half[k];
-    const uint32_t hit = (nh & 1u) ? copy_span<true>(b.src[k], b.dst[k], nh >> 1, block) : copy_span<false>(b.src[k], b.dst[k], nh >> 1, block);
-    if (st != nullptr) block_flag_commit<kCopyBlock>(hit, &st->overflow);
+    const uint64_t begun = __ballot(b.first_block[threadIdx.x & 63] <= blockIdx.x);
+    const int k = __builtin_amdgcn_readfirstlane(__popcll(begun) - 1);  // gradient 0 begins at workgroup 0: never -1
+    copy_and_probe(b.src[k], b.dst[k], b.numel_half[k], blockIdx.x - b.first_block[k], st);
+}
+
+// A gradient that has the launch to itself: nothing to look up, and arguments of 32 bytes instead of 1.8 KiB (with
+// those a launch back to back takes 4.5 us instead of 3.9 up to 1 Mi elements, 6.7 instead of 6.0 for 9 Mi in fp16).
+__global__ void __launch_bounds__(kCopyBlock)
+    grad_to_chunk_kernel(const void* src, uint16_t* dst, uint64_t numel_half, ps_step_state* st)
+{
+    copy_and_probe(src, dst, numel_half, blockIdx.x, st);
 }
 
 // ------------------------------------------------ device-resident step state
