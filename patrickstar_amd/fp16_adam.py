@@ -686,7 +686,7 @@ class FP16Adam(torch.optim.Optimizer):
         # which parameters are trainable is looked at every step, as the reference does (fp16_cpu_adam.py:569-571):
         # freezing or unfreezing a parameter between steps makes a new plan (descriptor tables, call pattern, and
         # whether every tensor can still share one step number)
-        if self._plan is None or tuple(p.requires_grad for p in self.param_groups[0]["params"]) != self._trainable_seen:
+        if self._plan is None or tuple([p.requires_grad for p in self.param_groups[0]["params"]]) != self._trainable_seen:
             self._make_plan()
         plan = self._plan
         if plan["kind"] == "empty":
