@@ -25,6 +25,30 @@ from .chunk_layout import (
     register_param,
 )
 
+# Where the three fp32 lists lie against one another.  A pass reads and writes the same element of all three at the same
+# time, and distances that are multiples of 128 MiB (which lists of power-of-two chunks back to back have) put those three
+# on the same memory banks.  64 Mi elements a list, distance over 256 MiB: 0 to 32 KiB 5.71-5.77 TB/s, 64 KiB 5.89, 256 KiB
+# 6.08, 1 MiB 6.27-6.29, 4 MiB 6.13-6.19, 6 to 17 MiB 6.26-6.35, 64 MiB 6.23, 128 MiB 5.84, 132 to 252 MiB 6.26-6.34; 9 MiB:
+# 6.28-6.31.  Lists that are allocations of their own lie as the allocator has it: 5.72 to 6.36 TB/s for the same list, by
+# what was allocated before.  At 9 MiB over a multiple of 64 MiB lists of 32 Mi to 256 Mi elements ran at 6.19-6.35 TB/s in
+# every process, against 5.73-6.35 on their own.  Up to 16 Mi elements the lists stay in the memory-side cache (8.3-8.7 TB/s
+# however they lie); from 384 Mi elements on lists of their own are as fast (6.28-6.35; 1.5 Gi elements in one allocation at
+# 8 MiB 6.10).
+ONE_ALLOCATION_BYTES = (80 << 20, 1 << 30)  # shortest and longest fp32 list that shares one
+LIST_PERIOD, LIST_CLEARANCE = 64 << 20, 9 << 20
+
+
+def list_distance(nbytes):
+    """How far apart to start the fp32 lists of ``nbytes`` bytes each: the least distance that is neither itself nor doubled
+    nearly a multiple of 128 MiB."""
+    past = nbytes % LIST_PERIOD
+    if past < LIST_CLEARANCE:
+        return nbytes - past + LIST_CLEARANCE
+    if past > LIST_PERIOD - LIST_CLEARANCE:
+        return nbytes - past + LIST_PERIOD + LIST_CLEARANCE
+    return nbytes
+
+
 class ChunkPosition:
     """The four chunks that sit at the same place of the four lists."""
 
@@ -76,7 +100,8 @@ class PatrickStarClient:
         # True: such a position's fp16 payload is in pinned host memory as well (the whole position is streamed);
         # False: it stays in HBM, where forward and backward use it (the only form a registered module can have)
         self.host_keeps_fp16 = True
-        self._slabs = []  # the allocations HBM-resident payloads are views of
+        self._slabs = []  # the lists' memory that HBM-resident payloads are views of
+        self._reserved = {}  # (state list, fp16 chunk id) -> (slab, element) for the state chunk of that position
         # called with (position index among fp16 chunks) -> True to keep that position in host memory
         self.host_chunk_policy: Optional[Callable[[int], bool]] = None
         default_opts = {"with_mem_saving_comm": False, "with_mem_cache": False, "with_async_move": False}
@@ -294,8 +319,8 @@ class PatrickStarClient:
 
         HBM-resident chunks of one list are carved out of ONE allocation per call (a slab): a few large
         allocations are backed by large physical fragments, which the streaming kernels need when few waves
-        are in flight (measured: 6.30 TB/s from slabs vs 6.01 TB/s from one allocation per chunk; skewing the
-        slabs' start addresses against each other by a few KiB made no measurable difference).
+        are in flight (measured: 6.30 TB/s from slabs vs 6.01 TB/s from one allocation per chunk).  The slabs of the
+        three fp32 lists, if they are long, are parts of one allocation and start ``list_distance`` apart.
         Positions selected by the host-chunk policy get their own pinned host allocations instead.
         """
         ids16 = self.chunk_tensor_index.chunk_type_to_chunk_id_list_map.get(ChunkType.PARAM_FP16, [])
@@ -322,12 +347,48 @@ class PatrickStarClient:
             def stride(c):
                 return -(-c.capacity // 512) * 512
 
-            slab = torch.zeros(sum(stride(c) for c in chunks), dtype=chunks[0].data_type, device=self.device)
+            if chunk_type in (ChunkType.MOMENTUM, ChunkType.VARIANCE):
+                chunks = self._take_reserved(chunk_type, chunks)
+                if not chunks:
+                    continue
+            n = sum(stride(c) for c in chunks)
+            positions = [self._fp16_chunk_of_position(c.chunk_id) for c in chunks] if chunk_type == ChunkType.PARAM_FP32 else []
+            rooms = self._fp32_lists(n) if positions and None not in positions else None
+            slab = rooms[0] if rooms else torch.zeros(n, dtype=chunks[0].data_type, device=self.device)
             self._slabs.append(slab)
             cursor = 0
-            for chunk in chunks:
+            for k, chunk in enumerate(chunks):
                 chunk.payload = slab.narrow(0, cursor, chunk.capacity)
+                if rooms:
+                    self._reserved[(ChunkType.MOMENTUM, positions[k])] = (rooms[1], cursor)
+                    self._reserved[(ChunkType.VARIANCE, positions[k])] = (rooms[2], cursor)
                 cursor += stride(chunk)
+
+    def _fp32_lists(self, n):
+        """Three zero-filled slabs of ``n`` floats, ``list_distance`` apart in one allocation: the fp32 parameters', and
+        room for the momentum and variance chunks of the same positions.  None: not worth it, or no memory for all three."""
+        if not ONE_ALLOCATION_BYTES[0] <= 4 * n <= ONE_ALLOCATION_BYTES[1]:
+            return None
+        distance = list_distance(4 * n) // 4
+        try:
+            whole = torch.zeros(2 * distance + n, dtype=torch.float, device=self.device)
+        except torch.OutOfMemoryError:
+            return None
+        # tensors in their own right, not views of one another, so that a payload's base is its own list
+        return [torch.empty(0, dtype=torch.float, device=self.device).set_(whole.untyped_storage(), k * distance, (n,)) for k in range(3)]
+
+    def _take_reserved(self, chunk_type, chunks):
+        """Give state chunks the room that was reserved beside their position's fp32 chunk; returns those that have none."""
+        rest = []
+        for chunk in chunks:
+            slab, at = self._reserved.pop((chunk_type, self._fp16_chunk_of_position(chunk.chunk_id)), (None, 0))
+            if slab is None:
+                rest.append(chunk)
+                continue
+            if not any(slab is known for known in self._slabs):
+                self._slabs.append(slab)
+            chunk.payload = slab.narrow(0, at, chunk.capacity)
+        return rest
 
     def chunk_ids_generator(self, chunk_type):
         for cid in self.chunk_tensor_index.chunk_type_to_chunk_id_list_map.get(chunk_type, []):
