@@ -338,20 +338,23 @@ void launch_small_step(int arith, const ChunkBatch& b, const SmallStep& a, const
         launch_small_step_arith<PS_ARITH_OPERATOR>(b, a, ga, fc, d_state, s);
 }
 
-template <int ARITH, int WD>
-void launch_tensors_wd(const TensorBatch& b, dim3 grid, const StepConsts& c, hipStream_t s)
+template <typename LIST>
+constexpr unsigned kListLds = std::is_same<LIST, NearBatch>::value ? kNearLdsBytes : kLdsBytes;
+
+template <int ARITH, int WD, typename LIST>
+void launch_tensors_wd(const LIST& b, dim3 grid, const StepConsts& c, hipStream_t s)
 {
     dim3 block(kBlock);
     if (c.unscale == UNSCALE_MUL)
-        hipLaunchKernelGGL((adam_tensors_kernel<ARITH, WD, UNSCALE_MUL>), grid, block, kLdsBytes, s, b, c);
+        hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_MUL>), grid, block, kListLds<LIST>, s, b, c);
     else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
-        hipLaunchKernelGGL((adam_tensors_kernel<ARITH, WD, UNSCALE_DIV>), grid, block, kLdsBytes, s, b, c);
+        hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_DIV>), grid, block, kListLds<LIST>, s, b, c);
     else
-        hipLaunchKernelGGL((adam_tensors_kernel<ARITH, WD, UNSCALE_NONE>), grid, block, kLdsBytes, s, b, c);
+        hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_NONE>), grid, block, kListLds<LIST>, s, b, c);
 }
 
-template <int ARITH>
-void launch_tensors_arith(const TensorBatch& b, dim3 grid, const StepConsts& c, hipStream_t s)
+template <int ARITH, typename LIST>
+void launch_tensors_arith(const LIST& b, dim3 grid, const StepConsts& c, hipStream_t s)
 {
     if (c.wd_mode == WD_DECOUPLED)
         launch_tensors_wd<ARITH, WD_DECOUPLED>(b, grid, c, s);
@@ -361,18 +364,18 @@ void launch_tensors_arith(const TensorBatch& b, dim3 grid, const StepConsts& c, 
         launch_tensors_wd<ARITH, WD_NONE>(b, grid, c, s);
 }
 
-template <int ARITH>
-void launch_tensors_gated_arith(const TensorBatch& b, dim3 grid, const GatedArgs& ga,
+template <int ARITH, typename LIST>
+void launch_tensors_gated_arith(const LIST& b, dim3 grid, const GatedArgs& ga,
                                 const ps_step_state* d_state, hipStream_t s)
 {
     dim3 block(kBlock);
     const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
     if (decay && ga.adamw)
-        hipLaunchKernelGGL((adam_tensors_gated_kernel<ARITH, WD_DECOUPLED>), grid, block, kLdsBytes, s, b, ga, d_state);
+        hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_DECOUPLED>), grid, block, kListLds<LIST>, s, b, ga, d_state);
     else if (decay)
-        hipLaunchKernelGGL((adam_tensors_gated_kernel<ARITH, WD_L2>), grid, block, kLdsBytes, s, b, ga, d_state);
+        hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_L2>), grid, block, kListLds<LIST>, s, b, ga, d_state);
     else
-        hipLaunchKernelGGL((adam_tensors_gated_kernel<ARITH, WD_NONE>), grid, block, kLdsBytes, s, b, ga, d_state);
+        hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_NONE>), grid, block, kListLds<LIST>, s, b, ga, d_state);
 }
 
 // The Python numbers of one step as they cross the boundary.
@@ -945,15 +948,98 @@ TensorItem tensor_item(const ps_chunk* tensors, const size_t* numels, int i, boo
 // max_classes > 0: a launch takes at most that many distinct classes; its tensors' numbers are then 0, 1, ... in the
 // order of their first tensor in the batch and classes.of[] says which of the items' classes each one is.
 struct BatchClasses {
-    int of[kTensorBatch];
+    int of[kNearBatch];
     int n;
 };
 
+// Number of a tensor's class in the launch that is being filled; -1: the launch holds as many classes as it may.
+int class_in_batch(BatchClasses& bc, int cls, int max_classes)
+{
+    if (max_classes <= 0) return cls;
+    for (int j = 0; j < bc.n; ++j)
+        if (bc.of[j] == cls) return j;
+    if (bc.n == max_classes) return -1;
+    bc.of[bc.n] = cls;
+    return bc.n++;
+}
+
+// Whether all of the items lie at the same place of their four lists (NearBatch): one distance from the fp32 parameter to
+// momentum and to variance, and the fp16 slot half as far along as the parameter.  `lists`: where offset 0 lies.
+bool near_lists(const std::vector<TensorItem>& items, const ps_chunk* tensors, ps_chunk* lists)
+{
+    const ps_chunk* low = nullptr;
+    for (const TensorItem& it : items)
+        if (!low || tensors[it.index].param_fp32 < low->param_fp32) low = &tensors[it.index];
+    if (!low) return false;
+    auto addr = [](const void* a) { return reinterpret_cast<uintptr_t>(a); };
+    if ((addr(low->param_fp32) | addr(low->exp_avg) | addr(low->exp_avg_sq)) & 3u || addr(low->param_fp16) & 1u) return false;
+    for (const TensorItem& it : items) {
+        const ps_chunk& t = tensors[it.index];
+        const uintptr_t d = addr(t.param_fp32) - addr(low->param_fp32);
+        if (d & 3u || d / 4 + it.head > kNumelMask || it.body > 0xFFFFFFFFu) return false;
+        if (addr(t.exp_avg) - addr(low->exp_avg) != d || addr(t.exp_avg_sq) - addr(low->exp_avg_sq) != d ||
+            addr(t.param_fp16) - addr(low->param_fp16) != d / 2)
+            return false;
+    }
+    *lists = *low;
+    return true;
+}
+
+constexpr size_t kMaxNearElements = (size_t)256 << 20;  // of a list that takes NearBatch: see there
+
+// The same for tensors of near_lists: a launch takes up to 208 of them, of up to 8 different lengths (within a tenth, and all
+// of up to 32 tiles together: a workgroup that finds nothing to do costs 0.2 ns).
+template <typename F>
+int for_each_near_batch(const std::vector<TensorItem>& items, const ps_chunk* tensors, const ps_chunk& lists, int first_tensor,
+                        int max_classes, F launch)
+{
+    constexpr size_t kShortTensorTiles = 32;
+    NearBatch b;
+    BatchClasses bc;
+    size_t next = 0;
+    while (next < items.size()) {
+        memset(&b, 0, sizeof(b));
+        memset(&bc, 0, sizeof(bc));
+        b.lists = lists;
+        b.first_call = -1;
+        for (uint32_t& s : b.start) s = 0xFFFFFFFFu;
+        size_t groups = 0;
+        int in_batch = 0, segments = 0;
+        for (; next < items.size() && in_batch < kNearBatch; ++in_batch, ++next) {
+            const TensorItem& it = items[next];
+            const uint32_t width = segments ? b.seg[segments - 1].width : 0;
+            const bool opens = !segments || !(it.tiles * 10 >= (size_t)width * 9 || width <= kShortTensorTiles);
+            const size_t wide = opens ? std::max<size_t>(it.tiles, 2) : width;
+            if ((opens && segments == kSegments) || groups + wide > kMaxGridX) break;
+            const int cls = class_in_batch(bc, it.cls, max_classes);
+            if (cls < 0) break;
+            if (opens) {
+                const uint32_t magic = (uint32_t)((((uint64_t)1 << 32) + wide - 1) / wide);
+                if (segments) b.start[segments - 1] = (uint32_t)groups;
+                b.seg[segments++] = Segment{(uint32_t)groups, (uint32_t)in_batch, (uint32_t)wide, magic};
+            }
+            groups += wide;
+            const uint64_t at = (uint64_t)(tensors[it.index].param_fp32 - lists.param_fp32) + it.head;
+            b.at[in_batch] = at | ((uint64_t)cls << 40) | ((uint64_t)it.head << 56);
+            b.numel[in_batch] = (uint32_t)it.body;
+            if (it.index == first_tensor) b.first_call = in_batch;
+        }
+        launch(b, dim3((unsigned)groups), bc);
+        PS_HIP(hipGetLastError());
+    }
+    return 0;
+}
+
 template <typename F>
 int for_each_tensor_batch(std::vector<TensorItem>& items, const ps_chunk* tensors, int first_tensor, int max_classes,
-                          F launch)
+                          F launch, bool grad_f32 = false)
 {
     std::stable_sort(items.begin(), items.end(), [](const TensorItem& a, const TensorItem& b) { return a.tiles > b.tiles; });
+    size_t elements = 0;
+    for (const TensorItem& it : items) elements += it.head + it.body;
+    ps_chunk lists;
+    if (!grad_f32 && elements <= kMaxNearElements && near_lists(items, tensors, &lists))
+        return for_each_near_batch(items, tensors, lists, first_tensor, max_classes, launch);
     constexpr size_t kShortTensorTiles = 256;
     TensorBatch b;
     BatchClasses bc;
@@ -967,16 +1053,8 @@ int for_each_tensor_batch(std::vector<TensorItem>& items, const ps_chunk* tensor
         while (next < items.size() && in_batch < kTensorBatch &&
                (items[next].tiles * 10 >= widest * 9 || widest <= kShortTensorTiles)) {
             const TensorItem& it = items[next];
-            int cls = it.cls;
-            if (max_classes > 0) {
-                int j = 0;
-                while (j < bc.n && bc.of[j] != it.cls) ++j;
-                if (j == bc.n) {
-                    if (bc.n == max_classes) break;  // the next launch starts with this tensor
-                    bc.of[bc.n++] = it.cls;
-                }
-                cls = j;
-            }
+            const int cls = class_in_batch(bc, it.cls, max_classes);
+            if (cls < 0) break;  // the next launch starts with this tensor
             ps_chunk t = tensors[it.index];
             t.param_fp32 += it.head;
             t.exp_avg += it.head;
@@ -1002,19 +1080,22 @@ int wd_mode_of(int arith, double wd, bool adamw)
     return decay ? (adamw ? WD_DECOUPLED : WD_L2) : WD_NONE;
 }
 
-template <int ARITH, int WD>
-void launch_tensors_planned_wd(const TensorBatch& b, dim3 grid, bool grad_f32,
+template <int ARITH, int WD, typename LIST>
+void launch_tensors_planned_wd(const LIST& b, dim3 grid, bool grad_f32,
                                const PlannedConsts* d_consts, const ps_step_state* d_state, hipStream_t s)
 {
     dim3 block(kBlock);
-    if (grad_f32)
-        hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
-    else
-        hipLaunchKernelGGL((adam_tensors_planned_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
+    if constexpr (std::is_same<LIST, TensorBatch>::value) {
+        if (grad_f32) {
+            hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((adam_tensors_planned_kernel<LIST, ARITH, WD>), grid, block, kListLds<LIST>, s, b, d_consts, d_state);
 }
 
-template <int ARITH>
-void launch_tensors_planned_arith(const TensorBatch& b, dim3 grid, int wd_mode, bool grad_f32,
+template <int ARITH, typename LIST>
+void launch_tensors_planned_arith(const LIST& b, dim3 grid, int wd_mode, bool grad_f32,
                                   const PlannedConsts* d_consts, const ps_step_state* d_state, hipStream_t s)
 {
     if (wd_mode == WD_DECOUPLED)
@@ -1066,19 +1147,22 @@ int key_arith(int key) { return key & 1; }
 bool key_grad_f32(int key) { return (key & 2) != 0; }
 static_assert(PS_ARITH_OPERATOR == 0 && PS_ARITH_TORCH == 1, "class_key keeps the arithmetic in one bit");
 
-template <int ARITH, int WD, int UNS>
-void launch_tensors_each_uns(const TensorBatch& b, dim3 grid, const ConstsBatch& cb, bool grad_f32,
+template <int ARITH, int WD, int UNS, typename LIST>
+void launch_tensors_each_uns(const LIST& b, dim3 grid, const ConstsBatch& cb, bool grad_f32,
                              hipStream_t s)
 {
     dim3 block(kBlock);
-    if (grad_f32)
-        hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
-    else
-        hipLaunchKernelGGL((adam_tensors_each_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
+    if constexpr (std::is_same<LIST, TensorBatch>::value) {
+        if (grad_f32) {
+            hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((adam_tensors_each_kernel<LIST, ARITH, WD, UNS>), grid, block, kListLds<LIST>, s, b, cb);
 }
 
-template <int ARITH, int WD>
-void launch_tensors_each_wd(const TensorBatch& b, dim3 grid, const ConstsBatch& cb,
+template <int ARITH, int WD, typename LIST>
+void launch_tensors_each_wd(const LIST& b, dim3 grid, const ConstsBatch& cb,
                             const Flavour& f, hipStream_t s)
 {
     if (f.unscale == UNSCALE_MUL)
@@ -1089,8 +1173,8 @@ void launch_tensors_each_wd(const TensorBatch& b, dim3 grid, const ConstsBatch& 
         launch_tensors_each_uns<ARITH, WD, UNSCALE_NONE>(b, grid, cb, f.grad_f32, s);
 }
 
-template <int ARITH>
-void launch_tensors_each_arith(const TensorBatch& b, dim3 grid, const ConstsBatch& cb,
+template <int ARITH, typename LIST>
+void launch_tensors_each_arith(const LIST& b, dim3 grid, const ConstsBatch& cb,
                                const Flavour& f, hipStream_t s)
 {
     if (f.wd_mode == WD_DECOUPLED)
@@ -1150,7 +1234,7 @@ int ps_adam_step_tensors(int optimizer_id, size_t step, double lr, double beta1,
     }
     for (int i = 0; i < n_tensors; ++i)
         if (numels[i] != 0) items.push_back(tensor_item(tensors, numels, i));
-    return for_each_tensor_batch(items, tensors, first_tensor, 0, [&](const TensorBatch& b, dim3 grid, const BatchClasses&) {
+    return for_each_tensor_batch(items, tensors, first_tensor, 0, [&](const auto& b, dim3 grid, const BatchClasses&) {
         if (d_state == nullptr) {
             if (arith == PS_ARITH_TORCH)
                 launch_tensors_arith<PS_ARITH_TORCH>(b, grid, c, s);
@@ -1238,7 +1322,7 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     }
                 const Flavour& f = flavours[j];
                 int rc = for_each_tensor_batch(items, tensors, -1, kLaunchClasses,
-                                               [&](const TensorBatch& b, dim3 grid, const BatchClasses& bc) {
+                                               [&](const auto& b, dim3 grid, const BatchClasses& bc) {
                     ConstsBatch cb;
                     memset(&cb, 0, sizeof(cb));
                     for (int q = 0; q < bc.n; ++q) cb.c[q] = consts[bc.of[q]];
@@ -1246,7 +1330,7 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                         launch_tensors_each_arith<PS_ARITH_TORCH>(b, grid, cb, f, s);
                     else
                         launch_tensors_each_arith<PS_ARITH_OPERATOR>(b, grid, cb, f, s);
-                });
+                }, f.grad_f32);
                 if (rc) return rc;
             }
             return 0;
@@ -1333,12 +1417,12 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     }
                     if (items.empty()) continue;
                     int rc = for_each_tensor_batch(items, tensors, -1, 0,
-                                                   [&](const TensorBatch& b, dim3 grid, const BatchClasses&) {
+                                                   [&](const auto& b, dim3 grid, const BatchClasses&) {
                         if (key_arith(key) == PS_ARITH_TORCH)
                             launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, wd_mode, grad_f32, table + window, d_state, s);
                         else
                             launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, wd_mode, grad_f32, table + window, d_state, s);
-                    });
+                    }, grad_f32);
                     if (rc) return rc;
                 }
             }

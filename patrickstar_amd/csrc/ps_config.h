@@ -17,6 +17,9 @@
 #ifndef PS_LDS_KB
 #define PS_LDS_KB 17  // KiB of (unused) dynamic LDS requested per workgroup: caps resident workgroups per CU at floor(160 / PS_LDS_KB) = 9
 #endif
+#ifndef PS_NEAR_LDS_KB
+#define PS_NEAR_LDS_KB 14  // the same for the one-launch tensor lists: 11 workgroups per CU (their waves take longer to their first load)
+#endif
 #ifndef PS_STREAMING
 #define PS_STREAMING 0  // bit 0: non-temporal loads, bit 1: non-temporal stores of chunk payloads (both slower on MI355X)
 #endif

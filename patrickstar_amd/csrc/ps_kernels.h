@@ -162,7 +162,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     StateView sv = view_state(st);  // asked for at once, as in tile_source
     asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
     if (__builtin_expect(sv.overflow, 0)) {
-        if (restore_leader()) restore_tiles(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
+        if (restore_leader(blockIdx.x)) restore_tiles(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
         return;
     }
     if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
@@ -222,6 +222,8 @@ struct TensorView {
     TileSource t;
     size_t numel;
     int head, cls;
+    bool first;      // the tensor is the step's first operator call
+    uint32_t x;      // this workgroup's number among those of its tensor
     ptrdiff_t tile;  // this workgroup's; -1: the elements in front of the tile grid
 };
 __device__ __forceinline__ TensorView tensor_view(const TensorBatch& b)
@@ -231,7 +233,70 @@ __device__ __forceinline__ TensorView tensor_view(const TensorBatch& b)
     w.numel = w.t.numel & kNumelMask;
     w.cls = (int)((w.t.numel >> 40) & 0xFFFFu);
     w.head = (int)(w.t.numel >> 56);
-    w.tile = (ptrdiff_t)blockIdx.x - (w.head ? 1 : 0);
+    w.first = (int)blockIdx.y == b.first_call;
+    w.x = blockIdx.x;
+    w.tile = (ptrdiff_t)w.x - (w.head ? 1 : 0);
+    return w;
+}
+
+// Tensors that lie at the same place of their four lists (the layout that PatrickStarClient makes: momentum and variance
+// mirror the parameters' chunks, and so do the lists' allocations): what differs from tensor to tensor is one offset and one
+// length, 12 bytes, and one launch takes up to 208 of them, of any lengths.
+//
+// The grid is one-dimensional.  Its workgroups are divided among up to 8 segments, tensors of nearly the same length
+// each; inside a segment the tensor is a division by the segment's width away (a multiplication by its reciprocal).  A wave
+// reaches its first data load after three rounds of scalar loads (segments, segment, tensor) and some 50 scalar
+// instructions, where TensorBatch needs one round, so 11 workgroups per CU instead of 9 keep as many loads in flight.
+//
+// What that buys is the ends of launches, 4 to 9 us each.  Device time in several launches (TensorBatch) / in one:
+// BERT-base, 199 tensors 517 / 500 us host-decided, 528 / 504 device-decided with a rate per layer; its upper half, 100
+// tensors 211 / 203 and 218 / 207; 12 layers of hidden size 64 14.6 / 5.8 and 20.4 / 10.6; 11 M elements with no two tensors
+// at the same phase 56.6 / 43.1.  With the cap of 9: BERT-base 508 and 520, with 12 533.  Longer lists gain less than the
+// longer way to the first load costs them: 335 M elements 1558 / 1572 host-decided, 1557 M (GPT-2 XL, 580 tensors, three launches)
+// 7226 / 7414, so lists of more than 256 Mi elements keep TensorBatch.
+constexpr int kNearBatch = 208;
+constexpr int kSegments = 8;
+struct Segment {
+    uint32_t start, first;  // workgroup and tensor it begins with
+    uint32_t width, magic;  // workgroups per tensor (2 at least); 2^32 / width, rounded up
+};
+struct NearBatch {
+    uint32_t start[kSegments];      // of the second segment, the third ...; behind the last one: 0xFFFFFFFF
+    Segment seg[kSegments];
+    ps_chunk lists;                 // where offset 0 lies in the four lists
+    uint64_t at[kNearBatch];        // low 40 bits: offset of the tile grid's origin; then class and head as in TensorBatch::lengths
+    uint32_t numel[kNearBatch];     // elements from the origin on
+    int first_call;
+};
+__device__ __forceinline__ TensorView tensor_view(const NearBatch& b)
+{
+    const uint32_t wg = blockIdx.x;
+    uint32_t k = 0;
+#pragma unroll
+    for (int j = 0; j < kSegments - 1; ++j)  // k += wg >= start[j]
+        asm("s_cmp_ge_u32 %1, %2\n\ts_addc_u32 %0, %0, 0" : "+s"(k) : "s"(wg), "s"(b.start[j]) : "scc");
+    Segment s = b.seg[k];
+    float *p32 = b.lists.param_fp32, *m32 = b.lists.exp_avg, *v32 = b.lists.exp_avg_sq;
+    uint16_t* h16 = b.lists.param_fp16;
+    int first_call = b.first_call;
+    asm volatile("" : "+s"(s.start), "+s"(s.first), "+s"(s.width), "+s"(s.magic), "+s"(p32), "+s"(m32), "+s"(v32), "+s"(h16), "+s"(first_call));
+    const uint32_t r = wg - s.start;
+    uint32_t q = __umulhi(r, s.magic);  // r / width, or one more: then the remainder is negative
+    if ((int32_t)(r - q * s.width) < 0) q -= 1;
+    const uint32_t index = s.first + q;
+    uint64_t at = b.at[index];
+    uint32_t numel = b.numel[index];
+    asm volatile("" : "+s"(at), "+s"(numel));
+    const uint64_t off = at & kNumelMask;
+    const uint32_t hi = (uint32_t)(at >> 32);
+    TensorView w;
+    w.first = (int)index == first_call;
+    w.numel = numel;
+    w.t = TileSource{p32 + off, m32 + off, v32 + off, h16 + off, numel};
+    w.cls = (int)((hi >> 8) & 0xFFFFu);
+    w.head = (int)(hi >> 24);
+    w.x = r - q * s.width;
+    w.tile = (int32_t)w.x - (w.head != 0);
     return w;
 }
 
@@ -253,10 +318,37 @@ __device__ __forceinline__ void adam_head(const StepConsts& c, const ps_chunk& t
     }
 }
 
+// One tile of a tensor, which is one operator call: all of its elements take the first call's scalars, or none.  As in
+// adam_tile_late_consts the constants are formed after the tile's loads have been issued.
+template <int ARITH, int WD, int UNS, typename MakeConsts>
+__device__ __forceinline__ void adam_tensor_tile(MakeConsts make_consts, const TensorView& w, bool first)
+{
+    const ps_chunk t = as_chunk(w.t);
+    const size_t base = (size_t)w.tile * kTile;
+    const int access = (uint32_t)w.tile < whole_tiles(w.numel) ? tile_access(t) : TILE_ELEMENTWISE;
+    if (access == TILE_ALIGNED) {
+        LaneTile r;
+        tile_load(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+        const StepConsts c = make_consts();
+        tile_finish<ARITH, WD, UNS>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r, t.param_fp32,
+                                    t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+    } else if (access == TILE_STATE_DWORD_ALIGNED) {
+        LaneTile r;
+        tile_load<true>(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+        const StepConsts c = make_consts();
+        tile_finish<ARITH, WD, UNS, true>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r,
+                                          t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+    } else if (base < w.numel) {  // (the grid is as wide as the longest tensor of the batch)
+        const StepConsts c = make_consts();
+        const size_t end = base + kTile < w.numel ? base + kTile : w.numel;
+        adam_tile_scalar<ARITH, WD, UNS>(c, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base, end, 0, first ? w.numel : 0);
+    }
+}
+
 // fp16 <- RNE(fp32) of this workgroup's tiles (a skipped step).
 __device__ __forceinline__ void restore_tensor_tiles(const ps_chunk& t, const TensorView& w)
 {
-    if (!restore_leader()) return;
+    if (!restore_leader(w.x)) return;
     if (w.tile >= 0) {
         restore_tiles(t.param_fp32, t.param_fp16, (size_t)w.tile * kTile, w.numel);
         return;
@@ -267,28 +359,26 @@ __device__ __forceinline__ void restore_tensor_tiles(const ps_chunk& t, const Te
     for (unsigned u = 1; u < kRestoreTiles; ++u) restore_tile(t.param_fp32, t.param_fp16, (size_t)(u * kRestoreStride - 1) * kTile, w.numel);
 }
 
-template <int ARITH, int WD, int UNS>
+template <typename LIST, int ARITH, int WD, int UNS>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_tensors_kernel(TensorBatch b, StepConsts c)
+    adam_tensors_kernel(LIST b, StepConsts c)
 {
     const TensorView w = tensor_view(b);
-    const bool first = (int)blockIdx.y == b.first_call;  // a tensor is one operator call: all of its tiles, or none
+    const bool first = w.first;  // a tensor is one operator call: all of its tiles, or none
     if (w.tile < 0) {
         adam_head<ARITH, WD, UNS>(c, as_chunk(w.t), w.head, first);
         return;
     }
-    const size_t base = (size_t)w.tile * kTile;
-    if (base >= w.numel) return;  // the grid is as wide as the longest tensor of the batch
-    adam_tile<ARITH, WD, UNS>(c, as_chunk(w.t), base, w.numel, 0, first ? w.numel : 0);
+    adam_tensor_tile<ARITH, WD, UNS>([&]() { return c; }, w, first);
 }
 
-template <int ARITH, int WD>
+template <typename LIST, int ARITH, int WD>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_tensors_gated_kernel(TensorBatch b, GatedArgs ga, const ps_step_state* __restrict__ st)
+    adam_tensors_gated_kernel(LIST b, GatedArgs ga, const ps_step_state* __restrict__ st)
 {
     const TensorView w = tensor_view(b);
     const ps_chunk t = as_chunk(w.t);
-    const bool first = (int)blockIdx.y == b.first_call;
+    const bool first = w.first;
     const size_t base = w.tile < 0 ? 0 : (size_t)w.tile * kTile;
     if (w.tile >= 0 && base >= w.numel) return;
     const StateView sv = view_state(st);
@@ -300,8 +390,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNSCALE_RUNTIME>(gated_consts<ARITH>(ga, sv, first), t, w.head, first);
         return;
     }
-    adam_tile_late_consts<ARITH, WD, UNSCALE_RUNTIME>([&]() { return gated_consts<ARITH>(ga, sv, first); }, t, base,
-                                                      w.numel, 0, first ? w.numel : 0);
+    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME>([&]() { return gated_consts<ARITH>(ga, sv, first); }, w, first);
 }
 
 // A step whose tensors carry their own step numbers and hyper-parameters: calls that come out with the same constants
@@ -315,12 +404,12 @@ constexpr int kLaunchClasses = 24;
 struct ConstsBatch {
     StepConsts c[kLaunchClasses];
 };
-static_assert(sizeof(TensorBatch) + sizeof(ConstsBatch) <= 4096, "kernel arguments of one launch");
+static_assert(sizeof(TensorBatch) + sizeof(ConstsBatch) <= 4096 && sizeof(NearBatch) + sizeof(ConstsBatch) <= 4096, "kernel arguments of one launch");
 
 // No tensor is "the first call" here: a first call that differs is a class of its own.
-template <int ARITH, int WD, int UNS>
+template <typename LIST, int ARITH, int WD, int UNS>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_tensors_each_kernel(TensorBatch b, ConstsBatch cb)
+    adam_tensors_each_kernel(LIST b, ConstsBatch cb)
 {
     const TensorView w = tensor_view(b);
     const ps_chunk t = as_chunk(w.t);
@@ -328,9 +417,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNS>(cb.c[w.cls], t, w.head, false);
         return;
     }
-    const size_t base = (size_t)w.tile * kTile;
-    if (base >= w.numel) return;  // the grid is as wide as the longest tensor of the batch
-    adam_tile_late_consts<ARITH, WD, UNS>([&]() { return cb.c[w.cls]; }, t, base, w.numel, 0, 0);
+    adam_tensor_tile<ARITH, WD, UNS>([&]() { return cb.c[w.cls]; }, w, false);
 }
 
 // The same for tensors whose gradient is binary32 and which have no binary16 copy (PS_TENSOR_GRAD_F32): the
@@ -354,9 +441,9 @@ struct PlannedConsts {
 };
 static_assert(sizeof(PlannedConsts) == 64, "one 64-byte record per class in the caller's workspace");
 
-template <int ARITH, int WD>
+template <typename LIST, int ARITH, int WD>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_tensors_planned_kernel(TensorBatch b, const PlannedConsts* __restrict__ consts,
+    adam_tensors_planned_kernel(LIST b, const PlannedConsts* __restrict__ consts,
                                 const ps_step_state* __restrict__ st)
 {
     const TensorView w = tensor_view(b);
@@ -371,7 +458,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNSCALE_RUNTIME>(consts[w.cls].c, t, w.head, false);
         return;
     }
-    adam_tile_late_consts<ARITH, WD, UNSCALE_RUNTIME>([&]() { return consts[w.cls].c; }, t, base, w.numel, 0, 0);
+    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME>([&]() { return consts[w.cls].c; }, w, false);
 }
 
 // PS_TENSOR_GRAD_F32 tensors of a device-decided step: a flagged step leaves them alone (there is no fp16 copy to

@@ -74,6 +74,7 @@ __device__ __forceinline__ void st_f4_as(float* p, float4v v)
 
 constexpr int kBlock = PS_BLOCK;
 constexpr unsigned kLdsBytes = PS_LDS_KB * 1024u;
+constexpr unsigned kNearLdsBytes = PS_NEAR_LDS_KB * 1024u;
 // Elements per lane per vector step.  8: one 16-byte access of fp16 and two
 // 16-byte accesses per fp32 array.  4: an 8-byte access of fp16 and one
 // 16-byte access per fp32 array.
@@ -415,7 +416,8 @@ __device__ __forceinline__ void restore_tile(const float* __restrict__ p32,
 // apart 579 / 499 / 513 us, 4 tiles 64 / 256 / 2048 apart 494 / 494 / 633.  (A launch of which every workgroup leaves at
 // once takes 441 us; the stand-alone write-back, uncapped, moves the same bytes in 495.)
 constexpr unsigned kRestoreTiles = 4, kRestoreStride = 32;
-__device__ __forceinline__ bool restore_leader() { return blockIdx.x % (kRestoreTiles * kRestoreStride) < kRestoreStride; }
+// x: the workgroup's number among those of its chunk or tensor
+__device__ __forceinline__ bool restore_leader(uint32_t x) { return x % (kRestoreTiles * kRestoreStride) < kRestoreStride; }
 
 // base: the first of the workgroup's tiles
 __device__ __forceinline__ void restore_tiles(const float* __restrict__ p32, uint16_t* __restrict__ h16, size_t base, size_t numel)
