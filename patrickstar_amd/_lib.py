@@ -4,6 +4,7 @@ There is no CPU fallback: if the library has not been built, loading raises.
 """
 import contextlib
 import ctypes
+import functools
 import os
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -178,6 +179,14 @@ def load():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    import torch  # noqa: F401  (the binding uses its libraries)
+
+    try:
+        from . import _binding
+    except ImportError as e:
+        raise HipLibraryMissing(f"{PKG_DIR}/_binding.so: {e}; build it with `python -m patrickstar_amd.build`") from e
+    # adam_op.adam_update's arguments -> return code, or None where the call is not of the ordinary form (csrc/ps_binding.cpp)
+    lib.adam_update = functools.partial(_binding.adam_update, ctypes.cast(lib.ps_adam_update, ctypes.c_void_p).value)
     if lib.ps_abi_version() != PS_ABI_VERSION:
         raise HipLibraryMissing(
             f"{LIB_PATH} has ABI version {lib.ps_abi_version()}, expected {PS_ABI_VERSION}; rebuild it"

@@ -37,6 +37,20 @@ def adam_update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bia
     CPU tensors here, ``fp16_cpu_adam.py:222-225``); ``grads``: float32 or float16, never written;
     ``loss_scale <= 0``: no unscale.
     """
+    rc = _lib.load().adam_update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bias_correction, params, grads,
+                                 exp_avg, exp_avg_sq, loss_scale)
+    if rc is None:
+        rc = _update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bias_correction, params, grads, exp_avg,
+                     exp_avg_sq, loss_scale)
+    if rc:
+        _lib.check(rc, "adam_update")
+    return 0
+
+
+def _update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bias_correction, params, grads, exp_avg, exp_avg_sq,
+            loss_scale):
+    """adam_update of calls that are not of the ordinary form (plain tensors and numbers, on the current device), or that it
+    refuses."""
     n = params.numel()
     if not (
         params.is_cuda and grads.is_cuda and exp_avg.is_cuda and exp_avg_sq.is_cuda
@@ -48,14 +62,11 @@ def adam_update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bia
     ):
         _refuse(params, grads, exp_avg, exp_avg_sq)
     with _lib.on_device(params.device):
-        rc = _lib.load().ps_adam_update(
+        return _lib.load().ps_adam_update(
             optimizer_id, int(step), lr, beta1, beta2, epsilon, weight_decay, 1 if bias_correction else 0,
             params.data_ptr(), grads.data_ptr(), 1 if grads.dtype is _HALF else 0, exp_avg.data_ptr(),
             exp_avg_sq.data_ptr(), n, float(loss_scale), None, _lib.raw_stream(params.device),
         )
-    if rc:
-        _lib.check(rc, "adam_update")
-    return 0
 
 
 def _refuse(params, grads, exp_avg, exp_avg_sq):

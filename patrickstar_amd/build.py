@@ -1,4 +1,4 @@
-"""Builds libps_adam.so (the C-ABI HIP library) for gfx950 with hipcc, in-tree."""
+"""Builds libps_adam.so (the C-ABI HIP library) for gfx950 with hipcc and _binding.so (host code) with g++, in-tree."""
 import os
 import shutil
 import subprocess
@@ -7,6 +7,8 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)
 LIB_PATH = os.path.join(PKG_DIR, "libps_adam.so")
 SOURCES = [os.path.join(PKG_DIR, "csrc", "ps_adam.hip")]
+BINDING_SOURCE = os.path.join(PKG_DIR, "csrc", "ps_binding.cpp")
+BINDING_PATH = os.path.join(PKG_DIR, "_binding.so")
 INCLUDE = os.path.join(ROOT, "include")
 
 # -ffp-contract=off: fused multiply-adds are written out explicitly; the compiler must not add or remove any.
@@ -55,8 +57,36 @@ def compile_shared(sources, target, verbose=False, extra_flags=()):
     return target
 
 
+def build_binding(verbose=False):
+    """Compile the Python side of the operator call, host code only, into patrickstar_amd/_binding.so (returned)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    tmp = BINDING_PATH + f".{os.getpid()}.tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM"]
+    for path in [INCLUDE, sysconfig.get_paths()["include"], "/opt/rocm/include"]:
+        cmd += ["-I", path]
+    for path in cpp_extension.include_paths():
+        cmd += ["-isystem", path]
+    cmd += [BINDING_SOURCE, "-o", tmp]
+    for path in cpp_extension.library_paths():
+        cmd += ["-L", path]
+    cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    try:
+        subprocess.check_call(cmd)
+        os.replace(tmp, BINDING_PATH)
+    finally:
+        if os.path.exists(tmp):
+            os.remove(tmp)
+    return BINDING_PATH
+
+
 def build(verbose=False, extra_flags=()):
-    """Compile the package's HIP sources into patrickstar_amd/libps_adam.so (returned)."""
+    """Compile the package's HIP sources into patrickstar_amd/libps_adam.so (returned), and the binding beside it."""
+    build_binding(verbose)
     return compile_shared(SOURCES, LIB_PATH, verbose, extra_flags)
 
 
