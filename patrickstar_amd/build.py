@@ -15,6 +15,7 @@ INCLUDE = os.path.join(ROOT, "include")
 # -fhip-fp32-correctly-rounded-divide-sqrt: IEEE-rounded '/' and sqrtf (hipcc's default, stated on purpose).
 # Denormals are kept: -fgpu-flush-denormals-to-zero is not given.
 # packed-fp32 ops are switched off: the compiler otherwise pairs independent float ops into v_pk_* forms.
+# Kernels whose first arguments are plain numbers or pointers get up to 14 words of them preloaded into scalar registers.
 HIPCC_FLAGS = [
     "-O3",
     "-std=c++17",
@@ -28,6 +29,8 @@ HIPCC_FLAGS = [
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
+    "-mllvm",
+    "-amdgpu-kernarg-preload-count=16",
     "-Wall",
     "-Wextra",
     "-Wno-unused-function",

@@ -800,12 +800,12 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
         const int tail = last ? (int)(left - n_tiles * kTile) : 0;
         const int this_head = done == 0 ? (int)head : 0;
         const size_t at = head + done;
-        dim3 grid((unsigned)(n_tiles + 1)), block(kBlock);  // + 1: the workgroup that does head and tail
+        dim3 grid((unsigned)(n_tiles + (this_head + tail > 0 ? 1 : 0))), block(kBlock);  // + 1: the workgroup that does head and tail
         uint16_t* out = d_param_fp16_out ? d_param_fp16_out + at : nullptr;
 #define PS_FLAT_VEC_5(WD, UNS, HALF, OUT, DWORD)                                                              \
-    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD>), grid, block, kLdsBytes, s, c,       \
+    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD>), grid, block, kLdsBytes, s,          \
                        d_params + at, static_cast<const void*>(gbytes + at * gsz), d_exp_avg + at,            \
-                       d_exp_avg_sq + at, out, n_tiles, this_head, tail)
+                       d_exp_avg_sq + at, out, (uint32_t)n_tiles, this_head, tail, c)
 #define PS_FLAT_VEC_4(WD, UNS, HALF, OUT)                  \
     do {                                                   \
         if (state_aligned)                                 \
@@ -1450,7 +1450,7 @@ int ps_cast_fp32_to_fp16(const float* d_src, uint16_t* d_dst, size_t numel, ps_s
     if (!d_src || !d_dst) return fail(PS_ERR_BAD_ARG, "ps_cast_fp32_to_fp16: NULL pointer");
     size_t n_tiles = (numel + kTile - 1) / kTile;
     hipLaunchKernelGGL(cast_kernel, dim3(grid_1d(n_tiles, kBlock)), dim3(kBlock), 0,
-                       static_cast<hipStream_t>(stream), d_src, d_dst, numel, n_tiles);
+                       static_cast<hipStream_t>(stream), CastArgs{d_src, d_dst, numel, n_tiles});
     PS_HIP(hipGetLastError());
     return 0;
 }
@@ -1830,7 +1830,7 @@ int ps_grads_to_chunks(const ps_grad_copy* copies, int n_copies, ps_step_state* 
         if (in_batch == 0) continue;
         const dim3 grid((unsigned)blocks), block(kCopyBlock);
         if (in_batch == 1)
-            hipLaunchKernelGGL(grad_to_chunk_kernel, grid, block, 0, s, b.src[0], b.dst[0], b.numel_half[0], d_state);
+            hipLaunchKernelGGL(grad_to_chunk_kernel, grid, block, 0, s, GradCopy{b.src[0], b.dst[0], b.numel_half[0], d_state});
         else
             hipLaunchKernelGGL(grads_to_chunks_kernel, grid, block, 0, s, b, d_state);
         PS_HIP(hipGetLastError());

@@ -483,12 +483,16 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     restore_tile(ch.param_fp32, ch.param_fp16, (size_t)blockIdx.x * kTile, b.n[blockIdx.y]);
 }
 
+struct CastArgs {
+    const float* src;
+    uint16_t* dst;
+    size_t numel, n_tiles;
+};
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    cast_kernel(const float* __restrict__ src, uint16_t* __restrict__ dst, size_t numel,
-                size_t n_tiles)
+    cast_kernel(CastArgs a)
 {
-    for (size_t t = blockIdx.x; t < n_tiles; t += gridDim.x)
-        restore_tile(src, dst, t * (size_t)kTile, numel);
+    for (size_t t = blockIdx.x; t < a.n_tiles; t += gridDim.x)
+        restore_tile(a.src, a.dst, t * (size_t)kTile, a.numel);
 }
 
 // ------------------------------------------------- auxiliary (non-hot) kernels
@@ -523,20 +527,27 @@ __global__ void __launch_bounds__(kAuxBlock)
 // straight through.  The tile grid is laid over the ADDRESSES of the fp32 parameter: the pointers are those of the
 // parameter's first 1 KiB boundary, so every wave access covers one aligned KiB (tiles at another phase of a KiB
 // measured 6 to 8 % slower); the up to 255 elements in front of it (`head`) and the up to 255 behind the last whole
-// tile (`tail`) are done element-wise by one extra workgroup of the same launch.  Gradients are read only and must
-// share the parameter's 16-byte phase, as must the optional fp16 output.
+// tile (`tail`), if there are any, are done element-wise by one extra workgroup of the same launch.  Gradients are read
+// only and must share the parameter's 16-byte phase, as must the optional fp16 output.
+//
+// Addresses and lengths come first so that they are preloaded into scalar registers (-amdgpu-kernarg-preload-count): a
+// wave issues its data loads without waiting for its arguments, and the constants are loaded in their shadow.  Of a tensor
+// that is a launch of its own that is most of what is left beside the 1.7 us of an empty launch and the bytes: 147 K elements
+// 2.52 -> 2.31 us, 590 K 5.03 -> 4.55, 2.36 M 13.35 -> 13.0; from 4096 to 40 K 1.9 -> 2.0.  Kernels of short or lone
+// launches, which the preloading makes 0.1 to 0.25 us longer (the element-wise operator, the lone gradient copy, the cast), take
+// their arguments in a struct, which is not preloaded.
 // STATE_DWORD_ALIGNED: exp_avg / exp_avg_sq sit at another 16-byte phase than the parameter (any element offset).
 template <int WD, int UNS, bool GRAD_HALF, bool HAS_OUT, bool STATE_DWORD_ALIGNED>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_flat_vec_kernel(StepConsts c, float* p32, const void* grads, float* m32, float* v32,
+    adam_flat_vec_kernel(float* p32, const void* grads, float* m32, float* v32,
                          uint16_t* out16,  // may alias grads (fp16 gradients overwritten by fp16 parameters)
-                         size_t n_tiles, int head, int tail)
+                         uint32_t n_tiles, int head, int tail, StepConsts c)
 {
     static_assert(kBlock == 64 && kLaneElems == 4 && kUnroll == 1, "one wave, one 16-byte access per lane and fp32 array");
     const size_t t = blockIdx.x;
-    if (t == n_tiles) {
+    if (blockIdx.x == n_tiles) {
         for (int j = threadIdx.x; j < head + tail; j += kBlock) {
-            const ptrdiff_t i = j < head ? (ptrdiff_t)j - head : (ptrdiff_t)(n_tiles * kTile) + (j - head);
+            const ptrdiff_t i = j < head ? (ptrdiff_t)j - head : (ptrdiff_t)((size_t)n_tiles * kTile) + (j - head);
             float g = GRAD_HALF ? half_bits_to_float(static_cast<const uint16_t*>(grads)[i])
                                 : static_cast<const float*>(grads)[i];
             float p = p32[i], m = m32[i], v = v32[i];
@@ -850,10 +861,15 @@ __global__ void __launch_bounds__(kCopyBlock) grads_to_chunks_kernel(GradBatch b
 
 // A gradient that has the launch to itself: nothing to look up, and arguments of 32 bytes instead of 1.8 KiB (with
 // those a launch back to back takes 4.5 us instead of 3.9 up to 1 Mi elements, 6.7 instead of 6.0 for 9 Mi in fp16).
-__global__ void __launch_bounds__(kCopyBlock)
-    grad_to_chunk_kernel(const void* src, uint16_t* dst, uint64_t numel_half, ps_step_state* st)
+struct GradCopy {
+    const void* src;
+    uint16_t* dst;
+    uint64_t numel_half;
+    ps_step_state* st;
+};
+__global__ void __launch_bounds__(kCopyBlock) grad_to_chunk_kernel(GradCopy c)
 {
-    copy_and_probe(src, dst, numel_half, blockIdx.x, st);
+    copy_and_probe(c.src, c.dst, c.numel_half, blockIdx.x, c.st);
 }
 
 // ------------------------------------------------ device-resident step state
