@@ -213,10 +213,7 @@ int for_each_batch(const ChunkList& a, F launch)
 }
 
 // A list whose chunks follow one another at one distance, all of one length but perhaps the last (EvenChunk).
-struct EvenList {
-    ps_chunk first;
-    uint32_t stride, numel, last, short_by;
-};
+using EvenList = EvenBatch;
 //
 // Lists of up to this many elements take the kernels for it.  Longer ones are bound by memory from the first tile to the
 // last, and the general kernels are as fast or a little faster: host-decided 593.6 / 595.7 us for 128 Mi elements, 7226 /
@@ -390,21 +387,22 @@ void launch_gated_batch(int arith, const ChunkBatch& b, dim3 grid, size_t chunk_
         launch_gated_batch_arith<PS_ARITH_OPERATOR>(b, grid, chunk_numel, ga, fc, d_state, s);
 }
 
-template <int ARITH>
-void launch_small_step_arith(const ChunkBatch& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
+template <int ARITH, typename LIST>
+void launch_small_step_arith(const LIST& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
                              ps_step_state* d_state, hipStream_t s)
 {
     dim3 grid(1), block(kBlock, kSmallWaves);
     const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
     if (decay && ga.adamw)
-        hipLaunchKernelGGL((adam_small_step_kernel<ARITH, WD_DECOUPLED>), grid, block, 0, s, b, a, ga, fc, d_state);
+        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_DECOUPLED>), grid, block, 0, s, b, a, ga, fc, d_state);
     else if (decay)
-        hipLaunchKernelGGL((adam_small_step_kernel<ARITH, WD_L2>), grid, block, 0, s, b, a, ga, fc, d_state);
+        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_L2>), grid, block, 0, s, b, a, ga, fc, d_state);
     else
-        hipLaunchKernelGGL((adam_small_step_kernel<ARITH, WD_NONE>), grid, block, 0, s, b, a, ga, fc, d_state);
+        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_NONE>), grid, block, 0, s, b, a, ga, fc, d_state);
 }
 
-void launch_small_step(int arith, const ChunkBatch& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
+template <typename LIST>
+void launch_small_step(int arith, const LIST& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
                        ps_step_state* d_state, hipStream_t s)
 {
     if (arith == PS_ARITH_TORCH)
@@ -1983,6 +1981,12 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
         const GatedArgs ga = gated_args(*o, lr, epsilon, weight_decay, bias_correction, k.n_calls);
         const SmallStep step{(uint32_t)tiles, (uint32_t)(tiles * n_chunks), (uint32_t)((((uint64_t)1 << 32) + tiles - 1) / tiles), chunk_numel, probe != 0, d_log, log_capacity, operator_calls};
         const int arith = o->arith;
+        EvenList e;
+        if (even_list(a, kMaxEvenElementsGated, &e)) {
+            launch_small_step(arith, e, step, ga, k.in_batch(0, n_chunks), d_state, static_cast<hipStream_t>(stream));
+            PS_HIP(hipGetLastError());
+            return 0;
+        }
         return for_each_batch(a, [&](const ChunkBatch& b, dim3, int) {
             launch_small_step(arith, b, step, ga, k.in_batch(0, n_chunks), d_state, static_cast<hipStream_t>(stream));
         });

@@ -1255,19 +1255,36 @@ struct SmallTile {
     size_t base, numel;  // the tile's first element in its chunk; the chunk's elements
     uint32_t k;
 };
-__device__ __forceinline__ SmallTile small_tile(const ChunkBatch& b, const SmallStep& a, uint32_t t)
+// The chunks of an EvenChunk list: 48 bytes of arguments where ChunkBatch has 2560, which cost the host 0.35 us a launch (the smoke
+// test's list, 13.8 -> 13.4 us a step among others) and the kernel 0.4.
+struct EvenBatch {
+    ps_chunk first;
+    uint32_t stride, numel, last, short_by;
+};
+__device__ __forceinline__ void small_chunk(const ChunkBatch& b, SmallTile& w)
+{
+    w.c = b.c[w.k];
+    w.numel = b.n[w.k];
+}
+__device__ __forceinline__ void small_chunk(const EvenBatch& b, SmallTile& w)
+{
+    const size_t at = (size_t)b.stride * w.k;
+    w.c = ps_chunk{b.first.param_fp32 + at, b.first.exp_avg + at, b.first.exp_avg_sq + at, b.first.param_fp16 + at};
+    w.numel = b.numel - (w.k == b.last ? b.short_by : 0u);
+}
+template <typename LIST>
+__device__ __forceinline__ SmallTile small_tile(const LIST& b, const SmallStep& a, uint32_t t)
 {
     SmallTile w;
     w.k = a.per_tile ? __umulhi(t, a.per_tile) : t;  // t / tiles
-    w.c = b.c[w.k];
+    small_chunk(b, w);
     w.base = (size_t)(t - w.k * a.tiles) * kTile;
-    w.numel = b.n[w.k];
     return w;
 }
 
-template <int ARITH, int WD>
+template <typename LIST, int ARITH, int WD>
 __global__ void __launch_bounds__(64 * kSmallWaves)
-    adam_small_step_kernel(ChunkBatch b, SmallStep a, GatedArgs ga, FirstCall fc, ps_step_state* st)
+    adam_small_step_kernel(LIST b, SmallStep a, GatedArgs ga, FirstCall fc, ps_step_state* st)
 {
     static_assert(kBlock == 64 && kLaneElems == 4 && kUnroll == 1, "tiles of one wave, four elements per lane");
     __shared__ uint32_t wave_hit[kSmallWaves];
