@@ -1066,9 +1066,12 @@ __global__ void __launch_bounds__(64)
     const int64_t adam_step = st->adam_step;
     const double cur_scale = st->cur_scale;
     const bool bias = a.bias_correction != 0;
-    if (j < a.n && (pb.k[j].mode & PLAN_KIND_MASK) != PLAN_MUL) {
-        const PlanClass& k = pb.k[j];
-        const int kind = k.mode & PLAN_KIND_MASK;
+    PlanClass k;
+    memset(&k, 0, sizeof(k));
+    if (j < a.n) k = pb.k[j];
+    const int kind = k.mode & PLAN_KIND_MASK;
+    uint64_t multiplying = __ballot(kind == PLAN_MUL);
+    if (j < a.n && kind != PLAN_MUL) {
         const float clip = clamp_bound(a.grad_clamp, cur_scale, (k.mode & PLAN_GRAD_F32) != 0);
         const int64_t t = adam_step + 1 + k.d;
         PlannedConsts out;
@@ -1091,10 +1094,11 @@ __global__ void __launch_bounds__(64)
     }
     __syncthreads();
     if (j != 0) return;
-    // a call that multiplies needs the call before it: in order, by one lane
-    for (int i = 0; i < a.n; ++i) {
+    // a call that multiplies needs the call before it: in order, by one lane, which looks at those calls only (a look at each
+    // of the classes was a chain of waits: 14 classes of which none multiplies cost a step 4.2 us, now 2.7)
+    for (; multiplying != 0; multiplying &= multiplying - 1) {
+        const int i = (int)__builtin_ctzll(multiplying);
         const PlanClass& k = pb.k[i];
-        if ((k.mode & PLAN_KIND_MASK) != PLAN_MUL) continue;
         const float clip = clamp_bound(a.grad_clamp, cur_scale, (k.mode & PLAN_GRAD_F32) != 0);
         const int q = k.prev - a.first_class;  // an earlier class: of this launch, or of a launch before it
         const float p1 = q >= 0 ? b1t_of[q] : table[k.prev].beta1_t;
