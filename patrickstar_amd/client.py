@@ -101,7 +101,7 @@ class PatrickStarClient:
         # False: it stays in HBM, where forward and backward use it (the only form a registered module can have)
         self.host_keeps_fp16 = True
         self._slabs = []  # the lists' memory that HBM-resident payloads are views of
-        self._reserved = {}  # (state list, fp16 chunk id) -> (slab, element) for the state chunk of that position
+        self._reserved = {}  # (state list, fp16 chunk id) -> memory for the state chunk of that position
         # called with (position index among fp16 chunks) -> True to keep that position in host memory
         self.host_chunk_policy: Optional[Callable[[int], bool]] = None
         default_opts = {"with_mem_saving_comm": False, "with_mem_cache": False, "with_async_move": False}
@@ -352,16 +352,19 @@ class PatrickStarClient:
                 if not chunks:
                     continue
             n = sum(stride(c) for c in chunks)
-            positions = [self._fp16_chunk_of_position(c.chunk_id) for c in chunks] if chunk_type == ChunkType.PARAM_FP32 else []
-            rooms = self._fp32_lists(n) if positions and None not in positions else None
+            rooms = None
+            if chunk_type == ChunkType.PARAM_FP32 and all(c.data_type == torch.float for c in chunks):
+                positions = [self._fp16_chunk_of_position(c.chunk_id) for c in chunks]
+                if None not in positions:  # (an fp32 list driven on its own has no state lists either)
+                    rooms = self._fp32_lists(n)
             slab = rooms[0] if rooms else torch.zeros(n, dtype=chunks[0].data_type, device=self.device)
             self._slabs.append(slab)
             cursor = 0
             for k, chunk in enumerate(chunks):
                 chunk.payload = slab.narrow(0, cursor, chunk.capacity)
                 if rooms:
-                    self._reserved[(ChunkType.MOMENTUM, positions[k])] = (rooms[1], cursor)
-                    self._reserved[(ChunkType.VARIANCE, positions[k])] = (rooms[2], cursor)
+                    for state, room in ((ChunkType.MOMENTUM, rooms[1]), (ChunkType.VARIANCE, rooms[2])):
+                        self._reserved[(state, positions[k])] = room.narrow(0, cursor, chunk.capacity)
                 cursor += stride(chunk)
 
     def _fp32_lists(self, n):
@@ -381,13 +384,17 @@ class PatrickStarClient:
         """Give state chunks the room that was reserved beside their position's fp32 chunk; returns those that have none."""
         rest = []
         for chunk in chunks:
-            slab, at = self._reserved.pop((chunk_type, self._fp16_chunk_of_position(chunk.chunk_id)), (None, 0))
-            if slab is None:
+            room = None
+            if self._reserved:
+                position = next((cid for cid, states in self.chunk_tensor_index.param_chunk_id_to_os_chunk_id_map.items()
+                                 if states.get(chunk_type) == chunk.chunk_id), None)  # None: a list driven on its own
+                room = self._reserved.pop((chunk_type, position), None)
+            if room is None or room.numel() != chunk.capacity or room.dtype != chunk.data_type:
                 rest.append(chunk)
                 continue
-            if not any(slab is known for known in self._slabs):
-                self._slabs.append(slab)
-            chunk.payload = slab.narrow(0, at, chunk.capacity)
+            if not any(room._base is slab for slab in self._slabs):
+                self._slabs.append(room._base)
+            chunk.payload = room
         return rest
 
     def chunk_ids_generator(self, chunk_type):

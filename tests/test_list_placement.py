@@ -3,6 +3,7 @@ import pytest
 import torch
 
 import patrickstar_amd as ps
+from patrickstar_amd.chunk_layout import AccessType, ChunkType, ParamType, register_param
 from patrickstar_amd.client import LIST_CLEARANCE, LIST_PERIOD, list_distance
 
 MB = 1 << 20
@@ -43,3 +44,26 @@ def test_every_chunk_has_memory_of_its_own(numel, calls):
     apart = [(a[1].data_ptr() - a[0].data_ptr()) % LIST_PERIOD for a in where.values()]
     if 80 * MB <= 4 * numel * calls[0] <= 1024 * MB and calls != (1, 2):
         assert LIST_CLEARANCE <= apart[0] <= LIST_PERIOD - LIST_CLEARANCE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("with_parameters", [False, True])
+@pytest.mark.parametrize("chunk_type,dtype", [(ChunkType.MOMENTUM, torch.float), (ChunkType.VARIANCE, torch.float), (ChunkType.PARAM_FP32, torch.double)])
+def test_lists_driven_on_their_own_get_memory_of_their_own(chunk_type, dtype, with_parameters):
+    n = 24 * MB
+    client = ps.PatrickStarClient(0, n)
+    params = client.append_flat_chunks(1) if with_parameters else []
+    p = torch.nn.Parameter(torch.tensor([], dtype=dtype), requires_grad=False)
+    register_param(p, ParamType.CHUNK_BASED, dtype, "own")
+    p.ps_attr.reset_shape(torch.Size([n]))
+    client.append_tensor([p], dtype, AccessType.DATA, chunk_type)
+    own = client.access_data(p)
+    assert own.dtype == dtype and int(torch.count_nonzero(own)) == 0
+    own.fill_(3)
+    if params:
+        opt = ps.FP16Adam(client, params, loss_scaler=ps.LossScaler(8.0), lr=1e-3)
+        for q in (client.param_fp16_to_param_fp32_map[params[0]], opt.state[params[0]]["exp_avg"], opt.state[params[0]]["exp_avg_sq"], params[0]):
+            t = client.access_data(q)
+            assert t.numel() == n and int(torch.count_nonzero(t)) == 0
+        opt.step()
+        assert bool((own == 3).all())
