@@ -9,16 +9,16 @@
 //     instruction covers a contiguous span of whole cache lines;
 //   * one small tile (256 elements) per single-wave workgroup and a CAP on
 //     resident workgroups (9 per CU, enforced by requesting 17 KiB of unused
-//     dynamic LDS): the pass touches four arrays for reading and the same four
+//     dynamic LDS; 11 with the hint below): the pass touches four arrays for reading and the same four
 //     for writing, and HBM efficiency drops when the set of in-flight cache
 //     lines gets wide; a narrow, steadily advancing window per array gave
 //     6.3 TB/s where the fully occupied machine gave 5.3 TB/s (a plain
 //     1-read-1-write copy peaks at 6.3-6.4 TB/s on the same GPU);
 //   * chunk descriptors travel in the kernel-argument segment (64 per launch),
 //     so a wave's first data load depends on one scalar load, not two;
-//   * plain (temporal) loads/stores: non-temporal loads cost 6 % at this
-//     operating point (20-25 % with fully occupied CUs), non-temporal stores
-//     change nothing.
+//   * lists too long for the caches stream past them: non-temporal loads AND
+//     stores, and 11 instead of 9 workgroups per CU, 6.6 TB/s where plain
+//     accesses gave 6.25 (either hint alone gains nothing or loses 6 %).
 //
 // Arithmetic contract (ps_arith.h).  Operator arithmetic: bit-exact with the
 // explicit-intrinsic body of the reference operator
@@ -212,6 +212,55 @@ int for_each_batch(const ChunkList& a, F launch)
     return 0;
 }
 
+size_t elements(const ChunkList& a)
+{
+    size_t n = 0;
+    for (int i = 0; i < a.n_chunks; ++i) n += a.numel_of(i);
+    return n;
+}
+
+// ---- streaming past the caches
+//
+// A pass over a list uses nothing twice, but its loads and stores go through the L2 and the memory-side cache like any
+// other: what a kernel has written waits there, is written back when something else needs the room or the kernel ends, and
+// is in the way of the loads.  With the non-temporal hint on loads AND stores (and 11 workgroups per CU instead of 9) it
+// leaves at once.  24 x 64 Mi elements 7211 -> 6848 us host-decided, a device-decided step with its probe 7713 -> 7266; 8 x 64 Mi
+// 2374 -> 2234 and 2572 -> 2394; one 64 Mi chunk 295 -> 280 and 324 -> 304.  The hint on the loads alone makes the same steps 6 %
+// slower, on the stores alone nothing.
+//
+// Steps over a list that stays in the memory-side cache from one step to the next (256 MiB) want it there: the same state
+// again and again, without / with the hint, host-decided 16 Mi elements 53 / 71 us, 24 Mi 105 / 106, 28 Mi 127 / 123, 32 Mi 150 / 142;
+// device-decided 24 Mi 115 / 118, 28 Mi 136 / 138, 32 Mi 157 / 157, 48 Mi 244 / 230.  The probe alone at 32 Mi 10.2 / 9.0.  A tensor of the
+// operator comes with others, and its launch ends when its stores have left the L2: 144 K elements 2.33 / 2.41 us, 576 K 4.50 / 3.68,
+// 2.25 Mi 13.0 / 11.5; the tensors of a module of 5.3 M elements one after the other 67 / 68, of 11 M 166 / 139.
+//
+// A store that fills a 64-byte line in part only must not leave at once: lists whose phases differ by 16 or 32 bytes ran
+// 5 to 6 % slower with the hint, by 64 6 % faster.
+constexpr size_t kStreamElements = (size_t)28 << 20, kStreamElementsGated = (size_t)32 << 20, kScanStreamElements = (size_t)32 << 20,
+                 kFlatStreamElements = (size_t)256 << 10;
+bool whole_lines(const void* p32, const void* m32, const void* v32, const void* h16)
+{
+    return ((reinterpret_cast<uintptr_t>(p32) | reinterpret_cast<uintptr_t>(m32) | reinterpret_cast<uintptr_t>(v32) |
+             reinterpret_cast<uintptr_t>(h16)) & 63u) == 0;
+}
+bool streams(const ChunkList& a, bool gated)
+{
+    if (elements(a) < (gated ? kStreamElementsGated : kStreamElements)) return false;
+    for (int i = 0; i < a.n_chunks; ++i)
+        if (!whole_lines(a.chunks[i].param_fp32, a.chunks[i].exp_avg, a.chunks[i].exp_avg_sq, a.chunks[i].param_fp16)) return false;
+    return true;
+}
+
+// launch(std::true_type or std::false_type): whether the kernel is the one with the non-temporal hint.
+template <typename F>
+void with_hint(bool nt, F launch)
+{
+    if (nt)
+        launch(std::true_type{});
+    else
+        launch(std::false_type{});
+}
+
 // A list whose chunks follow one another at one distance, all of one length but perhaps the last (EvenChunk).
 using EvenList = EvenBatch;
 //
@@ -289,102 +338,114 @@ int make_calls(Calls& out, const ps_call_pattern* calls, int64_t n_chunks_total,
 }
 
 template <int ARITH, int WD>
-void launch_adam_batch_wd(const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc, hipStream_t s)
+void launch_adam_batch_wd(const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc, bool nt, hipStream_t s)
 {
-    dim3 block(kBlock);
-    if (c.unscale == UNSCALE_MUL)
-        hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_MUL>), grid, block, kLdsBytes, s, b, c, fc);
-    else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)  // the torch formula never divides
-        hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_DIV>), grid, block, kLdsBytes, s, b, c, fc);
-    else
-        hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_NONE>), grid, block, kLdsBytes, s, b, c, fc);
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        dim3 block(kBlock);
+        if (c.unscale == UNSCALE_MUL)
+            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_MUL, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, c, fc);
+        else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)  // the torch formula never divides
+            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_DIV, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, c, fc);
+        else
+            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, c, fc);
+    });
 }
 
 template <int ARITH>
-void launch_adam_batch_arith(const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc, hipStream_t s)
+void launch_adam_batch_arith(const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc, bool nt, hipStream_t s)
 {
     if (c.wd_mode == WD_DECOUPLED)
-        launch_adam_batch_wd<ARITH, WD_DECOUPLED>(b, grid, c, fc, s);
+        launch_adam_batch_wd<ARITH, WD_DECOUPLED>(b, grid, c, fc, nt, s);
     else if (c.wd_mode == WD_L2)
-        launch_adam_batch_wd<ARITH, WD_L2>(b, grid, c, fc, s);
+        launch_adam_batch_wd<ARITH, WD_L2>(b, grid, c, fc, nt, s);
     else
-        launch_adam_batch_wd<ARITH, WD_NONE>(b, grid, c, fc, s);
+        launch_adam_batch_wd<ARITH, WD_NONE>(b, grid, c, fc, nt, s);
 }
 
 #define PS_EVEN(e) (e).first.param_fp32, (e).first.exp_avg, (e).first.exp_avg_sq, (e).first.param_fp16, (e).stride, (e).numel, (e).last, (e).short_by
 
 template <int ARITH, int WD>
-void launch_even_wd(const EvenList& e, const StepConsts& c, const FirstCall& fc, hipStream_t s)
+void launch_even_wd(const EvenList& e, const StepConsts& c, const FirstCall& fc, bool nt, hipStream_t s)
 {
-    const dim3 grid = even_grid(e, kTile), block(kBlock);
-    if (c.unscale == UNSCALE_MUL)
-        hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_MUL>), grid, block, kLdsBytes, s, PS_EVEN(e), c, fc);
-    else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
-        hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_DIV>), grid, block, kLdsBytes, s, PS_EVEN(e), c, fc);
-    else
-        hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_NONE>), grid, block, kLdsBytes, s, PS_EVEN(e), c, fc);
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        const dim3 grid = even_grid(e, kTile), block(kBlock);
+        if (c.unscale == UNSCALE_MUL)
+            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_MUL, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), c, fc);
+        else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
+            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_DIV, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), c, fc);
+        else
+            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), c, fc);
+    });
 }
 
 template <int ARITH>
-void launch_even_arith(const EvenList& e, const StepConsts& c, const FirstCall& fc, hipStream_t s)
+void launch_even_arith(const EvenList& e, const StepConsts& c, const FirstCall& fc, bool nt, hipStream_t s)
 {
     if (c.wd_mode == WD_DECOUPLED)
-        launch_even_wd<ARITH, WD_DECOUPLED>(e, c, fc, s);
+        launch_even_wd<ARITH, WD_DECOUPLED>(e, c, fc, nt, s);
     else if (c.wd_mode == WD_L2)
-        launch_even_wd<ARITH, WD_L2>(e, c, fc, s);
+        launch_even_wd<ARITH, WD_L2>(e, c, fc, nt, s);
     else
-        launch_even_wd<ARITH, WD_NONE>(e, c, fc, s);
+        launch_even_wd<ARITH, WD_NONE>(e, c, fc, nt, s);
 }
 
 template <int ARITH>
 void launch_even_gated(const EvenList& e, size_t chunk_numel, const GatedArgs& ga, const FirstCall& fc,
-                       const ps_step_state* d_state, hipStream_t s)
+                       const ps_step_state* d_state, bool nt, hipStream_t s)
 {
-    const dim3 grid = even_grid(e, kTile), block(kBlock);
-    const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
-    if (decay && ga.adamw)
-        hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_DECOUPLED>), grid, block, kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
-    else if (decay)
-        hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_L2>), grid, block, kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
-    else
-        hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_NONE>), grid, block, kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        const dim3 grid = even_grid(e, kTile), block(kBlock);
+        const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
+        if (decay && ga.adamw)
+            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_DECOUPLED, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+        else if (decay)
+            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_L2, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+        else
+            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+    });
 }
 
 // `c` must have been built for `arith` (finish_consts / torch_consts).  `fc`: which elements of the
 // batch the step's first operator call covers; the torch formula has no such distinction.
-void launch_adam_batch(int arith, const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc,
+void launch_adam_batch(int arith, const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc, bool nt,
                        hipStream_t s)
 {
     if (arith == PS_ARITH_TORCH)
-        launch_adam_batch_arith<PS_ARITH_TORCH>(b, grid, c, kNoFirstCall, s);
+        launch_adam_batch_arith<PS_ARITH_TORCH>(b, grid, c, kNoFirstCall, nt, s);
     else
-        launch_adam_batch_arith<PS_ARITH_OPERATOR>(b, grid, c, fc, s);
+        launch_adam_batch_arith<PS_ARITH_OPERATOR>(b, grid, c, fc, nt, s);
 }
 
 template <int ARITH>
 void launch_gated_batch_arith(const ChunkBatch& b, dim3 grid, size_t chunk_numel,
                               const GatedArgs& ga, const FirstCall& fc, const ps_step_state* d_state,
-                              hipStream_t s)
+                              bool nt, hipStream_t s)
 {
-    dim3 block(kBlock);
-    // the operator tests its float weight decay "> 0" (cpu_adam.cpp:42), the torch formula "!= 0"
-    const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
-    if (decay && ga.adamw)
-        hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_DECOUPLED>), grid, block, kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
-    else if (decay)
-        hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_L2>), grid, block, kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
-    else
-        hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_NONE>), grid, block, kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        dim3 block(kBlock);
+        // the operator tests its float weight decay "> 0" (cpu_adam.cpp:42), the torch formula "!= 0"
+        const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
+        if (decay && ga.adamw)
+            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_DECOUPLED, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+        else if (decay)
+            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_L2, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+        else
+            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+    });
 }
 
 void launch_gated_batch(int arith, const ChunkBatch& b, dim3 grid, size_t chunk_numel,
                         const GatedArgs& ga, const FirstCall& fc, const ps_step_state* d_state,
-                        hipStream_t s)
+                        bool nt, hipStream_t s)
 {
     if (arith == PS_ARITH_TORCH)
-        launch_gated_batch_arith<PS_ARITH_TORCH>(b, grid, chunk_numel, ga, kNoFirstCall, d_state, s);
+        launch_gated_batch_arith<PS_ARITH_TORCH>(b, grid, chunk_numel, ga, kNoFirstCall, d_state, nt, s);
     else
-        launch_gated_batch_arith<PS_ARITH_OPERATOR>(b, grid, chunk_numel, ga, fc, d_state, s);
+        launch_gated_batch_arith<PS_ARITH_OPERATOR>(b, grid, chunk_numel, ga, fc, d_state, nt, s);
 }
 
 template <int ARITH, typename LIST>
@@ -411,44 +472,50 @@ void launch_small_step(int arith, const LIST& b, const SmallStep& a, const Gated
         launch_small_step_arith<PS_ARITH_OPERATOR>(b, a, ga, fc, d_state, s);
 }
 
-template <typename LIST>
-constexpr unsigned kListLds = std::is_same<LIST, NearBatch>::value ? kNearLdsBytes : kLdsBytes;
+template <typename LIST, bool NT>
+constexpr unsigned kListLds = std::is_same<LIST, NearBatch>::value ? (NT ? kStreamNearLdsBytes : kNearLdsBytes) : (NT ? kStreamLdsBytes : kLdsBytes);
 
 template <int ARITH, int WD, typename LIST>
-void launch_tensors_wd(const LIST& b, dim3 grid, const StepConsts& c, hipStream_t s)
+void launch_tensors_wd(const LIST& b, dim3 grid, const StepConsts& c, bool nt, hipStream_t s)
 {
-    dim3 block(kBlock);
-    if (c.unscale == UNSCALE_MUL)
-        hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_MUL>), grid, block, kListLds<LIST>, s, b, c);
-    else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
-        hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_DIV>), grid, block, kListLds<LIST>, s, b, c);
-    else
-        hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_NONE>), grid, block, kListLds<LIST>, s, b, c);
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        dim3 block(kBlock);
+        if (c.unscale == UNSCALE_MUL)
+            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_MUL, NT>), grid, block, (kListLds<LIST, NT>), s, b, c);
+        else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
+            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_DIV, NT>), grid, block, (kListLds<LIST, NT>), s, b, c);
+        else
+            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_NONE, NT>), grid, block, (kListLds<LIST, NT>), s, b, c);
+    });
 }
 
 template <int ARITH, typename LIST>
-void launch_tensors_arith(const LIST& b, dim3 grid, const StepConsts& c, hipStream_t s)
+void launch_tensors_arith(const LIST& b, dim3 grid, const StepConsts& c, bool nt, hipStream_t s)
 {
     if (c.wd_mode == WD_DECOUPLED)
-        launch_tensors_wd<ARITH, WD_DECOUPLED>(b, grid, c, s);
+        launch_tensors_wd<ARITH, WD_DECOUPLED>(b, grid, c, nt, s);
     else if (c.wd_mode == WD_L2)
-        launch_tensors_wd<ARITH, WD_L2>(b, grid, c, s);
+        launch_tensors_wd<ARITH, WD_L2>(b, grid, c, nt, s);
     else
-        launch_tensors_wd<ARITH, WD_NONE>(b, grid, c, s);
+        launch_tensors_wd<ARITH, WD_NONE>(b, grid, c, nt, s);
 }
 
 template <int ARITH, typename LIST>
 void launch_tensors_gated_arith(const LIST& b, dim3 grid, const GatedArgs& ga,
-                                const ps_step_state* d_state, hipStream_t s)
+                                const ps_step_state* d_state, bool nt, hipStream_t s)
 {
-    dim3 block(kBlock);
-    const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
-    if (decay && ga.adamw)
-        hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_DECOUPLED>), grid, block, kListLds<LIST>, s, b, ga, d_state);
-    else if (decay)
-        hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_L2>), grid, block, kListLds<LIST>, s, b, ga, d_state);
-    else
-        hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_NONE>), grid, block, kListLds<LIST>, s, b, ga, d_state);
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        dim3 block(kBlock);
+        const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
+        if (decay && ga.adamw)
+            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_DECOUPLED, NT>), grid, block, (kListLds<LIST, NT>), s, b, ga, d_state);
+        else if (decay)
+            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_L2, NT>), grid, block, (kListLds<LIST, NT>), s, b, ga, d_state);
+        else
+            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_NONE, NT>), grid, block, (kListLds<LIST, NT>), s, b, ga, d_state);
+    });
 }
 
 // The Python numbers of one step as they cross the boundary.
@@ -864,6 +931,8 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
     const size_t head = (size_t)((kTile - (reinterpret_cast<uintptr_t>(d_params) / sizeof(float)) % kTile) % kTile);
     // one tile per workgroup: a tensor beyond the launch grid (2^39 elements) goes in several launches
     const size_t max_tiles = kMaxGridX - 1;
+    const bool nt = numel >= kFlatStreamElements && whole_lines(d_params + head, d_exp_avg + head, d_exp_avg_sq + head,
+                                                                 d_param_fp16_out ? d_param_fp16_out + head : nullptr);
     size_t done = 0;  // elements behind the head that earlier launches of this call have covered
     const size_t body = numel - head;
     do {
@@ -875,10 +944,17 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
         const size_t at = head + done;
         dim3 grid((unsigned)(n_tiles + (this_head + tail > 0 ? 1 : 0))), block(kBlock);  // + 1: the workgroup that does head and tail
         uint16_t* out = d_param_fp16_out ? d_param_fp16_out + at : nullptr;
-#define PS_FLAT_VEC_5(WD, UNS, HALF, OUT, DWORD)                                                              \
-    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD>), grid, block, kLdsBytes, s,          \
+#define PS_FLAT_VEC_6(WD, UNS, HALF, OUT, DWORD, NT)                                                              \
+    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s,          \
                        d_params + at, static_cast<const void*>(gbytes + at * gsz), d_exp_avg + at,            \
                        d_exp_avg_sq + at, out, (uint32_t)n_tiles, this_head, tail, c)
+#define PS_FLAT_VEC_5(WD, UNS, HALF, OUT, DWORD)           \
+    do {                                                   \
+        if (nt)                                            \
+            PS_FLAT_VEC_6(WD, UNS, HALF, OUT, DWORD, true);  \
+        else                                               \
+            PS_FLAT_VEC_6(WD, UNS, HALF, OUT, DWORD, false); \
+    } while (0)
 #define PS_FLAT_VEC_4(WD, UNS, HALF, OUT)                  \
     do {                                                   \
         if (state_aligned)                                 \
@@ -917,6 +993,7 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
 #undef PS_FLAT_VEC_3
 #undef PS_FLAT_VEC_4
 #undef PS_FLAT_VEC_5
+#undef PS_FLAT_VEC_6
         PS_HIP(hipGetLastError());
         done += n_tiles * kTile + tail;
     } while (done < body);
@@ -944,18 +1021,19 @@ int ps_adam_step_chunks(int optimizer_id, size_t step, double lr, double beta1, 
         c = operator_step_consts(*o, step, hp, k.n_calls);
     if (!zeros_are_a_fixed_point(c)) a.used = nullptr;  // the padding is computed like everything else
     const int arith = o->arith;
+    const bool nt = streams(a, false);
     hipStream_t s = static_cast<hipStream_t>(stream);
     EvenList e;
     if (even_list(a, kMaxEvenElements, &e)) {
         if (arith == PS_ARITH_TORCH)
-            launch_even_arith<PS_ARITH_TORCH>(e, c, kNoFirstCall, s);
+            launch_even_arith<PS_ARITH_TORCH>(e, c, kNoFirstCall, nt, s);
         else
-            launch_even_arith<PS_ARITH_OPERATOR>(e, c, k.in_batch(0, n_chunks), s);
+            launch_even_arith<PS_ARITH_OPERATOR>(e, c, k.in_batch(0, n_chunks), nt, s);
         PS_HIP(hipGetLastError());
         return 0;
     }
     return for_each_batch(a, [&](const ChunkBatch& b, dim3 grid, int first) {
-        launch_adam_batch(arith, b, grid, c, k.in_batch(first, (int)grid.y), s);
+        launch_adam_batch(arith, b, grid, c, k.in_batch(first, (int)grid.y), nt, s);
     });
 }
 
@@ -975,18 +1053,19 @@ int ps_adam_step_chunks_gated(int optimizer_id, double lr, double epsilon, doubl
     const GatedArgs ga = gated_args(*o, lr, epsilon, weight_decay, bias_correction, k.n_calls);
     const int arith = o->arith;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool nt = streams(a, true);
     // (whether the padding may be left alone depends on the device-resident scalars: the kernel decides)
     EvenList e;
     if (even_list(a, kMaxEvenElementsGated, &e)) {
         if (arith == PS_ARITH_TORCH)
-            launch_even_gated<PS_ARITH_TORCH>(e, chunk_numel, ga, kNoFirstCall, d_state, s);
+            launch_even_gated<PS_ARITH_TORCH>(e, chunk_numel, ga, kNoFirstCall, d_state, nt, s);
         else
-            launch_even_gated<PS_ARITH_OPERATOR>(e, chunk_numel, ga, k.in_batch(0, n_chunks), d_state, s);
+            launch_even_gated<PS_ARITH_OPERATOR>(e, chunk_numel, ga, k.in_batch(0, n_chunks), d_state, nt, s);
         PS_HIP(hipGetLastError());
         return 0;
     }
     return for_each_batch(a, [&](const ChunkBatch& b, dim3 grid, int first) {
-        launch_gated_batch(arith, b, grid, chunk_numel, ga, k.in_batch(first, (int)grid.y), d_state, s);
+        launch_gated_batch(arith, b, grid, chunk_numel, ga, k.in_batch(first, (int)grid.y), d_state, nt, s);
     });
 }
 
@@ -1028,6 +1107,21 @@ TensorItem tensor_item(const ps_chunk* tensors, const size_t* numels, int i, boo
     if (head > numels[i]) head = numels[i];
     const size_t body = numels[i] - head;
     return TensorItem{i, (uint32_t)head, body, (head ? 1 : 0) + (body + kTile - 1) / kTile, 0};
+}
+
+// (of tensors, the tiles start at the parameter's KiB boundary)
+bool streams(const ps_chunk* tensors, const size_t* numels, int n_tensors, bool gated)
+{
+    size_t total = 0;
+    for (int i = 0; i < n_tensors; ++i) total += numels[i];
+    if (total < (gated ? kStreamElementsGated : kStreamElements)) return false;
+    for (int i = 0; i < n_tensors; ++i) {
+        if (numels[i] < (size_t)kTile) continue;
+        const size_t head = tensor_item(tensors, numels, i).head;
+        const ps_chunk& t = tensors[i];
+        if (!whole_lines(t.param_fp32 + head, t.exp_avg + head, t.exp_avg_sq + head, t.param_fp16 + head)) return false;
+    }
+    return true;
 }
 
 // Calls launch(batch, grid, classes) for groups of the given tensors (all of them non-empty): longest first; one launch
@@ -1173,28 +1267,31 @@ int wd_mode_of(int arith, double wd, bool adamw)
 
 template <int ARITH, int WD, typename LIST>
 void launch_tensors_planned_wd(const LIST& b, dim3 grid, bool grad_f32,
-                               const PlannedConsts* d_consts, const ps_step_state* d_state, hipStream_t s)
+                               const PlannedConsts* d_consts, const ps_step_state* d_state, bool nt, hipStream_t s)
 {
-    dim3 block(kBlock);
-    if constexpr (std::is_same<LIST, TensorBatch>::value) {
-        if (grad_f32) {
-            hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
-            return;
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        dim3 block(kBlock);
+        if constexpr (std::is_same<LIST, TensorBatch>::value) {
+            if (grad_f32) {
+                hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
+                return;
+            }
         }
-    }
-    hipLaunchKernelGGL((adam_tensors_planned_kernel<LIST, ARITH, WD>), grid, block, kListLds<LIST>, s, b, d_consts, d_state);
+        hipLaunchKernelGGL((adam_tensors_planned_kernel<LIST, ARITH, WD, NT>), grid, block, (kListLds<LIST, NT>), s, b, d_consts, d_state);
+    });
 }
 
 template <int ARITH, typename LIST>
 void launch_tensors_planned_arith(const LIST& b, dim3 grid, int wd_mode, bool grad_f32,
-                                  const PlannedConsts* d_consts, const ps_step_state* d_state, hipStream_t s)
+                                  const PlannedConsts* d_consts, const ps_step_state* d_state, bool nt, hipStream_t s)
 {
     if (wd_mode == WD_DECOUPLED)
-        launch_tensors_planned_wd<ARITH, WD_DECOUPLED>(b, grid, grad_f32, d_consts, d_state, s);
+        launch_tensors_planned_wd<ARITH, WD_DECOUPLED>(b, grid, grad_f32, d_consts, d_state, nt, s);
     else if (wd_mode == WD_L2)
-        launch_tensors_planned_wd<ARITH, WD_L2>(b, grid, grad_f32, d_consts, d_state, s);
+        launch_tensors_planned_wd<ARITH, WD_L2>(b, grid, grad_f32, d_consts, d_state, nt, s);
     else
-        launch_tensors_planned_wd<ARITH, WD_NONE>(b, grid, grad_f32, d_consts, d_state, s);
+        launch_tensors_planned_wd<ARITH, WD_NONE>(b, grid, grad_f32, d_consts, d_state, nt, s);
 }
 
 // Numbers the distinct records (classes of calls) of a step by their bytes; records are zero-filled before they are
@@ -1240,40 +1337,43 @@ static_assert(PS_ARITH_OPERATOR == 0 && PS_ARITH_TORCH == 1, "class_key keeps th
 
 template <int ARITH, int WD, int UNS, typename LIST>
 void launch_tensors_each_uns(const LIST& b, dim3 grid, const ConstsBatch& cb, bool grad_f32,
-                             hipStream_t s)
+                             bool nt, hipStream_t s)
 {
-    dim3 block(kBlock);
-    if constexpr (std::is_same<LIST, TensorBatch>::value) {
-        if (grad_f32) {
-            hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
-            return;
+    with_hint(nt, [&](auto hint) {
+        constexpr bool NT = decltype(hint)::value;
+        dim3 block(kBlock);
+        if constexpr (std::is_same<LIST, TensorBatch>::value) {
+            if (grad_f32) {
+                hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
+                return;
+            }
         }
-    }
-    hipLaunchKernelGGL((adam_tensors_each_kernel<LIST, ARITH, WD, UNS>), grid, block, kListLds<LIST>, s, b, cb);
+        hipLaunchKernelGGL((adam_tensors_each_kernel<LIST, ARITH, WD, UNS, NT>), grid, block, (kListLds<LIST, NT>), s, b, cb);
+    });
 }
 
 template <int ARITH, int WD, typename LIST>
 void launch_tensors_each_wd(const LIST& b, dim3 grid, const ConstsBatch& cb,
-                            const Flavour& f, hipStream_t s)
+                            const Flavour& f, bool nt, hipStream_t s)
 {
     if (f.unscale == UNSCALE_MUL)
-        launch_tensors_each_uns<ARITH, WD, UNSCALE_MUL>(b, grid, cb, f.grad_f32, s);
+        launch_tensors_each_uns<ARITH, WD, UNSCALE_MUL>(b, grid, cb, f.grad_f32, nt, s);
     else if (ARITH == PS_ARITH_OPERATOR && f.unscale == UNSCALE_DIV)  // the torch formula never divides
-        launch_tensors_each_uns<ARITH, WD, UNSCALE_DIV>(b, grid, cb, f.grad_f32, s);
+        launch_tensors_each_uns<ARITH, WD, UNSCALE_DIV>(b, grid, cb, f.grad_f32, nt, s);
     else
-        launch_tensors_each_uns<ARITH, WD, UNSCALE_NONE>(b, grid, cb, f.grad_f32, s);
+        launch_tensors_each_uns<ARITH, WD, UNSCALE_NONE>(b, grid, cb, f.grad_f32, nt, s);
 }
 
 template <int ARITH, typename LIST>
 void launch_tensors_each_arith(const LIST& b, dim3 grid, const ConstsBatch& cb,
-                               const Flavour& f, hipStream_t s)
+                               const Flavour& f, bool nt, hipStream_t s)
 {
     if (f.wd_mode == WD_DECOUPLED)
-        launch_tensors_each_wd<ARITH, WD_DECOUPLED>(b, grid, cb, f, s);
+        launch_tensors_each_wd<ARITH, WD_DECOUPLED>(b, grid, cb, f, nt, s);
     else if (f.wd_mode == WD_L2)
-        launch_tensors_each_wd<ARITH, WD_L2>(b, grid, cb, f, s);
+        launch_tensors_each_wd<ARITH, WD_L2>(b, grid, cb, f, nt, s);
     else
-        launch_tensors_each_wd<ARITH, WD_NONE>(b, grid, cb, f, s);
+        launch_tensors_each_wd<ARITH, WD_NONE>(b, grid, cb, f, nt, s);
 }
 
 }  // namespace
@@ -1325,17 +1425,18 @@ int ps_adam_step_tensors(int optimizer_id, size_t step, double lr, double beta1,
     }
     for (int i = 0; i < n_tensors; ++i)
         if (numels[i] != 0) items.push_back(tensor_item(tensors, numels, i));
+    const bool nt = streams(tensors, numels, n_tensors, d_state != nullptr);
     return for_each_tensor_batch(items, tensors, first_tensor, 0, [&](const auto& b, dim3 grid, const BatchClasses&) {
         if (d_state == nullptr) {
             if (arith == PS_ARITH_TORCH)
-                launch_tensors_arith<PS_ARITH_TORCH>(b, grid, c, s);
+                launch_tensors_arith<PS_ARITH_TORCH>(b, grid, c, nt, s);
             else
-                launch_tensors_arith<PS_ARITH_OPERATOR>(b, grid, c, s);
+                launch_tensors_arith<PS_ARITH_OPERATOR>(b, grid, c, nt, s);
         } else {
             if (arith == PS_ARITH_TORCH)
-                launch_tensors_gated_arith<PS_ARITH_TORCH>(b, grid, ga, d_state, s);
+                launch_tensors_gated_arith<PS_ARITH_TORCH>(b, grid, ga, d_state, nt, s);
             else
-                launch_tensors_gated_arith<PS_ARITH_OPERATOR>(b, grid, ga, d_state, s);
+                launch_tensors_gated_arith<PS_ARITH_OPERATOR>(b, grid, ga, d_state, nt, s);
         }
     });
 }
@@ -1371,6 +1472,7 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
             return fail(PS_ERR_BAD_ARG, "d_workspace must be 16-byte aligned");
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool nt = streams(tensors, numels, n_tensors, d_state != nullptr);
     const bool bias = bias_correction != 0;
     auto arith_of = [&](int i) { return each[i].arithmetic < 0 ? o->arith : each[i].arithmetic; };
     auto grad_f32_of = [&](int i) { return (each[i].flags & PS_TENSOR_GRAD_F32) != 0; };
@@ -1418,9 +1520,9 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     memset(&cb, 0, sizeof(cb));
                     for (int q = 0; q < bc.n; ++q) cb.c[q] = consts[bc.of[q]];
                     if (f.arith == PS_ARITH_TORCH)
-                        launch_tensors_each_arith<PS_ARITH_TORCH>(b, grid, cb, f, s);
+                        launch_tensors_each_arith<PS_ARITH_TORCH>(b, grid, cb, f, nt, s);
                     else
-                        launch_tensors_each_arith<PS_ARITH_OPERATOR>(b, grid, cb, f, s);
+                        launch_tensors_each_arith<PS_ARITH_OPERATOR>(b, grid, cb, f, nt, s);
                 }, f.grad_f32);
                 if (rc) return rc;
             }
@@ -1510,9 +1612,9 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     int rc = for_each_tensor_batch(items, tensors, -1, 0,
                                                    [&](const auto& b, dim3 grid, const BatchClasses&) {
                         if (key_arith(key) == PS_ARITH_TORCH)
-                            launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, wd_mode, grad_f32, table + window, d_state, s);
+                            launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, wd_mode, grad_f32, table + window, d_state, nt, s);
                         else
-                            launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, wd_mode, grad_f32, table + window, d_state, s);
+                            launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, wd_mode, grad_f32, table + window, d_state, nt, s);
                     }, grad_f32);
                     if (rc) return rc;
                 }
@@ -1609,12 +1711,14 @@ int ps_adam_step_hybrid(int optimizer_id, size_t step, double lr, double beta1, 
         // the resident chunks' kernels, queued next on the caller's stream, do NOT hold the copies back
         if (int rc = p->begin(caller)) return rc;
     }
+    // (beside host chunks the link sets the pace, and 11 workgroups per CU here leave less room for theirs: 17.97 -> 18.10 ms)
+    const bool nt = !stream_host && streams(resident, d_state != nullptr);
     int rc = for_each_batch(resident, [&](const ChunkBatch& b, dim3 grid, int first) {
         const FirstCall fc = k.in_batch(first, (int)grid.y);
         if (d_state == nullptr)
-            launch_adam_batch(arith, b, grid, c_resident, fc, caller);
+            launch_adam_batch(arith, b, grid, c_resident, fc, nt, caller);
         else
-            launch_gated_batch(arith, b, grid, chunk_numel, ga, fc, d_state, caller);
+            launch_gated_batch(arith, b, grid, chunk_numel, ga, fc, d_state, nt, caller);
     });
     if (!stream_host) return rc;
 
@@ -1646,9 +1750,9 @@ int ps_adam_step_hybrid(int optimizer_id, size_t step, double lr, double beta1, 
         dim3 grid((unsigned)((numel + kTile - 1) / kTile), 1);
         const FirstCall fc = k.in_batch((int64_t)n_chunks + k_host, 1);
         if (d_state == nullptr)
-            launch_adam_batch(PS_ARITH_OPERATOR, b, grid, c_host, fc, p->compute);
+            launch_adam_batch(PS_ARITH_OPERATOR, b, grid, c_host, fc, false, p->compute);
         else  // the staged copy ends at `numel`: nothing behind it for the kernel to decide about
-            launch_gated_batch(PS_ARITH_OPERATOR, b, grid, numel, ga, fc, d_state, p->compute);
+            launch_gated_batch(PS_ARITH_OPERATOR, b, grid, numel, ga, fc, d_state, false, p->compute);
         PS_HIP(hipGetLastError());
         PS_HIP(hipEventRecord(p->compute_done[s], p->compute));
 
@@ -1669,9 +1773,9 @@ int ps_adam_step_hybrid(int optimizer_id, size_t step, double lr, double beta1, 
             rc = for_each_batch(host, [&](const ChunkBatch& b, dim3 grid, int first) {
                 const FirstCall fc = k.in_batch((int64_t)n_chunks + first, (int)grid.y);
                 if (d_state == nullptr)
-                    launch_adam_batch(PS_ARITH_OPERATOR, b, grid, c_host, fc, p->compute);
+                    launch_adam_batch(PS_ARITH_OPERATOR, b, grid, c_host, fc, false, p->compute);
                 else  // chunk_numel 0: as on a staged copy, what lies behind the used part is not looked at
-                    launch_gated_batch(PS_ARITH_OPERATOR, b, grid, 0, ga, fc, d_state, p->compute);
+                    launch_gated_batch(PS_ARITH_OPERATOR, b, grid, 0, ga, fc, d_state, false, p->compute);
             });
     } else {
         for (int i = 0; i < n_host_chunks && rc == 0; ++i) rc = stream_chunk(i);
@@ -1848,15 +1952,20 @@ int ps_overflow_scan_chunks(const ps_chunk* chunks, int n_chunks, size_t chunk_n
     ChunkList a;
     if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kScanTile, true)) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool nt = elements(a) >= kScanStreamElements;
     EvenList e;
     if (even_list(a, kMaxEvenElementsGated, &e, true)) {
-        hipLaunchKernelGGL(scan_even_chunks_kernel, even_grid(e, kScanTile), dim3(kScanBlock), kScanLdsBytes, s, e.first.param_fp16, e.stride,
-                           e.numel, e.last, e.short_by, d_state);
+        with_hint(nt, [&](auto hint) {
+            hipLaunchKernelGGL((scan_even_chunks_kernel<decltype(hint)::value>), even_grid(e, kScanTile), dim3(kScanBlock), kScanLdsBytes, s,
+                               e.first.param_fp16, e.stride, e.numel, e.last, e.short_by, d_state);
+        });
         PS_HIP(hipGetLastError());
         return 0;
     }
     return for_each_batch(a, [&](const ChunkBatch& b, dim3 grid, int) {
-        hipLaunchKernelGGL(scan_chunks_kernel, grid, dim3(kScanBlock), kScanLdsBytes, s, b, d_state);
+        with_hint(nt, [&](auto hint) {
+            hipLaunchKernelGGL((scan_chunks_kernel<decltype(hint)::value>), grid, dim3(kScanBlock), kScanLdsBytes, s, b, d_state);
+        });
     });
 }
 

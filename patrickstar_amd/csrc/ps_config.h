@@ -20,8 +20,11 @@
 #ifndef PS_NEAR_LDS_KB
 #define PS_NEAR_LDS_KB 14  // the same for the one-launch tensor lists: 11 workgroups per CU (their waves take longer to their first load)
 #endif
-#ifndef PS_STREAMING
-#define PS_STREAMING 0  // bit 0: non-temporal loads, bit 1: non-temporal stores of chunk payloads (both slower on MI355X)
+#ifndef PS_STREAM_LDS_KB
+#define PS_STREAM_LDS_KB 14  // PS_LDS_KB of the kernels that stream past the caches: 11 workgroups per CU
+#endif
+#ifndef PS_STREAM_NEAR_LDS_KB
+#define PS_STREAM_NEAR_LDS_KB 12  // PS_NEAR_LDS_KB of those: 13 workgroups per CU
 #endif
 // Launch shape of the inf/nan probe kernels (pure read streams).  Measured on 3.2 GB of fp16 payloads: single-wave
 // workgroups with 8 loads per lane and 6 resident workgroups per CU read 6.85 TB/s; 256 threads x 4 loads, uncapped,

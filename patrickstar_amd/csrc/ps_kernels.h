@@ -60,7 +60,7 @@ __device__ __forceinline__ CallSpan call_span(const FirstCall& fc)
 
 // Host-decided step: all scalars arrive as kernel arguments and the
 // arithmetic variant is a compile-time property of the kernel.
-template <int ARITH, int WD, int UNS>
+template <int ARITH, int WD, int UNS, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_chunks_kernel(ChunkBatch b, StepConsts c, FirstCall fc)
 {
@@ -69,8 +69,10 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     const CallSpan s = call_span(fc);
     const size_t base = (size_t)blockIdx.x * kTile;
     if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
-        adam_tile_vec<ARITH, WD, UNS>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, t.p32,
-                                      t.m32, t.v32, t.h16, base);
+        LaneTile r;
+        tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
+        tile_finish<ARITH, WD, UNS, false, NT>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r,
+                                               t.p32, t.m32, t.v32, t.h16, base);
         return;
     }
     if (base >= t.numel) return;  // the grid is as wide as the longest chunk of the batch
@@ -95,7 +97,7 @@ __device__ __forceinline__ EvenChunk even_chunk(float* p32, float* m32, float* v
     return EvenChunk{p32 + at, m32 + at, v32 + at, h16 + at, (size_t)(numel - (blockIdx.y == last ? short_by : 0u))};
 }
 
-template <int ARITH, int WD, int UNS>
+template <int ARITH, int WD, int UNS, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_even_chunks_kernel(float* p32, float* m32, float* v32, uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last,
                             uint32_t short_by, StepConsts c, FirstCall fc)
@@ -104,11 +106,11 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     const size_t base = (size_t)blockIdx.x * kTile;
     if (blockIdx.x < whole_tiles(t.numel)) {
         LaneTile r;
-        tile_load(r, t.p32, t.m32, t.v32, t.h16, base);
+        tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
         __builtin_amdgcn_sched_barrier(0);  // the loads in front of the wait for the arguments behind the preloaded ones
         const CallSpan s = call_span(fc);
         if (!s.cut) {
-            tile_finish<ARITH, WD, UNS>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r, t.p32,
+            tile_finish<ARITH, WD, UNS, false, NT>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r, t.p32,
                                         t.m32, t.v32, t.h16, base);
             return;
         }
@@ -193,7 +195,7 @@ __host__ __device__ inline bool zeros_are_a_fixed_point(const StepConsts& c)
     return c.eps > 0.0f && (s - s) == 0.0f;  // every term finite (no NaN, and no infinities: inf - inf is NaN)
 }
 
-template <int ARITH, int WD>
+template <int ARITH, int WD, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_chunks_gated_kernel(ChunkBatch b, size_t chunk_numel, GatedArgs ga, FirstCall fc,
                              const ps_step_state* __restrict__ st)
@@ -209,9 +211,9 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     }
     if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
         LaneTile r;
-        tile_load(r, t.p32, t.m32, t.v32, t.h16, base);
+        tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
         const StepConsts c = gated_consts<ARITH>(ga, sv, s.here);
-        tile_finish<ARITH, WD, UNSCALE_RUNTIME>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r,
+        tile_finish<ARITH, WD, UNSCALE_RUNTIME, false, NT>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r,
                                                 t.p32, t.m32, t.v32, t.h16, base);
         return;
     }
@@ -225,7 +227,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
                                                       numel, s.here ? fc.lo : 0, s.here ? fc.hi : 0);
 }
 
-template <int ARITH, int WD>
+template <int ARITH, int WD, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_even_chunks_gated_kernel(float* p32, float* m32, float* v32, uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last,
                                   uint32_t short_by, const ps_step_state* __restrict__ st, size_t chunk_numel, GatedArgs ga, FirstCall fc)
@@ -240,12 +242,12 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     }
     if (blockIdx.x < whole_tiles(t.numel)) {
         LaneTile r;
-        tile_load(r, t.p32, t.m32, t.v32, t.h16, base);
+        tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
         __builtin_amdgcn_sched_barrier(0);
         const CallSpan s = call_span(fc);
         if (!s.cut) {
             const StepConsts c = gated_consts<ARITH>(ga, sv, s.here);
-            tile_finish<ARITH, WD, UNSCALE_RUNTIME>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv,
+            tile_finish<ARITH, WD, UNSCALE_RUNTIME, false, NT>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv,
                                                     r, t.p32, t.m32, t.v32, t.h16, base);
             return;
         }
@@ -396,7 +398,7 @@ __device__ __forceinline__ void adam_head(const StepConsts& c, const ps_chunk& t
 
 // One tile of a tensor, which is one operator call: all of its elements take the first call's scalars, or none.  As in
 // adam_tile_late_consts the constants are formed after the tile's loads have been issued.
-template <int ARITH, int WD, int UNS, typename MakeConsts>
+template <int ARITH, int WD, int UNS, bool NT, typename MakeConsts>
 __device__ __forceinline__ void adam_tensor_tile(MakeConsts make_consts, const TensorView& w, bool first)
 {
     const ps_chunk t = as_chunk(w.t);
@@ -404,15 +406,15 @@ __device__ __forceinline__ void adam_tensor_tile(MakeConsts make_consts, const T
     const int access = (uint32_t)w.tile < whole_tiles(w.numel) ? tile_access(t) : TILE_ELEMENTWISE;
     if (access == TILE_ALIGNED) {
         LaneTile r;
-        tile_load(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+        tile_load<false, NT>(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
         const StepConsts c = make_consts();
-        tile_finish<ARITH, WD, UNS>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r, t.param_fp32,
+        tile_finish<ARITH, WD, UNS, false, NT>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r, t.param_fp32,
                                     t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
     } else if (access == TILE_STATE_DWORD_ALIGNED) {
         LaneTile r;
-        tile_load<true>(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+        tile_load<true, NT>(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
         const StepConsts c = make_consts();
-        tile_finish<ARITH, WD, UNS, true>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r,
+        tile_finish<ARITH, WD, UNS, true, NT>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r,
                                           t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
     } else if (base < w.numel) {  // (the grid is as wide as the longest tensor of the batch)
         const StepConsts c = make_consts();
@@ -435,7 +437,7 @@ __device__ __forceinline__ void restore_tensor_tiles(const ps_chunk& t, const Te
     for (unsigned u = 1; u < kRestoreTiles; ++u) restore_tile(t.param_fp32, t.param_fp16, (size_t)(u * kRestoreStride - 1) * kTile, w.numel);
 }
 
-template <typename LIST, int ARITH, int WD, int UNS>
+template <typename LIST, int ARITH, int WD, int UNS, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_tensors_kernel(LIST b, StepConsts c)
 {
@@ -445,10 +447,10 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNS>(c, as_chunk(w.t), w.head, first);
         return;
     }
-    adam_tensor_tile<ARITH, WD, UNS>([&]() { return c; }, w, first);
+    adam_tensor_tile<ARITH, WD, UNS, NT>([&]() { return c; }, w, first);
 }
 
-template <typename LIST, int ARITH, int WD>
+template <typename LIST, int ARITH, int WD, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_tensors_gated_kernel(LIST b, GatedArgs ga, const ps_step_state* __restrict__ st)
 {
@@ -466,7 +468,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNSCALE_RUNTIME>(gated_consts<ARITH>(ga, sv, first), t, w.head, first);
         return;
     }
-    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME>([&]() { return gated_consts<ARITH>(ga, sv, first); }, w, first);
+    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME, NT>([&]() { return gated_consts<ARITH>(ga, sv, first); }, w, first);
 }
 
 // A step whose tensors carry their own step numbers and hyper-parameters: calls that come out with the same constants
@@ -483,7 +485,7 @@ struct ConstsBatch {
 static_assert(sizeof(TensorBatch) + sizeof(ConstsBatch) <= 4096 && sizeof(NearBatch) + sizeof(ConstsBatch) <= 4096, "kernel arguments of one launch");
 
 // No tensor is "the first call" here: a first call that differs is a class of its own.
-template <typename LIST, int ARITH, int WD, int UNS>
+template <typename LIST, int ARITH, int WD, int UNS, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_tensors_each_kernel(LIST b, ConstsBatch cb)
 {
@@ -493,7 +495,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNS>(cb.c[w.cls], t, w.head, false);
         return;
     }
-    adam_tensor_tile<ARITH, WD, UNS>([&]() { return cb.c[w.cls]; }, w, false);
+    adam_tensor_tile<ARITH, WD, UNS, NT>([&]() { return cb.c[w.cls]; }, w, false);
 }
 
 // The same for tensors whose gradient is binary32 and which have no binary16 copy (PS_TENSOR_GRAD_F32): the
@@ -517,7 +519,7 @@ struct PlannedConsts {
 };
 static_assert(sizeof(PlannedConsts) == 64, "one 64-byte record per class in the caller's workspace");
 
-template <typename LIST, int ARITH, int WD>
+template <typename LIST, int ARITH, int WD, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_tensors_planned_kernel(LIST b, const PlannedConsts* __restrict__ consts,
                                 const ps_step_state* __restrict__ st)
@@ -534,7 +536,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         adam_head<ARITH, WD, UNSCALE_RUNTIME>(consts[w.cls].c, t, w.head, false);
         return;
     }
-    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME>([&]() { return consts[w.cls].c; }, w, false);
+    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME, NT>([&]() { return consts[w.cls].c; }, w, false);
 }
 
 // PS_TENSOR_GRAD_F32 tensors of a device-decided step: a flagged step leaves them alone (there is no fp16 copy to
@@ -613,7 +615,7 @@ __global__ void __launch_bounds__(kAuxBlock)
 // launches, which the preloading makes 0.1 to 0.25 us longer (the element-wise operator, the lone gradient copy, the cast), take
 // their arguments in a struct, which is not preloaded.
 // STATE_DWORD_ALIGNED: exp_avg / exp_avg_sq sit at another 16-byte phase than the parameter (any element offset).
-template <int WD, int UNS, bool GRAD_HALF, bool HAS_OUT, bool STATE_DWORD_ALIGNED>
+template <int WD, int UNS, bool GRAD_HALF, bool HAS_OUT, bool STATE_DWORD_ALIGNED, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     adam_flat_vec_kernel(float* p32, const void* grads, float* m32, float* v32,
                          uint16_t* out16,  // may alias grads (fp16 gradients overwritten by fp16 parameters)
@@ -639,10 +641,10 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     uint2v w;
     float4v gv;
     if (GRAD_HALF)
-        w = *(const guint2v*)(static_cast<const uint16_t*>(grads) + i);
+        w = NT ? __builtin_nontemporal_load((const guint2v*)(static_cast<const uint16_t*>(grads) + i)) : *(const guint2v*)(static_cast<const uint16_t*>(grads) + i);
     else
-        gv = ld_f4(static_cast<const float*>(grads) + i);
-    float4v p = ld_f4(p32 + i), m = ld_f4_as<STATE_DWORD_ALIGNED>(m32 + i), v = ld_f4_as<STATE_DWORD_ALIGNED>(v32 + i);
+        gv = ld_f4<NT>(static_cast<const float*>(grads) + i);
+    float4v p = ld_f4<NT>(p32 + i), m = ld_f4_as<STATE_DWORD_ALIGNED, NT>(m32 + i), v = ld_f4_as<STATE_DWORD_ALIGNED, NT>(v32 + i);
     float g[4];
     if (GRAD_HALF) {
         g[0] = half_bits_to_float(w[0] & 0xFFFFu);
@@ -663,14 +665,17 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         v[e] = ve;
         h[e] = float_to_half_bits(pe);
     }
-    st_f4(p32 + i, p);
-    st_f4_as<STATE_DWORD_ALIGNED>(m32 + i, m);
-    st_f4_as<STATE_DWORD_ALIGNED>(v32 + i, v);
+    st_f4<NT>(p32 + i, p);
+    st_f4_as<STATE_DWORD_ALIGNED, NT>(m32 + i, m);
+    st_f4_as<STATE_DWORD_ALIGNED, NT>(v32 + i, v);
     if (HAS_OUT) {
         uint2v o;
         o[0] = h[0] | (h[1] << 16);
         o[1] = h[2] | (h[3] << 16);
-        *(guint2v*)(out16 + i) = o;
+        if (NT)
+            __builtin_nontemporal_store(o, (guint2v*)(out16 + i));
+        else
+            *(guint2v*)(out16 + i) = o;
     }
 }
 
@@ -736,7 +741,7 @@ typedef uint4v __attribute__((aligned(4))) uint4v_word_aligned;
 // As a loop over single elements such a tile was a chain of up to 64 waits for memory, and the launch was no faster
 // than that chain: 12.2 us for 3 chunks of 6267 halves (2.8 us now), 70.1 us for the four part-filled chunks of a
 // BERT-base-sized module (62.6 us now; 109 M halves, read while the update before it is still being written back).
-template <typename Element, int BLOCK, int UNROLL>
+template <typename Element, int BLOCK, int UNROLL, bool NT = false>
 __device__ __forceinline__ uint32_t scan_tile(const Element* __restrict__ x, size_t numel, size_t tile)
 {
     constexpr bool kHalf = sizeof(Element) == 2;
@@ -758,7 +763,7 @@ __device__ __forceinline__ uint32_t scan_tile(const Element* __restrict__ x, siz
     if ((((uintptr_t)x) & 15u) == 0 && left >= kElems) {
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
-            w[u] = ld_u4(reinterpret_cast<const uint16_t*>(t + (size_t)(u * BLOCK + threadIdx.x) * kVec));
+            w[u] = ld_u4<NT>(reinterpret_cast<const uint16_t*>(t + (size_t)(u * BLOCK + threadIdx.x) * kVec));
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u) hit |= nonfinite(w[u]);
         return hit;
@@ -799,18 +804,20 @@ __global__ void __launch_bounds__(kScanBlock)
     block_flag_commit<kScanBlock>(hit, &st->overflow);
 }
 
+template <bool NT>
 __global__ void __launch_bounds__(kScanBlock)
     scan_chunks_kernel(ChunkBatch b, ps_step_state* st)
 {
-    uint32_t hit = scan_tile<uint16_t, kScanBlock, kScanUnroll>(b.c[blockIdx.y].param_fp16, b.n[blockIdx.y], blockIdx.x);
+    uint32_t hit = scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(b.c[blockIdx.y].param_fp16, b.n[blockIdx.y], blockIdx.x);
     block_flag_commit<kScanBlock>(hit, &st->overflow);
 }
 
+template <bool NT>
 __global__ void __launch_bounds__(kScanBlock)
     scan_even_chunks_kernel(const uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last, uint32_t short_by, ps_step_state* st)
 {
     const uint32_t n = numel - (blockIdx.y == last ? short_by : 0u);
-    uint32_t hit = scan_tile<uint16_t, kScanBlock, kScanUnroll>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x);
+    uint32_t hit = scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x);
     block_flag_commit<kScanBlock>(hit, &st->overflow);
 }
 

@@ -21,60 +21,61 @@ typedef PS_GLOBAL float4v gfloat4v;
 typedef PS_GLOBAL uint4v guint4v;
 typedef PS_GLOBAL uint2v guint2v;
 
+// NT: with the non-temporal hint.
+template <bool NT = false>
 __device__ __forceinline__ float4v ld_f4(const float* p)
 {
-#if PS_STREAMING & 1
-    return __builtin_nontemporal_load((const gfloat4v*)(p));
-#else
-    return *(const gfloat4v*)(p);
-#endif
+    return NT ? __builtin_nontemporal_load((const gfloat4v*)(p)) : *(const gfloat4v*)(p);
 }
+template <bool NT = false>
 __device__ __forceinline__ void st_f4(float* p, float4v v)
 {
-#if PS_STREAMING & 2
-    __builtin_nontemporal_store(v, (gfloat4v*)(p));
-#else
-    *(gfloat4v*)(p) = v;
-#endif
+    if (NT)
+        __builtin_nontemporal_store(v, (gfloat4v*)(p));
+    else
+        *(gfloat4v*)(p) = v;
 }
+template <bool NT = false>
 __device__ __forceinline__ uint4v ld_u4(const uint16_t* p)
 {
-#if PS_STREAMING & 1
-    return __builtin_nontemporal_load((const guint4v*)(p));
-#else
-    return *(const guint4v*)(p);
-#endif
+    return NT ? __builtin_nontemporal_load((const guint4v*)(p)) : *(const guint4v*)(p);
 }
+template <bool NT = false>
 __device__ __forceinline__ void st_u4(uint16_t* p, uint4v v)
 {
-#if PS_STREAMING & 2
-    __builtin_nontemporal_store(v, (guint4v*)(p));
-#else
-    *(guint4v*)(p) = v;
-#endif
+    if (NT)
+        __builtin_nontemporal_store(v, (guint4v*)(p));
+    else
+        *(guint4v*)(p) = v;
 }
 
 // 16 bytes at an address that is only 4-byte aligned (multi-dword global accesses need dword alignment only): for
 // momentum / variance tensors that sit at another 16-byte phase than their parameter.
 typedef float4v __attribute__((aligned(4))) float4v_dword_aligned;
-template <bool DWORD_ALIGNED>
+typedef PS_GLOBAL float4v_dword_aligned gfloat4v_dword_aligned;
+template <bool DWORD_ALIGNED, bool NT = false>
 __device__ __forceinline__ float4v ld_f4_as(const float* p)
 {
-    if (DWORD_ALIGNED) return *(const PS_GLOBAL float4v_dword_aligned*)(p);
-    return ld_f4(p);
+    if (!DWORD_ALIGNED) return ld_f4<NT>(p);
+    if (NT) return __builtin_nontemporal_load((const gfloat4v_dword_aligned*)(p));
+    return *(const gfloat4v_dword_aligned*)(p);
 }
-template <bool DWORD_ALIGNED>
+template <bool DWORD_ALIGNED, bool NT = false>
 __device__ __forceinline__ void st_f4_as(float* p, float4v v)
 {
-    if (DWORD_ALIGNED)
-        *(PS_GLOBAL float4v_dword_aligned*)(p) = v;
+    if (!DWORD_ALIGNED)
+        st_f4<NT>(p, v);
+    else if (NT)
+        __builtin_nontemporal_store(v, (gfloat4v_dword_aligned*)(p));
     else
-        st_f4(p, v);
+        *(gfloat4v_dword_aligned*)(p) = v;
 }
 
 constexpr int kBlock = PS_BLOCK;
 constexpr unsigned kLdsBytes = PS_LDS_KB * 1024u;
 constexpr unsigned kNearLdsBytes = PS_NEAR_LDS_KB * 1024u;
+constexpr unsigned kStreamLdsBytes = PS_STREAM_LDS_KB * 1024u;
+constexpr unsigned kStreamNearLdsBytes = PS_STREAM_NEAR_LDS_KB * 1024u;
 // Elements per lane per vector step.  8: one 16-byte access of fp16 and two
 // 16-byte accesses per fp32 array.  4: an 8-byte access of fp16 and one
 // 16-byte access per fp32 array.
@@ -91,41 +92,70 @@ struct HalfWords {
     uint32_t w[kWords];
 };
 
+template <bool NT = false>
 __device__ __forceinline__ HalfWords ld_halves(const uint16_t* p)
 {
     HalfWords r;
     if (kWords == 4) {
-        uint4v t = ld_u4(p);
+        uint4v t = ld_u4<NT>(p);
 #pragma unroll
         for (int k = 0; k < kWords; ++k) r.w[k] = t[k];
     } else {
-#if PS_STREAMING & 1
-        uint2v t = __builtin_nontemporal_load((const guint2v*)(p));
-#else
-        uint2v t = *(const guint2v*)(p);
-#endif
+        uint2v t = NT ? __builtin_nontemporal_load((const guint2v*)(p)) : *(const guint2v*)(p);
 #pragma unroll
         for (int k = 0; k < kWords; ++k) r.w[k] = t[k];
     }
     return r;
 }
 
+template <bool NT = false>
 __device__ __forceinline__ void st_halves(uint16_t* p, const HalfWords& r)
 {
     if (kWords == 4) {
         uint4v t;
 #pragma unroll
         for (int k = 0; k < kWords; ++k) t[k] = r.w[k];
-        st_u4(p, t);
+        st_u4<NT>(p, t);
     } else {
         uint2v t;
 #pragma unroll
         for (int k = 0; k < kWords; ++k) t[k] = r.w[k];
-#if PS_STREAMING & 2
-        __builtin_nontemporal_store(t, (guint2v*)(p));
-#else
-        *(guint2v*)(p) = t;
-#endif
+        if (NT)
+            __builtin_nontemporal_store(t, (guint2v*)(p));
+        else
+            *(guint2v*)(p) = t;
+    }
+}
+
+// Stores of one lane's share of a tile; `first`: the tile's first element, the same in every lane.  With the hint they are buffer
+// stores, whose cache policy is an operand: a plain store's hint is metadata, which the compiler drops where it merges the
+// stores of several branches (of every kernel that decides on the device how to unscale).
+constexpr int kBufferFlags = 0x00027000;  // raw buffer, 32-bit data format
+constexpr int kCacheNt = 2;               // cache policy: non-temporal
+template <bool DWORD_ALIGNED, bool NT>
+__device__ __forceinline__ void st_tile(float* first, int q, float4v v)
+{
+    if (NT) {
+        const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(first, 0, kTile * (int)sizeof(float), kBufferFlags);
+        uint4v w;
+        __builtin_memcpy(&w, &v, sizeof(w));
+        __builtin_amdgcn_raw_buffer_store_b128(w, b, (int)(threadIdx.x * kLaneElems + 4 * q) * 4, 0, kCacheNt);
+    } else {
+        st_f4_as<DWORD_ALIGNED>(first + (size_t)threadIdx.x * kLaneElems + 4 * q, v);
+    }
+}
+template <bool NT>
+__device__ __forceinline__ void st_tile_halves(uint16_t* first, const HalfWords& r)
+{
+    if (NT) {
+        static_assert(kWords == 2, "8 bytes of fp16 a lane");
+        const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(first, 0, kTile * (int)sizeof(uint16_t), kBufferFlags);
+        uint2v w;
+        w[0] = r.w[0];
+        w[1] = r.w[1];
+        __builtin_amdgcn_raw_buffer_store_b64(w, b, (int)threadIdx.x * 8, 0, kCacheNt);
+    } else {
+        st_halves(first + (size_t)threadIdx.x * kLaneElems, r);
     }
 }
 
@@ -171,25 +201,25 @@ __device__ __forceinline__ void lane_math(const StepConsts& c, float step_size, 
 // branch on the arithmetic variant.
 // The loads of one whole, aligned tile: all of them issued back to back, nothing waited for.
 // STATE_DWORD_ALIGNED: exp_avg / exp_avg_sq are only 4-byte aligned (the parameter lists are aligned as always).
-template <bool STATE_DWORD_ALIGNED = false>
+template <bool STATE_DWORD_ALIGNED = false, bool NT = false>
 __device__ __forceinline__ void tile_load(LaneTile& r, const float* __restrict__ p32, const float* __restrict__ m32,
                                           const float* __restrict__ v32, const uint16_t* __restrict__ h16, size_t base)
 {
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
         size_t i = base + ((size_t)u * kBlock + threadIdx.x) * kLaneElems;
-        r.g[u] = ld_halves(h16 + i);
+        r.g[u] = ld_halves<NT>(h16 + i);
 #pragma unroll
-        for (int q = 0; q < kQuads; ++q) r.p[u][q] = ld_f4(p32 + i + 4 * q);
+        for (int q = 0; q < kQuads; ++q) r.p[u][q] = ld_f4<NT>(p32 + i + 4 * q);
 #pragma unroll
-        for (int q = 0; q < kQuads; ++q) r.m[u][q] = ld_f4_as<STATE_DWORD_ALIGNED>(m32 + i + 4 * q);
+        for (int q = 0; q < kQuads; ++q) r.m[u][q] = ld_f4_as<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(m32 + i + 4 * q);
 #pragma unroll
-        for (int q = 0; q < kQuads; ++q) r.v[u][q] = ld_f4_as<STATE_DWORD_ALIGNED>(v32 + i + 4 * q);
+        for (int q = 0; q < kQuads; ++q) r.v[u][q] = ld_f4_as<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(v32 + i + 4 * q);
     }
 }
 
 // Arithmetic and stores of a tile whose loads are under way.
-template <int ARITH, int WD, int UNS, bool STATE_DWORD_ALIGNED = false>
+template <int ARITH, int WD, int UNS, bool STATE_DWORD_ALIGNED = false, bool NT = false>
 __device__ __forceinline__ void tile_finish(const StepConsts& c, float step_size, float bc2inv, LaneTile& r,
                                             float* __restrict__ p32, float* __restrict__ m32,
                                             float* __restrict__ v32, uint16_t* __restrict__ h16, size_t base)
@@ -205,14 +235,14 @@ __device__ __forceinline__ void tile_finish(const StepConsts& c, float step_size
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-        size_t i = base + ((size_t)u * kBlock + threadIdx.x) * kLaneElems;
+        const size_t first = base + (size_t)u * kBlock * kLaneElems;  // the wave's, the same in every lane
 #pragma unroll
-        for (int q = 0; q < kQuads; ++q) st_f4(p32 + i + 4 * q, r.p[u][q]);
-#pragma unroll
-        for (int q = 0; q < kQuads; ++q) st_f4_as<STATE_DWORD_ALIGNED>(m32 + i + 4 * q, r.m[u][q]);
-#pragma unroll
-        for (int q = 0; q < kQuads; ++q) st_f4_as<STATE_DWORD_ALIGNED>(v32 + i + 4 * q, r.v[u][q]);
-        st_halves(h16 + i, r.h[u]);
+        for (int q = 0; q < kQuads; ++q) {
+            st_tile<false, NT>(p32 + first, q, r.p[u][q]);
+            st_tile<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(m32 + first, q, r.m[u][q]);
+            st_tile<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(v32 + first, q, r.v[u][q]);
+        }
+        st_tile_halves<NT>(h16 + first, r.h[u]);
     }
 }
 
