@@ -206,7 +206,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     StateView sv = view_state(st);  // asked for at once, as in tile_source
     asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
     if (__builtin_expect(sv.overflow, 0)) {
-        if (restore_leader(blockIdx.x)) restore_tiles(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
+        if (restore_leader(blockIdx.x)) restore_tiles<NT>(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
         return;
     }
     if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     StateView sv = view_state(st);
     asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
     if (__builtin_expect(sv.overflow, 0)) {
-        if (restore_leader(blockIdx.x)) restore_tiles(t.p32, t.h16, base, t.numel);
+        if (restore_leader(blockIdx.x)) restore_tiles<NT>(t.p32, t.h16, base, t.numel);
         return;
     }
     if (blockIdx.x < whole_tiles(t.numel)) {
@@ -424,11 +424,12 @@ __device__ __forceinline__ void adam_tensor_tile(MakeConsts make_consts, const T
 }
 
 // fp16 <- RNE(fp32) of this workgroup's tiles (a skipped step).
+template <bool NT>
 __device__ __forceinline__ void restore_tensor_tiles(const ps_chunk& t, const TensorView& w)
 {
     if (!restore_leader(w.x)) return;
     if (w.tile >= 0) {
-        restore_tiles(t.param_fp32, t.param_fp16, (size_t)w.tile * kTile, w.numel);
+        restore_tiles<NT>(t.param_fp32, t.param_fp16, (size_t)w.tile * kTile, w.numel);
         return;
     }
     // workgroup 0 of a tensor with elements in front of its tile grid: those, and the tiles it leads
@@ -461,7 +462,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     if (w.tile >= 0 && base >= w.numel) return;
     const StateView sv = view_state(st);
     if (__builtin_expect(sv.overflow, 0)) {
-        restore_tensor_tiles(t, w);
+        restore_tensor_tiles<NT>(t, w);
         return;
     }
     if (w.tile < 0) {
@@ -529,7 +530,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     const size_t base = w.tile < 0 ? 0 : (size_t)w.tile * kTile;
     if (w.tile >= 0 && base >= w.numel) return;
     if (__builtin_expect(st->overflow, 0)) {
-        restore_tensor_tiles(t, w);
+        restore_tensor_tiles<NT>(t, w);
         return;
     }
     if (w.tile < 0) {

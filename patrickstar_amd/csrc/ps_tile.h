@@ -445,11 +445,13 @@ __device__ __forceinline__ void restore_tile(const float* __restrict__ p32,
 // consecutive ones: 1197).  8 x 64 Mi elements, 3.2 GB, under the cap of 9: 950 us with a tile each; 2 / 4 / 8 tiles 32
 // apart 579 / 499 / 513 us, 4 tiles 64 / 256 / 2048 apart 494 / 494 / 633.  (A launch of which every workgroup leaves at
 // once takes 441 us; the stand-alone write-back, uncapped, moves the same bytes in 495.)
+// With the non-temporal hint (in the kernels of long lists) a skipped step over 8 x 64 Mi elements, probe included, 651 -> 613 us.
 constexpr unsigned kRestoreTiles = 4, kRestoreStride = 32;
 // x: the workgroup's number among those of its chunk or tensor
 __device__ __forceinline__ bool restore_leader(uint32_t x) { return x % (kRestoreTiles * kRestoreStride) < kRestoreStride; }
 
 // base: the first of the workgroup's tiles
+template <bool NT = false>
 __device__ __forceinline__ void restore_tiles(const float* __restrict__ p32, uint16_t* __restrict__ h16, size_t base, size_t numel)
 {
     static_assert(kLaneElems == 4 && kUnroll == 1, "one 16-byte load per lane and tile");
@@ -458,14 +460,14 @@ __device__ __forceinline__ void restore_tiles(const float* __restrict__ p32, uin
         const size_t i = base + (size_t)threadIdx.x * kLaneElems;
         float4v a[kRestoreTiles];
 #pragma unroll
-        for (unsigned u = 0; u < kRestoreTiles; ++u) a[u] = ld_f4(p32 + i + u * step);
+        for (unsigned u = 0; u < kRestoreTiles; ++u) a[u] = ld_f4<NT>(p32 + i + u * step);
         __builtin_amdgcn_sched_barrier(0);  // the compiler converts each tile before it asks for the next otherwise
 #pragma unroll
         for (unsigned u = 0; u < kRestoreTiles; ++u) {
             HalfWords out;
             out.w[0] = float_to_half_bits(a[u][0]) | (float_to_half_bits(a[u][1]) << 16);
             out.w[1] = float_to_half_bits(a[u][2]) | (float_to_half_bits(a[u][3]) << 16);
-            st_halves(h16 + i + u * step, out);
+            st_tile_halves<NT>(h16 + base + u * step, out);
         }
         return;
     }
