@@ -9,13 +9,14 @@
 //     instruction covers a contiguous span of whole cache lines;
 //   * one small tile (256 elements) per single-wave workgroup and a CAP on
 //     resident workgroups (9 per CU, enforced by requesting 17 KiB of unused
-//     dynamic LDS; 11 with the hint below): the pass touches four arrays for reading and the same four
-//     for writing, and HBM efficiency drops when the set of in-flight cache
+//     dynamic LDS; 11 with the hint below): the pass touches four arrays for
+//     reading and the same four for writing, and HBM efficiency drops when the set of in-flight cache
 //     lines gets wide; a narrow, steadily advancing window per array gave
 //     6.3 TB/s where the fully occupied machine gave 5.3 TB/s (a plain
 //     1-read-1-write copy peaks at 6.3-6.4 TB/s on the same GPU);
 //   * chunk descriptors travel in the kernel-argument segment (64 per launch),
-//     so a wave's first data load depends on one scalar load, not two;
+//     so a wave's first data load depends on one scalar load, not two; evenly
+//     spaced chunks need 12 words, preloaded into scalar registers;
 //   * lists too long for the caches stream past them: non-temporal loads AND
 //     stores, and 11 instead of 9 workgroups per CU, 6.6 TB/s where plain
 //     accesses gave 6.25 (either hint alone gains nothing or loses 6 %).
@@ -265,7 +266,7 @@ void with_hint(bool nt, F launch)
 using EvenList = EvenBatch;
 //
 // Lists of up to this many elements take the kernels for it.  Longer ones are bound by memory from the first tile to the
-// last, and the general kernels are as fast or a little faster: host-decided 593.6 / 595.7 us for 128 Mi elements, 7226 /
+// last, and the general kernels are as fast or a little faster; with plain accesses host-decided 593.6 / 595.7 us for 128 Mi elements, 7226 /
 // 7236 for 1.5 Gi; device-decided 596.3 / 593.5 and 7176 / 7209, for 512 Mi 2377 / 2376.
 constexpr size_t kMaxEvenElements = (size_t)96 << 20, kMaxEvenElementsGated = (size_t)256 << 20;
 bool even_list(const ChunkList& a, size_t most, EvenList* out, bool fp16_only = false)

@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
 // PatrickStarClient allocates.  Addresses, distance and lengths are 12 words (with the step state's address 14), which are
 // preloaded into scalar registers, so a wave asks for its data, or for the step state, before it has waited for anything.
 //
-// Device time, descriptors / preloaded, host-decided: 128 K elements 2.60 / 2.36 us, 1 Mi 7.98 / 7.64, 4 Mi 23.3 / 22.7, 16 Mi
+// Device time with plain accesses, descriptors / preloaded, host-decided: 128 K elements 2.60 / 2.36 us, 1 Mi 7.98 / 7.64, 4 Mi 23.3 / 22.7, 16 Mi
 // 77.4 / 77.2; device-decided, with the probe and the scale update: 128 K 9.27 / 8.65, 1 Mi 15.4 / 13.8, 4 Mi 31.4 / 29.3, 16 Mi
 // 89.6 / 87.4, 64 Mi 327.3 / 324.3; the probe alone 2.19 / 1.87 at 1 Mi, 6.24 / 5.85 at 16 Mi.
 struct EvenChunk {
@@ -326,7 +326,8 @@ __device__ __forceinline__ TensorView tensor_view(const TensorBatch& b)
 // reaches its first data load after three rounds of scalar loads (segments, segment, tensor) and some 50 scalar
 // instructions, where TensorBatch needs one round, so 11 workgroups per CU instead of 9 keep as many loads in flight.
 //
-// What that buys is the ends of launches, 4 to 9 us each.  Device time in several launches (TensorBatch) / in one:
+// What that buys is the ends of launches, 4 to 9 us each.  Device time in several launches (TensorBatch) / in one, with plain
+// accesses (long lists that stream past the caches: 13 workgroups per CU, BERT-base 460 us, its upper half 182):
 // BERT-base, 199 tensors 517 / 500 us host-decided, 528 / 504 device-decided with a rate per layer; its upper half, 100
 // tensors 211 / 203 and 218 / 207; 12 layers of hidden size 64 14.6 / 5.8 and 20.4 / 10.6; 11 M elements with no two tensors
 // at the same phase 56.6 / 43.1.  With the cap of 9: BERT-base 508 and 520, with 12 533.  Longer lists gain less than the
