@@ -26,20 +26,23 @@ from .chunk_layout import (
 )
 
 # Where the three fp32 lists lie against one another.  A pass reads and writes the same element of all three at the same
-# time, and distances that are multiples of 128 MiB (which lists of power-of-two chunks back to back have) put those three
-# on the same memory banks.  64 Mi elements a list, distance over 256 MiB: 0 to 32 KiB 5.71-5.77 TB/s, 64 KiB 5.89, 256 KiB
-# 6.08, 1 MiB 6.27-6.29, 4 MiB 6.13-6.19, 6 to 17 MiB 6.26-6.35, 64 MiB 6.23, 128 MiB 5.84, 132 to 252 MiB 6.26-6.34; 9 MiB:
-# 6.28-6.31.  Lists that are allocations of their own lie as the allocator has it: 5.72 to 6.36 TB/s for the same list, by
-# what was allocated before.  At 9 MiB over a multiple of 64 MiB lists of 32 Mi to 256 Mi elements ran at 6.19-6.35 TB/s in
-# every process, against 5.73-6.35 on their own.  Up to 16 Mi elements the lists stay in the memory-side cache (8.3-8.7 TB/s
-# however they lie); from 384 Mi elements on lists of their own are as fast (6.28-6.35; 1.5 Gi elements in one allocation at
-# 8 MiB 6.10).
-ONE_ALLOCATION_BYTES = (80 << 20, 1 << 30)  # shortest and longest fp32 list that shares one
+# time.  With plain accesses distances that are multiples of 128 MiB (which lists of power-of-two chunks back to back have)
+# put those three on the same memory banks: 64 Mi elements a list, distance over 256 MiB, 0 to 32 KiB 5.71-5.77 TB/s, 64 KiB
+# 5.89, 1 MiB 6.27-6.29, 6 to 17 MiB 6.26-6.35, 64 MiB 6.23, 128 MiB 5.84.  Steps that stream past the caches (28 Mi elements and
+# up) run at 6.4 to 6.8 TB/s at every distance from 0 to 126 MiB, in no order that two processes share; what is left of the rule
+# shows in whole steps, each list in an allocation of its own / momentum and variance in one at any place / in one and clear
+# of the parameters, us: 24 Mi elements (plain) 113.9 / 114.4 / 112.7, 64 Mi 288.3 / 282.0 / 283.5, 2 x 64 Mi 572 / 569 / 561,
+# 4 x 64 Mi 1142 / 1119 / 1114, BERT-base with a rate per layer 504 / 508 / 502; 32 Mi 141 / 144 / 144.  (All three lists in
+# one allocation, the state's part kept from before there is an optimizer: the same within 1 %.)  Up to 16 Mi elements the
+# lists stay in the memory-side cache (8.3-8.7 TB/s however they lie).  Without the upper line 6 x 64 Mi gain 1.0 to 1.6 %,
+# 12 x 64 Mi 0.6 to 1.8, 8 x 64 Mi nothing, and 24 x 64 Mi lose 0.8 to 1.3.
+CLEAR_LIST_BYTES = (80 << 20, 1 << 30)  # shortest and longest fp32 list that is laid clear of the others
 LIST_PERIOD, LIST_CLEARANCE = 64 << 20, 9 << 20
+LIST_SLACK = 4 * LIST_CLEARANCE + (2 << 20)  # what list_shift may take
 
 
 def list_distance(nbytes):
-    """How far apart to start the fp32 lists of ``nbytes`` bytes each: the least distance that is neither itself nor doubled
+    """How far apart to start fp32 lists of ``nbytes`` bytes each: the least distance that is neither itself nor doubled
     nearly a multiple of 128 MiB."""
     past = nbytes % LIST_PERIOD
     if past < LIST_CLEARANCE:
@@ -47,6 +50,15 @@ def list_distance(nbytes):
     if past > LIST_PERIOD - LIST_CLEARANCE:
         return nbytes - past + LIST_PERIOD + LIST_CLEARANCE
     return nbytes
+
+
+def list_shift(apart, distance):
+    """How far into their allocation to lay two lists that start ``distance`` apart, where that allocation starts ``apart``
+    bytes from the list both are to be clear of (in whole MiB, at most ``LIST_SLACK``)."""
+    shift = 0
+    while any(min(at % LIST_PERIOD, -at % LIST_PERIOD) < LIST_CLEARANCE for at in (apart + shift, apart + shift + distance)):
+        shift += 1 << 20
+    return shift
 
 
 class ChunkPosition:
@@ -101,7 +113,6 @@ class PatrickStarClient:
         # False: it stays in HBM, where forward and backward use it (the only form a registered module can have)
         self.host_keeps_fp16 = True
         self._slabs = []  # the lists' memory that HBM-resident payloads are views of
-        self._reserved = {}  # (state list, fp16 chunk id) -> memory for the state chunk of that position
         # called with (position index among fp16 chunks) -> True to keep that position in host memory
         self.host_chunk_policy: Optional[Callable[[int], bool]] = None
         default_opts = {"with_mem_saving_comm": False, "with_mem_cache": False, "with_async_move": False}
@@ -319,8 +330,8 @@ class PatrickStarClient:
 
         HBM-resident chunks of one list are carved out of ONE allocation per call (a slab): a few large
         allocations are backed by large physical fragments, which the streaming kernels need when few waves
-        are in flight (measured: 6.30 TB/s from slabs vs 6.01 TB/s from one allocation per chunk).  The slabs of the
-        three fp32 lists, if they are long, are parts of one allocation and start ``list_distance`` apart.
+        are in flight (measured: 6.30 TB/s from slabs vs 6.01 TB/s from one allocation per chunk).  The slabs of momentum
+        and variance, if they are long, are parts of one allocation, laid clear of the fp32 parameters' (``_state_slabs``).
         Positions selected by the host-chunk policy get their own pinned host allocations instead.
         """
         ids16 = self.chunk_tensor_index.chunk_type_to_chunk_id_list_map.get(ChunkType.PARAM_FP16, [])
@@ -337,65 +348,54 @@ class PatrickStarClient:
                 chunk.allocate_payload("cpu", pin_memory=True)
             else:
                 pending.setdefault(chunk.chunk_type, []).append(chunk)
+
+        # every payload starts on a 512-element boundary of its slab (>= 1 KiB for every dtype), so that odd
+        # chunk sizes do not push later chunks off the alignment the vector kernels want
+        def stride(c):
+            return -(-c.capacity // 512) * 512
+
+        state_slabs = {}
+        momentum, variance = pending.get(ChunkType.MOMENTUM, []), pending.get(ChunkType.VARIANCE, [])
+        if self.device.type != "cpu" and momentum and [c.capacity for c in momentum] == [c.capacity for c in variance]:
+            state_slabs = self._state_slabs(momentum, variance, sum(stride(c) for c in momentum))
         for chunk_type, chunks in pending.items():
             if self.device.type == "cpu":
                 for chunk in chunks:
                     chunk.allocate_payload(self.device)
                 continue
-            # every payload starts on a 512-element boundary of its slab (>= 1 KiB for every dtype), so that odd
-            # chunk sizes do not push later chunks off the alignment the vector kernels want
-            def stride(c):
-                return -(-c.capacity // 512) * 512
-
-            if chunk_type in (ChunkType.MOMENTUM, ChunkType.VARIANCE):
-                chunks = self._take_reserved(chunk_type, chunks)
-                if not chunks:
-                    continue
-            n = sum(stride(c) for c in chunks)
-            rooms = None
-            if chunk_type == ChunkType.PARAM_FP32 and all(c.data_type == torch.float for c in chunks):
-                positions = [self._fp16_chunk_of_position(c.chunk_id) for c in chunks]
-                if None not in positions:  # (an fp32 list driven on its own has no state lists either)
-                    rooms = self._fp32_lists(n)
-            slab = rooms[0] if rooms else torch.zeros(n, dtype=chunks[0].data_type, device=self.device)
+            slab = state_slabs.get(chunk_type)
+            if slab is None:
+                slab = torch.zeros(sum(stride(c) for c in chunks), dtype=chunks[0].data_type, device=self.device)
             self._slabs.append(slab)
             cursor = 0
-            for k, chunk in enumerate(chunks):
+            for chunk in chunks:
                 chunk.payload = slab.narrow(0, cursor, chunk.capacity)
-                if rooms:
-                    for state, room in ((ChunkType.MOMENTUM, rooms[1]), (ChunkType.VARIANCE, rooms[2])):
-                        self._reserved[(state, positions[k])] = room.narrow(0, cursor, chunk.capacity)
                 cursor += stride(chunk)
 
-    def _fp32_lists(self, n):
-        """Three zero-filled slabs of ``n`` floats, ``list_distance`` apart in one allocation: the fp32 parameters', and
-        room for the momentum and variance chunks of the same positions.  None: not worth it, or no memory for all three."""
-        if not ONE_ALLOCATION_BYTES[0] <= 4 * n <= ONE_ALLOCATION_BYTES[1]:
-            return None
-        distance = list_distance(4 * n) // 4
+    def _state_slabs(self, momentum, variance, n):
+        """{list: zero-filled slab of ``n`` floats} for momentum and variance chunks of the same positions: parts of one
+        allocation, clear of the fp32 parameters' list and of one another.  Empty: not worth it, not such lists, or no memory
+        for the gaps."""
+        if not CLEAR_LIST_BYTES[0] <= 4 * n <= CLEAR_LIST_BYTES[1] or any(c.data_type != torch.float for c in momentum + variance):
+            return {}
+        index = self.chunk_tensor_index
+        position_of = {(kind, cid): cid16 for cid16, states in index.param_chunk_id_to_os_chunk_id_map.items() for kind, cid in states.items()}
+        positions = [position_of.get((ChunkType.MOMENTUM, c.chunk_id)) for c in momentum]
+        if None in positions or positions != [position_of.get((ChunkType.VARIANCE, c.chunk_id)) for c in variance]:
+            return {}  # (lists driven on their own have no positions)
+        distance = list_distance(4 * n)
         try:
-            whole = torch.zeros(2 * distance + n, dtype=torch.float, device=self.device)
+            whole = torch.zeros((distance + 4 * n + LIST_SLACK) // 4, dtype=torch.float, device=self.device)
         except torch.OutOfMemoryError:
-            return None
+            return {}
+        ids16 = index.chunk_type_to_chunk_id_list_map[ChunkType.PARAM_FP16]
+        ids32 = index.chunk_type_to_chunk_id_list_map.get(ChunkType.PARAM_FP32, [])
+        place = ids16.index(positions[0])
+        master = self.chunk_list[ids32[place]].payload if place < len(ids32) else None
+        shift = 0 if master is None else list_shift(whole.data_ptr() - master.data_ptr(), distance)
         # tensors in their own right, not views of one another, so that a payload's base is its own list
-        return [torch.empty(0, dtype=torch.float, device=self.device).set_(whole.untyped_storage(), k * distance, (n,)) for k in range(3)]
-
-    def _take_reserved(self, chunk_type, chunks):
-        """Give state chunks the room that was reserved beside their position's fp32 chunk; returns those that have none."""
-        rest = []
-        for chunk in chunks:
-            room = None
-            if self._reserved:
-                position = next((cid for cid, states in self.chunk_tensor_index.param_chunk_id_to_os_chunk_id_map.items()
-                                 if states.get(chunk_type) == chunk.chunk_id), None)  # None: a list driven on its own
-                room = self._reserved.pop((chunk_type, position), None)
-            if room is None or room.numel() != chunk.capacity or room.dtype != chunk.data_type:
-                rest.append(chunk)
-                continue
-            if not any(room._base is slab for slab in self._slabs):
-                self._slabs.append(room._base)
-            chunk.payload = room
-        return rest
+        return {kind: torch.empty(0, dtype=torch.float, device=self.device).set_(whole.untyped_storage(), at // 4, (n,))
+                for kind, at in ((ChunkType.MOMENTUM, shift), (ChunkType.VARIANCE, shift + distance))}
 
     def chunk_ids_generator(self, chunk_type):
         for cid in self.chunk_tensor_index.chunk_type_to_chunk_id_list_map.get(chunk_type, []):
