@@ -379,19 +379,25 @@ class PatrickStarClient:
         if not CLEAR_LIST_BYTES[0] <= 4 * n <= CLEAR_LIST_BYTES[1] or any(c.data_type != torch.float for c in momentum + variance):
             return {}
         index = self.chunk_tensor_index
-        position_of = {(kind, cid): cid16 for cid16, states in index.param_chunk_id_to_os_chunk_id_map.items() for kind, cid in states.items()}
-        positions = [position_of.get((ChunkType.MOMENTUM, c.chunk_id)) for c in momentum]
-        if None in positions or positions != [position_of.get((ChunkType.VARIANCE, c.chunk_id)) for c in variance]:
-            return {}  # (lists driven on their own have no positions)
+        place16 = {cid: k for k, cid in enumerate(index.chunk_type_to_chunk_id_list_map.get(ChunkType.PARAM_FP16, []))}
+        place_of = {(kind, cid): place16[cid16] for cid16, states in index.param_chunk_id_to_os_chunk_id_map.items()
+                    for kind, cid in states.items()}
+        places = []
+        for kind, chunks in ((ChunkType.MOMENTUM, momentum), (ChunkType.VARIANCE, variance)):
+            if any((kind, c.chunk_id) not in place_of for c in chunks):
+                return {}  # (lists driven on their own have no positions)
+            # in the order of the parameters' chunks, whatever the order in which the optimizer was given them
+            chunks.sort(key=lambda c: place_of[(kind, c.chunk_id)])
+            places.append([place_of[(kind, c.chunk_id)] for c in chunks])
+        if places[0] != places[1]:
+            return {}
         distance = list_distance(4 * n)
         try:
             whole = torch.zeros((distance + 4 * n + LIST_SLACK) // 4, dtype=torch.float, device=self.device)
         except torch.OutOfMemoryError:
             return {}
-        ids16 = index.chunk_type_to_chunk_id_list_map[ChunkType.PARAM_FP16]
         ids32 = index.chunk_type_to_chunk_id_list_map.get(ChunkType.PARAM_FP32, [])
-        place = ids16.index(positions[0])
-        master = self.chunk_list[ids32[place]].payload if place < len(ids32) else None
+        master = self.chunk_list[ids32[places[0][0]]].payload if places[0][0] < len(ids32) else None
         shift = 0 if master is None else list_shift(whole.data_ptr() - master.data_ptr(), distance)
         # tensors in their own right, not views of one another, so that a payload's base is its own list
         return {kind: torch.empty(0, dtype=torch.float, device=self.device).set_(whole.untyped_storage(), at // 4, (n,))

@@ -51,6 +51,16 @@ def test_state_of_the_positions_an_optimizer_is_given(numel, of_three):
     assert opt.state[params[-1]]["exp_avg"] is not None
 
 
+def test_state_lies_in_the_order_of_the_parameters_chunks():
+    client = ps.PatrickStarClient(0, 24 * MB, device="meta")
+    params = client.append_flat_chunks(4)
+    ps.FP16Adam(client, [params[k] for k in (2, 0, 3, 1)], loss_scaler=ps.LossScaler(8.0), lr=1e-3)
+    payload = [[client.chunk_list[cid].payload for cid in (pos.fp32, pos.exp_avg, pos.exp_avg_sq)] for pos in client.positions()]
+    for k, (p, m, v) in enumerate(payload):
+        assert p.storage_offset() - payload[0][0].storage_offset() == k * 24 * MB
+        assert m.storage_offset() - payload[0][1].storage_offset() == v.storage_offset() - payload[0][2].storage_offset() == k * 24 * MB
+
+
 def test_a_master_chunk_that_is_allocated_again_brings_no_state():
     numel = 32 * MB
     client = ps.PatrickStarClient(0, numel, device="meta")
