@@ -37,6 +37,11 @@ HIPCC_FLAGS = [
 ]
 
 
+def is_built():
+    """Whether everything that build() makes is there."""
+    return all(os.path.exists(path) for path in (LIB_PATH, BINDING_PATH))
+
+
 def hipcc_path():
     for cand in (shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
         if cand and os.path.exists(cand):

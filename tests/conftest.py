@@ -13,12 +13,12 @@ def pytest_configure(config):
 
 
 def pytest_sessionstart(session):
-    """A fresh checkout has no built library (built files are not in the history): compile it once, here on the host,
-    before the tests that load it.  Where the library is already there (every GPU run: it travels with the tree)
+    """A fresh checkout has nothing built (built files are not in the history): compile once, here on the host,
+    before the tests that load it.  Where library and binding are already there (every GPU run: they travel with the tree)
     nothing happens."""
-    from patrickstar_amd import _lib, build
+    from patrickstar_amd import build
 
-    if os.path.exists(_lib.LIB_PATH):
+    if build.is_built():
         return
     try:
         build.hipcc_path()
