@@ -203,12 +203,17 @@ def _load_binding():
     does the same through the same library in more host time (3 us of 6.4 are spent on what the binding saves)."""
     import torch  # noqa: F401  (the binding uses its libraries)
 
+    from . import build
+
     try:
         from . import _binding
     except ImportError as e:
         reason = str(e)
     else:
-        return _binding
+        made_for = (getattr(_binding, "abi_version", None), getattr(_binding, "built_for", None))
+        if made_for == (PS_ABI_VERSION, build.built_for()):
+            return _binding
+        reason = f"{_binding.__file__} was built for ABI version {made_for[0]}, {made_for[1]}"
     warnings.warn(f"adam_update goes without its compiled call ({reason}); build it with `python -m patrickstar_amd.build`",
                   RuntimeWarning, stacklevel=3)
     return None

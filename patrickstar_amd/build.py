@@ -2,6 +2,7 @@
 import os
 import shutil
 import subprocess
+import sys
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)
@@ -65,6 +66,13 @@ def compile_shared(sources, target, verbose=False, extra_flags=()):
     return target
 
 
+def built_for():
+    """What a binding that is compiled now can be used with."""
+    import torch
+
+    return f"Python {sys.version_info[0]}.{sys.version_info[1]}, torch {torch.__version__}"
+
+
 def build_binding(verbose=False):
     """Compile the Python side of the operator call, host code only, into patrickstar_amd/_binding.so (returned)."""
     import sysconfig
@@ -72,7 +80,8 @@ def build_binding(verbose=False):
     from torch.utils import cpp_extension
 
     tmp = BINDING_PATH + f".{os.getpid()}.tmp"
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM"]
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f'-DPS_BUILT_FOR="{built_for()}"']
     for path in [INCLUDE, sysconfig.get_paths()["include"], "/opt/rocm/include"]:
         cmd += ["-I", path]
     for path in cpp_extension.include_paths():

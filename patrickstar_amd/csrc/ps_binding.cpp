@@ -101,4 +101,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", nullptr, 0, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding() { return PyModule_Create(&module); }
+// abi_version: of the library whose ps_adam_update it calls by its address; built_for: the Python and torch it was compiled with.
+PyMODINIT_FUNC PyInit__binding()
+{
+    PyObject* m = PyModule_Create(&module);
+    if (m && (PyModule_AddIntConstant(m, "abi_version", PS_ABI_VERSION) || PyModule_AddStringConstant(m, "built_for", PS_BUILT_FOR))) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

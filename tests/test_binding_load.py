@@ -1,6 +1,8 @@
 """The compiled operator call is a shorter way to the library, not a part of it: the package loads without it, or beside one
 that was made for something else."""
 import sys
+import types
+import warnings
 
 import pytest
 
@@ -22,6 +24,30 @@ def test_the_library_loads_without_the_binding(fresh):
         lib = _lib.load()
     assert lib.ps_abi_version() == _lib.PS_ABI_VERSION
     assert lib.adam_update(*range(13)) is None  # "not of the ordinary form": the caller goes on to the general path
+
+
+@pytest.mark.parametrize(
+    "made_for",
+    [dict(), dict(abi_version=_lib.PS_ABI_VERSION - 1, built_for=build.built_for()), dict(abi_version=_lib.PS_ABI_VERSION, built_for="Python 3.9, torch 2.4.0")],
+)
+def test_a_binding_made_for_something_else_is_not_called(fresh, made_for):
+    """It calls ps_adam_update by its address, through the signature it was compiled with."""
+    other = types.ModuleType("patrickstar_amd._binding")
+    other.__file__ = "_binding.so"
+    other.adam_update = lambda *a: pytest.fail("called")
+    other.__dict__.update(made_for)
+    fresh.setitem(sys.modules, "patrickstar_amd._binding", other)
+    fresh.setattr(ps, "_binding", other, raising=False)
+    with pytest.warns(RuntimeWarning, match="was built for ABI version"):
+        lib = _lib.load()
+    assert lib.adam_update(*range(13)) is None
+
+
+def test_the_binding_of_this_build_is_used(fresh):
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        lib = _lib.load()
+    assert lib.adam_update.func is ps._binding.adam_update
 
 
 def test_a_tree_with_the_library_alone_is_not_built(monkeypatch, tmp_path):
