@@ -1,4 +1,5 @@
 """Builds libps_adam.so (the C-ABI HIP library) for gfx950 with hipcc and _binding.so (host code) with g++, in-tree."""
+import contextlib
 import os
 import shutil
 import subprocess
@@ -50,19 +51,35 @@ def hipcc_path():
     raise RuntimeError("hipcc not found: the HIP library cannot be built")
 
 
-def compile_shared(sources, target, verbose=False, extra_flags=()):
-    """hipcc the given sources into one shared library with this package's flags."""
-    # compile beside the target and rename: a process that has the old library mapped keeps its own copy
-    tmp = target + f".{os.getpid()}.tmp"
-    cmd = [hipcc_path(), *HIPCC_FLAGS, *extra_flags, "-I", INCLUDE, *sources, "-o", tmp]
+@contextlib.contextmanager
+def _replacing(*targets):
+    """Paths beside the targets to build into; they take the targets' places together, once all of them are built.  (A process
+    that has an old file mapped keeps its own copy.)"""
+    made = [f"{target}.{os.getpid()}.tmp" for target in targets]
+    try:
+        yield made
+        for path, target in zip(made, targets):
+            os.replace(path, target)
+    finally:
+        for path in made:
+            if os.path.exists(path):
+                os.remove(path)
+
+
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
-    try:
-        subprocess.check_call(cmd)
-        os.replace(tmp, target)
-    finally:
-        if os.path.exists(tmp):
-            os.remove(tmp)
+    subprocess.check_call(cmd)
+
+
+def _compile_hip(sources, out, verbose, extra_flags):
+    _run([hipcc_path(), *HIPCC_FLAGS, *extra_flags, "-I", INCLUDE, *sources, "-o", out], verbose)
+
+
+def compile_shared(sources, target, verbose=False, extra_flags=()):
+    """hipcc the given sources into one shared library with this package's flags."""
+    with _replacing(target) as (out,):
+        _compile_hip(sources, out, verbose, extra_flags)
     return target
 
 
@@ -73,38 +90,37 @@ def built_for():
     return f"Python {sys.version_info[0]}.{sys.version_info[1]}, torch {torch.__version__}"
 
 
-def build_binding(verbose=False):
-    """Compile the Python side of the operator call, host code only, into patrickstar_amd/_binding.so (returned)."""
+def _compile_binding(out, verbose):
     import sysconfig
 
     from torch.utils import cpp_extension
 
-    tmp = BINDING_PATH + f".{os.getpid()}.tmp"
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            f'-DPS_BUILT_FOR="{built_for()}"']
     for path in [INCLUDE, sysconfig.get_paths()["include"], "/opt/rocm/include"]:
         cmd += ["-I", path]
     for path in cpp_extension.include_paths():
         cmd += ["-isystem", path]
-    cmd += [BINDING_SOURCE, "-o", tmp]
+    cmd += [BINDING_SOURCE, "-o", out]
     for path in cpp_extension.library_paths():
         cmd += ["-L", path]
-    cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    try:
-        subprocess.check_call(cmd)
-        os.replace(tmp, BINDING_PATH)
-    finally:
-        if os.path.exists(tmp):
-            os.remove(tmp)
+    _run(cmd + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"], verbose)
+
+
+def build_binding(verbose=False):
+    """Compile the Python side of the operator call, host code only, into patrickstar_amd/_binding.so (returned)."""
+    with _replacing(BINDING_PATH) as (out,):
+        _compile_binding(out, verbose)
     return BINDING_PATH
 
 
 def build(verbose=False, extra_flags=()):
-    """Compile the package's HIP sources into patrickstar_amd/libps_adam.so (returned), and the binding beside it."""
-    build_binding(verbose)
-    return compile_shared(SOURCES, LIB_PATH, verbose, extra_flags)
+    """Compile the package's HIP sources into patrickstar_amd/libps_adam.so (returned), and the binding beside it.  Neither
+    replaces what is there before both are compiled: the binding calls into the library it was built with."""
+    with _replacing(BINDING_PATH, LIB_PATH) as (binding, library):
+        _compile_binding(binding, verbose)
+        _compile_hip(SOURCES, library, verbose, extra_flags)
+    return LIB_PATH
 
 
 if __name__ == "__main__":

@@ -1,5 +1,7 @@
 """The compiled operator call is a shorter way to the library, not a part of it: the package loads without it, or beside one
 that was made for something else."""
+import os
+import subprocess
 import sys
 import types
 import warnings
@@ -54,3 +56,26 @@ def test_a_tree_with_the_library_alone_is_not_built(monkeypatch, tmp_path):
     assert build.is_built()
     monkeypatch.setattr(build, "BINDING_PATH", str(tmp_path / "_binding.so"))
     assert not build.is_built()
+
+
+@pytest.mark.parametrize("fails", ["g++", "hipcc"])
+def test_a_build_that_fails_leaves_both_files_as_they_were(monkeypatch, tmp_path, fails):
+    for name in ("LIB_PATH", "BINDING_PATH"):
+        path = tmp_path / os.path.basename(getattr(build, name))
+        path.write_text("old")
+        monkeypatch.setattr(build, name, str(path))
+
+    def compiler(cmd):
+        if fails in os.path.basename(cmd[0]):
+            raise subprocess.CalledProcessError(1, cmd)
+        with open(cmd[cmd.index("-o") + 1], "w") as f:
+            f.write("new")
+
+    monkeypatch.setattr(build.subprocess, "check_call", compiler)
+    monkeypatch.setattr(build, "hipcc_path", lambda: "/opt/rocm/bin/hipcc")
+    with pytest.raises(subprocess.CalledProcessError):
+        build.build()
+    assert {p.name: p.read_text() for p in tmp_path.iterdir()} == {"libps_adam.so": "old", "_binding.so": "old"}
+    fails = "nothing"
+    assert build.build() == build.LIB_PATH
+    assert {p.name: p.read_text() for p in tmp_path.iterdir()} == {"libps_adam.so": "new", "_binding.so": "new"}
