@@ -10,6 +10,9 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <cstdio>
+#include <exception>
+
 #include <ATen/core/Tensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -68,27 +71,40 @@ PyObject* adam_update(PyObject*, PyObject* const* args, Py_ssize_t n)
         !number(args[3], lr) || !number(args[4], beta1) || !number(args[5], beta2) || !number(args[6], eps) || !number(args[7], wd) ||
         !number(args[13], scale) || (args[8] != Py_True && args[8] != Py_False))
         Py_RETURN_NONE;
-    int rc;
+    const at::Tensor *p, *g, *m, *v;
+    void *pp, *gp, *mp, *vp, *stream;
+    int64_t numel = 0;
+    int half;
     try {
-        const at::Tensor *p, *g, *m, *v;
         int device = -1;
-        int64_t numel = 0;
         if (!plain(args[9], at::kFloat, at::kFloat, device, numel, p) || !plain(args[10], at::kFloat, at::kHalf, device, numel, g) ||
             !plain(args[11], at::kFloat, at::kFloat, device, numel, m) || !plain(args[12], at::kFloat, at::kFloat, device, numel, v) ||
             device != c10::hip::current_device())
             Py_RETURN_NONE;
-        void *pp = p->data_ptr(), *gp = g->data_ptr(), *mp = m->data_ptr(), *vp = v->data_ptr();
-        const int half = g->scalar_type() == at::kHalf;
-        void* stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-        const auto call = reinterpret_cast<decltype(&ps_adam_update)>(address);
-        const int bias = args[8] == Py_True;
-        Py_BEGIN_ALLOW_THREADS  // a launch waits where the queue is full
-        rc = call((int)id, (size_t)step, lr, beta1, beta2, eps, wd, bias, static_cast<float*>(pp), gp, half, static_cast<float*>(mp),
-                  static_cast<float*>(vp), (size_t)numel, scale, nullptr, stream);
-        Py_END_ALLOW_THREADS
+        pp = p->data_ptr(), gp = g->data_ptr(), mp = m->data_ptr(), vp = v->data_ptr();
+        half = g->scalar_type() == at::kHalf;
+        stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
     } catch (...) {  // a tensor without memory of its own (vmap, meta): the general path says so
         PyErr_Clear();
         Py_RETURN_NONE;
+    }
+    const auto call = reinterpret_cast<decltype(&ps_adam_update)>(address);
+    const int bias = args[8] == Py_True;
+    int rc = 0;
+    char thrown[256] = "";  // by a call that was begun: it is an error, and not made again by the general path
+    Py_BEGIN_ALLOW_THREADS  // a launch waits where the queue is full; no exception passes this block's end
+    try {
+        rc = call((int)id, (size_t)step, lr, beta1, beta2, eps, wd, bias, static_cast<float*>(pp), gp, half, static_cast<float*>(mp),
+                  static_cast<float*>(vp), (size_t)numel, scale, nullptr, stream);
+    } catch (const std::exception& e) {
+        std::snprintf(thrown, sizeof(thrown), "adam_update: %s", e.what());
+    } catch (...) {
+        std::snprintf(thrown, sizeof(thrown), "adam_update: unknown exception");
+    }
+    Py_END_ALLOW_THREADS
+    if (thrown[0]) {
+        PyErr_SetString(PyExc_RuntimeError, thrown);
+        return nullptr;
     }
     return PyLong_FromLong(rc);
 }
