@@ -1110,14 +1110,17 @@ TensorItem tensor_item(const ps_chunk* tensors, const size_t* numels, int i, boo
     return TensorItem{i, (uint32_t)head, body, (head ? 1 : 0) + (body + kTile - 1) / kTile, 0};
 }
 
-// (of tensors, the tiles start at the parameter's KiB boundary)
-bool streams(const ps_chunk* tensors, const size_t* numels, int n_tensors, bool gated)
+// The same of tensors, whose tiles start at the parameter's KiB boundary.  Those with binary32 gradients (grad_f32(i)) never take
+// the hint: they don't count.
+template <typename F>
+bool streams(const ps_chunk* tensors, const size_t* numels, int n_tensors, bool gated, F grad_f32)
 {
     size_t total = 0;
-    for (int i = 0; i < n_tensors; ++i) total += numels[i];
+    for (int i = 0; i < n_tensors; ++i)
+        if (!grad_f32(i)) total += numels[i];
     if (total < (gated ? kStreamElementsGated : kStreamElements)) return false;
     for (int i = 0; i < n_tensors; ++i) {
-        if (numels[i] < (size_t)kTile) continue;
+        if (numels[i] < (size_t)kTile || grad_f32(i)) continue;
         const size_t head = tensor_item(tensors, numels, i).head;
         const ps_chunk& t = tensors[i];
         if (!whole_lines(t.param_fp32 + head, t.exp_avg + head, t.exp_avg_sq + head, t.param_fp16 + head)) return false;
@@ -1426,7 +1429,7 @@ int ps_adam_step_tensors(int optimizer_id, size_t step, double lr, double beta1,
     }
     for (int i = 0; i < n_tensors; ++i)
         if (numels[i] != 0) items.push_back(tensor_item(tensors, numels, i));
-    const bool nt = streams(tensors, numels, n_tensors, d_state != nullptr);
+    const bool nt = streams(tensors, numels, n_tensors, d_state != nullptr, [](int) { return false; });
     return for_each_tensor_batch(items, tensors, first_tensor, 0, [&](const auto& b, dim3 grid, const BatchClasses&) {
         if (d_state == nullptr) {
             if (arith == PS_ARITH_TORCH)
@@ -1473,10 +1476,10 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
             return fail(PS_ERR_BAD_ARG, "d_workspace must be 16-byte aligned");
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool nt = streams(tensors, numels, n_tensors, d_state != nullptr);
     const bool bias = bias_correction != 0;
     auto arith_of = [&](int i) { return each[i].arithmetic < 0 ? o->arith : each[i].arithmetic; };
     auto grad_f32_of = [&](int i) { return (each[i].flags & PS_TENSOR_GRAD_F32) != 0; };
+    const bool nt = streams(tensors, numels, n_tensors, d_state != nullptr, grad_f32_of);
     try {
         // Calls that come out with the same constants form a class; class_of[i] says which one tensor i belongs to.
         std::vector<int> class_of((size_t)n_tensors, -1);

@@ -1,5 +1,6 @@
 """Long lists whose tiles fill whole 64-byte lines are stepped and probed with the non-temporal hint, by kernels of their own; the
-same numbers at a phase of 32 bytes take the others and have to be left with the same bits."""
+same numbers at a phase of 32 bytes take the others and have to be left with the same bits.  (That these lists take two routes is
+checked in test_routes.py.)"""
 import ctypes
 
 import pytest
@@ -55,7 +56,9 @@ def test_chunk_lists(numel, chunks, mirrored, decided, arithmetic, scale, adamw,
             _lib.check(rc, "step")
         adam_op.destroy_adam(OPT)
         if scaler is not None:
-            assert scaler.skipped_steps == (1 if decided == "flagged" else 0) if hasattr(scaler, "skipped_steps") else True
+            state = _lib.ps_step_state()
+            _lib.check(lib.ps_state_read(scaler.state_ptr, ctypes.byref(state), s), "ps_state_read")
+            assert state.skipped_steps == (1 if decided == "flagged" else 0)
             lists.append(scaler._state.clone())
         got.append(lists)
     _same(*got)
