@@ -91,7 +91,8 @@ PyObject* adam_update(PyObject*, PyObject* const* args, Py_ssize_t n)
     const auto call = reinterpret_cast<decltype(&ps_adam_update)>(address);
     const int bias = args[8] == Py_True;
     int rc = 0;
-    char thrown[256] = "";  // by a call that was begun: it is an error, and not made again by the general path
+    char thrown[256];  // by a call that was begun: it is an error, and not made again by the general path
+    thrown[0] = 0;
     Py_BEGIN_ALLOW_THREADS  // a launch waits where the queue is full; no exception passes this block's end
     try {
         rc = call((int)id, (size_t)step, lr, beta1, beta2, eps, wd, bias, static_cast<float*>(pp), gp, half, static_cast<float*>(mp),
