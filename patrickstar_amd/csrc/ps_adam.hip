@@ -945,23 +945,18 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
         const size_t at = head + done;
         dim3 grid((unsigned)(n_tiles + (this_head + tail > 0 ? 1 : 0))), block(kBlock);  // + 1: the workgroup that does head and tail
         uint16_t* out = d_param_fp16_out ? d_param_fp16_out + at : nullptr;
-#define PS_FLAT_VEC_6(WD, UNS, HALF, OUT, DWORD, NT)                                                              \
-    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s,          \
-                       d_params + at, static_cast<const void*>(gbytes + at * gsz), d_exp_avg + at,            \
+#define PS_FLAT_VEC_5(WD, UNS, HALF, OUT, DWORD, NT)                                                                            \
+    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, \
+                       d_params + at, static_cast<const void*>(gbytes + at * gsz), d_exp_avg + at,                              \
                        d_exp_avg_sq + at, out, (uint32_t)n_tiles, this_head, tail, c)
-#define PS_FLAT_VEC_5(WD, UNS, HALF, OUT, DWORD)           \
-    do {                                                   \
-        if (nt)                                            \
-            PS_FLAT_VEC_6(WD, UNS, HALF, OUT, DWORD, true);  \
-        else                                               \
-            PS_FLAT_VEC_6(WD, UNS, HALF, OUT, DWORD, false); \
-    } while (0)
-#define PS_FLAT_VEC_4(WD, UNS, HALF, OUT)                  \
-    do {                                                   \
-        if (state_aligned)                                 \
-            PS_FLAT_VEC_5(WD, UNS, HALF, OUT, false);      \
-        else                                               \
-            PS_FLAT_VEC_5(WD, UNS, HALF, OUT, true);       \
+#define PS_FLAT_VEC_4(WD, UNS, HALF, OUT)                    \
+    do {                                                     \
+        if (!state_aligned)                                  \
+            PS_FLAT_VEC_5(WD, UNS, HALF, OUT, true, false);  \
+        else if (nt)                                         \
+            PS_FLAT_VEC_5(WD, UNS, HALF, OUT, false, true);  \
+        else                                                 \
+            PS_FLAT_VEC_5(WD, UNS, HALF, OUT, false, false); \
     } while (0)
 #define PS_FLAT_VEC_3(WD, UNS, HALF)                       \
     do {                                                   \
@@ -994,7 +989,6 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
 #undef PS_FLAT_VEC_3
 #undef PS_FLAT_VEC_4
 #undef PS_FLAT_VEC_5
-#undef PS_FLAT_VEC_6
         PS_HIP(hipGetLastError());
         done += n_tiles * kTile + tail;
     } while (done < body);

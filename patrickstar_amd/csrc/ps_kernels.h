@@ -411,13 +411,19 @@ __device__ __forceinline__ void adam_tensor_tile(MakeConsts make_consts, const T
         const StepConsts c = make_consts();
         tile_finish<ARITH, WD, UNS, false, NT>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r, t.param_fp32,
                                     t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
-    } else if (access == TILE_STATE_DWORD_ALIGNED) {
-        LaneTile r;
-        tile_load<true, NT>(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
-        const StepConsts c = make_consts();
-        tile_finish<ARITH, WD, UNS, true, NT>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r,
-                                          t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
-    } else if (base < w.numel) {  // (the grid is as wide as the longest tensor of the batch)
+        return;
+    }
+    if constexpr (!NT) {  // (tensors that stream past the caches have whole lines)
+        if (access == TILE_STATE_DWORD_ALIGNED) {
+            LaneTile r;
+            tile_load<true>(r, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+            const StepConsts c = make_consts();
+            tile_finish<ARITH, WD, UNS, true>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, r,
+                                              t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base);
+            return;
+        }
+    }
+    if (base < w.numel) {  // (the grid is as wide as the longest tensor of the batch)
         const StepConsts c = make_consts();
         const size_t end = base + kTile < w.numel ? base + kTile : w.numel;
         adam_tile_scalar<ARITH, WD, UNS>(c, t.param_fp32, t.exp_avg, t.exp_avg_sq, t.param_fp16, base, end, 0, first ? w.numel : 0);

@@ -40,35 +40,28 @@ __device__ __forceinline__ uint4v ld_u4(const uint16_t* p)
 {
     return NT ? __builtin_nontemporal_load((const guint4v*)(p)) : *(const guint4v*)(p);
 }
-template <bool NT = false>
-__device__ __forceinline__ void st_u4(uint16_t* p, uint4v v)
-{
-    if (NT)
-        __builtin_nontemporal_store(v, (guint4v*)(p));
-    else
-        *(guint4v*)(p) = v;
-}
+__device__ __forceinline__ void st_u4(uint16_t* p, uint4v v) { *(guint4v*)(p) = v; }
 
 // 16 bytes at an address that is only 4-byte aligned (multi-dword global accesses need dword alignment only): for
-// momentum / variance tensors that sit at another 16-byte phase than their parameter.
+// momentum / variance tensors that sit at another 16-byte phase than their parameter.  (Never with the hint, which is for tiles of
+// whole 64-byte lines.)
 typedef float4v __attribute__((aligned(4))) float4v_dword_aligned;
 typedef PS_GLOBAL float4v_dword_aligned gfloat4v_dword_aligned;
 template <bool DWORD_ALIGNED, bool NT = false>
 __device__ __forceinline__ float4v ld_f4_as(const float* p)
 {
-    if (!DWORD_ALIGNED) return ld_f4<NT>(p);
-    if (NT) return __builtin_nontemporal_load((const gfloat4v_dword_aligned*)(p));
-    return *(const gfloat4v_dword_aligned*)(p);
+    static_assert(!(DWORD_ALIGNED && NT), "the hint is for whole lines");
+    if (DWORD_ALIGNED) return *(const gfloat4v_dword_aligned*)(p);
+    return ld_f4<NT>(p);
 }
 template <bool DWORD_ALIGNED, bool NT = false>
 __device__ __forceinline__ void st_f4_as(float* p, float4v v)
 {
-    if (!DWORD_ALIGNED)
-        st_f4<NT>(p, v);
-    else if (NT)
-        __builtin_nontemporal_store(v, (gfloat4v_dword_aligned*)(p));
-    else
+    static_assert(!(DWORD_ALIGNED && NT), "the hint is for whole lines");
+    if (DWORD_ALIGNED)
         *(gfloat4v_dword_aligned*)(p) = v;
+    else
+        st_f4<NT>(p, v);
 }
 
 constexpr int kBlock = PS_BLOCK;
@@ -108,22 +101,18 @@ __device__ __forceinline__ HalfWords ld_halves(const uint16_t* p)
     return r;
 }
 
-template <bool NT = false>
 __device__ __forceinline__ void st_halves(uint16_t* p, const HalfWords& r)
 {
     if (kWords == 4) {
         uint4v t;
 #pragma unroll
         for (int k = 0; k < kWords; ++k) t[k] = r.w[k];
-        st_u4<NT>(p, t);
+        st_u4(p, t);
     } else {
         uint2v t;
 #pragma unroll
         for (int k = 0; k < kWords; ++k) t[k] = r.w[k];
-        if (NT)
-            __builtin_nontemporal_store(t, (guint2v*)(p));
-        else
-            *(guint2v*)(p) = t;
+        *(guint2v*)(p) = t;
     }
 }
 
@@ -135,6 +124,7 @@ constexpr int kCacheNt = 2;               // cache policy: non-temporal
 template <bool DWORD_ALIGNED, bool NT>
 __device__ __forceinline__ void st_tile(float* first, int q, float4v v)
 {
+    static_assert(!(DWORD_ALIGNED && NT), "the hint is for whole lines");
     if (NT) {
         const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(first, 0, kTile * (int)sizeof(float), kBufferFlags);
         uint4v w;
@@ -212,9 +202,9 @@ __device__ __forceinline__ void tile_load(LaneTile& r, const float* __restrict__
 #pragma unroll
         for (int q = 0; q < kQuads; ++q) r.p[u][q] = ld_f4<NT>(p32 + i + 4 * q);
 #pragma unroll
-        for (int q = 0; q < kQuads; ++q) r.m[u][q] = ld_f4_as<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(m32 + i + 4 * q);
+        for (int q = 0; q < kQuads; ++q) r.m[u][q] = ld_f4_as<STATE_DWORD_ALIGNED, NT>(m32 + i + 4 * q);
 #pragma unroll
-        for (int q = 0; q < kQuads; ++q) r.v[u][q] = ld_f4_as<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(v32 + i + 4 * q);
+        for (int q = 0; q < kQuads; ++q) r.v[u][q] = ld_f4_as<STATE_DWORD_ALIGNED, NT>(v32 + i + 4 * q);
     }
 }
 
@@ -239,8 +229,8 @@ __device__ __forceinline__ void tile_finish(const StepConsts& c, float step_size
 #pragma unroll
         for (int q = 0; q < kQuads; ++q) {
             st_tile<false, NT>(p32 + first, q, r.p[u][q]);
-            st_tile<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(m32 + first, q, r.m[u][q]);
-            st_tile<STATE_DWORD_ALIGNED, NT && !STATE_DWORD_ALIGNED>(v32 + first, q, r.v[u][q]);
+            st_tile<STATE_DWORD_ALIGNED, NT>(m32 + first, q, r.m[u][q]);
+            st_tile<STATE_DWORD_ALIGNED, NT>(v32 + first, q, r.v[u][q]);
         }
         st_tile_halves<NT>(h16 + first, r.h[u]);
     }

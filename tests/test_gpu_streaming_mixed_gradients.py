@@ -13,7 +13,7 @@ OPT = 8201
 
 
 def _tensors(sizes, scale, phases):
-    gen = torch.Generator(device="cuda").manual_seed(sum(sizes) % 1000)
+    gen = torch.Generator(device="cuda").manual_seed(sum(n for n, _ in sizes) % 1000)
     out = []
     for (n, wide), phase in zip(sizes, phases):
         p, m, v, g = (torch.empty(n + 64, device="cuda").normal_(0, f, generator=gen)[phase : phase + n] for f in (0.02, 1e-4, 1e-3, 1e-3 * scale))
