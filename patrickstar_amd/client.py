@@ -25,18 +25,19 @@ from .chunk_layout import (
     register_param,
 )
 
-# Where the three fp32 lists lie against one another.  A pass reads and writes the same element of all three at the same
-# time.  With plain accesses distances that are multiples of 128 MiB (which lists of power-of-two chunks back to back have)
-# put those three on the same memory banks: 64 Mi elements a list, distance over 256 MiB, 0 to 32 KiB 5.71-5.77 TB/s, 64 KiB
-# 5.89, 1 MiB 6.27-6.29, 6 to 17 MiB 6.26-6.35, 64 MiB 6.23, 128 MiB 5.84.  Steps that stream past the caches (28 Mi elements and
-# up) run at 6.4 to 6.8 TB/s at every distance from 0 to 126 MiB, in no order that two processes share; what is left of the rule
-# shows in whole steps, each list in an allocation of its own / momentum and variance in one at any place, us: 64 Mi elements
-# 288.3 / 282.0, 2 x 64 Mi 572 / 569, 4 x 64 Mi 1142 / 1119, 24 Mi (plain) 113.9 / 114.4, 32 Mi 141 / 144; at the least shift that is
-# clear of the parameters / at the one below, on another box: 24 Mi 114.9 / 112.2, 64 Mi 285.1 / 282.5, 2 x 64 Mi 562.7 / 560.2,
-# 4 x 64 Mi 1119 / 1112, BERT-base with a rate per layer 502.1 / 500.4.  (All three lists in
-# one allocation, the state's part kept from before there is an optimizer: 111.0, 281.5, 558.7, 1113, 500.4.)  Up to 16 Mi elements the
-# lists stay in the memory-side cache (8.3-8.7 TB/s however they lie).  Without the upper line 6 x 64 Mi gain 1.0 to 1.6 %,
-# 12 x 64 Mi 0.6 to 1.8, 8 x 64 Mi nothing, and 24 x 64 Mi lose 0.8 to 1.3.
+# Where the three fp32 lists lie against one another.  A pass reads and writes the same element of all three at the same time.
+# With plain accesses distances that are multiples of 128 MiB (which lists of power-of-two chunks back to back have) put those
+# three on the same memory banks: 64 Mi elements a list, distance over 256 MiB, 0 to 32 KiB 5.71-5.77 TB/s, 64 KiB 5.89, 1 MiB
+# 6.27-6.29, 6 to 17 MiB 6.26-6.35, 64 MiB 6.23, 128 MiB 5.84.  Steps that stream past the caches (28 Mi elements and up) run
+# at 6.4 to 6.8 TB/s at every distance from 0 to 126 MiB, in no order that two processes share; what is left of the rule shows
+# in whole steps, each list in an allocation of its own / momentum and variance in one at any place, us: 64 Mi elements 288.3
+# / 282.0, 2 x 64 Mi 572 / 569, 4 x 64 Mi 1142 / 1119, 24 Mi (plain) 113.9 / 114.4, 32 Mi 141 / 144, GPT-2 small in two chunks
+# 542.9 / 531.3 (by the rule 527.1, all three lists in one allocation 525.1); at the least shift that is clear of the
+# parameters / at the one below, on another box: 24 Mi 114.9 / 112.2, 64 Mi 285.1 / 282.5, 2 x 64 Mi 562.7 / 560.2, 4 x 64 Mi
+# 1119 / 1112, BERT-base with a rate per layer 502.1 / 500.4.  (All three lists in one allocation, the state's part kept from
+# before there is an optimizer: 111.0, 281.5, 558.7, 1113, 500.4.)  Up to 16 Mi elements the lists stay in the memory-side
+# cache (8.3-8.7 TB/s however they lie).  Without the upper line 6 x 64 Mi gain 1.0 to 1.6 %, 12 x 64 Mi 0.6 to 1.8, 8 x 64 Mi
+# nothing, and 24 x 64 Mi lose 0.8 to 1.3.
 CLEAR_LIST_BYTES = (80 << 20, 1 << 30)  # shortest and longest fp32 list that is laid clear of the others
 LIST_PERIOD, LIST_CLEARANCE = 64 << 20, 9 << 20
 LIST_SLACK = LIST_PERIOD + 2 * LIST_CLEARANCE + (1 << 20)

@@ -230,8 +230,12 @@ size_t elements(const ChunkList& a)
 // slower, on the stores alone nothing.
 //
 // Steps over a list that stays in the memory-side cache from one step to the next (256 MiB) want it there: the same state
-// again and again, without / with the hint, host-decided 16 Mi elements 53 / 71 us, 24 Mi 105 / 106, 28 Mi 127 / 123, 32 Mi 150 / 142;
-// device-decided 24 Mi 115 / 118, 28 Mi 136 / 138, 32 Mi 157 / 157, 48 Mi 244 / 230.  The probe alone at 32 Mi 10.2 / 9.0.  A tensor of the
+// again and again, without / with the hint, host-decided 8 Mi elements 28.3 / 36.6 us, 16 Mi 53.6 / 70.2, 20 Mi 87.7 / 88.7, 24 Mi
+// 105.8 / 106.2, 28 Mi 129.2 / 125.8, 32 Mi 149.0 / 139.6; device-decided 24 Mi 115 / 118, 28 Mi 136 / 138, 32 Mi 157 / 157, 48 Mi 244 / 230.  The
+// lines are where a step that finds its list there stops to lose.  One that doesn't, because forward and backward went over
+// more than the cache holds, would gain below them as well (lists in turn, 1 GiB of them: 1 Mi 7.66 / 6.75, 8 Mi 39.8 / 37.4, 16 Mi
+// 79.2 / 71.4, 24 Mi 113.8 / 106.3; device-decided with the probe 16 Mi 89.9 / 82.0); a call does not know which it is, and below 20 Mi
+// the loss is the larger.  The probe alone at 32 Mi 10.2 / 9.0.  A tensor of the
 // operator comes with others, and its launch ends when its stores have left the L2: 144 K elements 2.33 / 2.41 us, 576 K 4.50 / 3.68,
 // 2.25 Mi 13.0 / 11.5; the tensors of a module of 5.3 M elements one after the other 67 / 68, of 11 M 166 / 139.
 //
@@ -264,10 +268,11 @@ void with_hint(bool nt, F launch)
 
 // A list whose chunks follow one another at one distance, all of one length but perhaps the last (EvenChunk).
 using EvenList = EvenBatch;
-//
+
 // Lists of up to this many elements take the kernels for it.  Longer ones are bound by memory from the first tile to the
-// last, and the general kernels are as fast or a little faster; with plain accesses host-decided 593.6 / 595.7 us for 128 Mi elements, 7226 /
-// 7236 for 1.5 Gi; device-decided 596.3 / 593.5 and 7176 / 7209, for 512 Mi 2377 / 2376.
+// last: even / general kernels host-decided 558.1 / 559.2 us for 128 Mi elements, 2216 / 2217 for 512 Mi, 6719 / 6734 for 1.5 Gi;
+// device-decided with the probe 1189.7 / 1193.6 for 256 Mi, 2368 / 2373 and 7154 / 7138.  (The lines are from plain accesses, where the
+// general kernels were a little faster from there on: 7226 / 7236 and 7176 / 7209 for 1.5 Gi.)
 constexpr size_t kMaxEvenElements = (size_t)96 << 20, kMaxEvenElementsGated = (size_t)256 << 20;
 bool even_list(const ChunkList& a, size_t most, EvenList* out, bool fp16_only = false)
 {

@@ -83,9 +83,9 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
 // PatrickStarClient allocates.  Addresses, distance and lengths are 12 words (with the step state's address 14), which are
 // preloaded into scalar registers, so a wave asks for its data, or for the step state, before it has waited for anything.
 //
-// Device time with plain accesses, descriptors / preloaded, host-decided: 128 K elements 2.60 / 2.36 us, 1 Mi 7.98 / 7.64, 4 Mi 23.3 / 22.7, 16 Mi
+// Device time, descriptors / preloaded, host-decided: 128 K elements 2.60 / 2.36 us, 1 Mi 7.98 / 7.64, 4 Mi 23.3 / 22.7, 16 Mi
 // 77.4 / 77.2; device-decided, with the probe and the scale update: 128 K 9.27 / 8.65, 1 Mi 15.4 / 13.8, 4 Mi 31.4 / 29.3, 16 Mi
-// 89.6 / 87.4, 64 Mi 327.3 / 324.3; the probe alone 2.19 / 1.87 at 1 Mi, 6.24 / 5.85 at 16 Mi.
+// 89.6 / 87.4; 64 Mi, with the hint, 306.8 / 305.5; the probe alone 2.19 / 1.87 at 1 Mi, 6.24 / 5.85 at 16 Mi.
 struct EvenChunk {
     float *p32, *m32, *v32;
     uint16_t* h16;
@@ -319,20 +319,21 @@ __device__ __forceinline__ TensorView tensor_view(const TensorBatch& b)
 
 // Tensors that lie at the same place of their four lists (the layout that PatrickStarClient makes: momentum and variance
 // mirror the parameters' chunks, and so do the lists' allocations): what differs from tensor to tensor is one offset and one
-// length, 12 bytes, and one launch takes up to 208 of them, of any lengths.
+// length, 12 bytes, and one launch takes up to 208 of them, in up to 8 groups of nearly the same length (host-decided, with
+// numbers of their own: of up to 24 classes).
 //
 // The grid is one-dimensional.  Its workgroups are divided among up to 8 segments, tensors of nearly the same length
 // each; inside a segment the tensor is a division by the segment's width away (a multiplication by its reciprocal).  A wave
 // reaches its first data load after three rounds of scalar loads (segments, segment, tensor) and some 50 scalar
 // instructions, where TensorBatch needs one round, so 11 workgroups per CU instead of 9 keep as many loads in flight.
 //
-// What that buys is the ends of launches, 4 to 9 us each.  Device time in several launches (TensorBatch) / in one, with plain
-// accesses (long lists that stream past the caches: 13 workgroups per CU, BERT-base 460 us, its upper half 182):
-// BERT-base, 199 tensors 517 / 500 us host-decided, 528 / 504 device-decided with a rate per layer; its upper half, 100
-// tensors 211 / 203 and 218 / 207; 12 layers of hidden size 64 14.6 / 5.8 and 20.4 / 10.6; 11 M elements with no two tensors
-// at the same phase 56.6 / 43.1.  With the cap of 9: BERT-base 508 and 520, with 12 533.  Longer lists gain less than the
-// longer way to the first load costs them: 335 M elements 1558 / 1572 host-decided, 1557 M (GPT-2 XL, 580 tensors, three launches)
-// 7226 / 7414, so lists of more than 256 Mi elements keep TensorBatch.
+// What that buys is the ends of launches, 4 to 9 us each.  Device time in several launches (TensorBatch) / in one, us, lists
+// from 28 Mi elements (device-decided 32 Mi) on with the non-temporal hint, where 13 workgroups per CU are resident: BERT-base, 199
+// tensors, 463.8 / 459.2 host-decided, 474.7 / 461.0 device-decided with a rate per layer; its upper half, 100 tensors 185.2 / 181.3
+// and 192.0 / 184.5; 12 layers of hidden size 64 12.9 / 5.1 and 17.6 / 8.6; 11 M elements with no two tensors at the same phase
+// 52.6 / 39.6.  (With plain accesses BERT-base took 517 / 500, under a cap of 9 508, of 12 533.)  Longer lists gain less than
+// the longer way to the first load costs them: 335 M elements 1408 / 1423 host-decided, 1426 / 1416 device-decided, 1557 M (GPT-2 XL,
+// 580 tensors, three launches) 6568 / 6629 and 6640 / 6612, so lists of more than 256 Mi elements keep TensorBatch.
 constexpr int kNearBatch = 208;
 constexpr int kSegments = 8;
 struct Segment {
@@ -485,7 +486,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
 // record of the launch's constants each tensor of the batch uses.  What a launch cannot mix is what the kernels are
 // compiled for: the arithmetic, the weight-decay form and the way of unscaling.
 // Host-decided: the constants of up to kLaunchClasses classes travel with the launch (a launch's arguments stay
-// under 4 KiB: 2568 bytes of descriptors, 24 x 56 of constants).
+// under 4 KiB: 2696 bytes of NearBatch, which is the larger of the two lists, and 24 x 56 of constants make 4040).
 constexpr int kLaunchClasses = 24;
 struct ConstsBatch {
     StepConsts c[kLaunchClasses];
