@@ -91,6 +91,16 @@ def test_long_tensor_lists_stream_past_the_caches(entry, gated, moved):
     assert not any(q.hint for q in steps(launches(entry, flat_rows(short), short, gated)))
 
 
+def test_the_lists_that_are_compared_with_the_oracle():
+    from test_gpu_streaming_oracle import SIZES
+
+    rows = flat_rows(SIZES)
+    assert [(q.hint, q.near) for q in launches("tensors", rows, SIZES)] == [(True, True)]
+    rows[-1][2] += 4 * 1024
+    found = launches("tensors", rows, SIZES)
+    assert len(found) > 1 and all(q.hint and not q.near for q in found)
+
+
 @pytest.mark.parametrize("n,head,hint", [(256 * 1024, 0, True), (256 * 1024 - 1, 0, False), (300_001, 3, True), (2 * MI + 255, 128, True)])
 def test_long_tensors_of_the_operator_stream_past_the_caches(n, head, hint):
     at = (256 - head) % 256
