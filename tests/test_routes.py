@@ -32,6 +32,7 @@ class Launch:
         at, n = name.end(), int(name[1])
         self.name, rest = mangled[at : at + n], mangled[at + n :]
         self.near = "NearBatch" in rest
+        self.evenly = "even" in self.name or "EvenBatch" in rest
         self.hint = "Lb1EEEv" in rest  # the last template argument
         self.grid, self.lds = grid, lds
 
@@ -123,3 +124,34 @@ def test_tensors_with_binary32_gradients_have_no_say_in_the_hint(gated):
     rows[2] = [a + 16 for a in rows[2]]
     found = steps(launches("each", rows, sizes, gated, [False, False, True]))
     assert [q.hint for q in found if "f32grad" not in q.name] == [True]
+
+
+# --------------------------------------------------- chunks at one distance, tensors at the same place of their lists
+
+
+def test_chunks_at_one_distance_and_the_same_in_the_opposite_order():
+    from test_gpu_even_chunk_lists import LISTS
+
+    for chunks, n, last, _ in LISTS.values():
+        stride = -(-n // 512) * 512
+        rows = [[P + 4 * stride * k, M + 4 * stride * k, V + 4 * stride * k, H + 2 * stride * k] for k in range(chunks)]
+        numels = [n] * (chunks - 1) + [last]
+        for gated in (False, True):
+            short = gated and chunks * -(-n // 256) <= 80  # one workgroup does the whole step
+            (even,) = steps(launches("chunks", rows, numels, gated))
+            general = steps(launches("chunks", rows[::-1], numels[::-1], gated))
+            assert even.name == ("adam_small_step_kernel" if short else "adam_even_chunks_gated_kernel" if gated else "adam_even_chunks_kernel")
+            assert even.evenly and not any(q.evenly for q in general), (chunks, n, gated)
+
+
+def test_tensors_at_the_same_place_of_their_lists_and_one_that_is_not():
+    from test_gpu_near_tensor_lists import SHAPES
+
+    for name, sizes in SHAPES.items():
+        rows = flat_rows(sizes)
+        moved = [list(row) for row in rows]
+        moved[max(k for k, n in enumerate(sizes) if n)][2] += 4 + (1 << 38)
+        for entry in ("tensors", "each"):
+            for gated in (False, True):
+                assert all(q.near for q in steps(launches(entry, rows, sizes, gated))), name
+                assert len(sizes) == 1 or not any(q.near for q in steps(launches(entry, moved, sizes, gated))), name
