@@ -33,7 +33,7 @@ from .chunk_layout import (
 # in whole steps, each list in an allocation of its own / momentum and variance in one at any place, us: 64 Mi elements 288.3
 # / 282.0, 2 x 64 Mi 572 / 569, 4 x 64 Mi 1142 / 1119, 24 Mi (plain) 113.9 / 114.4, 32 Mi 141 / 144, GPT-2 small in two chunks
 # 542.9 / 531.3 (by the rule 527.1, all three lists in one allocation 525.1); at the least shift that is clear of the
-# parameters / at the one below, on another box: 24 Mi 114.9 / 112.2, 64 Mi 285.1 / 282.5, 2 x 64 Mi 562.7 / 560.2, 4 x 64 Mi
+# parameters / at the one below, on another GPU: 24 Mi 114.9 / 112.2, 64 Mi 285.1 / 282.5, 2 x 64 Mi 562.7 / 560.2, 4 x 64 Mi
 # 1119 / 1112, BERT-base with a rate per layer 502.1 / 500.4.  (All three lists in one allocation, the state's part kept from
 # before there is an optimizer: 111.0, 281.5, 558.7, 1113, 500.4.)  Up to 16 Mi elements the lists stay in the memory-side
 # cache (8.3-8.7 TB/s however they lie).  Without the upper line 6 x 64 Mi gain 1.0 to 1.6 %, 12 x 64 Mi 0.6 to 1.8, 8 x 64 Mi

@@ -6,13 +6,15 @@ import threading
 import pytest
 import torch
 
-from patrickstar_amd import _binding, _lib, adam_op
+from patrickstar_amd import _lib, adam_op
 
 pytestmark = pytest.mark.gpu
 
 
 def test_an_exception_is_an_error_of_the_call(monkeypatch):
     _lib.load()
+    from patrickstar_amd import _binding
+
     throws = ctypes.cast(ctypes.CDLL("libstdc++.so.6")._ZSt17__throw_bad_allocv, ctypes.c_void_p).value  # std::__throw_bad_alloc()
     t = [torch.ones(8, device="cuda") for _ in range(4)]
     args = (7802, 1, 1e-3, 0.9, 0.999, 1e-8, 0.0, True, *t, 8.0)

@@ -18,10 +18,12 @@ MI = 1 << 20
 P, M, V, H = (1 << 40, 2 << 40, 3 << 40, 4 << 40)
 
 
+_FOLDER = tempfile.TemporaryDirectory()
+
+
 @functools.lru_cache(maxsize=None)
 def _stand_in():
-    folder = tempfile.mkdtemp()
-    path = os.path.join(folder, "launches.so")
+    path = os.path.join(_FOLDER.name, "launches.so")
     subprocess.check_call(["gcc", "-O1", "-fPIC", "-shared", "-o", path, os.path.join(HERE, "launches.c")])
     return path
 
