@@ -190,6 +190,7 @@ def load():
         lib.adam_update = _no_binding
     else:
         lib.adam_update = functools.partial(binding.adam_update, ctypes.cast(lib.ps_adam_update, ctypes.c_void_p).value)
+        lib.compiled = _Compiled(binding, lib) if all(hasattr(binding, name) for name in _Compiled.NAMES) else None
     _lib = lib
     return lib
 
@@ -198,9 +199,24 @@ def _no_binding(*args):
     return None
 
 
+class _Compiled:
+    """What the binding has besides ``adam_update`` (csrc/ps_binding.cpp): ``lib.compiled``, if it was built with the library."""
+
+    NAMES = ("step_chunks", "step_dynamic", "quiet", "same_flags", "read_numbers", "write_steps")
+
+    def __init__(self, binding, lib):
+        def of(call, entry):
+            return functools.partial(call, ctypes.cast(entry, ctypes.c_void_p).value)
+
+        self.step_chunks = of(binding.step_chunks, lib.ps_adam_step_chunks)
+        self.step_dynamic = of(binding.step_dynamic, lib.ps_adam_step_chunks_dynamic)
+        self.quiet, self.same_flags = binding.quiet, binding.same_flags
+        self.read_numbers, self.write_steps = binding.read_numbers, binding.write_steps
+
+
 def _load_binding():
-    """The compiled operator call, or None with a warning: adam_op then makes every call through its general path, which
-    does the same through the same library in more host time (3 us of 6.4 are spent on what the binding saves)."""
+    """The compiled calls, or None with a warning: adam_op and FP16Adam then make every call through their general paths, which
+    do the same through the same library in more host time (3 us of 6.4 an operator's call, 8 of 13 a step)."""
     import torch  # noqa: F401  (the binding uses its libraries)
 
     from . import build
