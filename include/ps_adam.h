@@ -493,6 +493,18 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
                                 const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
                                 int64_t log_capacity, int64_t operator_calls, ps_stream_t stream);
 
+/*
+ * The same with 256 bytes of device memory (64-byte aligned, all zero before the first call) that the workgroups of a launch
+ * agree through: lists of up to 400 tiles of 256 elements then take one launch, done by many workgroups.  It belongs to
+ * d_state: calls that share it must be ordered as calls on d_state must, and nothing else may write to it.  NULL: as above.
+ */
+#define PS_STEP_SCRATCH_BYTES 256
+int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
+                                        const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
+                                        const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
+                                        int64_t log_capacity, int64_t operator_calls, void* d_scratch, size_t scratch_bytes,
+                                        ps_stream_t stream);
+
 /* Copy *d_state to host memory and wait for it: the only synchronising call. */
 int ps_state_read(const ps_step_state* d_state, ps_step_state* host_out, ps_stream_t stream);
 

@@ -16,6 +16,7 @@ PS_ERR_BAD_ARG, PS_ERR_UNKNOWN_ID, PS_ERR_NO_DEVICE = -10001, -10002, -10003
 PS_ARITH_OPERATOR, PS_ARITH_TORCH = 0, 1
 PS_TENSOR_GRAD_F32 = 1
 PS_ABI_VERSION = 5
+PS_STEP_SCRATCH_BYTES = 256
 
 
 class ps_chunk(ctypes.Structure):
@@ -155,6 +156,7 @@ SIGNATURES = {
     "ps_grad_to_chunk": (_i, [_vp, _i, _vp, _sz, _vp, _vp]),
     "ps_scaler_update": (_i, [_vp, _i, _vp, _i64, _i64, _vp]),
     "ps_adam_step_chunks_dynamic": (_i, [_i, _d, _d, _d, _i, _vp, _i, _sz, _vp, _vp, _i, _vp, _vp, _i64, _i64, _vp]),
+    "ps_adam_step_chunks_dynamic_scratch": (_i, [_i, _d, _d, _d, _i, _vp, _i, _sz, _vp, _vp, _i, _vp, _vp, _i64, _i64, _vp, _sz, _vp]),
     "ps_state_read": (_i, [_vp, ctypes.POINTER(ps_step_state), _vp]),
 }
 
@@ -209,7 +211,7 @@ class _Compiled:
             return functools.partial(call, ctypes.cast(entry, ctypes.c_void_p).value)
 
         self.step_chunks = of(binding.step_chunks, lib.ps_adam_step_chunks)
-        self.step_dynamic = of(binding.step_dynamic, lib.ps_adam_step_chunks_dynamic)
+        self.step_dynamic = of(binding.step_dynamic, lib.ps_adam_step_chunks_dynamic_scratch)
         self.quiet, self.same_flags = binding.quiet, binding.same_flags
         self.read_numbers, self.write_steps = binding.read_numbers, binding.write_steps
 

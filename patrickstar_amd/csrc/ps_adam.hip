@@ -456,26 +456,26 @@ void launch_gated_batch(int arith, const ChunkBatch& b, dim3 grid, size_t chunk_
 
 template <int ARITH, typename LIST>
 void launch_small_step_arith(const LIST& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
-                             ps_step_state* d_state, hipStream_t s)
+                             ps_step_state* d_state, StepScratch* scratch, hipStream_t s)
 {
-    dim3 grid(1), block(kBlock, kSmallWaves);
+    dim3 grid(scratch ? (a.n_tiles + kSmallSpan - 1) / kSmallSpan : 1), block(kBlock, kSmallWaves);
     const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
     if (decay && ga.adamw)
-        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_DECOUPLED>), grid, block, 0, s, b, a, ga, fc, d_state);
+        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_DECOUPLED>), grid, block, 0, s, b, a, ga, fc, d_state, scratch);
     else if (decay)
-        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_L2>), grid, block, 0, s, b, a, ga, fc, d_state);
+        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_L2>), grid, block, 0, s, b, a, ga, fc, d_state, scratch);
     else
-        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_NONE>), grid, block, 0, s, b, a, ga, fc, d_state);
+        hipLaunchKernelGGL((adam_small_step_kernel<LIST, ARITH, WD_NONE>), grid, block, 0, s, b, a, ga, fc, d_state, scratch);
 }
 
 template <typename LIST>
 void launch_small_step(int arith, const LIST& b, const SmallStep& a, const GatedArgs& ga, const FirstCall& fc,
-                       ps_step_state* d_state, hipStream_t s)
+                       ps_step_state* d_state, StepScratch* scratch, hipStream_t s)
 {
     if (arith == PS_ARITH_TORCH)
-        launch_small_step_arith<PS_ARITH_TORCH>(b, a, ga, kNoFirstCall, d_state, s);
+        launch_small_step_arith<PS_ARITH_TORCH>(b, a, ga, kNoFirstCall, d_state, scratch, s);
     else
-        launch_small_step_arith<PS_ARITH_OPERATOR>(b, a, ga, fc, d_state, s);
+        launch_small_step_arith<PS_ARITH_OPERATOR>(b, a, ga, fc, d_state, scratch, s);
 }
 
 template <typename LIST, bool NT>
@@ -2072,10 +2072,11 @@ int ps_scaler_update(ps_step_state* d_state, int flag_mode, ps_scale_record* d_l
     return 0;
 }
 
-int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
-                                const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
-                                const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
-                                int64_t log_capacity, int64_t operator_calls, ps_stream_t stream)
+int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
+                                        const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
+                                        const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
+                                        int64_t log_capacity, int64_t operator_calls, void* d_scratch, size_t scratch_bytes,
+                                        ps_stream_t stream)
 {
     auto o = find_opt(optimizer_id);
     if (!o) return fail(PS_ERR_UNKNOWN_ID, "optimizer id %d was never created", optimizer_id);
@@ -2083,24 +2084,32 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
     if (d_log != nullptr && log_capacity <= 0)
         return fail(PS_ERR_BAD_ARG, "log_capacity must be positive when d_log is given");
     if (operator_calls < 0) return fail(PS_ERR_BAD_ARG, "operator_calls = %lld is negative", (long long)operator_calls);
+    if (d_scratch != nullptr && (scratch_bytes < sizeof(StepScratch) || reinterpret_cast<uintptr_t>(d_scratch) % 64))
+        return fail(PS_ERR_BAD_ARG, "d_scratch holds %zu bytes at %p; it needs %zu, 64-byte aligned", scratch_bytes, d_scratch, sizeof(StepScratch));
     ChunkList a;
     if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kTile)) return rc;
     Calls k;
     if (int rc = make_calls(k, calls, n_chunks, chunk_numel)) return rc;
-    size_t tiles = 0;
-    for (int i = 0; i < n_chunks; ++i) tiles = std::max(tiles, (a.numel_of(i) + kTile - 1) / kTile);
-    if (n_chunks <= kBatch && tiles > 0 && tiles <= kSmallTiles / n_chunks) {
+    StepScratch* const scratch = static_cast<StepScratch*>(d_scratch);
+    size_t longest = 0;
+    for (int i = 0; i < n_chunks; ++i) longest = std::max(longest, a.numel_of(i));
+    const size_t tiles = (longest + kTile - 1) / kTile;
+    if (n_chunks <= kBatch && tiles > 0 && tiles <= (scratch ? kSmallTiles : kSmallTilesAlone) / n_chunks) {
         const GatedArgs ga = gated_args(*o, lr, epsilon, weight_decay, bias_correction, k.n_calls);
-        const SmallStep step{(uint32_t)tiles, (uint32_t)(tiles * n_chunks), (uint32_t)((((uint64_t)1 << 32) + tiles - 1) / tiles), chunk_numel, probe != 0, d_log, log_capacity, operator_calls};
+        const uint32_t scans = (uint32_t)((longest + kSmallScan - 1) / kSmallScan);
+        auto reciprocal = [](size_t n) { return (uint32_t)((((uint64_t)1 << 32) + n - 1) / n); };
+        const SmallStep step{(uint32_t)tiles, (uint32_t)(tiles * n_chunks), reciprocal(tiles), scans, probe ? scans * n_chunks : 0, reciprocal(scans),
+                             chunk_numel, d_log, log_capacity, operator_calls};
         const int arith = o->arith;
+        hipStream_t s = static_cast<hipStream_t>(stream);
         EvenList e;
         if (even_list(a, kMaxEvenElementsGated, &e)) {
-            launch_small_step(arith, e, step, ga, k.in_batch(0, n_chunks), d_state, static_cast<hipStream_t>(stream));
+            launch_small_step(arith, e, step, ga, k.in_batch(0, n_chunks), d_state, scratch, s);
             PS_HIP(hipGetLastError());
             return 0;
         }
         return for_each_batch(a, [&](const ChunkBatch& b, dim3, int) {
-            launch_small_step(arith, b, step, ga, k.in_batch(0, n_chunks), d_state, static_cast<hipStream_t>(stream));
+            launch_small_step(arith, b, step, ga, k.in_batch(0, n_chunks), d_state, scratch, s);
         });
     }
     if (probe)
@@ -2109,6 +2118,15 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
                                            chunk_numel, used_numel, calls, d_state, stream))
         return rc;
     return ps_scaler_update(d_state, PS_FLAG_FROM_DEVICE, d_log, log_capacity, operator_calls, stream);
+}
+
+int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
+                                const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
+                                const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
+                                int64_t log_capacity, int64_t operator_calls, ps_stream_t stream)
+{
+    return ps_adam_step_chunks_dynamic_scratch(optimizer_id, lr, epsilon, weight_decay, bias_correction, chunks, n_chunks, chunk_numel, used_numel,
+                                               calls, probe, d_state, d_log, log_capacity, operator_calls, nullptr, 0, stream);
 }
 
 int ps_state_read(const ps_step_state* d_state, ps_step_state* host_out, ps_stream_t stream)

@@ -202,24 +202,25 @@ PyObject* step_chunks(PyObject*, PyObject* const* args, Py_ssize_t n)
     });
 }
 
-// (address of ps_adam_step_chunks_dynamic, device, list_of's, lr, eps, weight decay, probe, state, log, its capacity, operator calls) -> its
-// return code, or None
+// (address of ps_adam_step_chunks_dynamic_scratch, device, list_of's, lr, eps, weight decay, probe, state, log, its capacity, operator
+// calls, scratch) -> its return code, or None
 PyObject* step_dynamic(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     long long address, capacity, operator_calls;
     List l;
     double lr, eps, wd;
-    void *state, *log, *stream;
-    if (n != 16 || !integer(args[0], 1, INT64_MAX, address) || !list_of(args + 2, l) || !number(args[8], lr) || !number(args[9], eps) ||
+    void *state, *log, *scratch, *stream;
+    if (n != 17 || !integer(args[0], 1, INT64_MAX, address) || !list_of(args + 2, l) || !number(args[8], lr) || !number(args[9], eps) ||
         !number(args[10], wd) || (args[11] != Py_True && args[11] != Py_False) || !integer(args[14], 0, INT64_MAX, capacity) ||
         !integer(args[15], 0, INT64_MAX, operator_calls) || !current_stream(args[1], stream) || !device_bytes(args[12], args[1], state) ||
-        !device_bytes(args[13], args[1], log) || !state)
+        !device_bytes(args[13], args[1], log) || !state ||
+        !device_bytes(args[16], args[1], scratch))
         Py_RETURN_NONE;
-    const auto call = reinterpret_cast<decltype(&ps_adam_step_chunks_dynamic)>(address);
+    const auto call = reinterpret_cast<decltype(&ps_adam_step_chunks_dynamic_scratch)>(address);
     const int probe = args[11] == Py_True;
     return called("step_dynamic", [&] {
         return call((int)l.id, lr, eps, wd, 1, l.chunks, (int)l.n, (size_t)l.numel, l.used, l.calls, probe, static_cast<ps_step_state*>(state),
-                    static_cast<ps_scale_record*>(log), capacity, operator_calls, stream);
+                    static_cast<ps_scale_record*>(log), capacity, operator_calls, scratch, scratch ? PS_STEP_SCRATCH_BYTES : 0, stream);
     });
 }
 

@@ -41,8 +41,14 @@
 #ifndef PS_COPY_BLOCK
 #define PS_COPY_BLOCK 256  // threads per workgroup of the backward-side gradient copy (64: 43 us instead of 40 for 64 Mi fp16 elements off the slot's phase)
 #endif
+#ifndef PS_SMALL_WAVES
+#define PS_SMALL_WAVES 16  // waves of a workgroup of the step in one launch: one for the state, the others a tile each
+#endif
 #ifndef PS_SMALL_TILES
-#define PS_SMALL_TILES 80  // longest list (256-element tiles) that one workgroup probes, steps and rescales in one launch
+#define PS_SMALL_TILES 400  // longest list (256-element tiles) that is probed, stepped and rescaled in one launch
+#endif
+#ifndef PS_SMALL_TILES_ALONE
+#define PS_SMALL_TILES_ALONE 80  // the same by one workgroup, where the caller has no scratch memory for several to share
 #endif
 #if PS_MAX_WAVES_PER_EU > 0
 #define PS_OCCUPANCY __attribute__((amdgpu_waves_per_eu(1, PS_MAX_WAVES_PER_EU)))

@@ -1249,116 +1249,366 @@ __global__ void __launch_bounds__(64)
 
 // ------------------------------------------- a whole device-decided step over a short chunk list
 //
-// Probe, update (or restore) and scale update of a list of at most kSmallTiles tiles by ONE workgroup of 16 waves.  As
-// three kernels they take three launches whatever the list's length, and the GPU waits for each.  The probe's flag crosses
-// the waves through LDS; waves 0 to 14 then go over the tiles, the last one meanwhile forms the next state, which
-// replaces the old one when nobody reads that any more.
-// Bound by the host and one launch up to about 80 tiles, by one CU's arithmetic (4 us + 0.12 us a tile, 12.8 us for 75
-// tiles) from there on; the three kernels take 10.6 us and the gaps between them.  FP16Adam.step(), in one launch / in three:
-// waited for, at 1 / 30 / 60 / 75 / 81 / 90 / 120 tiles 25.4 / 25.4 / 28.7 / 30.5 / 30.8 / 33.9 / 36.2 us against 29.8 to
-// 30.7 at all of them; among other steps 14.5 / 13.9 / 13.7 / 13.8 / 13.8 / 16.7 / 19.0 against 18.5 to 20.7.  The line is
-// the last length at which a step that is waited for is no slower (by more than the 0.4 us that runs differ by) and the
-// kernel still hides behind the host's work for the next step.
-constexpr int kSmallWaves = 16;
-constexpr unsigned kSmallTiles = PS_SMALL_TILES;
+// Probe, update (or restore) and scale update in one launch.  As three kernels they take three launches whatever the list's
+// length, and the GPU waits for each.  The list is divided among workgroups of 15 waves with a tile (256 elements) each and a
+// sixteenth that forms the step's constants and the next state.  EVERY workgroup probes the whole list, so that none has to
+// wait for another.
+//
+// No workgroup waits, so the order in which they run is open, and one that starts late can find fp16 gradients already
+// replaced by parameters.  What it finds then must not mislead it:
+//   * clean step: a parameter that is inf or nan as binary16 looks like an overflow.  The wave that stores such a one first marks
+//     the step as clean (StepScratch::clean); who finds an overflow looks there before it believes it.
+//   * overflow: the gradient that says so may have been replaced.  A workgroup that has found it marks the step
+//     (StepScratch::dirty) before it restores anything; who finds no overflow looks there before it believes it.
+// A mark is stored with device scope and complete before the stores it announces are issued; a look is a device-scope load
+// that depends on what the probe's loads brought.  Whoever has read a replaced value therefore sees the mark that came before it, and by
+// induction over the workgroups' decisions all of them decide what the gradients alone say.  Marks carry the number
+// of the launch (StepScratch::epoch), so nobody has to clear them.
+//
+// The state is replaced by the workgroup that took the last ticket; a ticket is taken when a workgroup has the state in its
+// registers.  Tickets and looks cost a trip to memory each, in the shadow of the probe and of the arithmetic.  A list
+// that one workgroup does alone needs neither, and no scratch.
+//
+// Bound by one CU's reads of the whole list (133 GB/s, 3.1 us for every 800 tiles) and by a chain of trips to memory: arguments,
+// state or gradients, mark, stores.  Device time of a step back to back, by one workgroup / three kernels / this: 1 tile 4.3 / - / 4.8 us,
+// 75 tiles 12.45 / 8.5 / 6.9, 120 - / 8.5 / 7.2, 240 - / 8.6 / 8.0, 480 - / 8.9 / 9.4, 800 - / 9.2 / 10.8, 1600 - / 9.7 / 13.8.  Among
+// other steps that is what FP16Adam.step() takes, if the host's part is not longer (4.6 us for one launch, 8.9 for three): 75 tiles 12.45
+// by one workgroup, 8.9 by three kernels, 6.7 by this, 240 tiles 8.9 / 7.7, 480 tiles 8.9 / 9.3; waited for, 75 tiles 27 / 22.3 / 18.9, 240
+// tiles 22.3 / 19.7, 480 tiles 22.3 / 21.4.  The line (kSmallTiles) lies where neither is the longer one.
+// Workgroups of 4 / 6 / 8 / 12 / 16 waves: 75 tiles 7.6 / 6.9 / 6.6 / 7.2 / 6.9, 480 tiles 15.2 / 12.1 / 10.9 / 9.5 / 9.5; two or
+// four tiles a wave 480 tiles 9.8 / 13.8.
+constexpr int kSmallWaves = PS_SMALL_WAVES;
+constexpr uint32_t kSmallSpan = kSmallWaves - 1;  // tiles that a workgroup has in hand at a time
+constexpr uint32_t kSmallScan = 4096;             // halves that a wave probes at a time: eight 16-byte loads a lane
+constexpr unsigned kSmallTiles = PS_SMALL_TILES, kSmallTilesAlone = PS_SMALL_TILES_ALONE;
 struct SmallStep {
     uint32_t tiles, n_tiles;  // of one chunk (as wide as the widest, like the grid of the chunk-list kernels), of the list
     uint32_t per_tile;        // 2^32 / tiles, rounded up: t * per_tile / 2^32 is t / tiles for every t of so short a list; 0: one tile each
+    uint32_t scans, n_scans, per_scan;  // the same in spans of kSmallScan; n_scans 0: no probe
     size_t chunk_numel;
-    int probe;
     ps_scale_record* log;
     int64_t log_capacity, operator_calls;
 };
 
-struct SmallTile {
-    ps_chunk c;
-    size_t base, numel;  // the tile's first element in its chunk; the chunk's elements
-    uint32_t k;
+// What the workgroups of one launch share (PS_STEP_SCRATCH_BYTES, the caller's, zero at first).
+struct StepScratch {
+    uint64_t epoch;  // launches so far
+    uint64_t pad0[15];
+    uint32_t tickets;  // 0 between launches
+    uint32_t pad1[15];
+    uint64_t dirty, clean;  // epoch + 1 of the latest launch that was marked so
+    uint64_t pad2[6];
 };
+static_assert(sizeof(StepScratch) == PS_STEP_SCRATCH_BYTES, "the caller's allocation");
+
 // The chunks of an EvenChunk list: 48 bytes of arguments where ChunkBatch has 2560, which cost the host 0.35 us a launch (the smoke
 // test's list, 13.8 -> 13.4 us a step among others) and the kernel 0.4.
 struct EvenBatch {
     ps_chunk first;
     uint32_t stride, numel, last, short_by;
 };
-__device__ __forceinline__ void small_chunk(const ChunkBatch& b, SmallTile& w)
+__device__ __forceinline__ void small_chunk(const ChunkBatch& b, uint32_t k, ps_chunk& c, uint32_t& numel)
 {
-    w.c = b.c[w.k];
-    w.numel = b.n[w.k];
+    c = b.c[k];
+    numel = (uint32_t)b.n[k];
 }
-__device__ __forceinline__ void small_chunk(const EvenBatch& b, SmallTile& w)
+__device__ __forceinline__ void small_chunk(const EvenBatch& b, uint32_t k, ps_chunk& c, uint32_t& numel)
 {
-    const size_t at = (size_t)b.stride * w.k;
-    w.c = ps_chunk{b.first.param_fp32 + at, b.first.exp_avg + at, b.first.exp_avg_sq + at, b.first.param_fp16 + at};
-    w.numel = b.numel - (w.k == b.last ? b.short_by : 0u);
+    const size_t at = (size_t)b.stride * k;
+    c = ps_chunk{b.first.param_fp32 + at, b.first.exp_avg + at, b.first.exp_avg_sq + at, b.first.param_fp16 + at};
+    numel = b.numel - (k == b.last ? b.short_by : 0u);
 }
+
+// ---- the probe: a binary16 value times zero is a NaN iff it is inf or nan, and a NaN stays one through every sum: one packed
+// instruction for two values, where the masks of nonfinite_halves take seven.  (The probe of a list that is read once by the
+// whole GPU hides them; here a CU reads all of it.)
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+struct SmallScan {
+    uint4v w[kSmallScan / 512];
+    uint32_t odd;
+};
 template <typename LIST>
-__device__ __forceinline__ SmallTile small_tile(const LIST& b, const SmallStep& a, uint32_t t)
+__device__ __forceinline__ void small_scan_load(SmallScan& r, const LIST& b, const SmallStep& a, uint32_t i)
 {
-    SmallTile w;
-    w.k = a.per_tile ? __umulhi(t, a.per_tile) : t;  // t / tiles
-    small_chunk(b, w);
-    w.base = (size_t)(t - w.k * a.tiles) * kTile;
-    return w;
+    // each workgroup begins somewhere else: all of them at the same lines of one L2 channel take their time
+    uint32_t s = i + blockIdx.x;
+    while (s >= a.n_scans) s -= a.n_scans;
+    const uint32_t k = a.per_scan ? __umulhi(s, a.per_scan) : s, base = (s - k * a.scans) * kSmallScan;
+    ps_chunk chunk;
+    uint32_t numel;
+    small_chunk(b, k, chunk, numel);
+    r.odd = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kSmallScan / 512; ++u) r.w[u] = uint4v{0, 0, 0, 0};
+    if (base >= numel) return;
+    const PS_GLOBAL char* h = (const PS_GLOBAL char*)(chunk.param_fp16 + base);
+    const uint32_t here = numel - base < kSmallScan ? numel - base : kSmallScan, n_vec = here / 8, behind = 8 * n_vec + threadIdx.x;
+    // lanes behind the end read what is in front of it again
+    if (n_vec != 0) {
+#pragma unroll
+        for (uint32_t u = 0; u < kSmallScan / 512; ++u) {
+            const uint32_t v = u * 64 + threadIdx.x;
+            r.w[u] = *(const PS_GLOBAL uint4v_half_aligned*)(h + (v < n_vec ? v : n_vec - 1) * 16);
+        }
+    }
+    r.odd = *(const PS_GLOBAL uint16_t*)(h + (behind < here ? behind : here - 1) * 2);
+}
+__device__ __forceinline__ half2v small_scan_add(const SmallScan& r, half2v sum)
+{
+    const half2v zero = {0, 0};
+#pragma unroll
+    for (uint32_t u = 0; u < kSmallScan / 512; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t two = r.w[u][k];  // (a bit_cast of the vector's element is one of its first)
+            sum = __builtin_elementwise_fma(__builtin_bit_cast(half2v, two), zero, sum);
+        }
+    return __builtin_elementwise_fma(__builtin_bit_cast(half2v, r.odd), zero, sum);
+}
+
+// ---- one lane's share of a tile: elements base + 4 * lane + e of a whole one, base + lane + 64 * e of any other
+struct SmallShare {
+    ps_chunk c;             // addresses of the tile's first element
+    uint32_t base, numel;   // the tile's first element in its chunk; the chunk's elements
+    uint32_t end;           // of what is updated, counted from base
+    bool whole, here;       // with vector accesses; its chunk holds elements of the step's first operator call
+    uint32_t g[4], h[4];    // g of a whole tile: two words of pairs, as they were loaded
+    float old[4], p[4], m[4], v[4];
+};
+template <typename T>
+__device__ __forceinline__ PS_GLOBAL T* small_at(const void* first, uint32_t i)
+{
+    return (PS_GLOBAL T*)((PS_GLOBAL char*)first + i * (uint32_t)sizeof(T));
+}
+
+// Elements of a tile that is not whole: all in flight; lanes behind the end read the last element again and store nothing.
+__device__ __forceinline__ void small_load_single(SmallShare& o)
+{
+    if (o.end == 0) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t at = threadIdx.x + e * kBlock, i = at < o.end ? at : o.end - 1;
+        o.g[e] = *small_at<uint16_t>(o.c.param_fp16, i);
+        o.old[e] = *small_at<float>(o.c.param_fp32, i);
+        o.m[e] = *small_at<float>(o.c.exp_avg, i);
+        o.v[e] = *small_at<float>(o.c.exp_avg_sq, i);
+    }
+}
+
+template <typename LIST>
+__device__ __forceinline__ void small_load(SmallShare& o, const LIST& b, const SmallStep& a, const FirstCall& fc, uint32_t t)
+{
+    const uint32_t k = a.per_tile ? __umulhi(t, a.per_tile) : t, tile = t - k * a.tiles;
+    small_chunk(b, k, o.c, o.numel);
+    o.base = tile * kTile;
+    o.c.param_fp32 += o.base;
+    o.c.exp_avg += o.base;
+    o.c.exp_avg_sq += o.base;
+    o.c.param_fp16 += o.base;
+    o.here = fc.chunk == (int)k;
+    const bool cut = o.here && tile >= fc.lo_tile && tile < fc.hi_tile && !(tile >= fc.in_lo && tile < fc.in_hi);
+    o.whole = o.base + kTile <= o.numel && !cut && aligned16(o.c.param_fp32, o.c.exp_avg, o.c.exp_avg_sq, o.c.param_fp16);
+    if (o.whole) {
+        o.end = kTile;
+        const uint2v g = *small_at<uint2v>(o.c.param_fp16, threadIdx.x);
+        const float4v p = *small_at<float4v>(o.c.param_fp32, threadIdx.x), m = *small_at<float4v>(o.c.exp_avg, threadIdx.x),
+                      v = *small_at<float4v>(o.c.exp_avg_sq, threadIdx.x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            o.g[e] = g[e & 1];
+            o.old[e] = p[e], o.m[e] = m[e], o.v[e] = v[e];
+        }
+        return;
+    }
+    o.end = o.base >= o.numel ? 0 : o.numel - o.base < kTile ? o.numel - o.base : kTile;
+    small_load_single(o);
+}
+
+template <int ARITH, int WD, int UNS>
+__device__ __forceinline__ void small_math(SmallShare& o, const StepConsts& c, const FirstCall& fc)
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const size_t i = o.base + (o.whole ? 4 * threadIdx.x + e : threadIdx.x + e * kBlock);
+        const bool first = o.here && i >= fc.lo && i < fc.hi;
+        const float g = half_bits_to_float((o.whole ? o.g[e >> 1] >> (16 * (e & 1)) : o.g[e]) & 0xFFFFu);
+        o.p[e] = o.old[e];
+        adam_element<ARITH, WD, UNS>(c, first ? c.first_step_size : c.step_size, first ? c.first_bc2inv : c.bc2inv, g, o.p[e], o.m[e], o.v[e]);
+        o.h[e] = float_to_half_bits(o.p[e]);
+    }
+}
+
+// The constants of the step as the workgroup's waves share them.
+struct SmallConsts {
+    StepConsts c;
+    int keeps_zeros_here, keeps_zeros;  // zeros_are_a_fixed_point, of chunks with and without elements of the first call
+};
+template <int ARITH, int WD>
+__device__ __forceinline__ void small_update(SmallShare& o, const SmallConsts& k, const SmallStep& a, const FirstCall& fc)
+{
+    if (!o.whole && o.base + kTile > o.numel && o.numel < a.chunk_numel && !(o.here ? k.keeps_zeros_here : k.keeps_zeros)) {
+        // the padding is computed, as in adam_chunks_gated_kernel
+        o.end = (uint32_t)(a.chunk_numel - o.base < kTile ? a.chunk_numel - o.base : kTile);
+        small_load_single(o);
+    }
+    if (k.c.unscale == UNSCALE_MUL)
+        small_math<ARITH, WD, UNSCALE_MUL>(o, k.c, fc);
+    else if (ARITH == PS_ARITH_OPERATOR && k.c.unscale == UNSCALE_DIV)
+        small_math<ARITH, WD, UNSCALE_DIV>(o, k.c, fc);
+    else
+        small_math<ARITH, WD, UNSCALE_NONE>(o, k.c, fc);
+}
+
+__device__ __forceinline__ void small_store(const SmallShare& o)
+{
+    if (o.whole) {
+        *small_at<float4v>(o.c.param_fp32, threadIdx.x) = float4v{o.p[0], o.p[1], o.p[2], o.p[3]};
+        *small_at<float4v>(o.c.exp_avg, threadIdx.x) = float4v{o.m[0], o.m[1], o.m[2], o.m[3]};
+        *small_at<float4v>(o.c.exp_avg_sq, threadIdx.x) = float4v{o.v[0], o.v[1], o.v[2], o.v[3]};
+        *small_at<uint2v>(o.c.param_fp16, threadIdx.x) = uint2v{o.h[0] | (o.h[1] << 16), o.h[2] | (o.h[3] << 16)};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t i = threadIdx.x + e * kBlock;
+        if (i >= o.end) continue;
+        *small_at<float>(o.c.param_fp32, i) = o.p[e];
+        *small_at<float>(o.c.exp_avg, i) = o.m[e];
+        *small_at<float>(o.c.exp_avg_sq, i) = o.v[e];
+        *small_at<uint16_t>(o.c.param_fp16, i) = (uint16_t)o.h[e];
+    }
+}
+
+// fp16 <- RNE(fp32): a skipped step.  (`end` is still that of the chunk's elements.)
+__device__ __forceinline__ void small_restore(const SmallShare& o)
+{
+    uint32_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) h[e] = float_to_half_bits(o.old[e]);
+    if (o.whole) {
+        *small_at<uint2v>(o.c.param_fp16, threadIdx.x) = uint2v{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t i = threadIdx.x + e * kBlock;
+        if (i < o.end && o.base + i < o.numel) *small_at<uint16_t>(o.c.param_fp16, i) = (uint16_t)h[e];
+    }
+}
+
+// Stores with device scope, complete before anything behind it is issued.
+__device__ __forceinline__ void small_mark(uint64_t* mark, uint64_t epoch)
+{
+    if (threadIdx.x == 0) __hip_atomic_store(mark, epoch + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
+}
+
+// __syncthreads() for what crosses the waves here, LDS words: loads, stores and the ticket in flight are not waited for.
+__device__ __forceinline__ void small_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    asm volatile("" ::: "memory");  // nor does the compiler move a load or store across
 }
 
 template <typename LIST, int ARITH, int WD>
 __global__ void __launch_bounds__(64 * kSmallWaves)
-    adam_small_step_kernel(LIST b, SmallStep a, GatedArgs ga, FirstCall fc, ps_step_state* st)
+    adam_small_step_kernel(LIST b, SmallStep a, GatedArgs ga, FirstCall fc, ps_step_state* st, StepScratch* scratch)
 {
-    static_assert(kBlock == 64 && kLaneElems == 4 && kUnroll == 1, "tiles of one wave, four elements per lane");
-    __shared__ uint32_t wave_hit[kSmallWaves];
-    __shared__ ps_step_state next;
+    static_assert(kBlock == 64 && kTile == 256, "tiles of one wave, four elements per lane");
+    __shared__ uint32_t wave_hit[64];
+    __shared__ uint32_t flagged, verdict, mark_low, mark_high;
+    __shared__ SmallConsts consts;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.y), lane = threadIdx.x;
-    const StateView sv = view_state(st);
-    uint32_t hit = 0;
-    if (a.probe) {
-        for (uint32_t t = wave; t < a.n_tiles; t += kSmallWaves) {
-            const SmallTile w = small_tile(b, a, t);
-            if (w.base >= w.numel) continue;
-            const PS_GLOBAL uint16_t* h = (const PS_GLOBAL uint16_t*)w.c.param_fp16 + w.base;
-            if (w.base + kTile <= w.numel && ((uintptr_t)w.c.param_fp16 & 7u) == 0) {
-                const uint2v x = ((const guint2v*)h)[lane];
-                hit |= nonfinite_halves(x[0]) | nonfinite_halves(x[1]);
-                continue;
-            }
-            const uint32_t n = w.numel - w.base < kTile ? (uint32_t)(w.numel - w.base) : kTile;
-#pragma unroll
-            for (int e = 0; e < kTile / kBlock; ++e) hit |= nonfinite_halves(h[lane + e * kBlock < n ? lane + e * kBlock : n - 1]);
+    const bool several = gridDim.x > 1;
+    if (wave == kSmallSpan) {
+        // ---- the state's wave
+        const ps_step_state now = *st;
+        uint64_t epoch = 0;
+        uint32_t ticket = 0;
+        const StateView sv = view_state(&now);
+        if (several) {
+            epoch = scratch->epoch;
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // all of the state is here: behind the ticket it may change
+            PS_GLOBAL uint32_t* tickets = (PS_GLOBAL uint32_t*)&scratch->tickets;
+            asm volatile("" : "+v"(tickets));  // (of an address known to be uniform the compiler waits for the result at once)
+            if (lane == 0) ticket = __hip_atomic_fetch_add(tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+        const StepConsts c_rest = gated_consts<ARITH>(ga, sv, false);
+        StepConsts c = c_rest;
+        // the first call's pair is formed if the list holds any of that call
+        if (fc.chunk >= 0 && ARITH == PS_ARITH_OPERATOR && ga.n_calls > 1)
+            bias_scalars((float)ga.lr, sv.b1t_next, sv.b2t_next, ga.bias_correction != 0, &c.first_step_size, &c.first_bc2inv);
+        if (lane == 0) {
+            consts.c = c;
+            consts.keeps_zeros = zeros_are_a_fixed_point(c_rest);
+            consts.keeps_zeros_here = zeros_are_a_fixed_point(c);
+            flagged = sv.overflow;
+            mark_low = (uint32_t)epoch, mark_high = (uint32_t)(epoch >> 32);
+        }
+        small_barrier();
+        bool overflow = sv.overflow != 0 || __any(lane < kSmallSpan && wave_hit[lane] != 0);
+        uint64_t mark = 0;
+        const bool marks = several && a.n_scans != 0 && !sv.overflow;
+        if (marks) mark = __hip_atomic_load(overflow ? &scratch->clean : &scratch->dirty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const ps_step_state clean = scaler_updated(now, false, a.operator_calls);  // while the mark is on its way
+        if (marks) {
+            const bool marked = mark == epoch + 1;
+            if (overflow && !marked) small_mark(&scratch->dirty, epoch);
+            overflow = overflow != marked;
+        }
+        if (lane == 0) verdict = overflow;
+        small_barrier();
+        if (several && (uint32_t)__builtin_amdgcn_readfirstlane(ticket) != gridDim.x - 1) return;
+        const ps_step_state after = overflow ? scaler_updated(now, true, a.operator_calls) : clean;
+        if (lane == 0) {
+            scaler_store(st, after, a.log, a.log_capacity);
+            if (several) {
+                scratch->epoch = epoch + 1;
+                __hip_atomic_store(&scratch->tickets, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        return;
     }
-    // the constants do not wait for the flag; the first call's pair is formed if the list holds any of that call
-    const StepConsts c_rest = gated_consts<ARITH>(ga, sv, false);
-    const StepConsts c = fc.chunk >= 0 ? gated_consts<ARITH>(ga, sv, true) : c_rest;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) hit |= (uint32_t)__shfl_xor((int)hit, off, 64);
+    // ---- a wave with tiles
+    SmallShare o;
+    SmallScan scan;
+    half2v sum = {0, 0};
+    uint32_t t = blockIdx.x * kSmallSpan + wave;
+    const bool any_tile = t < a.n_tiles;
+    if (wave < a.n_scans) small_scan_load(scan, b, a, wave);
+    if (any_tile) small_load(o, b, a, fc, t);
+    if (wave < a.n_scans) sum = small_scan_add(scan, sum);
+    for (uint32_t i = wave + kSmallSpan; i < a.n_scans; i += kSmallSpan) {
+        small_scan_load(scan, b, a, i);
+        sum = small_scan_add(scan, sum);
+    }
+    const bool hit = __any(nonfinite_halves(__builtin_bit_cast(uint32_t, sum)) != 0);
     if (lane == 0) wave_hit[wave] = hit;
-    __syncthreads();
-    uint32_t any = sv.overflow;
+    small_barrier();
+    const bool known = __builtin_amdgcn_readfirstlane(flagged) != 0;
+    if (any_tile && !known) small_update<ARITH, WD>(o, consts, a, fc);
+    small_barrier();
+    const bool overflow = __builtin_amdgcn_readfirstlane(verdict) != 0;
+    if (!any_tile) return;
+    for (;;) {
+        if (overflow) {
+            small_restore(o);
+        } else {
+            if (several && a.n_scans != 0) {
+                uint32_t odd = 0;
 #pragma unroll
-    for (int w = 0; w < kSmallWaves; ++w) any |= wave_hit[w];
-    const bool overflow = __builtin_amdgcn_readfirstlane(any) != 0;
-    if (wave == kSmallWaves - 1) {
-        const ps_step_state after = scaler_updated(*st, overflow, a.operator_calls);
-        if (lane == 0) next = after;
-    } else {
-        for (uint32_t t = wave; t < a.n_tiles; t += kSmallWaves - 1) {
-            const SmallTile w = small_tile(b, a, t);
-            if (overflow) {
-                restore_tile(w.c.param_fp32, w.c.param_fp16, w.base, w.numel);
-                continue;
+                for (int e = 0; e < 4; ++e) odd |= nonfinite_halves(o.h[e]);
+                if (__builtin_expect(__any(odd != 0), 0)) small_mark(&scratch->clean, ((uint64_t)mark_high << 32) | mark_low);
             }
-            const bool here = fc.chunk == (int)w.k;
-            size_t numel = w.numel;
-            if (w.base + kTile > numel && numel < a.chunk_numel) {  // as in adam_chunks_gated_kernel
-                if (!zeros_are_a_fixed_point(here ? c : c_rest)) numel = a.chunk_numel;
-                if (w.base >= numel) continue;
-            }
-            adam_tile<ARITH, WD, UNSCALE_RUNTIME>(c, w.c, w.base, numel, here ? (size_t)fc.lo : 0, here ? (size_t)fc.hi : 0);
+            small_store(o);
         }
+        t += gridDim.x * kSmallSpan;
+        if (t >= a.n_tiles) return;
+        small_load(o, b, a, fc, t);
+        if (!overflow) small_update<ARITH, WD>(o, consts, a, fc);
     }
-    __syncthreads();
-    if (wave == kSmallWaves - 1 && lane == 0) scaler_store(st, next, a.log, a.log_capacity);
 }
 
 }  // namespace

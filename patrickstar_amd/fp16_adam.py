@@ -790,7 +790,8 @@ class FP16Adam(torch.optim.Optimizer):
             scan = bool(self.scan_in_step)
             if not self._is_one_call(scan):
                 return False
-            rc = compiled.step_dynamic(*where, lr, eps, weight_decay, scan, scaler._state, scaler._log, scaler._log_capacity, self._operator_calls)
+            rc = compiled.step_dynamic(*where, lr, eps, weight_decay, scan, scaler._state, scaler._log, scaler._log_capacity, self._operator_calls,
+                                       scaler._scratch)
             if rc is None:
                 return False
             if rc != 0:
@@ -858,13 +859,13 @@ class FP16Adam(torch.optim.Optimizer):
                     and self._is_one_call(scan)
                 ):
                     # HBM-resident chunks, all of them whole: probe, step and scale update in one call
-                    _lib.check(
-                        self._lib.ps_adam_step_chunks_dynamic(
-                            self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls,
-                            int(scan), scaler.state_ptr, *scaler.log_arguments(), self._operator_calls, stream,
-                        ),
-                        "ps_adam_step_chunks_dynamic",
-                    )
+                    args = (self.opt_id, lr, eps, weight_decay, 1, table, n_dev, chunk_numel, self._used, self._calls, int(scan),
+                            scaler.state_ptr, *scaler.log_arguments(), self._operator_calls)
+                    if scaler._scratch is None:
+                        rc = self._lib.ps_adam_step_chunks_dynamic(*args, stream)
+                    else:
+                        rc = self._lib.ps_adam_step_chunks_dynamic_scratch(*args, scaler._scratch.data_ptr(), _lib.PS_STEP_SCRATCH_BYTES, stream)
+                    _lib.check(rc, "ps_adam_step_chunks_dynamic")
                     self._steps_dirty = True
                     return loss
                 if scan:

@@ -58,6 +58,8 @@ class DynamicLossScaler:
     by a factor that is not a power of two is rounded like a float from there on.
     """
 
+    _scratch = None  # device tensor beside the state, which the workgroups of one launch agree through
+
     def __init__(
         self,
         init_scale=2**32,
@@ -116,6 +118,7 @@ class DynamicLossScaler:
         lib = _lib.load()
         device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
         self._state = torch.zeros(ctypes.sizeof(_lib.ps_step_state), dtype=torch.uint8, device=device)
+        self._scratch = torch.zeros(_lib.PS_STEP_SCRATCH_BYTES, dtype=torch.uint8, device=device)
         i = self._init
         if not i["scale_window"] > 0:
             raise ValueError(f"scale_window must be positive, got {i['scale_window']}")
