@@ -1225,7 +1225,9 @@ __device__ __forceinline__ ps_step_state scaler_updated(ps_step_state s, bool ov
     return s;
 }
 
-// One lane's work: the state as it now is, and the log's record of the iteration.
+// One lane's work: the state as it now is, and the log's record of the iteration.  Field by field, as far as scaler_updated changes them:
+// the reserved arrays of a state that is stored as a whole go through memory (3 KiB of LDS for every workgroup of a kernel that does
+// so, 64 KiB and scratch memory in adam_small_step_kernel: 75 tiles 7.0 -> 6.4 us, waited for 18.9 -> 17.6, 240 tiles 7.6 -> 6.5; three launches of 4096 tiles 12.1 -> 10.9).
 __device__ __forceinline__ void scaler_store(ps_step_state* st, const ps_step_state& s, ps_scale_record* log, int64_t log_capacity)
 {
     if (log != nullptr && log_capacity > 0) {
@@ -1235,7 +1237,27 @@ __device__ __forceinline__ void scaler_store(ps_step_state* st, const ps_step_st
         r.scale_is_int = (uint32_t)s.scale_is_int;
         log[(s.cur_iter - 1) % log_capacity] = r;
     }
-    *st = s;
+    st->cur_scale = s.cur_scale;
+    st->cur_iter = s.cur_iter;
+    st->last_overflow_iter = s.last_overflow_iter;
+    st->adam_step = s.adam_step;
+    st->skipped_steps = s.skipped_steps;
+    st->cur_hysteresis = s.cur_hysteresis;
+    st->scale_is_int = s.scale_is_int;
+    st->overflow = s.overflow;
+    st->last_skipped = s.last_skipped;
+    st->beta1_t_next = s.beta1_t_next;
+    st->beta2_t_next = s.beta2_t_next;
+    st->bias_correction1_next = s.bias_correction1_next;
+    st->bias_correction2_next = s.bias_correction2_next;
+    st->operator_step = s.operator_step;
+    st->beta1_t_cur = s.beta1_t_cur;
+    st->beta2_t_cur = s.beta2_t_cur;
+    st->beta1_t_rest = s.beta1_t_rest;
+    st->beta2_t_rest = s.beta2_t_rest;
+    st->operator_beta1 = s.operator_beta1;
+    st->operator_beta2 = s.operator_beta2;
+    st->pending_operator_step = s.pending_operator_step;
 }
 
 __global__ void __launch_bounds__(64)
@@ -1271,7 +1293,8 @@ __global__ void __launch_bounds__(64)
 //
 // Bound by one CU's reads of the whole list (133 GB/s, 3.1 us for every 800 tiles) and by a chain of trips to memory: arguments,
 // state or gradients, mark, stores.  Device time of a step back to back, by one workgroup / three kernels / this: 1 tile 4.3 / - / 4.8 us,
-// 75 tiles 12.45 / 8.5 / 6.9, 120 - / 8.5 / 7.2, 240 - / 8.6 / 8.0, 480 - / 8.9 / 9.4, 800 - / 9.2 / 10.8, 1600 - / 9.7 / 13.8.  Among
+// 75 tiles 12.45 / 8.5 / 6.9, 120 - / 8.5 / 7.2, 240 - / 8.6 / 8.0, 480 - / 8.9 / 9.4, 800 - / 9.2 / 10.8, 1600 - / 9.7 / 13.8 (all with
+// the state in memory: see scaler_store).  Among
 // other steps that is what FP16Adam.step() takes, if the host's part is not longer (4.6 us for one launch, 8.9 for three): 75 tiles 12.45
 // by one workgroup, 8.9 by three kernels, 6.7 by this, 240 tiles 8.9 / 7.7, 480 tiles 8.9 / 9.3; waited for, 75 tiles 27 / 22.3 / 18.9, 240
 // tiles 22.3 / 19.7, 480 tiles 22.3 / 21.4.  The line (kSmallTiles) lies where neither is the longer one.
