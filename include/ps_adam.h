@@ -494,11 +494,12 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
                                 int64_t log_capacity, int64_t operator_calls, ps_stream_t stream);
 
 /*
- * The same with 256 bytes of device memory (64-byte aligned, all zero before the first call) that the workgroups of a launch
- * agree through: lists of up to 400 tiles of 256 elements then take one launch, done by many workgroups.  It belongs to
+ * The same with PS_STEP_SCRATCH_BYTES of device memory (64-byte aligned, all zero before the first call) that the workgroups of a
+ * step agree through: lists of up to 280 tiles of 256 elements then take one launch, done by many workgroups, and with the
+ * probe lists of evenly spaced chunks (to 256 Mi elements) and other lists below 32 Mi elements two.  It belongs to
  * d_state: calls that share it must be ordered as calls on d_state must, and nothing else may write to it.  NULL: as above.
  */
-#define PS_STEP_SCRATCH_BYTES 256
+#define PS_STEP_SCRATCH_BYTES 448
 int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
                                         const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
                                         const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,

@@ -16,7 +16,7 @@ PS_ERR_BAD_ARG, PS_ERR_UNKNOWN_ID, PS_ERR_NO_DEVICE = -10001, -10002, -10003
 PS_ARITH_OPERATOR, PS_ARITH_TORCH = 0, 1
 PS_TENSOR_GRAD_F32 = 1
 PS_ABI_VERSION = 5
-PS_STEP_SCRATCH_BYTES = 256
+PS_STEP_SCRATCH_BYTES = 448
 
 
 class ps_chunk(ctypes.Structure):

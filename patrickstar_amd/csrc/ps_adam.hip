@@ -414,6 +414,48 @@ void launch_even_gated(const EvenList& e, size_t chunk_numel, const GatedArgs& g
     });
 }
 
+// The three forms of weight decay: launch(std::integral_constant<int, WD_...>).  The operator tests its float weight decay "> 0"
+// (cpu_adam.cpp:42), the torch formula "!= 0".
+template <int ARITH, typename F>
+void with_decay(const GatedArgs& ga, F launch)
+{
+    const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
+    if (decay && ga.adamw)
+        launch(std::integral_constant<int, WD_DECOUPLED>{});
+    else if (decay)
+        launch(std::integral_constant<int, WD_L2>{});
+    else
+        launch(std::integral_constant<int, WD_NONE>{});
+}
+
+template <bool NT>
+dim3 with_first(dim3 grid)
+{
+    return dim3(grid.x + kInFront<NT>, grid.y);
+}
+
+template <int ARITH>
+void launch_even_closing(const EvenList& e, size_t chunk_numel, const GatedArgs& ga, const FirstCall& fc, const Closing& cl, bool nt, hipStream_t s)
+{
+    with_hint(nt, [&](auto hint) {
+        with_decay<ARITH>(ga, [&](auto wd) {
+            constexpr bool NT = decltype(hint)::value;
+            constexpr int WD = decltype(wd)::value;
+            hipLaunchKernelGGL((adam_even_chunks_closing_kernel<ARITH, WD, NT>), with_first<NT>(even_grid(e, kTile)), dim3(kBlock), NT ? kStreamLdsBytes : kLdsBytes, s,
+                               PS_EVEN(e), &cl.x->opened, chunk_numel, ga, fc, cl);
+        });
+    });
+}
+
+template <int ARITH>
+void launch_closing_batch(const ChunkBatch& b, dim3 grid, size_t chunk_numel, const GatedArgs& ga, const FirstCall& fc, const Closing& cl, hipStream_t s)
+{
+    with_decay<ARITH>(ga, [&](auto wd) {
+        hipLaunchKernelGGL((adam_chunks_closing_kernel<ARITH, decltype(wd)::value>), with_first<false>(grid), dim3(kBlock), kLdsBytes, s, &cl.x->opened, b,
+                           chunk_numel, ga, fc, cl);
+    });
+}
+
 // `c` must have been built for `arith` (finish_consts / torch_consts).  `fc`: which elements of the
 // batch the step's first operator call covers; the torch formula has no such distinction.
 void launch_adam_batch(int arith, const ChunkBatch& b, dim3 grid, const StepConsts& c, const FirstCall& fc, bool nt,
@@ -2110,6 +2152,44 @@ int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsi
         }
         return for_each_batch(a, [&](const ChunkBatch& b, dim3, int) {
             launch_small_step(arith, b, step, ga, k.in_batch(0, n_chunks), d_state, scratch, s);
+        });
+    }
+    // Two launches: lists of evenly spaced chunks, and other lists below the line from which they stream past the caches.  (Beyond it the update's
+    // waves with descriptors, which read the copy behind them, lose what the third launch costs: 8 x 64 Mi elements in three / two
+    // 2423 / 2431 us, a skipped step 614 / 623.)
+    EvenList e;
+    const bool even = even_list(a, kMaxEvenElementsGated, &e);
+    if (probe && scratch && tiles > 0 && tiles <= kMaxGridX - kInFront<true> && (even || (n_chunks <= kBatch && elements(a) < kStreamElementsGated))) {
+        const GatedArgs ga = gated_args(*o, lr, epsilon, weight_decay, bias_correction, k.n_calls);
+        const Closing cl{d_state, scratch, d_log, log_capacity, operator_calls};
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        const bool torch = o->arith == PS_ARITH_TORCH;
+        const FirstCall fc = torch ? kNoFirstCall : k.in_batch(0, n_chunks);
+        if (even) {
+            const bool nt = streams(a, true);
+            with_hint(elements(a) >= kScanStreamElements, [&](auto hint) {
+                hipLaunchKernelGGL((open_even_chunks_kernel<decltype(hint)::value>), with_first<decltype(hint)::value>(even_grid(e, kScanTile)), dim3(kScanBlock), kScanLdsBytes, s,
+                                   e.first.param_fp16, e.stride, e.numel, e.last, e.short_by, d_state, scratch);
+            });
+            PS_HIP(hipGetLastError());
+            if (torch)
+                launch_even_closing<PS_ARITH_TORCH>(e, chunk_numel, ga, fc, cl, nt, s);
+            else
+                launch_even_closing<PS_ARITH_OPERATOR>(e, chunk_numel, ga, fc, cl, nt, s);
+            PS_HIP(hipGetLastError());
+            return 0;
+        }
+        ChunkList probed = a;
+        probed.tile = kScanTile;
+        if (int rc = for_each_batch(probed, [&](const ChunkBatch& b, dim3 grid, int) {
+                hipLaunchKernelGGL(open_chunks_kernel, with_first<false>(grid), dim3(kScanBlock), kScanLdsBytes, s, b, d_state, scratch);
+            }))
+            return rc;
+        return for_each_batch(a, [&](const ChunkBatch& b, dim3 grid, int) {
+            if (torch)
+                launch_closing_batch<PS_ARITH_TORCH>(b, grid, chunk_numel, ga, fc, cl, s);
+            else
+                launch_closing_batch<PS_ARITH_OPERATOR>(b, grid, chunk_numel, ga, fc, cl, s);
         });
     }
     if (probe)

@@ -45,7 +45,7 @@
 #define PS_SMALL_WAVES 16  // waves of a workgroup of the step in one launch: one for the state, the others a tile each
 #endif
 #ifndef PS_SMALL_TILES
-#define PS_SMALL_TILES 400  // longest list (256-element tiles) that is probed, stepped and rescaled in one launch
+#define PS_SMALL_TILES 280  // longest list (256-element tiles) that is probed, stepped and rescaled in one launch
 #endif
 #ifndef PS_SMALL_TILES_ALONE
 #define PS_SMALL_TILES_ALONE 80  // the same by one workgroup, where the caller has no scratch memory for several to share

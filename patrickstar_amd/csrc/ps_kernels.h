@@ -48,9 +48,8 @@ __device__ __forceinline__ uint32_t whole_tiles(size_t numel) { return (uint32_t
 struct CallSpan {
     bool here, inside, cut;
 };
-__device__ __forceinline__ CallSpan call_span(const FirstCall& fc)
+__device__ __forceinline__ CallSpan call_span(const FirstCall& fc, uint32_t tile)
 {
-    const uint32_t tile = blockIdx.x;
     CallSpan s;
     s.here = fc.chunk == (int)blockIdx.y;
     s.inside = s.here && tile >= fc.in_lo && tile < fc.in_hi;
@@ -66,7 +65,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
 {
     // b.n: the host has already decided whether the zeros behind a chunk's last tensor may be left alone
     const TileSource t = tile_source(b.c[blockIdx.y], b.n[blockIdx.y]);
-    const CallSpan s = call_span(fc);
+    const CallSpan s = call_span(fc, blockIdx.x);
     const size_t base = (size_t)blockIdx.x * kTile;
     if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
         LaneTile r;
@@ -108,7 +107,7 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         LaneTile r;
         tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
         __builtin_amdgcn_sched_barrier(0);  // the loads in front of the wait for the arguments behind the preloaded ones
-        const CallSpan s = call_span(fc);
+        const CallSpan s = call_span(fc, blockIdx.x);
         if (!s.cut) {
             tile_finish<ARITH, WD, UNS, false, NT>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv, r, t.p32,
                                         t.m32, t.v32, t.h16, base);
@@ -195,21 +194,17 @@ __host__ __device__ inline bool zeros_are_a_fixed_point(const StepConsts& c)
     return c.eps > 0.0f && (s - s) == 0.0f;  // every term finite (no NaN, and no infinities: inf - inf is NaN)
 }
 
+// One tile of a device-decided step, over a list with descriptors.
 template <int ARITH, int WD, bool NT>
-__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_chunks_gated_kernel(ChunkBatch b, size_t chunk_numel, GatedArgs ga, FirstCall fc,
-                             const ps_step_state* __restrict__ st)
+__device__ __forceinline__ void gated_tile(const TileSource& t, uint32_t tile, const CallSpan& s, size_t chunk_numel, const GatedArgs& ga,
+                                           const FirstCall& fc, const StateView& sv)
 {
-    const TileSource t = tile_source(b.c[blockIdx.y], b.n[blockIdx.y]);
-    const CallSpan s = call_span(fc);
-    const size_t base = (size_t)blockIdx.x * kTile;
-    StateView sv = view_state(st);  // asked for at once, as in tile_source
-    asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
+    const size_t base = (size_t)tile * kTile;
     if (__builtin_expect(sv.overflow, 0)) {
-        if (restore_leader(blockIdx.x)) restore_tiles<NT>(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
+        if (restore_leader(tile)) restore_tiles<NT>(t.p32, t.h16, base, t.numel);  // RNE(0) = 0 is already there
         return;
     }
-    if (blockIdx.x < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
+    if (tile < whole_tiles(t.numel) && !s.cut && aligned16(t)) {
         LaneTile r;
         tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
         const StepConsts c = gated_consts<ARITH>(ga, sv, s.here);
@@ -227,24 +222,39 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
                                                       numel, s.here ? fc.lo : 0, s.here ? fc.hi : 0);
 }
 
+// asked for at once, as in tile_source
+__device__ __forceinline__ void ask_for(StateView& sv)
+{
+    asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
+}
+
 template <int ARITH, int WD, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_even_chunks_gated_kernel(float* p32, float* m32, float* v32, uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last,
-                                  uint32_t short_by, const ps_step_state* __restrict__ st, size_t chunk_numel, GatedArgs ga, FirstCall fc)
+    adam_chunks_gated_kernel(ChunkBatch b, size_t chunk_numel, GatedArgs ga, FirstCall fc,
+                             const ps_step_state* __restrict__ st)
 {
-    const EvenChunk t = even_chunk(p32, m32, v32, h16, stride, numel, last, short_by);
-    const size_t base = (size_t)blockIdx.x * kTile;
+    const TileSource t = tile_source(b.c[blockIdx.y], b.n[blockIdx.y]);
+    const CallSpan s = call_span(fc, blockIdx.x);
     StateView sv = view_state(st);
-    asm volatile("" : "+s"(sv.overflow), "+s"(sv.cur_scale), "+s"(sv.b1t_next), "+s"(sv.b2t_next), "+s"(sv.b1t_rest), "+s"(sv.b2t_rest));
+    ask_for(sv);
+    gated_tile<ARITH, WD, NT>(t, blockIdx.x, s, chunk_numel, ga, fc, sv);
+}
+
+// The same over evenly spaced chunks.
+template <int ARITH, int WD, bool NT>
+__device__ __forceinline__ void even_gated_tile(const EvenChunk& t, uint32_t tile, size_t chunk_numel, const GatedArgs& ga, const FirstCall& fc,
+                                                const StateView& sv)
+{
+    const size_t base = (size_t)tile * kTile;
     if (__builtin_expect(sv.overflow, 0)) {
-        if (restore_leader(blockIdx.x)) restore_tiles<NT>(t.p32, t.h16, base, t.numel);
+        if (restore_leader(tile)) restore_tiles<NT>(t.p32, t.h16, base, t.numel);
         return;
     }
-    if (blockIdx.x < whole_tiles(t.numel)) {
+    if (tile < whole_tiles(t.numel)) {
         LaneTile r;
         tile_load<false, NT>(r, t.p32, t.m32, t.v32, t.h16, base);
         __builtin_amdgcn_sched_barrier(0);
-        const CallSpan s = call_span(fc);
+        const CallSpan s = call_span(fc, tile);
         if (!s.cut) {
             const StepConsts c = gated_consts<ARITH>(ga, sv, s.here);
             tile_finish<ARITH, WD, UNSCALE_RUNTIME, false, NT>(c, s.inside ? c.first_step_size : c.step_size, s.inside ? c.first_bc2inv : c.bc2inv,
@@ -254,11 +264,22 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     }
     const bool here = fc.chunk == (int)blockIdx.y;
     const StepConsts c = gated_consts<ARITH>(ga, sv, here);
-    size_t end = t.numel;  // as in adam_chunks_gated_kernel: zeros behind it that are no fixed point are computed
+    size_t end = t.numel;  // as in gated_tile: zeros behind it that are no fixed point are computed
     if (base + kTile > end && end < chunk_numel && !zeros_are_a_fixed_point(c)) end = chunk_numel;
     if (base >= end) return;
     adam_tile_scalar<ARITH, WD, UNSCALE_RUNTIME>(c, t.p32, t.m32, t.v32, t.h16, base, base + kTile < end ? base + kTile : end,
                                                  here ? fc.lo : 0, here ? fc.hi : 0);
+}
+
+template <int ARITH, int WD, bool NT>
+__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
+    adam_even_chunks_gated_kernel(float* p32, float* m32, float* v32, uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last,
+                                  uint32_t short_by, const ps_step_state* __restrict__ st, size_t chunk_numel, GatedArgs ga, FirstCall fc)
+{
+    const EvenChunk t = even_chunk(p32, m32, v32, h16, stride, numel, last, short_by);
+    StateView sv = view_state(st);
+    ask_for(sv);
+    even_gated_tile<ARITH, WD, NT>(t, blockIdx.x, chunk_numel, ga, fc, sv);
 }
 
 // ------------------------------------------------------- tensor-list kernels
@@ -1269,6 +1290,174 @@ __global__ void __launch_bounds__(64)
     if (threadIdx.x == 0) scaler_store(st, after, log, log_capacity);
 }
 
+// ------------------------------------------- a whole device-decided step in two launches
+//
+// Probe, update and scale update.  As three kernels the last one cannot begin before the update has ended, because the update's
+// waves read the state that it replaces, and it is a chain of its own: load, powers of the betas, store, 3.5 us behind its launch.
+// Here the probe's first workgroup copies what the update needs of the state into the caller's scratch memory, the update's waves
+// read the copy, and the update's first workgroup replaces the state while the others work.
+//
+// Bound by two launches and their ramps up to some 512 Ki elements, then by memory.  A step through FP16Adam.step(), three launches /
+// two: among others 128 Ki elements 8.7 / 7.0 us (the host's part), 512 Ki 9.0 / 6.8, 1 Mi 10.9 / 9.2, 4 Mi 25.6 / 21.5, 16 Mi 75.7 / 71.9,
+// 64 Mi 306.9 / 304, 200 Mi 921.9 / 922.3; waited for 128 Ki 20.6 / 18.8, 1 Mi 24.5 / 21.7.
+//
+// What the probe finds goes to a word of the scratch that the step before has cleared: one of two, in turn (a workgroup of the update
+// clears the word of the step to come while others still read this step's).  The state's own flag, which copies of gradients
+// may have raised before, travels with the copy.
+
+// The state as the probe found it, as far as the update needs it.  The operator's arithmetic takes the first 64 bytes, one line
+// and one load: as a copy of the whole state, five lines of which every wave looked at, the update of 8 x 64 Mi
+// elements took 2358 us instead of 2276.
+struct OpenedStep {
+    double cur_scale;
+    float beta1, beta2, b1t_next, b2t_next, b1t_rest, b2t_rest;
+    uint32_t overflow;
+    uint32_t turn;    // steps & 1 of this step
+    uint32_t hit[2];  // the probe of step number `steps` found an inf or a nan: [steps & 1]
+    uint32_t pad[4];
+    double beta1_f64, beta2_f64, bc1_next, bc2_next;
+    uint32_t pad2[8];
+};
+static_assert(sizeof(OpenedStep) == 128, "two lines");
+
+// What the workgroups of a step share (PS_STEP_SCRATCH_BYTES, the caller's, zero at first).
+struct StepScratch {
+    // steps in one launch: adam_small_step_kernel
+    uint64_t epoch;  // launches so far
+    uint64_t pad0[15];
+    uint32_t tickets;  // 0 between launches
+    uint32_t pad1[15];
+    uint64_t dirty, clean;  // epoch + 1 of the latest launch that was marked so
+    uint64_t pad2[6];
+    // steps in two launches
+    OpenedStep opened;
+    uint64_t steps;  // so far
+    uint64_t pad3[7];
+};
+static_assert(sizeof(StepScratch) == PS_STEP_SCRATCH_BYTES, "the caller's allocation");
+
+// Workgroups in front of every chunk's tiles: the first of all opens or closes the step, the others leave at once.  Lists that stream past
+// the caches: as many as there are shader engines (8 XCDs of 4), which workgroups go round, so that every tile runs where it runs
+// without them; one / 32 200 Mi elements 924.3 / 922.3 us (921.9 without any, in three launches), 4 Mi 21.5 / 22.3.
+template <bool NT>
+constexpr uint32_t kInFront = NT ? 32 : 1;
+__device__ __forceinline__ bool first_of_all() { return (blockIdx.x | blockIdx.y) == 0; }
+
+// The probe's first workgroup.
+__device__ __forceinline__ void open_step(const ps_step_state* st, StepScratch* x)
+{
+    const StateView sv = view_state(st);
+    const uint32_t turn = (uint32_t)x->steps & 1u;
+    if (threadIdx.x != 0) return;
+    OpenedStep& o = x->opened;  // (hit is written by the others)
+    o.cur_scale = sv.cur_scale;
+    o.beta1 = sv.beta1, o.beta2 = sv.beta2;
+    o.b1t_next = sv.b1t_next, o.b2t_next = sv.b2t_next;
+    o.b1t_rest = sv.b1t_rest, o.b2t_rest = sv.b2t_rest;
+    o.overflow = sv.overflow;
+    o.turn = turn;
+    o.beta1_f64 = sv.beta1_f64, o.beta2_f64 = sv.beta2_f64;
+    o.bc1_next = sv.bc1_next, o.bc2_next = sv.bc2_next;
+}
+__device__ __forceinline__ void probe_commit(uint32_t hit, StepScratch* x)
+{
+    if (__builtin_expect(__any(hit != 0), 0) && threadIdx.x == 0) x->opened.hit[x->steps & 1u] = 1u;
+}
+
+template <bool NT>
+__global__ void __launch_bounds__(kScanBlock)
+    open_even_chunks_kernel(const uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last, uint32_t short_by, const ps_step_state* st, StepScratch* x)
+{
+    static_assert(kScanBlock == 64, "one wave");
+    if (__builtin_expect(blockIdx.x < kInFront<NT>, 0)) {
+        if (first_of_all()) open_step(st, x);
+        return;
+    }
+    const uint32_t n = numel - (blockIdx.y == last ? short_by : 0u);
+    probe_commit(scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x - kInFront<NT>), x);
+}
+
+__global__ void __launch_bounds__(kScanBlock)
+    open_chunks_kernel(ChunkBatch b, const ps_step_state* st, StepScratch* x)
+{
+    if (__builtin_expect(blockIdx.x < kInFront<false>, 0)) {
+        if (first_of_all()) open_step(st, x);
+        return;
+    }
+    probe_commit(scan_tile<uint16_t, kScanBlock, kScanUnroll>(b.c[blockIdx.y].param_fp16, b.n[blockIdx.y], blockIdx.x - kInFront<false>), x);
+}
+
+// What a wave of the update reads: the copy, with the flag as the probe left it.
+template <int ARITH>
+__device__ __forceinline__ StateView view_opened(const OpenedStep* __restrict__ x)
+{
+    StateView sv;
+    sv.cur_scale = x->cur_scale;
+    sv.beta1 = x->beta1, sv.beta2 = x->beta2;
+    sv.b1t_next = x->b1t_next, sv.b2t_next = x->b2t_next;
+    sv.b1t_rest = x->b1t_rest, sv.b2t_rest = x->b2t_rest;
+    sv.overflow = x->overflow;
+    uint32_t turn = x->turn, even = x->hit[0], odd = x->hit[1];
+    if (ARITH == PS_ARITH_TORCH) {
+        sv.beta1_f64 = x->beta1_f64, sv.beta2_f64 = x->beta2_f64;
+        sv.bc1_next = x->bc1_next, sv.bc2_next = x->bc2_next;
+    }
+    ask_for(sv);
+    asm volatile("" : "+s"(turn), "+s"(even), "+s"(odd));
+    sv.overflow |= turn ? odd : even;
+    return sv;
+}
+
+// The update's first workgroup.
+struct Closing {
+    ps_step_state* st;
+    StepScratch* x;
+    ps_scale_record* log;
+    int64_t log_capacity, operator_calls;
+};
+__device__ __forceinline__ void close_step(const Closing& c)
+{
+    const ps_step_state now = *c.st;
+    const uint64_t steps = c.x->steps;
+    const uint32_t even = c.x->opened.hit[0], odd = c.x->opened.hit[1];
+    const bool overflow = (now.overflow | (steps & 1u ? odd : even)) != 0;
+    const ps_step_state after = scaler_updated(now, overflow, c.operator_calls);
+    if (threadIdx.x == 0) {
+        scaler_store(c.st, after, c.log, c.log_capacity);
+        c.x->opened.hit[~steps & 1u] = 0;
+        c.x->steps = steps + 1;
+    }
+}
+
+template <int ARITH, int WD, bool NT>
+__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
+    adam_even_chunks_closing_kernel(float* p32, float* m32, float* v32, uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last,
+                                    uint32_t short_by, const OpenedStep* __restrict__ x, size_t chunk_numel, GatedArgs ga, FirstCall fc, Closing c)
+{
+    if (__builtin_expect(blockIdx.x < kInFront<NT>, 0)) {
+        if (first_of_all()) close_step(c);
+        return;
+    }
+    const EvenChunk t = even_chunk(p32, m32, v32, h16, stride, numel, last, short_by);
+    const StateView sv = view_opened<ARITH>(x);
+    even_gated_tile<ARITH, WD, NT>(t, blockIdx.x - kInFront<NT>, chunk_numel, ga, fc, sv);
+}
+
+template <int ARITH, int WD>
+__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
+    adam_chunks_closing_kernel(const OpenedStep* __restrict__ x, ChunkBatch b, size_t chunk_numel, GatedArgs ga, FirstCall fc, Closing c)
+{
+    if (__builtin_expect(blockIdx.x < kInFront<false>, 0)) {
+        if (first_of_all()) close_step(c);
+        return;
+    }
+    const uint32_t tile = blockIdx.x - kInFront<false>;
+    const TileSource t = tile_source(b.c[blockIdx.y], b.n[blockIdx.y]);
+    const CallSpan s = call_span(fc, tile);
+    const StateView sv = view_opened<ARITH>(x);
+    gated_tile<ARITH, WD, false>(t, tile, s, chunk_numel, ga, fc, sv);
+}
+
 // ------------------------------------------- a whole device-decided step over a short chunk list
 //
 // Probe, update (or restore) and scale update in one launch.  As three kernels they take three launches whatever the list's
@@ -1292,14 +1481,11 @@ __global__ void __launch_bounds__(64)
 // that one workgroup does alone needs neither, and no scratch.
 //
 // Bound by one CU's reads of the whole list (133 GB/s, 3.1 us for every 800 tiles) and by a chain of trips to memory: arguments,
-// state or gradients, mark, stores.  Device time of a step back to back, by one workgroup / three kernels / this: 1 tile 4.3 / - / 4.8 us,
-// 75 tiles 12.45 / 8.5 / 6.9, 120 - / 8.5 / 7.2, 240 - / 8.6 / 8.0, 480 - / 8.9 / 9.4, 800 - / 9.2 / 10.8, 1600 - / 9.7 / 13.8 (all with
-// the state in memory: see scaler_store).  Among
-// other steps that is what FP16Adam.step() takes, if the host's part is not longer (4.6 us for one launch, 8.9 for three): 75 tiles 12.45
-// by one workgroup, 8.9 by three kernels, 6.7 by this, 240 tiles 8.9 / 7.7, 480 tiles 8.9 / 9.3; waited for, 75 tiles 27 / 22.3 / 18.9, 240
-// tiles 22.3 / 19.7, 480 tiles 22.3 / 21.4.  The line (kSmallTiles) lies where neither is the longer one.
-// Workgroups of 4 / 6 / 8 / 12 / 16 waves: 75 tiles 7.6 / 6.9 / 6.6 / 7.2 / 6.9, 480 tiles 15.2 / 12.1 / 10.9 / 9.5 / 9.5; two or
-// four tiles a wave 480 tiles 9.8 / 13.8.
+// state or gradients, mark, stores.  A step through FP16Adam.step() among others, two launches / this: 73 tiles 6.9 / 5.8 us, 120
+// 7.2 / 6.2, 180 7.2 / 6.5, 240 7.1 / 6.6, 300 7.2 / 6.9, 360 7.2 / 7.0; waited for 73 tiles 18.3 / 17.8, 180 18.7 / 18.6, 240 18.5 / 18.5, 300
+// 18.3 / 18.7, 360 18.2 / 19.2.  The line (kSmallTiles) lies where neither is the longer one.  (By one workgroup 75 tiles took 12.45.)
+// Device time in workgroups of 4 / 6 / 8 / 12 / 16 waves, with the state in memory (scaler_store): 75 tiles 7.6 / 6.9 / 6.6 / 7.2 / 6.9, 480
+// tiles 15.2 / 12.1 / 10.9 / 9.5 / 9.5; two or four tiles a wave 480 tiles 9.8 / 13.8.
 constexpr int kSmallWaves = PS_SMALL_WAVES;
 constexpr uint32_t kSmallSpan = kSmallWaves - 1;  // tiles that a workgroup has in hand at a time
 constexpr uint32_t kSmallScan = 4096;             // halves that a wave probes at a time: eight 16-byte loads a lane
@@ -1312,17 +1498,6 @@ struct SmallStep {
     ps_scale_record* log;
     int64_t log_capacity, operator_calls;
 };
-
-// What the workgroups of one launch share (PS_STEP_SCRATCH_BYTES, the caller's, zero at first).
-struct StepScratch {
-    uint64_t epoch;  // launches so far
-    uint64_t pad0[15];
-    uint32_t tickets;  // 0 between launches
-    uint32_t pad1[15];
-    uint64_t dirty, clean;  // epoch + 1 of the latest launch that was marked so
-    uint64_t pad2[6];
-};
-static_assert(sizeof(StepScratch) == PS_STEP_SCRATCH_BYTES, "the caller's allocation");
 
 // The chunks of an EvenChunk list: 48 bytes of arguments where ChunkBatch has 2560, which cost the host 0.35 us a launch (the smoke
 // test's list, 13.8 -> 13.4 us a step among others) and the kernel 0.4.
@@ -1470,7 +1645,7 @@ template <int ARITH, int WD>
 __device__ __forceinline__ void small_update(SmallShare& o, const SmallConsts& k, const SmallStep& a, const FirstCall& fc)
 {
     if (!o.whole && o.base + kTile > o.numel && o.numel < a.chunk_numel && !(o.here ? k.keeps_zeros_here : k.keeps_zeros)) {
-        // the padding is computed, as in adam_chunks_gated_kernel
+        // the padding is computed, as in gated_tile
         o.end = (uint32_t)(a.chunk_numel - o.base < kTile ? a.chunk_numel - o.base : kTile);
         small_load_single(o);
     }

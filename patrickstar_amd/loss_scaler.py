@@ -58,7 +58,7 @@ class DynamicLossScaler:
     by a factor that is not a power of two is rounded like a float from there on.
     """
 
-    _scratch = None  # device tensor beside the state, which the workgroups of one launch agree through
+    _scratch = None  # device tensor beside the state, which the workgroups of one step agree through
 
     def __init__(
         self,
@@ -117,8 +117,10 @@ class DynamicLossScaler:
             raise RuntimeError("DynamicLossScaler keeps its state on the GPU; no GPU is available")
         lib = _lib.load()
         device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
-        self._state = torch.zeros(ctypes.sizeof(_lib.ps_step_state), dtype=torch.uint8, device=device)
-        self._scratch = torch.zeros(_lib.PS_STEP_SCRATCH_BYTES, dtype=torch.uint8, device=device)
+        # one allocation and one fill for both
+        size = ctypes.sizeof(_lib.ps_step_state)
+        both = torch.zeros(size + _lib.PS_STEP_SCRATCH_BYTES, dtype=torch.uint8, device=device)
+        self._state, self._scratch = both[:size], both[size:]
         i = self._init
         if not i["scale_window"] > 0:
             raise ValueError(f"scale_window must be positive, got {i['scale_window']}")
