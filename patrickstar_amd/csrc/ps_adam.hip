@@ -256,6 +256,22 @@ bool streams(const ChunkList& a, bool gated)
     return true;
 }
 
+// Dynamic LDS of a launch of the update, one tile a workgroup: the request that caps the resident workgroups per CU, except where
+// all of the launch's workgroups fit the GPU at once (256 CUs with 32 waves each).  The cap keeps the window of lines in flight narrow
+// while workgroups follow one another; a launch that has no second round only waits for its first one to end.  Capped / not, device
+// time in a graph, host-decided step over one chunk of 768 Ki / 1 Mi / 1.5 Mi / 2 Mi elements in the caches 4.3 / 3.9, 5.2 / 4.6, 6.4 / 5.6, 7.6 / 6.4 us, in
+// memory 6.6 / 6.0, 7.9 / 7.8, 10.6 / 10.7, 13.4 / 13.8; device-decided, probe included, in the caches 7.1 / 6.5, 8.0 / 7.1, 9.5 / 8.2,
+// 11.4 / 9.7, in memory 8.9 / 8.3, 10.3 / 9.7, 13.0 / 12.8, 15.9 / 16.1.  Tensors with numbers of their own 1.07 M elements 6.4 / 5.8, 2.1 M 10.2 /
+// 8.5; one tensor of the operator 768 Ki 5.35 / 4.6, 1 Mi 6.35 / 6.15, 2 Mi 10.7 / 10.65, beyond the line 2.5 Mi 12.9 / 13.05.  Beyond it
+// the cap pays: one chunk of 3 Mi in memory 18.6 / 19.3, 16 Mi 53.3 / 54.8, 26 Mi 116 / 130.
+constexpr size_t kResidentTiles = PS_RESIDENT_TILES;
+unsigned capped_lds(dim3 grid, unsigned request) { return (size_t)grid.x * grid.y <= kResidentTiles ? 0 : request; }
+template <bool NT>
+unsigned capped_lds(dim3 grid)
+{
+    return capped_lds(grid, NT ? kStreamLdsBytes : kLdsBytes);
+}
+
 // launch(std::true_type or std::false_type): whether the kernel is the one with the non-temporal hint.
 template <typename F>
 void with_hint(bool nt, F launch)
@@ -350,11 +366,11 @@ void launch_adam_batch_wd(const ChunkBatch& b, dim3 grid, const StepConsts& c, c
         constexpr bool NT = decltype(hint)::value;
         dim3 block(kBlock);
         if (c.unscale == UNSCALE_MUL)
-            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_MUL, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, c, fc);
+            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_MUL, NT>), grid, block, capped_lds<NT>(grid), s, b, c, fc);
         else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)  // the torch formula never divides
-            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_DIV, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, c, fc);
+            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_DIV, NT>), grid, block, capped_lds<NT>(grid), s, b, c, fc);
         else
-            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, c, fc);
+            hipLaunchKernelGGL((adam_chunks_kernel<ARITH, WD, UNSCALE_NONE, NT>), grid, block, capped_lds<NT>(grid), s, b, c, fc);
     });
 }
 
@@ -378,11 +394,11 @@ void launch_even_wd(const EvenList& e, const StepConsts& c, const FirstCall& fc,
         constexpr bool NT = decltype(hint)::value;
         const dim3 grid = even_grid(e, kTile), block(kBlock);
         if (c.unscale == UNSCALE_MUL)
-            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_MUL, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), c, fc);
+            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_MUL, NT>), grid, block, capped_lds<NT>(grid), s, PS_EVEN(e), c, fc);
         else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
-            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_DIV, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), c, fc);
+            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_DIV, NT>), grid, block, capped_lds<NT>(grid), s, PS_EVEN(e), c, fc);
         else
-            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), c, fc);
+            hipLaunchKernelGGL((adam_even_chunks_kernel<ARITH, WD, UNSCALE_NONE, NT>), grid, block, capped_lds<NT>(grid), s, PS_EVEN(e), c, fc);
     });
 }
 
@@ -406,11 +422,11 @@ void launch_even_gated(const EvenList& e, size_t chunk_numel, const GatedArgs& g
         const dim3 grid = even_grid(e, kTile), block(kBlock);
         const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
         if (decay && ga.adamw)
-            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_DECOUPLED, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_DECOUPLED, NT>), grid, block, capped_lds<NT>(grid), s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
         else if (decay)
-            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_L2, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_L2, NT>), grid, block, capped_lds<NT>(grid), s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
         else
-            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
+            hipLaunchKernelGGL((adam_even_chunks_gated_kernel<ARITH, WD_NONE, NT>), grid, block, capped_lds<NT>(grid), s, PS_EVEN(e), d_state, chunk_numel, ga, fc);
     });
 }
 
@@ -441,7 +457,8 @@ void launch_even_closing(const EvenList& e, size_t chunk_numel, const GatedArgs&
         with_decay<ARITH>(ga, [&](auto wd) {
             constexpr bool NT = decltype(hint)::value;
             constexpr int WD = decltype(wd)::value;
-            hipLaunchKernelGGL((adam_even_chunks_closing_kernel<ARITH, WD, NT>), with_first<NT>(even_grid(e, kTile)), dim3(kBlock), NT ? kStreamLdsBytes : kLdsBytes, s,
+            const dim3 grid = even_grid(e, kTile);
+            hipLaunchKernelGGL((adam_even_chunks_closing_kernel<ARITH, WD, NT>), with_first<NT>(grid), dim3(kBlock), capped_lds<NT>(grid), s,
                                PS_EVEN(e), &cl.x->opened, chunk_numel, ga, fc, cl);
         });
     });
@@ -451,7 +468,7 @@ template <int ARITH>
 void launch_closing_batch(const ChunkBatch& b, dim3 grid, size_t chunk_numel, const GatedArgs& ga, const FirstCall& fc, const Closing& cl, hipStream_t s)
 {
     with_decay<ARITH>(ga, [&](auto wd) {
-        hipLaunchKernelGGL((adam_chunks_closing_kernel<ARITH, decltype(wd)::value>), with_first<false>(grid), dim3(kBlock), kLdsBytes, s, &cl.x->opened, b,
+        hipLaunchKernelGGL((adam_chunks_closing_kernel<ARITH, decltype(wd)::value>), with_first<false>(grid), dim3(kBlock), capped_lds<false>(grid), s, &cl.x->opened, b,
                            chunk_numel, ga, fc, cl);
     });
 }
@@ -478,11 +495,11 @@ void launch_gated_batch_arith(const ChunkBatch& b, dim3 grid, size_t chunk_numel
         // the operator tests its float weight decay "> 0" (cpu_adam.cpp:42), the torch formula "!= 0"
         const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
         if (decay && ga.adamw)
-            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_DECOUPLED, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_DECOUPLED, NT>), grid, block, capped_lds<NT>(grid), s, b, chunk_numel, ga, fc, d_state);
         else if (decay)
-            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_L2, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_L2, NT>), grid, block, capped_lds<NT>(grid), s, b, chunk_numel, ga, fc, d_state);
         else
-            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_NONE, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, b, chunk_numel, ga, fc, d_state);
+            hipLaunchKernelGGL((adam_chunks_gated_kernel<ARITH, WD_NONE, NT>), grid, block, capped_lds<NT>(grid), s, b, chunk_numel, ga, fc, d_state);
     });
 }
 
@@ -521,7 +538,11 @@ void launch_small_step(int arith, const LIST& b, const SmallStep& a, const Gated
 }
 
 template <typename LIST, bool NT>
-constexpr unsigned kListLds = std::is_same<LIST, NearBatch>::value ? (NT ? kStreamNearLdsBytes : kNearLdsBytes) : (NT ? kStreamLdsBytes : kLdsBytes);
+unsigned list_lds(dim3 grid)
+{
+    if (std::is_same<LIST, NearBatch>::value) return capped_lds(grid, NT ? kStreamNearLdsBytes : kNearLdsBytes);
+    return capped_lds<NT>(grid);
+}
 
 template <int ARITH, int WD, typename LIST>
 void launch_tensors_wd(const LIST& b, dim3 grid, const StepConsts& c, bool nt, hipStream_t s)
@@ -530,11 +551,11 @@ void launch_tensors_wd(const LIST& b, dim3 grid, const StepConsts& c, bool nt, h
         constexpr bool NT = decltype(hint)::value;
         dim3 block(kBlock);
         if (c.unscale == UNSCALE_MUL)
-            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_MUL, NT>), grid, block, (kListLds<LIST, NT>), s, b, c);
+            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_MUL, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, c);
         else if (ARITH == PS_ARITH_OPERATOR && c.unscale == UNSCALE_DIV)
-            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_DIV, NT>), grid, block, (kListLds<LIST, NT>), s, b, c);
+            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_DIV, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, c);
         else
-            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_NONE, NT>), grid, block, (kListLds<LIST, NT>), s, b, c);
+            hipLaunchKernelGGL((adam_tensors_kernel<LIST, ARITH, WD, UNSCALE_NONE, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, c);
     });
 }
 
@@ -558,11 +579,11 @@ void launch_tensors_gated_arith(const LIST& b, dim3 grid, const GatedArgs& ga,
         dim3 block(kBlock);
         const bool decay = ARITH == PS_ARITH_OPERATOR ? (float)ga.wd > 0.0f : ga.wd != 0.0;
         if (decay && ga.adamw)
-            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_DECOUPLED, NT>), grid, block, (kListLds<LIST, NT>), s, b, ga, d_state);
+            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_DECOUPLED, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, ga, d_state);
         else if (decay)
-            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_L2, NT>), grid, block, (kListLds<LIST, NT>), s, b, ga, d_state);
+            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_L2, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, ga, d_state);
         else
-            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_NONE, NT>), grid, block, (kListLds<LIST, NT>), s, b, ga, d_state);
+            hipLaunchKernelGGL((adam_tensors_gated_kernel<LIST, ARITH, WD_NONE, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, ga, d_state);
     });
 }
 
@@ -993,7 +1014,7 @@ int ps_adam_update(int optimizer_id, size_t step, float lr, float beta1, float b
         dim3 grid((unsigned)(n_tiles + (this_head + tail > 0 ? 1 : 0))), block(kBlock);  // + 1: the workgroup that does head and tail
         uint16_t* out = d_param_fp16_out ? d_param_fp16_out + at : nullptr;
 #define PS_FLAT_VEC_5(WD, UNS, HALF, OUT, DWORD, NT)                                                                            \
-    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD, NT>), grid, block, NT ? kStreamLdsBytes : kLdsBytes, s, \
+    hipLaunchKernelGGL((adam_flat_vec_kernel<WD, UNS, HALF, OUT, DWORD, NT>), grid, block, capped_lds<NT>(grid), s, \
                        d_params + at, static_cast<const void*>(gbytes + at * gsz), d_exp_avg + at,                              \
                        d_exp_avg_sq + at, out, (uint32_t)n_tiles, this_head, tail, c)
 #define PS_FLAT_VEC_4(WD, UNS, HALF, OUT)                    \
@@ -1319,11 +1340,11 @@ void launch_tensors_planned_wd(const LIST& b, dim3 grid, bool grad_f32,
         dim3 block(kBlock);
         if constexpr (std::is_same<LIST, TensorBatch>::value) {
             if (grad_f32) {
-                hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, kLdsBytes, s, b, d_consts, d_state);
+                hipLaunchKernelGGL((adam_tensors_planned_f32grad_kernel<ARITH, WD>), grid, block, capped_lds<false>(grid), s, b, d_consts, d_state);
                 return;
             }
         }
-        hipLaunchKernelGGL((adam_tensors_planned_kernel<LIST, ARITH, WD, NT>), grid, block, (kListLds<LIST, NT>), s, b, d_consts, d_state);
+        hipLaunchKernelGGL((adam_tensors_planned_kernel<LIST, ARITH, WD, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, d_consts, d_state);
     });
 }
 
@@ -1389,11 +1410,11 @@ void launch_tensors_each_uns(const LIST& b, dim3 grid, const ConstsBatch& cb, bo
         dim3 block(kBlock);
         if constexpr (std::is_same<LIST, TensorBatch>::value) {
             if (grad_f32) {
-                hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, kLdsBytes, s, b, cb);
+                hipLaunchKernelGGL((adam_tensors_each_f32grad_kernel<ARITH, WD, UNS>), grid, block, capped_lds<false>(grid), s, b, cb);
                 return;
             }
         }
-        hipLaunchKernelGGL((adam_tensors_each_kernel<LIST, ARITH, WD, UNS, NT>), grid, block, (kListLds<LIST, NT>), s, b, cb);
+        hipLaunchKernelGGL((adam_tensors_each_kernel<LIST, ARITH, WD, UNS, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, cb);
     });
 }
 

@@ -35,6 +35,9 @@
 #ifndef PS_SCAN_UNROLL
 #define PS_SCAN_UNROLL 8  // 16-byte loads per lane per tile
 #endif
+#ifndef PS_RESIDENT_TILES
+#define PS_RESIDENT_TILES 8192  // launches of up to so many workgroups of the update are not capped
+#endif
 #ifndef PS_SCAN_LDS_KB
 #define PS_SCAN_LDS_KB 26  // KiB of unused dynamic LDS per workgroup (0: no cap on resident workgroups)
 #endif
