@@ -506,6 +506,17 @@ int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsi
                                         int64_t log_capacity, int64_t operator_calls, void* d_scratch, size_t scratch_bytes,
                                         ps_stream_t stream);
 
+/*
+ * A whole device-decided step with per-tensor numbers: ps_overflow_scan_chunks over the chunk list, ps_adam_step_tensors_each with
+ * d_state, ps_scaler_update with PS_FLAG_FROM_DEVICE, as one call.  With the scratch memory above, tensors that lie at the same
+ * place of their four lists (to 256 Mi elements, of up to 48 distinct calls, none with PS_TENSOR_GRAD_F32) and up to 64 chunks
+ * the probe forms the constants and the update replaces the state; else, and with d_scratch NULL, it is those calls one after the other.
+ */
+int ps_adam_step_tensors_dynamic(int optimizer_id, int bias_correction, const ps_chunk* chunks, int n_chunks, size_t chunk_numel,
+                                 const size_t* used_numel, const ps_chunk* tensors, const size_t* numels, const ps_tensor_call* each,
+                                 int n_tensors, ps_step_state* d_state, ps_scale_record* d_log, int64_t log_capacity, int64_t operator_calls,
+                                 void* d_workspace, size_t workspace_bytes, void* d_scratch, size_t scratch_bytes, ps_stream_t stream);
+
 /* Copy *d_state to host memory and wait for it: the only synchronising call. */
 int ps_state_read(const ps_step_state* d_state, ps_step_state* host_out, ps_stream_t stream);
 

@@ -1331,9 +1331,10 @@ int wd_mode_of(int arith, double wd, bool adamw)
     return decay ? (adamw ? WD_DECOUPLED : WD_L2) : WD_NONE;
 }
 
+// `closing`: of a step whose launches read the copy of the state (NearBatch only); nullptr: they read the state.
 template <int ARITH, int WD, typename LIST>
 void launch_tensors_planned_wd(const LIST& b, dim3 grid, bool grad_f32,
-                               const PlannedConsts* d_consts, const ps_step_state* d_state, bool nt, hipStream_t s)
+                               const PlannedConsts* d_consts, const ps_step_state* d_state, const Closing* closing, bool nt, hipStream_t s)
 {
     with_hint(nt, [&](auto hint) {
         constexpr bool NT = decltype(hint)::value;
@@ -1344,20 +1345,27 @@ void launch_tensors_planned_wd(const LIST& b, dim3 grid, bool grad_f32,
                 return;
             }
         }
+        if constexpr (std::is_same<LIST, NearBatch>::value) {
+            if (closing) {
+                hipLaunchKernelGGL((adam_tensors_planned_closing_kernel<ARITH, WD, NT>), with_first<NT>(grid), block, (list_lds<LIST, NT>(grid)), s,
+                                   b, d_consts, &closing->x->opened, *closing);
+                return;
+            }
+        }
         hipLaunchKernelGGL((adam_tensors_planned_kernel<LIST, ARITH, WD, NT>), grid, block, (list_lds<LIST, NT>(grid)), s, b, d_consts, d_state);
     });
 }
 
 template <int ARITH, typename LIST>
 void launch_tensors_planned_arith(const LIST& b, dim3 grid, int wd_mode, bool grad_f32,
-                                  const PlannedConsts* d_consts, const ps_step_state* d_state, bool nt, hipStream_t s)
+                                  const PlannedConsts* d_consts, const ps_step_state* d_state, const Closing* closing, bool nt, hipStream_t s)
 {
     if (wd_mode == WD_DECOUPLED)
-        launch_tensors_planned_wd<ARITH, WD_DECOUPLED>(b, grid, grad_f32, d_consts, d_state, nt, s);
+        launch_tensors_planned_wd<ARITH, WD_DECOUPLED>(b, grid, grad_f32, d_consts, d_state, closing, nt, s);
     else if (wd_mode == WD_L2)
-        launch_tensors_planned_wd<ARITH, WD_L2>(b, grid, grad_f32, d_consts, d_state, nt, s);
+        launch_tensors_planned_wd<ARITH, WD_L2>(b, grid, grad_f32, d_consts, d_state, closing, nt, s);
     else
-        launch_tensors_planned_wd<ARITH, WD_NONE>(b, grid, grad_f32, d_consts, d_state, nt, s);
+        launch_tensors_planned_wd<ARITH, WD_NONE>(b, grid, grad_f32, d_consts, d_state, closing, nt, s);
 }
 
 // Numbers the distinct records (classes of calls) of a step by their bytes; records are zero-filled before they are
@@ -1512,10 +1520,48 @@ size_t ps_tensors_each_workspace_bytes(int n_tensors)
     return n_tensors > 0 ? (size_t)n_tensors * sizeof(PlannedConsts) : 0;
 }
 
-int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_chunk* tensors,
-                              const size_t* numels, const ps_tensor_call* each, int n_tensors,
-                              double loss_scale, ps_step_state* d_state, void* d_workspace,
-                              size_t workspace_bytes, ps_stream_t stream)
+namespace {
+
+int check_scratch(const void* d_scratch, size_t bytes)
+{
+    if (d_scratch != nullptr && (bytes < sizeof(StepScratch) || reinterpret_cast<uintptr_t>(d_scratch) % 64))
+        return fail(PS_ERR_BAD_ARG, "d_scratch holds %zu bytes at %p; it needs %zu, 64-byte aligned", bytes, d_scratch, sizeof(StepScratch));
+    return 0;
+}
+
+// The rest of a device-decided step with per-tensor numbers: the lists it probes, the scratch beside its state, and what its
+// scale update is told.
+struct WholeStep {
+    const ChunkList& probed;
+    StepScratch* scratch;
+    ps_scale_record* log;
+    int64_t log_capacity, operator_calls;
+};
+
+// Whether it is done in one launch and those of the update, the first of which replaces the state.
+bool opens_with_plan(const WholeStep& w, int n_classes, const std::vector<int>& class_keys, const ps_chunk* tensors, const size_t* numels, int n_tensors)
+{
+    const ChunkList& a = w.probed;
+    if (!w.scratch || n_classes > kOpenClasses || a.n_chunks < 1 || a.n_chunks > kBatch) return false;
+    size_t longest = 0, elements = 0;
+    for (int i = 0; i < a.n_chunks; ++i) longest = std::max(longest, a.numel_of(i));
+    if (longest == 0 || longest > 0xFFFFFFFFu) return false;
+    for (int key : class_keys)
+        if (key_grad_f32(key)) return false;
+    std::vector<TensorItem> items;
+    for (int i = 0; i < n_tensors; ++i) {
+        if (numels[i] == 0) continue;
+        items.push_back(tensor_item(tensors, numels, i));
+        elements += numels[i];
+    }
+    ps_chunk lists;
+    return elements <= kMaxNearElements && near_lists(items, tensors, &lists);  // (no item: false)
+}
+
+int step_tensors_each(int optimizer_id, int bias_correction, const ps_chunk* tensors,
+                      const size_t* numels, const ps_tensor_call* each, int n_tensors,
+                      double loss_scale, ps_step_state* d_state, void* d_workspace,
+                      size_t workspace_bytes, const WholeStep* whole, ps_stream_t stream)
 {
     auto o = find_opt(optimizer_id);
     if (!o) return fail(PS_ERR_UNKNOWN_ID, "optimizer id %d was never created", optimizer_id);
@@ -1635,27 +1681,60 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
         }
         PlannedConsts* table = static_cast<PlannedConsts*>(d_workspace);
         const int n_classes = (int)classes.size();
-        for (int first = 0; first < n_classes || first == 0; first += kPlanBatch) {
-            PlanBatch pb;
+        auto plan_args = [&](auto& pb, int first) {
+            constexpr int N = sizeof(pb.k) / sizeof(pb.k[0]);
             memset(&pb, 0, sizeof(pb));
             PlanArgs pa;
             memset(&pa, 0, sizeof(pa));
-            pa.n = std::min(kPlanBatch, n_classes - first);
+            pa.n = std::min(N, n_classes - first);
             for (int j = 0; j < pa.n; ++j) pb.k[j] = classes[first + j];
             pa.grad_clamp = o->grad_clamp;
             pa.adamw = o->adamw ? 1 : 0;
             pa.bias_correction = bias ? 1 : 0;
             pa.first_class = first;
-            pa.is_last_launch = first + kPlanBatch >= n_classes;
+            pa.is_last_launch = first + N >= n_classes;
             pa.last_operator_class = last_operator;
             if (last_operator >= 0) {
                 pa.last_d = classes[last_operator].d;
                 pa.last_beta1 = (float)classes[last_operator].beta1;
                 pa.last_beta2 = (float)classes[last_operator].beta2;
             }
-            hipLaunchKernelGGL(plan_consts_kernel, dim3(1), dim3(64), 0, s, pb, pa, d_state, table);
+            return pa;
+        };
+        Closing closing{};
+        const Closing* closes = nullptr;
+        if (whole && opens_with_plan(*whole, n_classes, class_keys, tensors, numels, n_tensors)) {
+            closing = Closing{d_state, whole->scratch, whole->log, whole->log_capacity, whole->operator_calls};
+            closes = &closing;
+            PlanBatchOf<kOpenClasses> pb;
+            const PlanArgs pa = plan_args(pb, 0);
+            const ChunkList& a = whole->probed;
+            ProbeList list;
+            memset(&list, 0, sizeof(list));
+            size_t longest = 0;
+            for (int i = 0; i < a.n_chunks; ++i) {
+                list.h[i] = a.chunks[i].param_fp16;
+                list.n[i] = (uint32_t)a.numel_of(i);
+                longest = std::max(longest, a.numel_of(i));
+            }
+            const dim3 grid((unsigned)((longest + kScanTile - 1) / kScanTile), (unsigned)a.n_chunks);
+            with_hint(elements(a) >= kScanStreamElements, [&](auto hint) {
+                constexpr bool NT = decltype(hint)::value;
+                hipLaunchKernelGGL((open_planned_kernel<NT>), with_first<NT>(grid), dim3(kScanBlock), kScanLdsBytes, s, list, pb, pa, d_state,
+                                   whole->scratch, table);
+            });
             PS_HIP(hipGetLastError());
-            if (n_classes == 0) break;
+        } else {
+            if (whole)
+                if (int rc = ps_overflow_scan_chunks(whole->probed.chunks, whole->probed.n_chunks, whole->probed.chunk_numel, whole->probed.used, d_state, stream))
+                    return rc;
+            for (int first = 0; first < n_classes || first == 0; first += kPlanBatch) {
+                PlanBatch pb;
+                const PlanArgs pa = plan_args(pb, first);
+                hipLaunchKernelGGL(plan_consts_kernel, dim3(1), dim3(64), 0, s, pb, pa, d_state, table);
+                PS_HIP(hipGetLastError());
+                if (n_classes == 0) break;
+            }
         }
         // One pass of launches per (arithmetic, weight-decay form); inside it, tensors of any class.  A launch names
         // its tensors' classes in 16 bits, relative to the window of 65536 records it is handed.
@@ -1678,18 +1757,47 @@ int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_ch
                     int rc = for_each_tensor_batch(items, tensors, -1, 0,
                                                    [&](const auto& b, dim3 grid, const BatchClasses&) {
                         if (key_arith(key) == PS_ARITH_TORCH)
-                            launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, wd_mode, grad_f32, table + window, d_state, nt, s);
+                            launch_tensors_planned_arith<PS_ARITH_TORCH>(b, grid, wd_mode, grad_f32, table + window, d_state, closes, nt, s);
                         else
-                            launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, wd_mode, grad_f32, table + window, d_state, nt, s);
+                            launch_tensors_planned_arith<PS_ARITH_OPERATOR>(b, grid, wd_mode, grad_f32, table + window, d_state, closes, nt, s);
+                        closing.st = nullptr;  // the first launch closes the step
                     }, grad_f32);
                     if (rc) return rc;
                 }
             }
         }
+        if (whole && !closes) return ps_scaler_update(d_state, PS_FLAG_FROM_DEVICE, whole->log, whole->log_capacity, whole->operator_calls, stream);
         return 0;
     } catch (const std::exception&) {  // nothing may throw across the boundary
         return fail(PS_ERR_BAD_ARG, "no host memory for a list of %d tensors", n_tensors);
     }
+}
+
+}  // namespace
+
+int ps_adam_step_tensors_each(int optimizer_id, int bias_correction, const ps_chunk* tensors,
+                              const size_t* numels, const ps_tensor_call* each, int n_tensors,
+                              double loss_scale, ps_step_state* d_state, void* d_workspace,
+                              size_t workspace_bytes, ps_stream_t stream)
+{
+    return step_tensors_each(optimizer_id, bias_correction, tensors, numels, each, n_tensors, loss_scale, d_state, d_workspace, workspace_bytes,
+                             nullptr, stream);
+}
+
+int ps_adam_step_tensors_dynamic(int optimizer_id, int bias_correction, const ps_chunk* chunks, int n_chunks, size_t chunk_numel,
+                                 const size_t* used_numel, const ps_chunk* tensors, const size_t* numels, const ps_tensor_call* each,
+                                 int n_tensors, ps_step_state* d_state, ps_scale_record* d_log, int64_t log_capacity, int64_t operator_calls,
+                                 void* d_workspace, size_t workspace_bytes, void* d_scratch, size_t scratch_bytes, ps_stream_t stream)
+{
+    if (!d_state) return fail(PS_ERR_BAD_ARG, "d_state is NULL");
+    if (d_log != nullptr && log_capacity <= 0)
+        return fail(PS_ERR_BAD_ARG, "log_capacity must be positive when d_log is given");
+    if (operator_calls < 0) return fail(PS_ERR_BAD_ARG, "operator_calls = %lld is negative", (long long)operator_calls);
+    if (int rc = check_scratch(d_scratch, scratch_bytes)) return rc;
+    ChunkList a;
+    if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kScanTile, true)) return rc;
+    const WholeStep whole{a, static_cast<StepScratch*>(d_scratch), d_log, log_capacity, operator_calls};
+    return step_tensors_each(optimizer_id, bias_correction, tensors, numels, each, n_tensors, -1.0, d_state, d_workspace, workspace_bytes, &whole, stream);
 }
 
 int ps_restore_fp16_chunks(const ps_chunk* chunks, int n_chunks, size_t chunk_numel,
@@ -2147,8 +2255,7 @@ int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsi
     if (d_log != nullptr && log_capacity <= 0)
         return fail(PS_ERR_BAD_ARG, "log_capacity must be positive when d_log is given");
     if (operator_calls < 0) return fail(PS_ERR_BAD_ARG, "operator_calls = %lld is negative", (long long)operator_calls);
-    if (d_scratch != nullptr && (scratch_bytes < sizeof(StepScratch) || reinterpret_cast<uintptr_t>(d_scratch) % 64))
-        return fail(PS_ERR_BAD_ARG, "d_scratch holds %zu bytes at %p; it needs %zu, 64-byte aligned", scratch_bytes, d_scratch, sizeof(StepScratch));
+    if (int rc = check_scratch(d_scratch, scratch_bytes)) return rc;
     ChunkList a;
     if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kTile)) return rc;
     Calls k;

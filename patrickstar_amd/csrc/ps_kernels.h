@@ -369,9 +369,8 @@ struct NearBatch {
     uint32_t numel[kNearBatch];     // elements from the origin on
     int first_call;
 };
-__device__ __forceinline__ TensorView tensor_view(const NearBatch& b)
+__device__ __forceinline__ TensorView tensor_view(const NearBatch& b, uint32_t wg)
 {
-    const uint32_t wg = blockIdx.x;
     uint32_t k = 0;
 #pragma unroll
     for (int j = 0; j < kSegments - 1; ++j)  // k += wg >= start[j]
@@ -400,6 +399,8 @@ __device__ __forceinline__ TensorView tensor_view(const NearBatch& b)
     w.tile = (int32_t)w.x - (w.head != 0);
     return w;
 }
+
+__device__ __forceinline__ TensorView tensor_view(const NearBatch& b) { return tensor_view(b, blockIdx.x); }
 
 // The elements in front of a tensor's tile grid: indices -head .. -1 relative to the descriptor's addresses.
 template <int ARITH, int WD, int UNS>
@@ -549,16 +550,13 @@ struct PlannedConsts {
 };
 static_assert(sizeof(PlannedConsts) == 64, "one 64-byte record per class in the caller's workspace");
 
-template <typename LIST, int ARITH, int WD, bool NT>
-__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
-    adam_tensors_planned_kernel(LIST b, const PlannedConsts* __restrict__ consts,
-                                const ps_step_state* __restrict__ st)
+template <int ARITH, int WD, bool NT, typename Flagged>
+__device__ __forceinline__ void planned_tensor(const TensorView& w, const PlannedConsts* __restrict__ consts, Flagged flagged)
 {
-    const TensorView w = tensor_view(b);
     const ps_chunk t = as_chunk(w.t);
     const size_t base = w.tile < 0 ? 0 : (size_t)w.tile * kTile;
     if (w.tile >= 0 && base >= w.numel) return;
-    if (__builtin_expect(st->overflow, 0)) {
+    if (__builtin_expect(flagged(), 0)) {
         restore_tensor_tiles<NT>(t, w);
         return;
     }
@@ -567,6 +565,14 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
         return;
     }
     adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME, NT>([&]() { return consts[w.cls].c; }, w, false);
+}
+
+template <typename LIST, int ARITH, int WD, bool NT>
+__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
+    adam_tensors_planned_kernel(LIST b, const PlannedConsts* __restrict__ consts,
+                                const ps_step_state* __restrict__ st)
+{
+    planned_tensor<ARITH, WD, NT>(tensor_view(b), consts, [&]() { return st->overflow != 0; });
 }
 
 // PS_TENSOR_GRAD_F32 tensors of a device-decided step: a flagged step leaves them alone (there is no fp16 copy to
@@ -1082,9 +1088,11 @@ struct PlanClass {
     int32_t prev;  // PLAN_MUL: the class (index in the table) of the call before it
 };
 constexpr int kPlanBatch = 64;  // one lane per class; 64 x 56 bytes of kernel arguments
-struct PlanBatch {
-    PlanClass k[kPlanBatch];
+template <int N>
+struct PlanBatchOf {
+    PlanClass k[N];
 };
+using PlanBatch = PlanBatchOf<kPlanBatch>;
 struct PlanArgs {
     double grad_clamp;
     int64_t last_d;             // of the step's last operator call
@@ -1095,10 +1103,11 @@ struct PlanArgs {
     float last_beta1, last_beta2;
 };
 
-__global__ void __launch_bounds__(64)
-    plan_consts_kernel(PlanBatch pb, PlanArgs a, ps_step_state* st, PlannedConsts* table)
+// By one wave.
+template <int N>
+__device__ __forceinline__ void plan_consts(const PlanBatchOf<N>& pb, const PlanArgs& a, ps_step_state* st, PlannedConsts* table)
 {
-    __shared__ float b1t_of[kPlanBatch], b2t_of[kPlanBatch];
+    __shared__ float b1t_of[N], b2t_of[N];
     const int j = threadIdx.x;
     const int64_t adam_step = st->adam_step;
     const double cur_scale = st->cur_scale;
@@ -1161,6 +1170,12 @@ __global__ void __launch_bounds__(64)
     st->pending_beta1 = a.last_beta1;
     st->pending_beta2 = a.last_beta2;
     st->pending_operator_step = adam_step + 1 + a.last_d;
+}
+
+__global__ void __launch_bounds__(64)
+    plan_consts_kernel(PlanBatch pb, PlanArgs a, ps_step_state* st, PlannedConsts* table)
+{
+    plan_consts(pb, a, st, table);
 }
 
 __global__ void state_set_scaler_kernel(ps_step_state* st, double cur_scale, int scale_is_int,
@@ -1456,6 +1471,47 @@ __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
     const CallSpan s = call_span(fc, tile);
     const StateView sv = view_opened<ARITH>(x);
     gated_tile<ARITH, WD, false>(t, tile, s, chunk_numel, ga, fc, sv);
+}
+
+// The same for a step whose tensors carry their own numbers, over tensors at the same place of their four lists: the probe's first
+// workgroup forms the constants as well (plan_consts), which are ready long before the probe of the lists that this is for has ended;
+// every launch of the update reads the copy, the first one closes the step.
+//
+// Device time of a step in a graph, four launches (probe, constants, update, scale update) / two, modules of BERT blocks with a rate per layer:
+// 268 K elements 11.9 / 8.5 us, 2.1 M 17.6 / 16.4, 5.3 M 33.1 / 30.1, 43 M 205 / 197, 109 M 498 / 491, 223 M 1014 / 1009.  Bound by the launches and the
+// chain of the constants up to some 1 M elements, then by memory.  Of the probe's lists only addresses and lengths travel, so that 48
+// distinct calls fit beside them; steps with more, and tensors with binary32 gradients, take the launches one by one.
+constexpr int kOpenClasses = 48;
+struct ProbeList {
+    const uint16_t* h[kBatch];
+    uint32_t n[kBatch];
+};
+
+template <bool NT>
+__global__ void __launch_bounds__(kScanBlock)
+    open_planned_kernel(ProbeList b, PlanBatchOf<kOpenClasses> pb, PlanArgs a, ps_step_state* st, StepScratch* x, PlannedConsts* table)
+{
+    if (__builtin_expect(blockIdx.x < kInFront<NT>, 0)) {
+        if (!first_of_all()) return;
+        open_step(st, x);
+        plan_consts(pb, a, st, table);
+        return;
+    }
+    probe_commit(scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(b.h[blockIdx.y], b.n[blockIdx.y], blockIdx.x - kInFront<NT>), x);
+}
+static_assert(sizeof(ProbeList) + sizeof(PlanBatchOf<kOpenClasses>) + sizeof(PlanArgs) + 24 <= 4096, "kernel arguments of one launch");
+
+template <int ARITH, int WD, bool NT>
+__global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
+    adam_tensors_planned_closing_kernel(NearBatch b, const PlannedConsts* __restrict__ consts, const OpenedStep* __restrict__ x, Closing c)
+{
+    if (__builtin_expect(blockIdx.x < kInFront<NT>, 0)) {
+        if (blockIdx.x == 0 && c.st != nullptr) close_step(c);  // (nullptr: a launch before this one has)
+        return;
+    }
+    planned_tensor<ARITH, WD, NT>(tensor_view(b, blockIdx.x - kInFront<NT>), consts, [&]() {
+        return (x->overflow | (x->turn ? x->hit[1] : x->hit[0])) != 0;
+    });
 }
 
 // ------------------------------------------- a whole device-decided step over a short chunk list

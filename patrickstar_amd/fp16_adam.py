@@ -731,6 +731,31 @@ class FP16Adam(torch.optim.Optimizer):
                 again.arithmetic, again.rest = self.arithmetic, plan["table"][5:]
         return plan["table"]
 
+    def _step_each_at_once(self, plan, stream):
+        """Probe, device-decided step and scale update as one call, where all chunks lie in HBM and PyTorch manages no tensor
+        itself.  False: nothing was done."""
+        if not self._is_one_call(True):
+            return False
+        table, n_dev, host_positions = self._tables or self._build_tables()
+        if host_positions or not n_dev:
+            return False
+        rows, numels, n, each, workspace, operator_calls, _, managed = self._each_table(plan)
+        scaler = self.loss_scaler
+        state = scaler.state_ptr
+        if managed or scaler._scratch is None:
+            return False
+        if scaler.before_flag is not None:
+            scaler.before_flag()
+        _lib.check(
+            self._lib.ps_adam_step_tensors_dynamic(
+                self.opt_id, 1, table, n_dev, self.client.default_chunk_size, self._used, rows, numels, each, n, state,
+                *scaler.log_arguments(), operator_calls, workspace.data_ptr(), workspace.numel(), scaler._scratch.data_ptr(),
+                _lib.PS_STEP_SCRATCH_BYTES, stream,
+            ),
+            "ps_adam_step_tensors_dynamic",
+        )
+        return True
+
     def _step_each(self, plan, stream):
         """One step through ``ps_adam_step_tensors_each``."""
         rows, numels, n, each, workspace, operator_calls, offsets, managed = self._each_table(plan)
@@ -842,9 +867,10 @@ class FP16Adam(torch.optim.Optimizer):
         with _lib.on_device(self.client.device):
             stream = _lib.current_stream_handle()
             if plan["kind"] == "each":
-                if self._dynamic and self.scan_in_step:
-                    self.check_overflow_chunks()
-                self._step_each(plan, stream)
+                if not (self._dynamic and self.scan_in_step and self._step_each_at_once(plan, stream)):
+                    if self._dynamic and self.scan_in_step:
+                        self.check_overflow_chunks()
+                    self._step_each(plan, stream)
                 self._steps_dirty = True
                 return loss
             hyper = plan["hyper"]
