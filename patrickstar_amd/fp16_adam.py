@@ -498,6 +498,8 @@ class FP16Adam(torch.optim.Optimizer):
         """Call after re-allocating chunk payloads."""
         self._tables = None
         self._each_static = None
+        if self._numbers is not None:
+            self._plan = None  # it may have its numbers there
         self._numbers = None
         if self._plan is not None and self._plan["kind"] == "each":
             self._plan["table"] = None

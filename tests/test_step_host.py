@@ -135,3 +135,18 @@ def test_numbers_read_by_the_binding_make_the_same_plan(seed, monkeypatch):
             x[i].step = y[i].step = 0
         assert bytes(x) == bytes(y)
     assert True in again and False in again
+
+
+def test_a_plan_whose_numbers_were_read_by_the_binding_outlives_new_payloads(monkeypatch):
+    _compiled()
+    _, _, optimizer = _tiny_optimizer()
+    params = list(optimizer.param_groups[0]["params"])
+    monkeypatch.setattr(optimizer, "_tensor_rows", lambda trainable: (None, None, len(trainable)))
+    for k in range(4):
+        for i, p in enumerate(params):
+            optimizer.state[p]["lr"] = 0.5 ** (k + i)
+        optimizer._make_plan()
+    assert optimizer._plan["kind"] == "each" and optimizer._plan["entries"] is None
+    optimizer.invalidate_tables()
+    each = optimizer._each_table(optimizer._plan or optimizer._make_plan())[3]
+    assert [e.lr for e in each] == [0.5 ** (3 + i) for i in range(len(params))]
