@@ -564,7 +564,13 @@ __device__ __forceinline__ void planned_tensor(const TensorView& w, const Planne
         adam_head<ARITH, WD, UNSCALE_RUNTIME>(consts[w.cls].c, t, w.head, false);
         return;
     }
-    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME, NT>([&]() { return consts[w.cls].c; }, w, false);
+    adam_tensor_tile<ARITH, WD, UNSCALE_RUNTIME, NT>(
+        [&]() {
+            __builtin_amdgcn_sched_barrier(0);  // all of the tile's loads in front of the first wait: with the torch
+            // formula the compiler waited behind the third of four, 109 M elements 516 -> 496 us, 223 M 1052 -> 1009
+            return consts[w.cls].c;
+        },
+        w, false);
 }
 
 template <typename LIST, int ARITH, int WD, bool NT>
