@@ -6,7 +6,7 @@ import ctypes
 import pytest
 import torch
 
-from patrickstar_amd import DynamicLossScaler, _lib, adam_op
+from patrickstar_amd import DynamicLossScaler, FP16Adam, PatrickStarClient, _lib, adam_op
 from test_gpu_near_tensor_lists import SHAPES, Lists
 
 pytestmark = pytest.mark.gpu
@@ -113,3 +113,44 @@ def test_it_shares_its_scratch_with_whole_list_steps_and_replays_in_a_graph():
             _compare(runs, k)
     for r in runs:
         adam_op.destroy_adam(r.opt)
+
+
+@pytest.mark.parametrize("arithmetic", ["operator", "torch"])
+@pytest.mark.parametrize("schedule", [False, True])
+def test_a_step_over_some_of_the_tensors_is_done_at_once(schedule, arithmetic, monkeypatch):
+    """One set of numbers for all that is trainable; without scratch memory the optimizer takes the probe, the step and the scale update."""
+    outs, states, calls = [], [], []
+    for at_once in (True, False):
+        torch.manual_seed(3)
+        client = PatrickStarClient(0, 40000)
+        with torch.device("cuda"):
+            model = torch.nn.Sequential(*[torch.nn.Linear(97, 101), torch.nn.Linear(101, 64), torch.nn.LayerNorm(64), torch.nn.Linear(64, 300)])
+        client.register_model(model)
+        params = list(model.parameters())
+        for p in params[:3]:
+            p.requires_grad_(False)
+        scaler = DynamicLossScaler(init_scale=2.0**10, scale_window=2)
+        optimizer = FP16Adam(client, params, loss_scaler=scaler, lr=1e-3, weight_decay=0.01, use_adamw=True, arithmetic=arithmetic)
+        if not at_once:
+            scaler._scratch = None
+        step_at_once = optimizer._step_each_at_once
+        monkeypatch.setattr(optimizer, "_step_each_at_once", lambda *args: calls.append(step_at_once(*args)) or calls[-1])
+        for k in range(8):
+            for p in params[3:]:
+                p.data.copy_(torch.linspace(-1, 1, p.numel(), device="cuda").view(p.shape) * (k + 1))
+                if schedule:
+                    optimizer.state[p]["lr"] = 1e-3 * 0.5**k
+            if k in (2, 3, 6):
+                params[4 if k == 3 else -1].data.view(-1)[0] = float("inf")
+            if k == 5:
+                params[3].requires_grad_(False)
+            optimizer.step()
+        outs.append([client.chunk_list[c].payload.clone() for pos in client.positions() for c in (pos.fp32, pos.exp_avg, pos.exp_avg_sq, pos.fp16)])
+        state = scaler._read()
+        # (the record of a step's last call, when pending_operator_step says that there is none)
+        fields = [name for name, *_ in state._fields_ if not name.startswith(("reserved", "pending_beta", "pad", "_"))]
+        states.append({name: getattr(state, name) for name in fields})
+        assert scaler.skipped_steps == 3 and optimizer.state[params[4]]["step"] == 5
+    assert calls == [True] * 8 + [False] * 8 and states[0] == states[1] and states[0]["pending_operator_step"] == 0
+    for x, y in zip(*outs):
+        assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
