@@ -235,14 +235,24 @@ size_t elements(const ChunkList& a)
 // lines are where a step that finds its list there stops to lose.  One that doesn't, because forward and backward went over
 // more than the cache holds, would gain below them as well (lists in turn, 1 GiB of them: 1 Mi 7.66 / 6.75, 8 Mi 39.8 / 37.4, 16 Mi
 // 79.2 / 71.4, 24 Mi 113.8 / 106.3; device-decided with the probe 16 Mi 89.9 / 82.0); a call does not know which it is, and below 20 Mi
-// the loss is the larger.  The probe alone at 32 Mi 10.2 / 9.0.  A tensor of the
+// the loss is the larger.  A tensor of the
 // operator comes with others, and its launch ends when its stores have left the L2: 144 K elements 2.33 / 2.41 us, 576 K 4.50 / 3.68,
 // 2.25 Mi 13.0 / 11.5; the tensors of a module of 5.3 M elements one after the other 67 / 68, of 11 M 166 / 139.
 //
+// The probe in front of an update reads what the update reads next: of a list it takes as much through the caches as the
+// memory-side one holds, where a streaming update finds it, and the rest past them.  Whole steps, everything past the caches / the first 112 Mi
+// elements through them: 31 Mi 148.5 / 142.9 us, 48 Mi 228 / 224, 80 Mi 373 / 358, 104 Mi 490 / 480, 136 Mi 642 / 627, 3 x 72 Mi 1018 / 1008, 8 x 64 Mi
+// 2419 / 2402; 199 tensors of BERT-base with a rate per layer 502.6 / 479.  (96 Mi and 128 Mi: the same within 0.3 %.)  A skipped step reads no
+// gradients again and pays for the slower probe: 48 Mi 62.6 / 64.3, 8 x 64 Mi 612 / 614; of lists beyond 256 Mi, where the gain is small, it is
+// 64 Mi, 2419 / 2409 and 612 / 612.5.
+//
 // A store that fills a 64-byte line in part only must not leave at once: lists whose phases differ by 16 or 32 bytes ran
 // 5 to 6 % slower with the hint, by 64 6 % faster.
-constexpr size_t kStreamElements = (size_t)28 << 20, kStreamElementsGated = (size_t)32 << 20, kScanStreamElements = (size_t)32 << 20,
+constexpr size_t kStreamElements = (size_t)28 << 20, kStreamElementsGated = (size_t)32 << 20, kScanKeepElements = (size_t)112 << 20,
+                 kScanKeepOfLong = (size_t)256 << 20, kScanKeepLong = (size_t)64 << 20,
                  kFlatStreamElements = (size_t)256 << 10;
+// How many tiles of the probe go through the caches.
+uint32_t probe_keeps(const ChunkList& a) { return (uint32_t)((elements(a) > kScanKeepOfLong ? kScanKeepLong : kScanKeepElements) / kScanTile); }
 bool whole_lines(const void* p32, const void* m32, const void* v32, const void* h16)
 {
     return ((reinterpret_cast<uintptr_t>(p32) | reinterpret_cast<uintptr_t>(m32) | reinterpret_cast<uintptr_t>(v32) |
@@ -1718,10 +1728,10 @@ int step_tensors_each(int optimizer_id, int bias_correction, const ps_chunk* ten
                 longest = std::max(longest, a.numel_of(i));
             }
             const dim3 grid((unsigned)((longest + kScanTile - 1) / kScanTile), (unsigned)a.n_chunks);
-            with_hint(elements(a) >= kScanStreamElements, [&](auto hint) {
+            with_hint(elements(a) > kScanKeepElements, [&](auto hint) {
                 constexpr bool NT = decltype(hint)::value;
                 hipLaunchKernelGGL((open_planned_kernel<NT>), with_first<NT>(grid), dim3(kScanBlock), kScanLdsBytes, s, list, pb, pa, d_state,
-                                   whole->scratch, table);
+                                   whole->scratch, table, probe_keeps(a));
             });
             PS_HIP(hipGetLastError());
         } else {
@@ -2126,19 +2136,20 @@ int ps_overflow_scan_chunks(const ps_chunk* chunks, int n_chunks, size_t chunk_n
     ChunkList a;
     if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kScanTile, true)) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool nt = elements(a) >= kScanStreamElements;
+    const bool nt = elements(a) > kScanKeepElements;
     EvenList e;
     if (even_list(a, kMaxEvenElementsGated, &e, true)) {
         with_hint(nt, [&](auto hint) {
             hipLaunchKernelGGL((scan_even_chunks_kernel<decltype(hint)::value>), even_grid(e, kScanTile), dim3(kScanBlock), kScanLdsBytes, s,
-                               e.first.param_fp16, e.stride, e.numel, e.last, e.short_by, d_state);
+                               e.first.param_fp16, e.stride, e.numel, e.last, e.short_by, d_state, probe_keeps(a));
         });
         PS_HIP(hipGetLastError());
         return 0;
     }
-    return for_each_batch(a, [&](const ChunkBatch& b, dim3 grid, int) {
+    return for_each_batch(a, [&](const ChunkBatch& b, dim3 grid, int first) {
         with_hint(nt, [&](auto hint) {
-            hipLaunchKernelGGL((scan_chunks_kernel<decltype(hint)::value>), grid, dim3(kScanBlock), kScanLdsBytes, s, b, d_state);
+            hipLaunchKernelGGL((scan_chunks_kernel<decltype(hint)::value>), grid, dim3(kScanBlock), kScanLdsBytes, s, b, d_state,
+                               first ? 0 : probe_keeps(a));
         });
     });
 }
@@ -2295,9 +2306,9 @@ int ps_adam_step_chunks_dynamic_scratch(int optimizer_id, double lr, double epsi
         const FirstCall fc = torch ? kNoFirstCall : k.in_batch(0, n_chunks);
         if (even) {
             const bool nt = streams(a, true);
-            with_hint(elements(a) >= kScanStreamElements, [&](auto hint) {
+            with_hint(elements(a) > kScanKeepElements, [&](auto hint) {
                 hipLaunchKernelGGL((open_even_chunks_kernel<decltype(hint)::value>), with_first<decltype(hint)::value>(even_grid(e, kScanTile)), dim3(kScanBlock), kScanLdsBytes, s,
-                                   e.first.param_fp16, e.stride, e.numel, e.last, e.short_by, d_state, scratch);
+                                   e.first.param_fp16, e.stride, e.numel, e.last, e.short_by, d_state, scratch, probe_keeps(a));
             });
             PS_HIP(hipGetLastError());
             if (torch)

@@ -846,20 +846,29 @@ __global__ void __launch_bounds__(kScanBlock)
     block_flag_commit<kScanBlock>(hit, &st->overflow);
 }
 
-template <bool NT>
-__global__ void __launch_bounds__(kScanBlock)
-    scan_chunks_kernel(ChunkBatch b, ps_step_state* st)
+// The probe's part of one workgroup, `width` tiles a chunk.  STREAMS: beyond the first `keep` tiles of the list past the caches
+// (kScanKeepElements).
+template <bool STREAMS>
+__device__ __forceinline__ uint32_t probe_tile(const uint16_t* h, size_t n, uint32_t tile, uint32_t width, uint32_t keep)
 {
-    uint32_t hit = scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(b.c[blockIdx.y].param_fp16, b.n[blockIdx.y], blockIdx.x);
+    if (STREAMS && blockIdx.y * width + tile >= keep) return scan_tile<uint16_t, kScanBlock, kScanUnroll, true>(h, n, tile);
+    return scan_tile<uint16_t, kScanBlock, kScanUnroll, false>(h, n, tile);
+}
+
+template <bool STREAMS>
+__global__ void __launch_bounds__(kScanBlock)
+    scan_chunks_kernel(ChunkBatch b, ps_step_state* st, uint32_t keep)
+{
+    uint32_t hit = probe_tile<STREAMS>(b.c[blockIdx.y].param_fp16, b.n[blockIdx.y], blockIdx.x, gridDim.x, keep);
     block_flag_commit<kScanBlock>(hit, &st->overflow);
 }
 
-template <bool NT>
+template <bool STREAMS>
 __global__ void __launch_bounds__(kScanBlock)
-    scan_even_chunks_kernel(const uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last, uint32_t short_by, ps_step_state* st)
+    scan_even_chunks_kernel(const uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last, uint32_t short_by, ps_step_state* st, uint32_t keep)
 {
     const uint32_t n = numel - (blockIdx.y == last ? short_by : 0u);
-    uint32_t hit = scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x);
+    uint32_t hit = probe_tile<STREAMS>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x, gridDim.x, keep);
     block_flag_commit<kScanBlock>(hit, &st->overflow);
 }
 
@@ -1387,7 +1396,8 @@ __device__ __forceinline__ void probe_commit(uint32_t hit, StepScratch* x)
 
 template <bool NT>
 __global__ void __launch_bounds__(kScanBlock)
-    open_even_chunks_kernel(const uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last, uint32_t short_by, const ps_step_state* st, StepScratch* x)
+    open_even_chunks_kernel(const uint16_t* h16, uint32_t stride, uint32_t numel, uint32_t last, uint32_t short_by, const ps_step_state* st, StepScratch* x,
+                            uint32_t keep)
 {
     static_assert(kScanBlock == 64, "one wave");
     if (__builtin_expect(blockIdx.x < kInFront<NT>, 0)) {
@@ -1395,7 +1405,7 @@ __global__ void __launch_bounds__(kScanBlock)
         return;
     }
     const uint32_t n = numel - (blockIdx.y == last ? short_by : 0u);
-    probe_commit(scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x - kInFront<NT>), x);
+    probe_commit(probe_tile<NT>(h16 + (size_t)stride * blockIdx.y, n, blockIdx.x - kInFront<NT>, gridDim.x - kInFront<NT>, keep), x);
 }
 
 __global__ void __launch_bounds__(kScanBlock)
@@ -1495,7 +1505,7 @@ struct ProbeList {
 
 template <bool NT>
 __global__ void __launch_bounds__(kScanBlock)
-    open_planned_kernel(ProbeList b, PlanBatchOf<kOpenClasses> pb, PlanArgs a, ps_step_state* st, StepScratch* x, PlannedConsts* table)
+    open_planned_kernel(ProbeList b, PlanBatchOf<kOpenClasses> pb, PlanArgs a, ps_step_state* st, StepScratch* x, PlannedConsts* table, uint32_t keep)
 {
     if (__builtin_expect(blockIdx.x < kInFront<NT>, 0)) {
         if (!first_of_all()) return;
@@ -1503,9 +1513,9 @@ __global__ void __launch_bounds__(kScanBlock)
         plan_consts(pb, a, st, table);
         return;
     }
-    probe_commit(scan_tile<uint16_t, kScanBlock, kScanUnroll, NT>(b.h[blockIdx.y], b.n[blockIdx.y], blockIdx.x - kInFront<NT>), x);
+    probe_commit(probe_tile<NT>(b.h[blockIdx.y], b.n[blockIdx.y], blockIdx.x - kInFront<NT>, gridDim.x - kInFront<NT>, keep), x);
 }
-static_assert(sizeof(ProbeList) + sizeof(PlanBatchOf<kOpenClasses>) + sizeof(PlanArgs) + 24 <= 4096, "kernel arguments of one launch");
+static_assert(sizeof(ProbeList) + sizeof(PlanBatchOf<kOpenClasses>) + sizeof(PlanArgs) + 32 <= 4096, "kernel arguments of one launch");
 
 template <int ARITH, int WD, bool NT>
 __global__ void __launch_bounds__(kBlock) PS_OCCUPANCY
