@@ -496,7 +496,7 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
 /*
  * The same with PS_STEP_SCRATCH_BYTES of device memory (64-byte aligned, all zero before the first call) that the workgroups of a
  * step agree through: lists of up to 280 tiles of 256 elements then take one launch, done by many workgroups, and with the
- * probe lists of evenly spaced chunks (to 256 Mi elements) and other lists below 32 Mi elements two.  It belongs to
+ * probe lists of evenly spaced chunks (to 256 Mi elements) and other lists below 28 Mi elements two.  It belongs to
  * d_state: calls that share it must be ordered as calls on d_state must, and nothing else may write to it.  NULL: as above.
  */
 #define PS_STEP_SCRATCH_BYTES 448

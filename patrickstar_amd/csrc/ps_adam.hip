@@ -230,12 +230,13 @@ size_t elements(const ChunkList& a)
 // slower, on the stores alone nothing.
 //
 // Steps over a list that stays in the memory-side cache from one step to the next (256 MiB) want it there: the same state
-// again and again, without / with the hint, host-decided 8 Mi elements 28.3 / 36.6 us, 16 Mi 53.6 / 70.2, 20 Mi 87.7 / 88.7, 24 Mi
-// 105.8 / 106.2, 28 Mi 129.2 / 125.8, 32 Mi 149.0 / 139.6; device-decided 24 Mi 115 / 118, 28 Mi 136 / 138, 32 Mi 157 / 157, 48 Mi 244 / 230.  The
-// lines are where a step that finds its list there stops to lose.  One that doesn't, because forward and backward went over
-// more than the cache holds, would gain below them as well (lists in turn, 1 GiB of them: 1 Mi 7.66 / 6.75, 8 Mi 39.8 / 37.4, 16 Mi
-// 79.2 / 71.4, 24 Mi 113.8 / 106.3; device-decided with the probe 16 Mi 89.9 / 82.0); a call does not know which it is, and below 20 Mi
-// the loss is the larger.  A tensor of the
+// again and again, without / with the hint, host-decided 8 Mi elements 28.8 / 36.7 us, 16 Mi 54.6 / 71.2, 20 Mi 85.8 / 90.1, 22 Mi 96.0 / 98.1,
+// 24 Mi 107.6 / 104.5, 26 Mi 117.9 / 114.3; device-decided (the probe without it) 16 Mi 59.6 / 72.9, 18 Mi 84.8 / 82.1, 20 Mi 91.0 / 91.4, 22 Mi
+// 99.8 / 100.6, 26 Mi 120.4 / 119.2, 31 Mi 151 / 143; tensors with numbers of their own 17.7 Mi 85.5 / 82.1 and 97.9 / 86.5.  The lines
+// lie where no step that finds its list there loses (host-decided from 24 Mi on, device-decided from 18 Mi on within 1 %).  One that does not, because forward and backward went over
+// more than the cache holds, gains from 1 Mi on (three lists in turn, host-decided: 4 Mi 16.1 / 20.2, 8 Mi 38.9 / 37.3, 16 Mi 82.4 / 72.8, 24 Mi 114.1 /
+// 105.2; device-decided 8 Mi 40.7 / 39.9, 16 Mi 83.6 / 74.0, 20 Mi 102.2 / 91.9, 26 Mi 133.7 / 119.2); a call does not know which it is, and below the
+// lines the loss is the larger.  A tensor of the
 // operator comes with others, and its launch ends when its stores have left the L2: 144 K elements 2.33 / 2.41 us, 576 K 4.50 / 3.68,
 // 2.25 Mi 13.0 / 11.5; the tensors of a module of 5.3 M elements one after the other 67 / 68, of 11 M 166 / 139.
 //
@@ -248,7 +249,7 @@ size_t elements(const ChunkList& a)
 //
 // A store that fills a 64-byte line in part only must not leave at once: lists whose phases differ by 16 or 32 bytes ran
 // 5 to 6 % slower with the hint, by 64 6 % faster.
-constexpr size_t kStreamElements = (size_t)28 << 20, kStreamElementsGated = (size_t)32 << 20, kScanKeepElements = (size_t)112 << 20,
+constexpr size_t kStreamElements = (size_t)28 << 20, kStreamElementsGated = (size_t)28 << 20, kScanKeepElements = (size_t)112 << 20,
                  kScanKeepOfLong = (size_t)256 << 20, kScanKeepLong = (size_t)64 << 20,
                  kFlatStreamElements = (size_t)256 << 10;
 // How many tiles of the probe go through the caches.

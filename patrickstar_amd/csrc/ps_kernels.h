@@ -349,7 +349,7 @@ __device__ __forceinline__ TensorView tensor_view(const TensorBatch& b)
 // instructions, where TensorBatch needs one round, so 11 workgroups per CU instead of 9 keep as many loads in flight.
 //
 // What that buys is the ends of launches, 4 to 9 us each.  Device time in several launches (TensorBatch) / in one, us, lists
-// from 28 Mi elements (device-decided 32 Mi) on with the non-temporal hint, where 13 workgroups per CU are resident: BERT-base, 199
+// from 28 Mi elements on with the non-temporal hint, where 13 workgroups per CU are resident: BERT-base, 199
 // tensors, 463.8 / 459.2 host-decided, 474.7 / 461.0 device-decided with a rate per layer; its upper half, 100 tensors 185.2 / 181.3
 // and 192.0 / 184.5; 12 layers of hidden size 64 12.9 / 5.1 and 17.6 / 8.6; 11 M elements with no two tensors at the same phase
 // 52.6 / 39.6.  (With plain accesses BERT-base took 517 / 500, under a cap of 9 508, of 12 533.)  Longer lists gain less than
