@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define PS_ABI_VERSION 5
+#define PS_ABI_VERSION 5 /* another number where a declaration or a structure changes, not where one is added */
 
 #define PS_ERR_BAD_ARG (-10001)     /* null pointer, negative count, unknown mode */
 #define PS_ERR_UNKNOWN_ID (-10002)  /* optimizer id was never created (the reference dereferences null here) */

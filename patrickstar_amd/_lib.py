@@ -169,7 +169,7 @@ class HipLibraryMissing(RuntimeError):
 
 
 def load():
-    """Load libps_adam.so once; raise HipLibraryMissing if it was never built."""
+    """Load libps_adam.so once; raise HipLibraryMissing if it was never built, or built for another version of this package."""
     global _lib
     if _lib is not None:
         return _lib
@@ -179,14 +179,16 @@ def load():
             "(hipcc, --offload-arch=gfx950). There is no CPU fallback for this path."
         )
     lib = ctypes.CDLL(LIB_PATH)
+    # the version first: of another one, some names may not exist.  (An entry point that is added does not change it.)
+    version = lib.ps_abi_version() if hasattr(lib, "ps_abi_version") else "none"
+    if version != PS_ABI_VERSION:
+        raise HipLibraryMissing(f"{LIB_PATH} has ABI version {version}, expected {PS_ABI_VERSION}; rebuild it")
     for name, (res, args) in SIGNATURES.items():
-        fn = getattr(lib, name)
+        fn = getattr(lib, name, None)
+        if fn is None:
+            raise HipLibraryMissing(f"{LIB_PATH} has no {name}: it is older than this package; rebuild it")
         fn.restype = res
         fn.argtypes = args
-    if lib.ps_abi_version() != PS_ABI_VERSION:
-        raise HipLibraryMissing(
-            f"{LIB_PATH} has ABI version {lib.ps_abi_version()}, expected {PS_ABI_VERSION}; rebuild it"
-        )
     binding = _load_binding()
     # adam_op.adam_update's arguments -> return code, or None where the call is not of the ordinary form (csrc/ps_binding.cpp)
     if binding is None:

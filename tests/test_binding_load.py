@@ -28,6 +28,19 @@ def test_the_library_loads_without_the_binding(fresh):
     assert lib.adam_update(*range(13)) is None  # "not of the ordinary form": the caller goes on to the general path
 
 
+@pytest.mark.parametrize("source,says", [
+    ("int ps_abi_version(void) { return %d; }" % (_lib.PS_ABI_VERSION - 1), f"has ABI version {_lib.PS_ABI_VERSION - 1}, expected {_lib.PS_ABI_VERSION}; rebuild it"),
+    ("int ps_abi_version(void) { return %d; }" % _lib.PS_ABI_VERSION, "has no ps_.*; rebuild it"), ("int other;", "rebuild it"),
+])
+def test_an_older_library_is_told_to_be_rebuilt(fresh, tmp_path, source, says):
+    """Of another version, or of this one before an entry point was added."""
+    (tmp_path / "old.c").write_text(source)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", str(tmp_path / "old.so")])
+    fresh.setattr(_lib, "LIB_PATH", str(tmp_path / "old.so"))
+    with pytest.raises(_lib.HipLibraryMissing, match=says):
+        _lib.load()
+
+
 @pytest.mark.parametrize(
     "made_for",
     [dict(), dict(abi_version=_lib.PS_ABI_VERSION - 1, built_for=build.built_for()), dict(abi_version=_lib.PS_ABI_VERSION, built_for="Python 3.9, torch 2.4.0")],
