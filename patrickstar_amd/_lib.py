@@ -190,12 +190,14 @@ def load():
         fn.restype = res
         fn.argtypes = args
     binding = _load_binding()
+    lib.compiled = None  # (a step looks here: a name that the library is asked for in vain costs 2 us)
     # adam_op.adam_update's arguments -> return code, or None where the call is not of the ordinary form (csrc/ps_binding.cpp)
     if binding is None:
         lib.adam_update = _no_binding
     else:
         lib.adam_update = functools.partial(binding.adam_update, ctypes.cast(lib.ps_adam_update, ctypes.c_void_p).value)
-        lib.compiled = _Compiled(binding, lib) if all(hasattr(binding, name) for name in _Compiled.NAMES) else None
+        if all(hasattr(binding, name) for name in _Compiled.NAMES):
+            lib.compiled = _Compiled(binding, lib)
     _lib = lib
     return lib
 

@@ -28,6 +28,14 @@ def test_the_library_loads_without_the_binding(fresh):
     assert lib.adam_update(*range(13)) is None  # "not of the ordinary form": the caller goes on to the general path
 
 
+def test_without_the_binding_no_step_asks_the_library_for_it(fresh):
+    """ctypes looks a name up in the library and all that it needs, again every time."""
+    fresh.setitem(sys.modules, "patrickstar_amd._binding", None)
+    with pytest.warns(RuntimeWarning):
+        lib = _lib.load()
+    assert vars(lib)["compiled"] is None
+
+
 @pytest.mark.parametrize("source,says", [
     ("int ps_abi_version(void) { return %d; }" % (_lib.PS_ABI_VERSION - 1), f"has ABI version {_lib.PS_ABI_VERSION - 1}, expected {_lib.PS_ABI_VERSION}; rebuild it"),
     ("int ps_abi_version(void) { return %d; }" % _lib.PS_ABI_VERSION, "has no ps_.*; rebuild it"), ("int other;", "rebuild it"),
