@@ -19,6 +19,7 @@ class Launch(ctypes.Structure):
 
 
 STATE, WORK = 1 << 30, 1 << 31  # addresses that nothing follows either
+SCRATCH = 1 << 29
 RATES = (1e-3, 0.9, 0.999, 1e-8, 0.01)
 
 
@@ -43,6 +44,8 @@ def main():
             if gated:
                 return lib.ps_adam_step_chunks_dynamic(1, 1e-3, 1e-8, 0.01, 1, table, n, longest, sizes, None, 1, state, None, 0, 1, None)
             return lib.ps_adam_step_chunks(1, 1, *RATES, 1, table, n, longest, sizes, None, 8.0, None)
+        if entry == "scratch":  # a device-decided step over chunks, with scratch memory
+            return lib.ps_adam_step_chunks_dynamic_scratch(1, 1e-3, 1e-8, 0.01, 1, table, n, max(numels), sizes, None, 1, state, None, 0, 1, SCRATCH, 448, None)
         if entry == "tensors":
             return lib.ps_adam_step_tensors(1, 1, *RATES, 1, table, sizes, n, None, 8.0, state, None)
         if entry == "each":

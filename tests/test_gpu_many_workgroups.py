@@ -1,4 +1,5 @@
-"""The scratch memory of device-decided steps."""
+"""The device-decided step of many workgroups in one launch: ragged, short, empty and unaligned chunks up to the end of its range.  That these lists
+are done so is checked in test_scratch_routes.py."""
 import pytest
 import torch
 
@@ -7,6 +8,21 @@ from patrickstar_amd import _lib, adam_op
 from test_gpu_short_lists import OPT
 
 pytestmark = pytest.mark.gpu
+MOST = 280 * 256  # elements of the longest list that is one launch
+
+# chunks, chunk length, used lengths (None: all full), element offset of the payloads in their allocations
+LISTS = [
+    (1, MOST, None, 0), (1, MOST, [MOST - 100], 3), (3, 16 * 256 + 1, None, 0), (7, 40 * 256 - 3, [40 * 256 - 3, 10000, 256, 255, 1, 0, 40 * 256 - 3], 0),
+    (64, 1000, None, 4), (2, 35000, [34999, 3], 1), (5, 56 * 256, [56 * 256, 1, 0, 4097, 4095], 2), (40, 7 * 256, [1792, 1, 256, 0] * 10, 0),
+]
+
+
+@pytest.mark.parametrize("case", LISTS, ids=[f"{c[0]}x{c[1]}at{c[3]}" for c in LISTS])
+@pytest.mark.parametrize("arithmetic,adamw,wd,clamp,scale,eps", [
+    (0, True, 0.01, 0.0, 2.0**12, 1e-8), (0, False, 0.01, 1.0, 1000.0, 1e-8), (1, True, 0.0, 0.0, 2**16, 1e-8), (0, True, 0.01, 0.0, 2.0**12, 0.0),
+])
+def test_one_launch_is_its_three_parts(case, arithmetic, adamw, wd, clamp, scale, eps):
+    scratch.test_one_launch_is_its_three_parts(case, arithmetic, adamw, wd, clamp, scale, eps)
 
 
 def test_scratch_one_byte_short_or_off_its_line_is_refused():
