@@ -486,8 +486,8 @@ int ps_scaler_update(ps_step_state* d_state, int flag_mode, ps_scale_record* d_l
 
 /* A whole device-decided step over HBM-resident chunks in one call: ps_overflow_scan_chunks (if probe
  * != 0), ps_adam_step_chunks_gated, ps_scaler_update(..., PS_FLAG_FROM_DEVICE, ...), with the same
- * results.  A list of at most 80 tiles of 256 elements (every chunk counted as long as the
- * longest) is one kernel launch instead of three.  All arguments are checked before anything is queued. */
+ * results.  A list of at most 64 chunks and 80 tiles of 256 elements (every chunk counted as long
+ * as the longest) is one kernel launch instead of three.  All arguments are checked before anything is queued. */
 int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, double weight_decay, int bias_correction,
                                 const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel,
                                 const ps_call_pattern* calls, int probe, ps_step_state* d_state, ps_scale_record* d_log,
@@ -495,8 +495,9 @@ int ps_adam_step_chunks_dynamic(int optimizer_id, double lr, double epsilon, dou
 
 /*
  * The same with PS_STEP_SCRATCH_BYTES of device memory (64-byte aligned, all zero before the first call) that the workgroups of a
- * step agree through: lists of up to 280 tiles of 256 elements then take one launch, done by many workgroups, and with the
- * probe lists of evenly spaced chunks (to 256 Mi elements) and other lists below 28 Mi elements two.  It belongs to
+ * step agree through: lists of at most 64 chunks and 280 tiles of 256 elements (every chunk counted as long as the longest) then take
+ * one launch, done by many workgroups, and with the probe lists of evenly spaced chunks (to 256 Mi elements) and other lists
+ * of at most 64 chunks and below 28 Mi elements two.  It belongs to
  * d_state: calls that share it must be ordered as calls on d_state must, and nothing else may write to it.  NULL: as above.
  */
 #define PS_STEP_SCRATCH_BYTES 448
