@@ -229,23 +229,30 @@ size_t elements(const ChunkList& a)
 // 2374 -> 2234 and 2572 -> 2394; one 64 Mi chunk 295 -> 280 and 324 -> 304.  The hint on the loads alone makes the same steps 6 %
 // slower, on the stores alone nothing.
 //
-// Steps over a list that stays in the memory-side cache from one step to the next (256 MiB) want it there: the same state
-// again and again, without / with the hint, host-decided 8 Mi elements 28.8 / 36.7 us, 16 Mi 54.6 / 71.2, 20 Mi 85.8 / 90.1, 22 Mi 96.0 / 98.1,
-// 24 Mi 107.6 / 104.5, 26 Mi 117.9 / 114.3; device-decided (the probe without it) 16 Mi 59.6 / 72.9, 18 Mi 84.8 / 82.1, 20 Mi 91.0 / 91.4, 22 Mi
-// 99.8 / 100.6, 26 Mi 120.4 / 119.2, 31 Mi 151 / 143; tensors with numbers of their own 17.7 Mi 85.5 / 82.1 and 97.9 / 86.5.  The lines
-// lie where no step that finds its list there loses (host-decided from 24 Mi on, device-decided from 18 Mi on within 1 %).  One that does not, because forward and backward went over
-// more than the cache holds, gains from 1 Mi on (three lists in turn, host-decided: 4 Mi 16.1 / 20.2, 8 Mi 38.9 / 37.3, 16 Mi 82.4 / 72.8, 24 Mi 114.1 /
-// 105.2; device-decided 8 Mi 40.7 / 39.9, 16 Mi 83.6 / 74.0, 20 Mi 102.2 / 91.9, 26 Mi 133.7 / 119.2); a call does not know which it is, and below the
-// lines the loss is the larger.  A tensor of the
-// operator comes with others, and its launch ends when its stores have left the L2: 144 K elements 2.33 / 2.41 us, 576 K 4.50 / 3.68,
-// 2.25 Mi 13.0 / 11.5; the tensors of a module of 5.3 M elements one after the other 67 / 68, of 11 M 166 / 139.
+// Steps over a list that stays in the memory-side cache from one step to the next (256 MiB) want it there; others, because forward and
+// backward went over more than the cache holds, do not, and a call does not know which it is.  Without / with the hint, the same list
+// again and again: host-decided 8 Mi elements 28.8 / 36.7 us, 16 Mi 65.7 / 69.7, 18 Mi 73.4 / 78.7, 20 Mi 90.8 / 88.1, 22 Mi 98.0 / 97.0, 24 Mi 108.2 /
+// 105.9, 26 Mi 118.3 / 115.4; device-decided 16 Mi 72.9 / 77.0, 18 Mi 79.8 / 85.9, 20 Mi 99.5 / 94.8, 22 Mi 104.4 / 103.9, 24 Mi 114.4 / 113.2, 26 Mi
+// 123.8 / 122.3; device-decided tensors with numbers of their own 17.5 Mi 80.1 / 87.0, 20 Mi 101.2 / 98.5, 23 Mi 115.7 / 111.6, 26 Mi 129.2 / 122.9 (runs
+// of one side differ by 2 to 8 us here, by 0.4 below).  Three lists in turn: host-decided 4 Mi 16.1 / 20.2, 8 Mi 38.9 / 37.3, 16 Mi 78.4 / 71.6, 24 Mi 112.8 / 106.8;
+// device-decided 8 Mi 40.7 / 39.9, 16 Mi 85.3 / 77.8, 20 Mi 104.9 / 95.8, 26 Mi 134.6 / 122.5; tensors 17.5 Mi 94.5 / 86.9, 23 Mi 125.1 / 111.1.
+// Up to some 18 Mi elements a list that is in the cache loses 5 to 27 % by the hint, and plain accesses stay.  From 20 to 24 Mi on the hint loses in neither state, and from there to the lines, 28 Mi for every kind of step, plain
+// accesses give up 1 to 5 % with the list in the cache and 5 to 11 % with it elsewhere: the lines are held by the tests of the routes, where
+// a list of 27 Mi does not stream.
+//
+// A tensor of the operator comes with others, and its launch ends when its stores have left the L2.  Tensors of one length one after the other,
+// without / with the hint, 600 MiB of them: 96 Ki elements 2.40 / 2.27 us, 128 Ki 2.56 / 2.35, 144 Ki 2.68 / 2.40, 192 Ki 2.93 / 2.57, 256 Ki 3.19 / 2.74, 576 Ki
+// 4.77 / 3.55; eight of them, in the caches: the same within 0.03 up to 224 Ki, 256 Ki 2.34 / 2.27, 576 Ki 3.70 / 3.34; one of 2.25 Mi 13.0 / 11.5.  The loop of a program
+// takes the host 3.7 us a call, which hides all of that below the line (256 Ki): modules of hidden size 384 and 448 with a line of 256 / 128 Ki
+// 816 / 823 and 426 / 427 us (runs differ by 16 to 40); in a graph 516 / 465 and 320 / 283.
 //
 // The probe in front of an update reads what the update reads next: of a list it takes as much through the caches as the
 // memory-side one holds, where a streaming update finds it, and the rest past them.  Whole steps, everything past the caches / the first 112 Mi
 // elements through them: 31 Mi 148.5 / 142.9 us, 48 Mi 228 / 224, 80 Mi 373 / 358, 104 Mi 490 / 480, 136 Mi 642 / 627, 3 x 72 Mi 1018 / 1008, 8 x 64 Mi
 // 2419 / 2402; 199 tensors of BERT-base with a rate per layer 502.6 / 479.  (96 Mi and 128 Mi: the same within 0.3 %.)  A skipped step reads no
-// gradients again and pays for the slower probe: 48 Mi 62.6 / 64.3, 8 x 64 Mi 612 / 614; of lists beyond 256 Mi, where the gain is small, it is
-// 64 Mi, 2419 / 2409 and 612 / 612.5.
+// gradients again and pays for the slower probe: 48 Mi 62.6 / 64.3.  Of lists beyond 256 Mi it is 64 Mi.  Everything past the caches / 64 / 112 Mi: 8 x 64 Mi
+// 2420.7 / 2411.5 / 2404.8 us, 5 x 56 Mi 1335.8 / 1328.5 / 1320.4, 12 x 64 Mi 3666.6 / 3661.1 / 3657.2; skipped 615.6 / 614.3 / 615.0, 339.5 / 341.3 / 341.3,
+// 922.2 / 918.6 / 918.4, where runs differ by 3 to 10: 112 Mi there as well would give a clean step 0.1 to 0.6 % more at no cost that shows.
 //
 // A store that fills a 64-byte line in part only must not leave at once: lists whose phases differ by 16 or 32 bytes ran
 // 5 to 6 % slower with the hint, by 64 6 % faster.
@@ -270,11 +277,12 @@ bool streams(const ChunkList& a, bool gated)
 // Dynamic LDS of a launch of the update, one tile a workgroup: the request that caps the resident workgroups per CU, except where
 // all of the launch's workgroups fit the GPU at once (256 CUs with 32 waves each).  The cap keeps the window of lines in flight narrow
 // while workgroups follow one another; a launch that has no second round only waits for its first one to end.  Capped / not, device
-// time in a graph, host-decided step over one chunk of 768 Ki / 1 Mi / 1.5 Mi / 2 Mi elements in the caches 4.3 / 3.9, 5.2 / 4.6, 6.4 / 5.6, 7.6 / 6.4 us, in
-// memory 6.6 / 6.0, 7.9 / 7.8, 10.6 / 10.7, 13.4 / 13.8; device-decided, probe included, in the caches 7.1 / 6.5, 8.0 / 7.1, 9.5 / 8.2,
-// 11.4 / 9.7, in memory 8.9 / 8.3, 10.3 / 9.7, 13.0 / 12.8, 15.9 / 16.1.  Tensors with numbers of their own 1.07 M elements 6.4 / 5.8, 2.1 M 10.2 /
+// time in a graph, host-decided step over one chunk of 768 Ki / 1 Mi / 1.25 Mi / 1.5 Mi / 2 Mi elements in the caches 4.3 / 3.9, 5.6 / 5.1, 6.3 / 5.6, 6.8 / 6.0,
+// 8.0 / 6.9 us, in memory 6.6 / 6.0, 8.0 / 7.9, 9.5 / 9.4, 10.8 / 10.8, 13.5 / 13.8; device-decided, probe included, in the caches 7.1 / 6.5, 8.6 / 7.9, 9.4 / 8.4,
+// 10.1 / 8.9, 11.9 / 10.3, in memory 8.9 / 8.3, 10.3 / 9.8, 11.9 / 11.6, 13.3 / 13.1, 16.1 / 16.4.  Tensors with numbers of their own 1.07 M elements 6.4 / 5.8, 2.1 M 10.2 /
 // 8.5; one tensor of the operator 768 Ki 5.35 / 4.6, 1 Mi 6.35 / 6.15, 2 Mi 10.7 / 10.65, beyond the line 2.5 Mi 12.9 / 13.05.  Beyond it
-// the cap pays: one chunk of 3 Mi in memory 18.6 / 19.3, 16 Mi 53.3 / 54.8, 26 Mi 116 / 130.
+// the cap pays: one chunk of 3 Mi in memory 18.6 / 19.3, 16 Mi 53.3 / 54.8, 26 Mi 116 / 130.  The line is that of lists in the caches: from 1.5 Mi elements
+// (host-decided; device-decided 1.75 Mi) up to it a list in memory loses up to 2.5 %, where one in the caches gains 11 to 13 %.
 constexpr size_t kResidentTiles = PS_RESIDENT_TILES;
 unsigned capped_lds(dim3 grid, unsigned request) { return (size_t)grid.x * grid.y <= kResidentTiles ? 0 : request; }
 template <bool NT>
