@@ -518,6 +518,14 @@ int ps_adam_step_tensors_dynamic(int optimizer_id, int bias_correction, const ps
                                  int n_tensors, ps_step_state* d_state, ps_scale_record* d_log, int64_t log_capacity, int64_t operator_calls,
                                  void* d_workspace, size_t workspace_bytes, void* d_scratch, size_t scratch_bytes, ps_stream_t stream);
 
+/*
+ * 1 if ps_adam_step_tensors_dynamic, given scratch memory, takes such lists in the probe's launch and those of the update, 0 if it makes its
+ * calls one after the other (the distinct calls and PS_TENSOR_GRAD_F32, which are left out of account here, may still have it do so).
+ * For steps whose tensors all share one set of numbers, which ps_adam_step_tensors does without forming constants first.
+ */
+int ps_tensors_at_once(const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel, const ps_chunk* tensors,
+                       const size_t* numels, int n_tensors);
+
 /* Copy *d_state to host memory and wait for it: the only synchronising call. */
 int ps_state_read(const ps_step_state* d_state, ps_step_state* host_out, ps_stream_t stream);
 

@@ -158,6 +158,7 @@ SIGNATURES = {
     "ps_adam_step_chunks_dynamic": (_i, [_i, _d, _d, _d, _i, _vp, _i, _sz, _vp, _vp, _i, _vp, _vp, _i64, _i64, _vp]),
     "ps_adam_step_chunks_dynamic_scratch": (_i, [_i, _d, _d, _d, _i, _vp, _i, _sz, _vp, _vp, _i, _vp, _vp, _i64, _i64, _vp, _sz, _vp]),
     "ps_adam_step_tensors_dynamic": (_i, [_i, _i, _vp, _i, _sz, _vp, _vp, _vp, _vp, _i, _vp, _vp, _i64, _i64, _vp, _sz, _vp, _sz, _vp]),
+    "ps_tensors_at_once": (_i, [_vp, _i, _sz, _vp, _vp, _vp, _i]),
     "ps_state_read": (_i, [_vp, ctypes.POINTER(ps_step_state), _vp]),
 }
 

@@ -1557,16 +1557,13 @@ struct WholeStep {
     int64_t log_capacity, operator_calls;
 };
 
-// Whether it is done in one launch and those of the update, the first of which replaces the state.
-bool opens_with_plan(const WholeStep& w, int n_classes, const std::vector<int>& class_keys, const ps_chunk* tensors, const size_t* numels, int n_tensors)
+// Whether such lists can be done in one launch and those of the update.
+bool lists_open_with_plan(const ChunkList& a, const ps_chunk* tensors, const size_t* numels, int n_tensors)
 {
-    const ChunkList& a = w.probed;
-    if (!w.scratch || n_classes > kOpenClasses || a.n_chunks < 1 || a.n_chunks > kBatch) return false;
+    if (a.n_chunks < 1 || a.n_chunks > kBatch) return false;
     size_t longest = 0, elements = 0;
     for (int i = 0; i < a.n_chunks; ++i) longest = std::max(longest, a.numel_of(i));
     if (longest == 0 || longest > 0xFFFFFFFFu) return false;
-    for (int key : class_keys)
-        if (key_grad_f32(key)) return false;
     std::vector<TensorItem> items;
     for (int i = 0; i < n_tensors; ++i) {
         if (numels[i] == 0) continue;
@@ -1575,6 +1572,15 @@ bool opens_with_plan(const WholeStep& w, int n_classes, const std::vector<int>& 
     }
     ps_chunk lists;
     return elements <= kMaxNearElements && near_lists(items, tensors, &lists);  // (no item: false)
+}
+
+// Whether it is done in one launch and those of the update, the first of which replaces the state.
+bool opens_with_plan(const WholeStep& w, int n_classes, const std::vector<int>& class_keys, const ps_chunk* tensors, const size_t* numels, int n_tensors)
+{
+    if (!w.scratch || n_classes > kOpenClasses) return false;
+    for (int key : class_keys)
+        if (key_grad_f32(key)) return false;
+    return lists_open_with_plan(w.probed, tensors, numels, n_tensors);
 }
 
 int step_tensors_each(int optimizer_id, int bias_correction, const ps_chunk* tensors,
@@ -1817,6 +1823,19 @@ int ps_adam_step_tensors_dynamic(int optimizer_id, int bias_correction, const ps
     if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kScanTile, true)) return rc;
     const WholeStep whole{a, static_cast<StepScratch*>(d_scratch), d_log, log_capacity, operator_calls};
     return step_tensors_each(optimizer_id, bias_correction, tensors, numels, each, n_tensors, -1.0, d_state, d_workspace, workspace_bytes, &whole, stream);
+}
+
+int ps_tensors_at_once(const ps_chunk* chunks, int n_chunks, size_t chunk_numel, const size_t* used_numel, const ps_chunk* tensors,
+                       const size_t* numels, int n_tensors)
+{
+    ChunkList a;
+    if (int rc = make_chunk_list(a, chunks, n_chunks, chunk_numel, used_numel, kScanTile, true)) return rc;
+    if (int rc = check_tensor_list(tensors, numels, n_tensors)) return rc;
+    try {
+        return lists_open_with_plan(a, tensors, numels, n_tensors) ? 1 : 0;
+    } catch (const std::exception&) {  // nothing may throw across the boundary
+        return fail(PS_ERR_BAD_ARG, "no host memory for a list of %d tensors", n_tensors);
+    }
 }
 
 int ps_restore_fp16_chunks(const ps_chunk* chunks, int n_chunks, size_t chunk_numel,

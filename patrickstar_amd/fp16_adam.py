@@ -244,6 +244,7 @@ class FP16Adam(torch.optim.Optimizer):
             _lib.check(self._lib.ps_adam_set_arithmetic(self.opt_id, _lib.PS_ARITH_TORCH), "ps_adam_set_arithmetic")
         self._tables = None
         self._tensor_table = None  # (ps_chunk rows, numels, count) when the step has to go tensor by tensor
+        self._at_once = None  # _tensors_at_once of those tables
         self._calls = None  # ps_call_pattern of one step (None: no operator call at all)
         self._stages = None  # the entry-point calls of a step that cannot be made as one (see _plan_stages)
         self._trainable_seen = None  # requires_grad of every parameter when the plan was made
@@ -331,7 +332,7 @@ class FP16Adam(torch.optim.Optimizer):
                         cl[pos.fp16].payload.data_ptr(),
                     ]
                 )
-        self._tensor_table = None
+        self._tensor_table = self._at_once = None
         if partly_frozen and not host_positions:
             self._tensor_table = self._tensor_rows(trainable)
         # The operator calls of one step: with the operator's arithmetic every trainable tensor is one, with the torch
@@ -745,6 +746,15 @@ class FP16Adam(torch.optim.Optimizer):
             plan["tensors"] = {"kind": "each", "trainable": trainable, "entries": entries, "table": None}
         return plan["tensors"]
 
+    def _tensors_at_once(self):
+        """Whether a uniform step over some of the tensors gains by being one call: else that is the three calls, with a kernel more
+        that forms every tensor's constants (226 chunks, 2.8 M elements 73.5 us as three calls, 89.7 as one; 90 chunks, 17.4 M 96.8
+        and 103.1; 314 M in 6 chunks 1468 and 1484; within the lines, 31.8 M, 146.3 and 143.6)."""
+        if self._at_once is None:
+            table, n_dev, _ = self._tables
+            self._at_once = bool(n_dev) and self._lib.ps_tensors_at_once(table, n_dev, self.client.default_chunk_size, self._used, *self._tensor_table) == 1
+        return self._at_once
+
     def _step_each_at_once(self, plan, stream):
         """Probe, device-decided step and scale update as one call, where all chunks lie in HBM and PyTorch manages no tensor
         itself.  False: nothing was done."""
@@ -908,7 +918,10 @@ class FP16Adam(torch.optim.Optimizer):
                     _lib.check(rc, "ps_adam_step_chunks_dynamic")
                     self._steps_dirty = True
                     return loss
-                if scan and self._stages is None and self._tensor_table is not None and self._step_each_at_once(self._tensors_of(plan), stream):
+                if (
+                    scan and self._stages is None and self._tensor_table is not None and self._tensors_at_once()
+                    and self._step_each_at_once(self._tensors_of(plan), stream)
+                ):
                     self._steps_dirty = True
                     return loss
                 if scan:

@@ -51,6 +51,12 @@ def main():
         if entry == "each":
             each = (_lib.ps_tensor_call * n)(*[(*RATES, 0 if gated else 1, -1, int(f)) for f in grad_f32])
             return lib.ps_adam_step_tensors_each(1, 1, table, sizes, each, n, 8.0, state, WORK, 64 * n, None)
+        if entry == "dynamic":  # a whole device-decided step over tensors, which are probed as chunks; one set of numbers
+            each = (_lib.ps_tensor_call * n)(*[(*RATES, 0, -1, 0)] * n)
+            rc = lib.ps_adam_step_tensors_dynamic(1, 1, table, n, max(numels), sizes, table, sizes, each, n, state, None, 0, n, WORK, 64 * n, SCRATCH, 448, None)
+            opened = count.value > 0 and b"open_planned" in launches[0].name
+            assert lib.ps_tensors_at_once(table, n, max(numels), sizes, table, sizes, n) == opened
+            return rc
         if entry == "operator":
             p, m, v, h = rows[0]
             return lib.ps_adam_update(1, 1, *RATES, 1, p, h, 1, m, v, numels[0], 8.0, None, None)
