@@ -697,7 +697,7 @@ class FP16Adam(torch.optim.Optimizer):
             if self._each_static is None:
                 # addresses, lengths, where the state lives and the workspace stay as they are while the same
                 # parameters are trainable (a learning-rate schedule makes a new plan before every step)
-                rows, numels, n = self._tensor_rows(trainable)
+                rows, numels, n = plan.get("rows") or self._tensor_rows(trainable)
                 on_host = {pos.fp16 for pos in self.client.positions() if pos.on_host}
                 index = self.client.chunk_tensor_index
                 host = [not self._torch_managed(p) and index.get_tensor_info(p.ps_attr.data_id()).chunk_id in on_host
@@ -743,7 +743,8 @@ class FP16Adam(torch.optim.Optimizer):
             again = plan.get("numbers")  # where the numbers are already
             trainable = self._trainable() if again is None else again.trainable
             entries = [(*plan["hyper"], self._offsets.get(p, 0)) for p in trainable] if again is None else None
-            plan["tensors"] = {"kind": "each", "trainable": trainable, "entries": entries, "table": None}
+            # (the rows of _build_tables are those of the same parameters, since PyTorch manages none of a uniform plan's)
+            plan["tensors"] = {"kind": "each", "trainable": trainable, "entries": entries, "table": None, "rows": self._tensor_table}
         return plan["tensors"]
 
     def _tensors_at_once(self):

@@ -24,9 +24,8 @@ class _Calls(_StepCalls):
         return 64 * n
 
 
-@pytest.mark.parametrize("layers,chunk_numel,calls", [(64, 64, ["ps_adam_step_tensors_dynamic"]), (65, 64, CALLS), (130, 64, CALLS), (130, 1000, ["ps_adam_step_tensors_dynamic"])])
-def test_more_chunks_than_one_launch_probes_take_the_three_calls(monkeypatch, layers, chunk_numel, calls):
-    """Of 65 chunks on the one call forms constants in a launch of its own: it is a launch longer than the others."""
+def _step_over_some(monkeypatch, layers, chunk_numel):
+    """(optimizer, library, parameters), one parameter frozen"""
     client = ps.PatrickStarClient(0, chunk_numel, device="cpu")
     model = torch.nn.Sequential(*[torch.nn.Linear(8, 7) for _ in range(layers)])  # 63 elements
     client.register_model(model)
@@ -41,6 +40,13 @@ def test_more_chunks_than_one_launch_probes_take_the_three_calls(monkeypatch, la
     size = ctypes.sizeof(_lib.ps_step_state)
     both = torch.zeros(size + _lib.PS_STEP_SCRATCH_BYTES, dtype=torch.uint8)
     scaler._state, scaler._scratch = both[:size], both[size:]
+    return optimizer, library, params
+
+
+@pytest.mark.parametrize("layers,chunk_numel,calls", [(64, 64, ["ps_adam_step_tensors_dynamic"]), (65, 64, CALLS), (130, 64, CALLS), (130, 1000, ["ps_adam_step_tensors_dynamic"])])
+def test_more_chunks_than_one_launch_probes_take_the_three_calls(monkeypatch, layers, chunk_numel, calls):
+    """Of 65 chunks on the one call forms constants in a launch of its own: it is a launch longer than the others."""
+    optimizer, library, params = _step_over_some(monkeypatch, layers, chunk_numel)
 
     def made():
         library.names.clear()
@@ -65,3 +71,18 @@ def test_the_library_says_which_lists_open_with_the_plan(sizes, moved, opens):
         rows[1][2] += 1 << 38
     found = launches("dynamic", rows, sizes, True)  # (which compares the answer with what was launched)
     assert (found[0].name == "open_planned_kernel") == opens
+
+
+def test_the_addresses_of_the_tensors_are_looked_up_once(monkeypatch):
+    """Four views of every tensor: most of the host's part of the first step over some of them."""
+    optimizer, library, params = _step_over_some(monkeypatch, 8, 1000)
+    looked, rows = [], optimizer._tensor_rows
+    monkeypatch.setattr(optimizer, "_tensor_rows", lambda trainable, *slot: looked.append(list(trainable)) or rows(trainable, *slot))
+    for k in range(3):
+        for p in params:
+            optimizer.state[p]["lr"] = 0.5**k
+        optimizer.step()
+    assert library.names.count("ps_adam_step_tensors_dynamic") == 3 and looked == [params[:1] + params[2:]]
+    optimizer.invalidate_tables()
+    optimizer.step()
+    assert len(looked) == 2 and library.names.count("ps_adam_step_tensors_dynamic") == 4
