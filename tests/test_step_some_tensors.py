@@ -86,3 +86,18 @@ def test_the_addresses_of_the_tensors_are_looked_up_once(monkeypatch):
     optimizer.invalidate_tables()
     optimizer.step()
     assert len(looked) == 2 and library.names.count("ps_adam_step_tensors_dynamic") == 4
+
+
+@pytest.mark.parametrize("arithmetic", ["operator", "torch"])
+def test_the_records_of_one_set_of_numbers_are_those_of_every_tensor(monkeypatch, arithmetic):
+    optimizer, _, params = _step_over_some(monkeypatch, 8, 1000)
+    optimizer.arithmetic = arithmetic
+    for p in params:
+        for key, value in dict(lr=0.25, betas=[0, 0.5], eps=1, weight_decay=3e-2).items():
+            optimizer.state[p][key] = value
+    optimizer.step()
+    plan = optimizer._tensors_of(optimizer._plan)
+    general = {key: value for key, value in plan.items() if key != "rows"}
+    a, b = [optimizer._each_table(dict(one, table=None)) for one in (plan, general)]
+    assert bytes(a[3]) == bytes(b[3]) and len(bytes(a[3])) == 56 * 15
+    assert a[:3] == b[:3] and a[4:] == b[4:] and a[5] == (15 if arithmetic == "operator" else 0)
