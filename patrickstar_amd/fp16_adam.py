@@ -717,7 +717,7 @@ class FP16Adam(torch.optim.Optimizer):
                 lr, (beta1, beta2), eps, weight_decay, _ = entries[0]
                 arithmetic = _lib.PS_ARITH_OPERATOR if self.arithmetic == "operator" else _lib.PS_ARITH_TORCH
                 same = bytes(_lib.ps_tensor_call(lr, beta1, beta2, eps, weight_decay, 0, arithmetic, 0))
-                each = (_lib.ps_tensor_call * n).from_buffer_copy(same * n)  # (199 records field by field: 0.15 ms)
+                each = (_lib.ps_tensor_call * n).from_buffer_copy(same * n)  # (199 records field by field: 0.1 ms)
                 offsets = [e[4] for e in entries]
                 for i, d in enumerate(offsets):
                     if d:
